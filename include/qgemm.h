@@ -165,7 +165,9 @@ int qgemm_tile_map(uint32_t wg, uint32_t tiles_m, uint32_t tiles_n, uint32_t gro
 
 /* Tuning / diagnostics (no reference counterpart: the reference picks its tile at compile time,
  * src/include/gemm_config.h:30-36).
- * qgemm_set_option(key, value): "force_split" (K slices, 0 = heuristic), "group_m", "kmajor", "stagger", "k_rot",
+ * qgemm_set_option(key, value): "force_split" (K slices, 0 = heuristic), "group_m", "kmajor", "any_shape" (operands whose K
+ *   bytes are no multiple of 16, or whose rows or pointers are unaligned: 0 the scalar kernel, 1 packed into the workspace
+ *   for the matrix cores where that is faster, 2 packed wherever possible), "stagger", "k_rot",
  *   "stagger_groups", "as_groups", "row_split" (0: one launch always; 1: the rows "a+b" or columns "a|b" of a partly
  *   empty last round of 256 x 256 tiles as a second launch where the estimate gains; 2 / 3: rows / columns wherever
  *   possible), "small_tiles" (0: 17 .. 256 rows against few columns keep a tall tile with a K split instead of several
@@ -189,6 +191,7 @@ int qgemm_last_config(char *buf, size_t buflen);
 
 /* Which kernel configuration the library would run for a problem with dense, 16-byte aligned operands: the name
  * qgemm_last_config would report after the call ("256x256_w2x2_solo", "128x128_w2x2_dma_tn_splitk2", ...;
+ * "strided_any_shape" for both forms of what option "any_shape" chooses between;
  * "transpose+<name>" when operands stored K-major go through the transpose kernels first).  Nothing is launched
  * and no device is needed (256 CUs are assumed before qgemm_init).  No reference counterpart: the reference picks
  * its tile at compile time (src/include/gemm_config.h:30-36).

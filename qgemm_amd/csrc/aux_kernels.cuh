@@ -36,7 +36,8 @@ __device__ inline void store_out(void *C, size_t idx, float v, int out_dtype) {
 
 // ---------------------------------------------------------------------------
 // Any-shape, any-stride GEMM: one thread per C element.  Carries the shapes the
-// MFMA kernel does not take (K not a multiple of 128 bytes).  Same arithmetic
+// MFMA kernels do not take and pack_kernel does not bring to them (very small ones,
+// fp8 with fp32 output, calls that have no workspace to pack into).  Same arithmetic
 // contract: int32 accumulation for int8, fp32 otherwise; block scales folded in
 // per `bk` K elements as (P * as) * bs  (hip_mix_gemm_kernel.cpp:231-244).
 // ---------------------------------------------------------------------------
@@ -139,6 +140,9 @@ __global__ void __launch_bounds__(256) transpose_kernel(const T *__restrict__ in
     }
 }
 
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));       // 16 bytes at any address
+typedef unsigned u32_any __attribute__((aligned(1)));
+
 // ---------------------------------------------------------------------------
 // Byte transpose for shapes with M % 16 == 0, N % 4 == 0 and 16-byte aligned rows (the fp8 / int8
 // operands of the reference layout).  128 x 128 tile, 256 threads.  A thread loads 4 x 4 bytes (four
@@ -146,25 +150,39 @@ __global__ void __launch_bounds__(256) transpose_kernel(const T *__restrict__ in
 // registers with byte permutes, and writes the four resulting dwords (4 consecutive m of one n)
 // into the LDS tile [n][m]; the tile leaves as 16-byte pieces of output rows, 128 bytes per row.
 // ---------------------------------------------------------------------------
-// One 128 x 128 tile of the byte transpose (tile_m, tile_n in tiles)
-__device__ inline void transpose_bytes_tile(const uint8_t *__restrict__ in, uint8_t *__restrict__ out, uint32_t M,
-                                            uint32_t N, uint32_t tile_m, uint32_t tile_n) {
+// One 128 x 128 tile of the byte transpose (tile_m, tile_n in tiles).  ALIGNED: M a multiple of 16, N of 4, aligned rows,
+// Mout == M.  Otherwise any M, N, ld, pitch and pointers: pieces that stick out go byte by byte, and the columns
+// M .. Mout - 1 of the output are filled with zeros.
+template <bool ALIGNED>
+__device__ inline void transpose_bytes_tile(const uint8_t *__restrict__ in, size_t ld, uint8_t *__restrict__ out, size_t pitch,
+                                            uint32_t M, uint32_t Mout, uint32_t N, uint32_t tile_m, uint32_t tile_n) {
 #if defined(__HIP_DEVICE_COMPILE__)
+    typedef typename std::conditional<ALIGNED, v4i, v4i_any>::type vec_t;
+    typedef typename std::conditional<ALIGNED, uint32_t, u32_any>::type word_t;
     constexpr int T = 128, PITCH = T + 16;        // bytes per LDS row
     __shared__ __attribute__((aligned(16))) uint8_t tile[T * PITCH];
     const uint32_t m0 = tile_m * T, n0 = tile_n * T;
     const int cg = threadIdx.x & 31, rg = threadIdx.x >> 5;      // 32 column groups of 4 bytes x 8 row groups of 16
     const uint32_t n = n0 + cg * 4;
+    auto load4 = [&](const uint8_t *src, bool row_in) -> uint32_t {        // four bytes of one row, zeros outside
+        if constexpr (ALIGNED) return *(const word_t *)src;
+        if (!row_in) return 0;
+        if (n + 4 <= N) return *(const word_t *)src;
+        uint32_t w = 0;
+        for (int e = 0; e < 3; ++e)
+            if (n + e < N) w |= (uint32_t)src[e] << (8 * e);
+        return w;
+    };
 #pragma unroll
     for (int ch = 0; ch < 4; ++ch) {
         const uint32_t m = m0 + rg * 16 + ch * 4;
         uint32_t a = 0, b = 0, c = 0, d = 0;
-        if (n < N && m < M) {                     // M % 4 == 0: the four rows are all inside or all outside
-            const uint8_t *src = in + (size_t)m * N + n;
-            a = *(const uint32_t *)src;
-            b = *(const uint32_t *)(src + N);
-            c = *(const uint32_t *)(src + 2 * (size_t)N);
-            d = *(const uint32_t *)(src + 3 * (size_t)N);
+        if (n < N && m < M) {                     // (aligned: M % 4 == 0, the four rows are all inside or all outside)
+            const uint8_t *src = in + (size_t)m * ld + n;
+            a = load4(src, true);
+            b = load4(src + ld, m + 1 < M);
+            c = load4(src + 2 * ld, m + 2 < M);
+            d = load4(src + 3 * ld, m + 3 < M);
         }
         // v_perm_b32: selector byte k picks byte k of the result out of {src1 bytes 0-3, src0 bytes 4-7}
         const uint32_t ab_lo = __builtin_amdgcn_perm(b, a, 0x05010400), ab_hi = __builtin_amdgcn_perm(b, a, 0x07030602);
@@ -183,14 +201,22 @@ __device__ inline void transpose_bytes_tile(const uint8_t *__restrict__ in, uint
     for (int ps = 0; ps < 4; ++ps) {
         const int r = row + ps * 32;
         const uint32_t on = n0 + r, om = m0 + piece * 16;
-        if (on < N && om < M) *(v4i *)(out + (size_t)on * M + om) = *(const v4i *)(tile + r * PITCH + piece * 16);
+        if (on >= N || om >= Mout) continue;
+        const uint8_t *src = tile + r * PITCH + piece * 16;
+        uint8_t *dst = out + (size_t)on * pitch + om;
+        if (ALIGNED || om + 16 <= Mout) {
+            *(vec_t *)dst = *(const v4i *)src;
+        } else {
+            for (uint32_t e = 0; om + e < Mout; ++e) dst[e] = src[e];
+        }
     }
 #endif
 }
 
+template <bool ALIGNED>
 __global__ void __launch_bounds__(256) transpose_bytes_kernel(const uint8_t *__restrict__ in, uint8_t *__restrict__ out,
                                                               uint32_t M, uint32_t N) {
-    transpose_bytes_tile(in, out, M, N, blockIdx.y, blockIdx.x);
+    transpose_bytes_tile<ALIGNED>(in, N, out, M, M, M, N, blockIdx.y, blockIdx.x);
 }
 
 // Two byte transposes in one launch (both operands of the reference fp8 layout: the second launch costs more
@@ -202,11 +228,12 @@ struct Transpose2Args {
 };
 __global__ void __launch_bounds__(256) transpose_bytes2_kernel(const Transpose2Args a) {
     const uint32_t which = blockIdx.x >= a.tiles0 ? 1u : 0u, t = blockIdx.x - (which ? a.tiles0 : 0u);
-    transpose_bytes_tile(a.in[which], a.out[which], a.M[which], a.N[which], t / a.tiles_n[which], t % a.tiles_n[which]);
+    transpose_bytes_tile<true>(a.in[which], a.N[which], a.out[which], a.M[which], a.M[which], a.M[which], a.N[which],
+                               t / a.tiles_n[which], t % a.tiles_n[which]);
 }
 
 // ---------------------------------------------------------------------------
-// 2-byte transpose for shapes with M % 8 == 0, N % 8 == 0 and 16-byte aligned rows (what
+// 2-byte transpose.  Written for shapes with M % 8 == 0, N % 8 == 0 and 16-byte aligned rows (what
 // matrix_transpose<bf16 / fp16> of the reference is called with, src/transpose/transpose.cu:60-74).
 // No LDS: a lane owns an 8 x 8 block.  It loads eight 16-byte row pieces, interleaves the 16-bit halves
 // of vertically adjacent dwords (one v_perm each: 32 per block), and the rest of the transposition is
@@ -215,17 +242,35 @@ __global__ void __launch_bounds__(256) transpose_bytes2_kernel(const Transpose2A
 // blocks, so every store instruction writes 128-byte pieces of 8 output rows.  A wave covers 64 x 64
 // elements, a workgroup of four waves 64 rows x 256 columns.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) transpose_u16_kernel(const uint16_t *__restrict__ in, uint16_t *__restrict__ out,
-                                                            uint32_t M, uint32_t N) {
+// ALIGNED: M and N multiples of 8, 16-byte aligned rows, Mout == M.  Otherwise any M, N, ld, pitch and element-aligned
+// pointers (through LDS one element per lane before: 1999 x 3001 11.4 -> 9.6 us): pieces that stick out go element by
+// element, the columns M .. Mout - 1 of the output are filled with zeros.
+template <bool ALIGNED>
+__device__ inline void transpose_u16_tile(const uint16_t *__restrict__ in, size_t ld, uint16_t *__restrict__ out, size_t pitch,
+                                          uint32_t M, uint32_t Mout, uint32_t N, uint32_t tile_m, uint32_t tile_n) {
 #if defined(__HIP_DEVICE_COMPILE__)
+    typedef typename std::conditional<ALIGNED, v4i, v4i_any>::type vec_t;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t m = blockIdx.y * 64 + (lane >> 3) * 8;                   // first of this lane's 8 rows
-    const uint32_t n = blockIdx.x * 256 + wave * 64 + (lane & 7) * 8;       // first of its 8 columns
-    if (m >= M || n >= N) return;                                           // blocks are wholly in or out
+    const uint32_t m = tile_m * 64 + (lane >> 3) * 8;                       // first of this lane's 8 rows
+    const uint32_t n = tile_n * 256 + wave * 64 + (lane & 7) * 8;           // first of its 8 columns
+    if (m >= Mout || n >= N) return;                                        // (aligned: blocks are wholly in or out)
+    const bool cols = ALIGNED || n + 8 <= N, rows = ALIGNED || m + 8 <= Mout;
     v4i row[8];
-    const uint16_t *src = in + (size_t)m * N + n;
+    const uint16_t *src = in + (size_t)m * ld + n;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) row[j] = *(const v4i *)(src + (size_t)j * N);
+    for (int j = 0; j < 8; ++j) {
+        if (!ALIGNED && m + j >= M) {
+            row[j] = v4i{0, 0, 0, 0};
+        } else if (cols) {
+            row[j] = *(const vec_t *)(src + (size_t)j * ld);
+        } else {
+            uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 7; ++e)
+                if (n + e < N) w[e >> 1] |= (uint32_t)src[(size_t)j * ld + e] << (16 * (e & 1));
+            row[j] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        }
+    }
     // pair[i][k] = columns 2k (low perm) and 2k+1 (high perm) of rows 2i, 2i+1
     uint32_t lo[4][4], hi[4][4];
 #pragma unroll
@@ -236,15 +281,95 @@ __global__ void __launch_bounds__(256) transpose_u16_kernel(const uint16_t *__re
             lo[i][k] = __builtin_amdgcn_perm(b, a, 0x05040100);     // (a.lo16, b.lo16)
             hi[i][k] = __builtin_amdgcn_perm(b, a, 0x07060302);     // (a.hi16, b.hi16)
         }
-    uint16_t *dst = out + (size_t)n * M + m;
+    uint16_t *dst = out + (size_t)n * pitch + m;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const v4i even = {(int)lo[0][k], (int)lo[1][k], (int)lo[2][k], (int)lo[3][k]};
-        const v4i odd = {(int)hi[0][k], (int)hi[1][k], (int)hi[2][k], (int)hi[3][k]};
-        *(v4i *)(dst + (size_t)(2 * k) * M) = even;
-        *(v4i *)(dst + (size_t)(2 * k + 1) * M) = odd;
+    for (int k = 0; k < 8; ++k) {
+        const v4i v = (k & 1) ? v4i{(int)hi[0][k >> 1], (int)hi[1][k >> 1], (int)hi[2][k >> 1], (int)hi[3][k >> 1]}
+                              : v4i{(int)lo[0][k >> 1], (int)lo[1][k >> 1], (int)lo[2][k >> 1], (int)lo[3][k >> 1]};
+        if (!cols && n + k >= N) break;
+        if (rows) {
+            *(vec_t *)(dst + (size_t)k * pitch) = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 7; ++e)
+                if (m + e < Mout) dst[(size_t)k * pitch + e] = (uint16_t)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
+        }
     }
 #endif
+}
+
+template <bool ALIGNED>
+__global__ void __launch_bounds__(256) transpose_u16_kernel(const uint16_t *__restrict__ in, uint16_t *__restrict__ out,
+                                                            uint32_t M, uint32_t N) {
+    transpose_u16_tile<ALIGNED>(in, N, out, M, M, M, N, blockIdx.y, blockIdx.x);
+}
+
+// ---------------------------------------------------------------------------
+// Operands that the MFMA kernels cannot read as they stand (K bytes not a multiple of 16, rows or pointers that are not
+// 16-byte aligned, B stored K x N with such rows): one launch brings one or both of them to rows of `pitch` bytes, K
+// contiguous, zeros behind the last element up to the pitch (a multiple of 128), so that the whole of K is whole K steps.
+// Bound by memory: every element is read and written once.  Loads are 16 bytes a lane at whatever address the row has
+// (the vector memory path takes any byte address; only the pieces that reach past a row's end go element by element).
+// ---------------------------------------------------------------------------
+struct PackOperand {
+    const char *src;
+    char *dst;
+    uint64_t ld;          // bytes between rows of the source (rows of the operand, or rows of k when k_major)
+    uint32_t rows, k;     // of the operand, elements
+    uint32_t pitch;       // bytes between rows of dst, a multiple of 128
+    uint32_t k_major;     // the source is K x rows
+    uint32_t blocks, tiles_k;      // workgroups of this operand; k_major: tiles along k (the slower index is the tile of rows)
+};
+struct PackArgs {
+    PackOperand op[2];
+};
+
+// rows of the operand as they are: 16 bytes of dst per lane and turn, four turns per workgroup
+template <int ES>
+__device__ inline void pack_rows(const PackOperand &o, uint32_t block) {
+    const uint32_t per_row = o.pitch / 16, kbytes = o.k * ES;
+    const uint32_t total = o.rows * per_row, first = block * 1024 + threadIdx.x;       // (the host keeps these below 2^32)
+    v4i v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t i = first + j * 256;
+        v[j] = v4i{0, 0, 0, 0};
+        if (i >= total) continue;
+        const uint32_t r = i / per_row, at = (i - r * per_row) * 16;
+        const char *src = o.src + r * o.ld + at;
+        if (at + 16 <= kbytes) {
+            v[j] = *(const v4i_any *)src;
+        } else if (at < kbytes) {
+            uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 16 / ES; ++e)
+                if (at + e * ES < kbytes) {
+                    const uint32_t x = ES == 2 ? (uint32_t)((const uint16_t *)src)[e] : (uint32_t)((const uint8_t *)src)[e];
+                    w[e * ES / 4] |= x << (8 * (e * ES % 4));
+                }
+            v[j] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t i = first + j * 256;
+        if (i < total) *(v4i *)(o.dst + (size_t)i * 16) = v[j];          // (rows of dst follow each other without a gap)
+    }
+}
+
+template <int ES>
+__global__ void __launch_bounds__(256) pack_kernel(const PackArgs a) {
+    const uint32_t which = blockIdx.x >= a.op[0].blocks ? 1u : 0u, block = blockIdx.x - (which ? a.op[0].blocks : 0u);
+    const PackOperand &o = a.op[which];
+    if (!o.k_major) {
+        pack_rows<ES>(o, block);
+        return;
+    }
+    const uint32_t tk = block % o.tiles_k, tr = block / o.tiles_k;
+    if constexpr (ES == 2)
+        transpose_u16_tile<false>((const uint16_t *)o.src, o.ld / 2, (uint16_t *)o.dst, o.pitch / 2, o.k, o.pitch / 2, o.rows, tk, tr);
+    else
+        transpose_bytes_tile<false>((const uint8_t *)o.src, o.ld, (uint8_t *)o.dst, o.pitch, o.k, o.pitch, o.rows, tk, tr);
 }
 
 // ---------------------------------------------------------------------------

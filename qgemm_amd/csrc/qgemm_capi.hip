@@ -70,6 +70,8 @@ struct Context {
     long row_split = 1;         // 0: never run the rows (or columns) of a last, mostly empty round of 256 x 256 tiles as a second launch;
                                 // 2 / 3: the rows / the columns always where the geometry allows it, whatever the estimate says
                                 // (for measurements)
+    long any_shape = 1;         // operands no MFMA kernel reads as they stand: 0: the scalar kernel, 1: packed for the MFMA kernels where
+                                // that is faster, 2: packed wherever possible (for measurements and tests)
     long kmajor = 1;            // 0: K-major operands (NN, reference fp8 layout) always go through the transposes; 2: never
                                 // where a K-major kernel fits the shape (for measurements and tests)
     std::string last_config;
@@ -975,6 +977,98 @@ int launch_nt(NtProblem q, hipStream_t stream) {
     return run_nt(q, pl, ws, stream);
 }
 
+// Is a product on the any-shape path large enough for the packing launch and the matrix cores?  The scalar kernel, one
+// thread per element, takes 2 us and 0.07 - 0.09 us per element of K, and no less than a microsecond per 0.8e6 products;
+// packing and the MFMA kernel take 5.5 - 9 us on products this small.  Graph replays, us, scalar / packed: 16 x 1001 bf16
+// K = 33 4.6 / 6.8, 65 6.6 / 7.1, 129 12.2 / 7.4; 1 x 1001 int8 65 6.0 / 7.6, 129 10.0 / 7.7; 256 x 257 bf16 33 6.4 / 8.5,
+// 65 10.5 / 8.8.  Large: 1531 x 4100 x 3004 int8 23 800 / 45 us, bf16 1999 x 1000 x 3001 2 750 / 30.
+bool pack_pays(size_t M, size_t N, size_t K) { return K >= 72 || (double)M * N * K >= 8e6; }
+
+// Operands that no MFMA kernel reads as they stand: pack_kernel writes what has to change into the workspace as rows of
+// whole 128-byte K steps (one launch for both operands), and the K-contiguous kernels take it from there.  a_src / b_src:
+// the operands as the caller has them, ld in bytes between rows, or, k_major, between rows of k.  q: everything else, with
+// the caller's K.  *taken = false, and nothing launched, where the scalar kernel is the one to run:
+//   * fp8 operands with fp32 output: the matrix core adds the products of an fp8 step with fewer bits than an fp32 sum
+//     keeps (1.5e-5 against 5e-8 of the result at K = 4096: nothing beside a 16-bit output's rounding, all of the error of an
+//     fp32 one), and these shapes have always been summed in fp32;
+//   * no room: the static scratch is too small, a stream capture forbids growing the workspace (the scalar kernel needs
+//     none), or the shape exceeds what the MFMA kernels index;
+//   * a product so small that the scalar kernel is done first (pack_pays).
+struct SourceOperand {
+    const void *p;
+    size_t ld;
+    bool k_major;
+};
+int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const SourceOperand &b_src, size_t K, hipStream_t stream,
+                  bool *taken) {
+    *taken = false;
+    const size_t eb = dtype_bytes(in_dtype);
+    if (!g_ctx.any_shape || (in_dtype == QGEMM_DT_F8E4M3 && q.out_dtype == QGEMM_DT_F32)) return QGEMM_OK;
+    if (g_ctx.any_shape == 1 && !pack_pays(q.M, q.N, K)) return QGEMM_OK;
+    if (q.M >= ((size_t)1 << 31) || q.N >= ((size_t)1 << 31) || K >= ((size_t)1 << 30)) return QGEMM_OK;
+    // (a K that ends inside a 16-byte piece has to end in zeros in both operands)
+    const bool whole = (K * eb) % 16 == 0;
+    const SourceOperand *src[2] = {&a_src, &b_src};
+    const size_t rows[2] = {q.M, q.N}, pitch = (K * eb + 127) / 128 * 128;
+    bool pack[2];
+    size_t room[2];
+    for (int i = 0; i < 2; ++i) {
+        pack[i] = !whole || src[i]->k_major || src[i]->ld % 16 != 0 || !aligned16(src[i]->p);
+        room[i] = pack[i] ? rows[i] * pitch : 0;
+        (i ? q.ldb_bytes : q.lda_bytes) = pack[i] ? pitch : src[i]->ld;
+    }
+    q.Kbytes = pack[0] && pack[1] ? pitch : K * eb;
+    q.kmaj = 0;
+    if (!mfma_shape_ok(q)) return QGEMM_OK;
+    Plan pl;
+    if (plan_nt(q, pl) != QGEMM_OK) return QGEMM_OK;
+    const size_t split_room = (pl.split_bytes + 255) / 256 * 256;
+    const size_t as_room = settle_scale_layout(q, pl) ? 0 : scales_room(q);
+    PackArgs pa;
+    std::memset(&pa, 0, sizeof(pa));
+    uint64_t blocks = 0;
+    for (int i = 0; i < 2; ++i) {
+        if (!pack[i]) continue;
+        PackOperand &o = pa.op[i];
+        o.src = (const char *)src[i]->p;
+        o.ld = src[i]->ld;
+        o.rows = (uint32_t)rows[i];
+        o.k = (uint32_t)K;
+        o.pitch = (uint32_t)pitch;
+        o.k_major = src[i]->k_major;
+        uint64_t n;
+        if (o.k_major) {        // tiles of 64 k x 256 rows (16-bit), 128 x 128 (bytes)
+            o.tiles_k = (uint32_t)(eb == 2 ? pitch / 2 / 64 : pitch / 128);
+            n = (uint64_t)o.tiles_k * (eb == 2 ? (rows[i] + 255) / 256 : (rows[i] + 127) / 128);
+        } else {
+            n = ((uint64_t)rows[i] * (pitch / 16) + 1023) / 1024;
+            if (n >= ((uint64_t)1 << 22)) return QGEMM_OK;          // (32-bit piece numbers in pack_rows)
+        }
+        o.blocks = (uint32_t)n;
+        blocks += n;
+    }
+    if (blocks >= ((uint64_t)1 << 31)) return QGEMM_OK;
+    void *ws = nullptr;
+    int st = ensure_workspace_locked(split_room + as_room + room[0] + room[1], stream, &ws);
+    if (st == QGEMM_ERR_ALLOC || st == QGEMM_ERR_SCRATCH_TOO_SMALL) return QGEMM_OK;
+    *taken = true;
+    if (st != QGEMM_OK) return st;
+    char *at = (char *)ws + split_room + as_room, *bt = at + room[0];
+    pa.op[0].dst = at;
+    pa.op[1].dst = bt;
+    q.A = pack[0] ? at : a_src.p;
+    q.B = pack[1] ? bt : b_src.p;
+    hipLaunchKernelGGL(eb == 2 ? pack_kernel<2> : pack_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, stream, pa);
+    if (hipGetLastError() != hipSuccess) return QGEMM_ERR_LAUNCH;
+    if (as_room) {
+        st = scales_rows_contiguous(q, (char *)ws + split_room, stream);
+        if (st != QGEMM_OK) return st;
+    }
+    st = run_nt(q, pl, ws, stream);
+    g_ctx.last_config = "strided_any_shape";        // (one name for both forms of the any-shape path, as qgemm_plan gives it)
+    return st;
+}
+
 template <int DT>
 int launch_strided_t(const StridedArgs &s, hipStream_t stream) {
     dim3 grid((s.N + 15) / 16, (s.M + 15) / 16);
@@ -999,32 +1093,23 @@ int launch_transpose(int elem_bytes, const void *in, void *out, size_t M, size_t
     if (M >= ((size_t)1 << 31) || N >= ((size_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
     dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
     if (grid.y > 65535u * 1024u) return QGEMM_ERR_TOO_LARGE;
-    if (elem_bytes == 1 && M % 16 == 0 && N % 4 == 0 && (uintptr_t)in % 4 == 0 && (uintptr_t)out % 16 == 0) {
-        dim3 g128((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128));
-        hipLaunchKernelGGL(transpose_bytes_kernel, g128, dim3(256), 0, stream, (const uint8_t *)in, (uint8_t *)out,
+    // Sizes or addresses that rule out aligned 16-byte pieces take the same tiles with pieces at any address, the ones on
+    // the edges element by element.
+    if (elem_bytes == 1) {
+        const bool aligned = M % 16 == 0 && N % 4 == 0 && (uintptr_t)in % 4 == 0 && (uintptr_t)out % 16 == 0;
+        const dim3 g((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128));
+        const auto kernel = aligned ? transpose_bytes_kernel<true> : transpose_bytes_kernel<false>;
+        hipLaunchKernelGGL(kernel, g, dim3(256), 0, stream, (const uint8_t *)in, (uint8_t *)out, (uint32_t)M, (uint32_t)N);
+    } else if (elem_bytes == 2) {
+        const bool aligned = M % 8 == 0 && N % 8 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 16 == 0;
+        const dim3 g((unsigned)((N + 255) / 256), (unsigned)((M + 63) / 64));
+        const auto kernel = aligned ? transpose_u16_kernel<true> : transpose_u16_kernel<false>;
+        hipLaunchKernelGGL(kernel, g, dim3(256), 0, stream, (const uint16_t *)in, (uint16_t *)out, (uint32_t)M, (uint32_t)N);
+    } else if (elem_bytes == 4) {
+        hipLaunchKernelGGL(transpose_kernel<uint32_t>, grid, dim3(256), 0, stream, (const uint32_t *)in, (uint32_t *)out,
                            (uint32_t)M, (uint32_t)N);
-        return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
-    }
-    if (elem_bytes == 2 && M % 8 == 0 && N % 8 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 16 == 0) {
-        dim3 g((unsigned)((N + 255) / 256), (unsigned)((M + 63) / 64));
-        hipLaunchKernelGGL(transpose_u16_kernel, g, dim3(256), 0, stream, (const uint16_t *)in, (uint16_t *)out,
-                           (uint32_t)M, (uint32_t)N);
-        return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
-    }
-    switch (elem_bytes) {
-        case 1:
-            hipLaunchKernelGGL(transpose_kernel<uint8_t>, grid, dim3(256), 0, stream, (const uint8_t *)in, (uint8_t *)out,
-                               (uint32_t)M, (uint32_t)N);
-            break;
-        case 2:
-            hipLaunchKernelGGL(transpose_kernel<uint16_t>, grid, dim3(256), 0, stream, (const uint16_t *)in,
-                               (uint16_t *)out, (uint32_t)M, (uint32_t)N);
-            break;
-        case 4:
-            hipLaunchKernelGGL(transpose_kernel<uint32_t>, grid, dim3(256), 0, stream, (const uint32_t *)in,
-                               (uint32_t *)out, (uint32_t)M, (uint32_t)N);
-            break;
-        default: return QGEMM_ERR_UNSUPPORTED;
+    } else {
+        return QGEMM_ERR_UNSUPPORTED;
     }
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }
@@ -1133,6 +1218,7 @@ QGEMM_EXPORT int qgemm_set_option(const char *key, long value) {
     } else if (!std::strcmp(key, "force_split")) g_ctx.force_split = value;
     else if (!std::strcmp(key, "group_m")) g_ctx.force_group_m = value;
     else if (!std::strcmp(key, "kmajor")) g_ctx.kmajor = value;
+    else if (!std::strcmp(key, "any_shape")) g_ctx.any_shape = value;
     else if (!std::strcmp(key, "stagger")) g_ctx.stagger = value;
     else if (!std::strcmp(key, "stagger_groups")) g_ctx.stagger_groups = value;
     else if (!std::strcmp(key, "c_plain")) g_ctx.c_plain = value;
@@ -1361,6 +1447,9 @@ QGEMM_EXPORT int qgemm_gemm(int in_dtype, int out_dtype, int layout_b, const voi
     }
 
     if (M >= ((size_t)1 << 32) || N >= ((size_t)1 << 32) || K >= ((size_t)1 << 32)) return QGEMM_ERR_TOO_LARGE;
+    bool taken = false;
+    st = launch_packed(q, in_dtype, {A, ldA * eb, false}, {B, ldB * eb, layout_b == QGEMM_B_KN}, K, stream, &taken);
+    if (taken) return st;
     StridedArgs s;
     std::memset(&s, 0, sizeof(s));
     s.A = A;
@@ -1495,6 +1584,10 @@ int scaled_gemm_entry(bool use_static, int in_dtype, int out_dtype, int scale_mo
     }
 
     if (M >= ((size_t)1 << 32) || N >= ((size_t)1 << 32) || K >= ((size_t)1 << 32)) return QGEMM_ERR_TOO_LARGE;
+    const bool km = layout == QGEMM_LAYOUT_REFERENCE;
+    bool taken = false;
+    st = launch_packed(q, in_dtype, {A, km ? M : K, km}, {B, km ? N : K, km}, K, stream, &taken);
+    if (taken) return st;
     StridedArgs s;
     std::memset(&s, 0, sizeof(s));
     s.A = A;
