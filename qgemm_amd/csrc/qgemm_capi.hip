@@ -1114,40 +1114,42 @@ int launch_transpose(int elem_bytes, const void *in, void *out, size_t M, size_t
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }
 
-template <int IN_DT>
+template <int IN_DT, int OUT_DT>
 int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
-    const uint64_t groups = (uint64_t)a.rows * ((a.cols + 3) / 4);
+    typedef Piece<IN_DT> P;
+    auto number = [&](uint32_t per_row) {       // see QuantArgs::per_row
+        a.per_row = std::max<uint32_t>(1, per_row);
+        a.inv = (uint32_t)std::min<uint64_t>(((uint64_t)1 << 32) / a.per_row, 0xFFFFFFFFu);
+        a.rows_per_slice = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(a.rows, ((uint64_t)1 << 31) / a.per_row));
+    };
     if (mode == QGEMM_QUANT_PER_MATRIX) {
         // two passes: partial maxima (one per workgroup) into the workspace, then scale and cast
-        const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(2048, (groups + 1023) / 1024));
+        number((a.cols + P::VEC - 1) / P::VEC);
+        const uint32_t slices = std::max<uint32_t>(1, (a.rows + a.rows_per_slice - 1) / a.rows_per_slice);
+        const uint64_t turns = ((uint64_t)a.rows_per_slice * a.per_row + 256 * kQuantTurn - 1) / (256 * kQuantTurn);
+        const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(1024, turns));
+        a.npartial = nblk * slices;
         void *ws = nullptr;
-        int st = ensure_workspace_locked(nblk * sizeof(float), stream, &ws);
+        int st = ensure_workspace_locked((size_t)a.npartial * sizeof(uint32_t), stream, &ws);
         if (st != QGEMM_OK) return st;
-        a.partial = (float *)ws;
-        a.npartial = nblk;
-        hipLaunchKernelGGL(quant_amax_kernel<IN_DT>, dim3(nblk), dim3(256), 0, stream, a);
-        const uint32_t nq = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(8192, (groups + 255) / 256));
-        hipLaunchKernelGGL(quant_matrix_kernel<IN_DT>, dim3(nq), dim3(256), 0, stream, a);
+        a.partial = (uint32_t *)ws;
+        hipLaunchKernelGGL(quant_amax_kernel<IN_DT>, dim3(nblk, slices), dim3(256), 0, stream, a);
+        const uint32_t nq = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(2048, turns));
+        hipLaunchKernelGGL((quant_matrix_kernel<IN_DT, OUT_DT>), dim3(nq, slices), dim3(256), 0, stream, a);
     } else if (mode == QGEMM_QUANT_BLOCK_1x128) {
-        const uint64_t nblocks = (uint64_t)a.rows * ((a.cols + 127) / 128);
-        if ((nblocks + 7) / 8 >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
-        const uint32_t nbc = a.cols / 128;
-        const bool whole = a.cols % 128 == 0 && a.ld % 4 == 0 && (uintptr_t)a.x % 16 == 0 && a.ldq % 4 == 0 &&
-                           (uintptr_t)a.q % 4 == 0 && a.out_dtype == QGEMM_DT_F8E4M3 && (nbc + 7) / 8 <= 65535 && a.rows > 0;
-        if (whole)
-            hipLaunchKernelGGL(quant_row_block_whole_kernel<IN_DT>, dim3(a.rows, (nbc + 7) / 8), dim3(256), 0, stream, a);
+        number((a.cols + 127) / 128);
+        const uint64_t blocks = (uint64_t)a.rows_per_slice * a.per_row;
+        const uint32_t slices = (a.rows + a.rows_per_slice - 1) / a.rows_per_slice, per_turn = 256 / P::LANES;
+        if (blocks >= (uint64_t)4096 * per_turn)
+            hipLaunchKernelGGL((quant_row_block_kernel<IN_DT, OUT_DT, 4>), dim3((unsigned)((blocks + 4 * per_turn - 1) / (4 * per_turn)), slices),
+                               dim3(256), 0, stream, a);
         else
-            hipLaunchKernelGGL(quant_row_block_kernel<IN_DT>, dim3((unsigned)((nblocks + 7) / 8)), dim3(256), 0, stream, a);
+            hipLaunchKernelGGL((quant_row_block_kernel<IN_DT, OUT_DT, 1>), dim3((unsigned)((blocks + per_turn - 1) / per_turn), slices),
+                               dim3(256), 0, stream, a);
     } else {
         const uint64_t nblocks = (uint64_t)((a.rows + 127) / 128) * ((a.cols + 127) / 128);
         if (nblocks >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
-        const bool whole = a.cols % 128 == 0 && a.rows % 128 == 0 && a.rows > 0 && a.cols > 0 && a.ld % 4 == 0 &&
-                           (uintptr_t)a.x % 16 == 0 && a.ldq % 4 == 0 && (uintptr_t)a.q % 4 == 0 &&
-                           a.out_dtype == QGEMM_DT_F8E4M3 && a.rows / 128 <= 65535;
-        if (whole)
-            hipLaunchKernelGGL(quant_square_block_whole_kernel<IN_DT>, dim3(a.cols / 128, a.rows / 128), dim3(256), 0, stream, a);
-        else
-            hipLaunchKernelGGL(quant_square_block_kernel<IN_DT>, dim3((unsigned)nblocks), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((quant_square_block_kernel<IN_DT, OUT_DT>), dim3((unsigned)nblocks), dim3(256), 0, stream, a);
     }
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }
@@ -1358,7 +1360,6 @@ QGEMM_EXPORT int qgemm_quantize(int in_dtype, int out_dtype, int mode, const voi
     a.ldq = ldq;
     a.scale_rs = scale_rs;
     a.scale_cs = scale_cs;
-    a.out_dtype = out_dtype;
     if (rows == 0 || cols == 0) {
         if (mode != QGEMM_QUANT_PER_MATRIX) return QGEMM_OK;
         // the scale of an empty matrix is the scale of a zero matrix: run the passes over nothing
@@ -1368,10 +1369,14 @@ QGEMM_EXPORT int qgemm_quantize(int in_dtype, int out_dtype, int mode, const voi
     }
     g_ctx.last_config = mode == QGEMM_QUANT_PER_MATRIX ? "quantize_per_matrix"
                         : (mode == QGEMM_QUANT_BLOCK_1x128 ? "quantize_1x128" : "quantize_128x128");
+    const bool f8 = out_dtype == QGEMM_DT_F8E4M3;
     switch (in_dtype) {
-        case QGEMM_DT_F32: return quantize_t<QGEMM_DT_F32>(mode, a, stream);
-        case QGEMM_DT_BF16: return quantize_t<QGEMM_DT_BF16>(mode, a, stream);
-        default: return quantize_t<QGEMM_DT_F16>(mode, a, stream);
+        case QGEMM_DT_F32:
+            return f8 ? quantize_t<QGEMM_DT_F32, QGEMM_DT_F8E4M3>(mode, a, stream) : quantize_t<QGEMM_DT_F32, QGEMM_DT_I8>(mode, a, stream);
+        case QGEMM_DT_BF16:
+            return f8 ? quantize_t<QGEMM_DT_BF16, QGEMM_DT_F8E4M3>(mode, a, stream) : quantize_t<QGEMM_DT_BF16, QGEMM_DT_I8>(mode, a, stream);
+        default:
+            return f8 ? quantize_t<QGEMM_DT_F16, QGEMM_DT_F8E4M3>(mode, a, stream) : quantize_t<QGEMM_DT_F16, QGEMM_DT_I8>(mode, a, stream);
     }
 }
 

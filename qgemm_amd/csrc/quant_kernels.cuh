@@ -3,9 +3,22 @@
 //   1 x 128 blocks  one scale per row and 128 columns      (the a_scale of hip_mix_gemm_kernel.cpp:149)
 //   128 x 128       one scale per 128 x 128 block          (the b_scale of hip_mix_gemm_kernel.cpp:137,164)
 // A block (or matrix) of zeros gets s = 1.  x / s is a true division and the rounding is to nearest even,
-// so the results are the bits the CPU quantisers give.  All three are bound by HBM traffic.
+// so the results are the bits the CPU quantisers give.
+//
+// What bounds them: memory, once the instructions per element are few.  16-bit input leaves 1.2 ns per element and CU at
+// the rate a copy reaches, a dozen vector instructions; element by element, with a test for NaN, infinity and zero and a
+// clamp around every quotient, it took 25 and the 1 x 128 quantiser of bf16 ran at 2.9 TB/s.  So:
+//   * a lane works on pieces of 16 bytes (8 16-bit or 4 fp32 elements), at any address, the row ends element by element;
+//   * maxima are integer maxima of the bits without the sign (two at a time for 16-bit input): the order of the numbers,
+//     with infinities and NaNs on top, so that one look at a block's maximum tells whether the plain form below will do;
+//   * plain form (a finite maximum: no element is NaN or infinite, no quotient exceeds the type's largest value): the
+//     quotient of |x| without special cases, the sign moved over afterwards; anything else takes the careful form.
+// Before and now, us (to fp8 unless said): 1 x 128 6144 x 7168 bf16 45.7 -> 28.4 (4.7 TB/s, what a copy reaches), 500 x 7200
+// 7.3 -> 5.7; 128 x 128 7168 x 6144 fp32 43.4 -> 39.6 (5.6 TB/s); per matrix 1531 x 3004 bf16 to int8 4.9 + 8.5 -> 4.2 + 6.6.
+// A decoder's 16 x 2048 stays at 2.8: one trip to memory and back.
 #pragma once
 #include "common.h"
+#include "aux_kernels.cuh"
 
 namespace qgemm {
 
@@ -13,294 +26,379 @@ struct QuantArgs {
     const void *x;        // rows x cols, row stride ld elements
     void *q;              // rows x cols bytes, row stride ldq
     float *scales;        // per matrix: 1 float; blocks: scales[ib*scale_rs + jb*scale_cs]
-    float *partial;       // per matrix: one partial maximum per workgroup of the first pass
+    uint32_t *partial;    // per matrix: one partial maximum per workgroup of the first pass (bits of |x|; bit 31: NaNs seen)
     uint32_t rows, cols, npartial;
     uint64_t ld, ldq, scale_rs, scale_cs;
-    int out_dtype;        // QGEMM_DT_I8 or QGEMM_DT_F8E4M3
+    // Work is numbered along rows in units of a piece (per matrix) or of a 1 x 128 block: `per_row` of them in a row,
+    // inv = floor(2^32 / per_row).  blockIdx.y counts slices of rows_per_slice rows, so that a number fits 32 bits.
+    uint32_t per_row, inv, rows_per_slice;
 };
 
-template <int IN_DT>
-__device__ inline float load_as_f32(const void *base, size_t idx) {
-    if constexpr (IN_DT == QGEMM_DT_F32) return ((const float *)base)[idx];
-    else if constexpr (IN_DT == QGEMM_DT_BF16)
-        return __builtin_bit_cast(float, (uint32_t)((const unsigned short *)base)[idx] << 16);
-    else return (float)((const _Float16 *)base)[idx];
-}
-
-// four consecutive elements; `vec` says the address is aligned for one vector load
-template <int IN_DT>
-__device__ inline v4f load4_as_f32(const void *base, size_t idx, bool vec, uint32_t valid) {
-    v4f r = {0, 0, 0, 0};
-    if (vec && valid >= 4) {
-        if constexpr (IN_DT == QGEMM_DT_F32) {
-            r = *(const v4f *)((const float *)base + idx);
-        } else {
-            const us4 h = *(const us4 *)((const unsigned short *)base + idx);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned short bits = h[i];     // (a bit_cast applied to a vector element reads element 0)
-                if constexpr (IN_DT == QGEMM_DT_BF16) r[i] = __builtin_bit_cast(float, (uint32_t)bits << 16);
-                else r[i] = (float)__builtin_bit_cast(_Float16, bits);
-            }
-        }
-        return r;
+// i / d and i % d with inv = min(floor(2^32 / d), 2^32 - 1): the estimate is at most one too small
+__device__ inline uint32_t div_by_inv(uint32_t i, uint32_t d, uint32_t inv, uint32_t &rem) {
+    uint32_t q = __umulhi(i, inv);
+    rem = i - q * d;
+    if (rem >= d) {
+        rem -= d;
+        ++q;
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if ((uint32_t)i < valid) r[i] = load_as_f32<IN_DT>(base, idx + i);
-    return r;
+    return q;
 }
 
-// |x| with NaN mapped to 0: a NaN never becomes the maximum (the CPU loop's `a > m` ignores it too)
-__device__ inline float abs_or_zero(float v) {
-    const float a = __builtin_fabsf(v);
-    return a == a ? a : 0.0f;
-}
+// ---- 16 bytes of input
+template <int IN_DT>
+struct Piece {
+    static constexpr int ES = IN_DT == QGEMM_DT_F32 ? 4 : 2, VEC = 16 / ES;
+    static constexpr int LANES = kScaleBlock / VEC;                  // lanes that cover the 128 columns of a block
+    static constexpr uint32_t INF = IN_DT == QGEMM_DT_F32 ? 0x7F800000u : (IN_DT == QGEMM_DT_BF16 ? 0x7F80u : 0x7C00u);
+
+    __device__ static float element(uint32_t bits) {
+        if constexpr (IN_DT == QGEMM_DT_F32) return __builtin_bit_cast(float, bits);
+        else if constexpr (IN_DT == QGEMM_DT_BF16) return __builtin_bit_cast(float, bits << 16);
+        else return (float)__builtin_bit_cast(_Float16, (unsigned short)bits);
+    }
+    // elements idx .. idx + VEC - 1; those from `valid` on are zeros and not read
+    __device__ static v4i load(const void *base, size_t idx, uint32_t valid) {
+        const char *p = (const char *)base + idx * ES;
+        if (valid >= (uint32_t)VEC) return *(const v4i_any *)p;
+        uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int e = 0; e < VEC - 1; ++e)
+            if ((uint32_t)e < valid) {
+                if constexpr (ES == 4) w[e] = ((const uint32_t *)p)[e];
+                else w[e >> 1] |= (uint32_t)((const uint16_t *)p)[e] << (16 * (e & 1));
+            }
+        return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+    }
+    __device__ static uint32_t bits(v4i r, int e) {
+        if constexpr (ES == 4) return (uint32_t)r[e];
+        else return ((uint32_t)r[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
+    }
+    // bits of the largest |x| of the piece, NaNs above everything
+    __device__ static uint32_t max_bits(v4i r) {
+        if constexpr (ES == 4) {
+            const uint32_t k = 0x7FFFFFFFu, a = r[0] & k, b = r[1] & k, c = r[2] & k, d = r[3] & k;
+            const uint32_t m = a > b ? a : b, n = c > d ? c : d;
+            return m > n ? m : n;
+        } else {
+            typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+            auto h = [&](int i) { return __builtin_bit_cast(us2, (uint32_t)r[i] & 0x7FFF7FFFu); };
+            const us2 m = __builtin_elementwise_max(__builtin_elementwise_max(h(0), h(1)), __builtin_elementwise_max(h(2), h(3)));
+            const uint32_t u = __builtin_bit_cast(uint32_t, m), hi = u >> 16, lo = u & 0xFFFFu;
+            return hi > lo ? hi : lo;
+        }
+    }
+    // the same over the elements that are numbers
+    __device__ static uint32_t max_bits_of_numbers(v4i r) {
+        uint32_t m = 0;
+        for (int e = 0; e < VEC; ++e) {
+            const uint32_t b = bits(r, e) & (ES == 4 ? 0x7FFFFFFFu : 0x7FFFu);
+            if (b <= INF && b > m) m = b;
+        }
+        return m;
+    }
+};
 
 // e4m3 (OCP): saturate to +-448, then round to nearest even; NaN -> 0x7F with the sign kept.
-// Two values per call: v_cvt_pk_fp8_f32 packs them into the low half of a dword.
-__device__ inline uint32_t f32x2_to_fp8(float a, float b) {
-    const bool na = a != a, nb = b != b;
-    const float ca = __builtin_fminf(__builtin_fmaxf(a, -448.0f), 448.0f);
-    const float cb = __builtin_fminf(__builtin_fmaxf(b, -448.0f), 448.0f);
-    uint32_t r = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(ca, cb, 0, false) & 0xFFFFu;
-    if (na) r = (r & 0xFF00u) | 0x7Fu | ((__builtin_bit_cast(uint32_t, a) >> 24) & 0x80u);
-    if (nb) r = (r & 0x00FFu) | ((0x7Fu | ((__builtin_bit_cast(uint32_t, b) >> 24) & 0x80u)) << 8);
-    return r;
+__device__ inline uint32_t f32_to_fp8_careful(float a) {
+    if (a != a) return 0x7Fu | ((__builtin_bit_cast(uint32_t, a) >> 24) & 0x80u);
+    const float c = __builtin_fminf(__builtin_fmaxf(a, -448.0f), 448.0f);
+    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c, c, 0, false) & 0xFFu;
 }
 
-__device__ inline uint32_t f32_to_i8(float v) {
+__device__ inline uint32_t f32_to_i8_careful(float v) {
     float r = __builtin_rintf(v);                 // ties to even
     r = r > 127.0f ? 127.0f : r;
     r = r < -127.0f ? -127.0f : r;
     return (uint32_t)(int)r & 0xFFu;              // NaN: the comparisons are false, the cast gives 0
 }
 
-// x / s for many x and one s (a scale: positive, finite).  The compiler expands every fp32 division into a
+// x / s for many x and one s (a scale: positive).  The compiler expands every fp32 division into a
 // reciprocal, two refinements of it and three of the quotient, all on values scaled by v_div_scale so that nothing
 // leaves the normal range.  With s between 2^-60 and 2^60 and |x| at most a few hundred s (the quantisers divide by
 // max|x| / 448 or / 127) that scaling is the identity unless the quotient is below 2^-100, which every output type
 // here turns into a zero of the quotient's sign whatever its low bits: so the reciprocal is refined once per scale
 // and the quotient steps are the same fused multiply-adds on the same values: the same bits as x / s, about half
-// the instructions per element.  Zeros, infinities and NaNs of x pass through as they are (what the division's
-// last step, v_div_fixup, does for a finite positive divisor); scales outside the range take the plain division.
+// the instructions per element.  (A zero comes out as +0: the callers carry the sign.)
 struct Divisor {
     float s, r;
-    bool in_range;
+    bool plain;           // the quotients may take the short way: s in range and every x finite
 };
-__device__ inline Divisor make_divisor(float s) {
+__device__ inline Divisor make_divisor(float s, bool finite) {
     Divisor d;
     d.s = s;
-    d.in_range = s >= 0x1p-60f && s <= 0x1p60f;
+    d.plain = finite && s >= 0x1p-60f && s <= 0x1p60f;
     const float r0 = __builtin_amdgcn_rcpf(s);
     d.r = __builtin_fmaf(__builtin_fmaf(-s, r0, 1.0f), r0, r0);
     return d;
 }
-__device__ inline float div_by(float x, const Divisor &d) {
-    if (!d.in_range) return x / d.s;
+__device__ inline float div_plain(float x, const Divisor &d) {
     float q = x * d.r;
     q = __builtin_fmaf(__builtin_fmaf(-d.s, q, x), d.r, q);
-    q = __builtin_fmaf(__builtin_fmaf(-d.s, q, x), d.r, q);
-    const float ax = __builtin_fabsf(x);
-    return (ax > 0.0f && ax < __builtin_inff()) ? q : x;
+    return __builtin_fmaf(__builtin_fmaf(-d.s, q, x), d.r, q);
 }
 
-// four quantised bytes of (v / s), packed little-endian
-__device__ inline uint32_t quant4(v4f v, const Divisor &dv, int out_dtype) {
-    const float a = div_by(v[0], dv), b = div_by(v[1], dv), c = div_by(v[2], dv), d = div_by(v[3], dv);
-    if (out_dtype == QGEMM_DT_F8E4M3) return f32x2_to_fp8(a, b) | (f32x2_to_fp8(c, d) << 16);
-    return f32_to_i8(a) | (f32_to_i8(b) << 8) | (f32_to_i8(c) << 16) | (f32_to_i8(d) << 24);
+// the VEC quantised bytes of a piece, element 0 in the low byte of component 0
+template <int IN_DT, int OUT_DT>
+__device__ inline v2i quant_piece(v4i r, const Divisor &dv) {
+    typedef Piece<IN_DT> P;
+    uint32_t w[2] = {0, 0};
+    if (dv.plain) {
+#pragma unroll
+        for (int h = 0; h < P::VEC / 4; ++h) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = P::element(P::bits(r, 4 * h + e));
+            if constexpr (OUT_DT == QGEMM_DT_F8E4M3) {
+                // |x| / s is at most 448 and half an ulp: it rounds to at most 448
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float q = div_plain(__builtin_fabsf(v[e]), dv);
+                    v[e] = P::ES == 4 ? __builtin_copysignf(q, v[e]) : q;
+                }
+                uint32_t p = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+                p = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], (int)p, true);
+                if constexpr (P::ES == 2)        // the four sign bits at once, out of the high bytes of the elements
+                    p |= __builtin_amdgcn_perm((uint32_t)r[2 * h + 1], (uint32_t)r[2 * h], 0x07050301) & 0x80808080u;
+                w[h] = p;
+            } else {
+                // adding 1.5 * 2^23 rounds to the nearest integer, ties to even, and leaves it in the low byte; |x| / s is
+                // at most 127 and half an ulp
+                uint32_t b[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) b[e] = __builtin_bit_cast(uint32_t, div_plain(v[e], dv) + 12582912.0f);
+                const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0400), hi = __builtin_amdgcn_perm(b[3], b[2], 0x0C0C0400);
+                w[h] = lo | (hi << 16);
+            }
+        }
+    } else {
+        for (int e = 0; e < P::VEC; ++e) {
+            const float v = P::element(P::bits(r, e)) / dv.s;
+            w[e >> 2] |= (OUT_DT == QGEMM_DT_F8E4M3 ? f32_to_fp8_careful(v) : f32_to_i8_careful(v)) << (8 * (e & 3));
+        }
+    }
+    return v2i{(int)w[0], (int)w[1]};
 }
 
-__device__ inline void store4(void *q, size_t idx, uint32_t packed, bool vec, uint32_t valid) {
-    if (vec && valid >= 4) {
-        *(uint32_t *)((uint8_t *)q + idx) = packed;
+template <int IN_DT>
+__device__ inline void store_piece(void *q, size_t idx, v2i w, uint32_t valid) {
+    typedef int v2i_any __attribute__((ext_vector_type(2), aligned(1)));
+    uint8_t *p = (uint8_t *)q + idx;
+    if (valid >= (uint32_t)Piece<IN_DT>::VEC) {
+        if constexpr (Piece<IN_DT>::VEC == 8) *(v2i_any *)p = w;
+        else *(u32_any *)p = (uint32_t)w[0];
         return;
     }
-    for (uint32_t i = 0; i < 4 && i < valid; ++i) ((uint8_t *)q)[idx + i] = (uint8_t)(packed >> (8 * i));
+    for (uint32_t e = 0; e < valid; ++e) p[e] = (uint8_t)((uint32_t)w[e >> 2] >> (8 * (e & 3)));
 }
 
-__device__ inline float wave_max(float m) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = __builtin_fmaxf(m, __shfl_xor(m, off, 64));
+// maximum over groups of 16, 32 or 64 neighbouring lanes, in every lane, on the vector ALU alone: lane exchanges inside a
+// row of 16 ride on the max instruction (DPP), rows are exchanged with lane swaps.  (Every __shfl_xor is a trip through
+// the LDS crossbar with its address arithmetic.)
+template <int LANES>
+__device__ inline uint32_t lanes_max(uint32_t m) {
+    auto with = [&](uint32_t o) { m = o > m ? o : m; };
+    auto dpp = [&](auto ctrl) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, decltype(ctrl)::value, 0xF, 0xF, true); };
+    with(dpp(std::integral_constant<int, 0xB1>{}));      // quad_perm [1,0,3,2]: lane ^ 1
+    with(dpp(std::integral_constant<int, 0x4E>{}));      // quad_perm [2,3,0,1]: lane ^ 2
+    with(dpp(std::integral_constant<int, 0x141>{}));     // row_half_mirror: lane -> 7 - lane within 8
+    with(dpp(std::integral_constant<int, 0x140>{}));     // row_mirror: lane -> 15 - lane within 16
+    if constexpr (LANES >= 32) {
+        const auto sw = __builtin_amdgcn_permlane16_swap(m, m, false, false);      // (R0 R0 R2 R2), (R1 R1 R3 R3)
+        const uint32_t a = sw[0], b = sw[1];
+        m = a > b ? a : b;
+    }
+    if constexpr (LANES == 64) {
+        const auto sw = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+        const uint32_t a = sw[0], b = sw[1];
+        m = a > b ? a : b;
+    }
     return m;
 }
 
-// maximum over each half of the wave (lanes 0-31, 32-63), in every lane, on the vector ALU alone: lane exchanges
-// inside a row of 16 ride on the max instruction (DPP), the two rows of a half are exchanged with one lane swap.
-// (Five __shfl_xor per block are five trips through the LDS crossbar with their address arithmetic.)
-__device__ inline float half_wave_max(float m) {
-    auto dpp = [](float v, auto ctrl) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xF, 0xF, true));
-    };
-    m = __builtin_fmaxf(m, dpp(m, std::integral_constant<int, 0xB1>{}));      // quad_perm [1,0,3,2]: lane ^ 1
-    m = __builtin_fmaxf(m, dpp(m, std::integral_constant<int, 0x4E>{}));      // quad_perm [2,3,0,1]: lane ^ 2
-    m = __builtin_fmaxf(m, dpp(m, std::integral_constant<int, 0x141>{}));     // row_half_mirror: lane -> 7 - lane within 8
-    m = __builtin_fmaxf(m, dpp(m, std::integral_constant<int, 0x140>{}));     // row_mirror: lane -> 15 - lane within 16
-    const unsigned u = __builtin_bit_cast(unsigned, m);
-    const auto sw = __builtin_amdgcn_permlane16_swap(u, u, false, false);      // (R0 R0 R2 R2), (R1 R1 R3 R3)
-    const unsigned even = sw[0], odd = sw[1];          // (a bit_cast applied to a vector element reads element 0)
-    return __builtin_fmaxf(__builtin_bit_cast(float, even), __builtin_bit_cast(float, odd));
+template <int OUT_DT>
+__device__ inline float scale_of(float amax) {
+    return amax > 0.0f ? amax / (OUT_DT == QGEMM_DT_F8E4M3 ? 448.0f : 127.0f) : 1.0f;
 }
 
-__device__ inline float scale_of(float amax, int out_dtype) {
-    return amax > 0.0f ? amax / (out_dtype == QGEMM_DT_F8E4M3 ? 448.0f : 127.0f) : 1.0f;
-}
+constexpr uint32_t kQuantNan = 0x80000000u;
+constexpr int kQuantTurn = 4;                    // pieces a lane has in flight (per-matrix passes)
 
-// ---- per matrix, pass 1: one partial maximum per workgroup (grid-stride over groups of 4 columns)
+// ---- per matrix, pass 1: one partial maximum per workgroup
 template <int IN_DT>
 __global__ void __launch_bounds__(256) quant_amax_kernel(const QuantArgs p) {
-    __shared__ float red[4];
-    const uint32_t groups_per_row = (p.cols + 3) / 4;
-    const bool vec = p.ld % 4 == 0 && (uintptr_t)p.x % 16 == 0;
-    float m = 0.0f;
-    // rows in turn over the workgroups, groups of four columns in turn over the threads: no division per element
-    for (uint32_t r = blockIdx.x; r < p.rows; r += gridDim.x) {
-        for (uint32_t g = threadIdx.x; g < groups_per_row; g += 256) {
-            const uint32_t c = g * 4;
-            const v4f v = load4_as_f32<IN_DT>(p.x, (size_t)r * p.ld + c, vec, p.cols - c);
+    typedef Piece<IN_DT> P;
+    __shared__ uint32_t red[4];
+    const uint32_t row0 = blockIdx.y * p.rows_per_slice;
+    const uint32_t rows = p.rows - row0 < p.rows_per_slice ? p.rows - row0 : p.rows_per_slice, total = rows * p.per_row;
+    uint32_t m = 0, nan = 0;
+    for (uint32_t first = blockIdx.x * 256 * kQuantTurn; first < total; first += gridDim.x * 256 * kQuantTurn) {
+        v4i v[kQuantTurn];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) m = __builtin_fmaxf(m, abs_or_zero(v[i]));
+        for (int j = 0; j < kQuantTurn; ++j) {
+            const uint32_t i = first + j * 256 + threadIdx.x;
+            v[j] = v4i{0, 0, 0, 0};
+            if (i < total) {
+                uint32_t c;
+                const uint32_t r = div_by_inv(i, p.per_row, p.inv, c);
+                v[j] = P::load(p.x, (size_t)(row0 + r) * p.ld + c * P::VEC, p.cols - c * P::VEC);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kQuantTurn; ++j) {
+            uint32_t b = P::max_bits(v[j]);
+            if (b > P::INF) {
+                nan = kQuantNan;
+                b = P::max_bits_of_numbers(v[j]);
+            }
+            m = b > m ? b : m;
         }
     }
-    m = wave_max(m);
+    m = lanes_max<64>(m) | (__any(nan != 0) ? kQuantNan : 0u);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0)
-        p.partial[blockIdx.x] = __builtin_fmaxf(__builtin_fmaxf(red[0], red[1]), __builtin_fmaxf(red[2], red[3]));
+    if (threadIdx.x == 0) {
+        uint32_t best = 0, any = 0;
+        for (int w = 0; w < 4; ++w) {
+            any |= red[w] & kQuantNan;
+            best = (red[w] & ~kQuantNan) > best ? (red[w] & ~kQuantNan) : best;
+        }
+        p.partial[blockIdx.y * gridDim.x + blockIdx.x] = best | any;
+    }
 }
 
 // ---- per matrix, pass 2: every workgroup reduces the partial maxima again (a few KB, L2 resident), then
 // quantises its share; workgroup 0 writes the scale
-template <int IN_DT>
+template <int IN_DT, int OUT_DT>
 __global__ void __launch_bounds__(256) quant_matrix_kernel(const QuantArgs p) {
-    __shared__ float red[4];
-    float m = 0.0f;
-    for (uint32_t i = threadIdx.x; i < p.npartial; i += 256) m = __builtin_fmaxf(m, p.partial[i]);
-    m = wave_max(m);
+    typedef Piece<IN_DT> P;
+    __shared__ uint32_t red[4];
+    uint32_t m = 0, nan = 0;
+    for (uint32_t i = threadIdx.x; i < p.npartial; i += 256) {
+        const uint32_t b = p.partial[i];
+        nan |= b & kQuantNan;
+        m = (b & ~kQuantNan) > m ? (b & ~kQuantNan) : m;
+    }
+    m = lanes_max<64>(m) | (__any(nan != 0) ? kQuantNan : 0u);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    const float amax = __builtin_fmaxf(__builtin_fmaxf(red[0], red[1]), __builtin_fmaxf(red[2], red[3]));
-    const float s = scale_of(amax, p.out_dtype);
-    if (blockIdx.x == 0 && threadIdx.x == 0) p.scales[0] = s;
-    const uint32_t groups_per_row = (p.cols + 3) / 4;
-    const bool vin = p.ld % 4 == 0 && (uintptr_t)p.x % 16 == 0;
-    const bool vout = p.ldq % 4 == 0 && (uintptr_t)p.q % 4 == 0;
-    const Divisor dv = make_divisor(s);
-    for (uint32_t r = blockIdx.x; r < p.rows; r += gridDim.x) {
-        for (uint32_t g = threadIdx.x; g < groups_per_row; g += 256) {
-            const uint32_t c = g * 4;
-            const v4f v = load4_as_f32<IN_DT>(p.x, (size_t)r * p.ld + c, vin, p.cols - c);
-            store4(p.q, (size_t)r * p.ldq + c, quant4(v, dv, p.out_dtype), vout, p.cols - c);
+    m = 0;
+    nan = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        nan |= red[w] & kQuantNan;
+        m = (red[w] & ~kQuantNan) > m ? (red[w] & ~kQuantNan) : m;
+    }
+    const float s = scale_of<OUT_DT>(P::element(m));
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.scales[0] = s;
+    const Divisor dv = make_divisor(s, m < P::INF && !nan);
+    const uint32_t row0 = blockIdx.y * p.rows_per_slice;
+    const uint32_t rows = p.rows - row0 < p.rows_per_slice ? p.rows - row0 : p.rows_per_slice, total = rows * p.per_row;
+    for (uint32_t first = blockIdx.x * 256 * kQuantTurn; first < total; first += gridDim.x * 256 * kQuantTurn) {
+        v4i v[kQuantTurn];
+        uint32_t r[kQuantTurn], c[kQuantTurn];
+#pragma unroll
+        for (int j = 0; j < kQuantTurn; ++j) {
+            const uint32_t i = first + j * 256 + threadIdx.x;
+            r[j] = div_by_inv(i, p.per_row, p.inv, c[j]);
+            v[j] = v4i{0, 0, 0, 0};
+            if (i < total) v[j] = P::load(p.x, (size_t)(row0 + r[j]) * p.ld + c[j] * P::VEC, p.cols - c[j] * P::VEC);
         }
+#pragma unroll
+        for (int j = 0; j < kQuantTurn; ++j)
+            if (first + j * 256 + threadIdx.x < total)
+                store_piece<IN_DT>(p.q, (size_t)(row0 + r[j]) * p.ldq + c[j] * P::VEC, quant_piece<IN_DT, OUT_DT>(v[j], dv),
+                                   p.cols - c[j] * P::VEC);
     }
 }
 
-// ---- 1 x 128 blocks: half a wave (32 lanes x 4 columns) per block, 8 blocks per workgroup
-template <int IN_DT>
+// scale and divisor of a block whose maximum is in every lane that works on it; `numbers`: the maximum without its NaNs
+template <int IN_DT, int OUT_DT, class F>
+__device__ inline Divisor block_divisor(uint32_t m, F numbers) {
+    const bool finite = m < Piece<IN_DT>::INF;
+    if (m > Piece<IN_DT>::INF) m = numbers();
+    return make_divisor(scale_of<OUT_DT>(Piece<IN_DT>::element(m)), finite);
+}
+
+// ---- 1 x 128 blocks: Piece::LANES lanes (16 or 32) per block and turn, U turns in flight per lane: four where there are
+// enough blocks to fill the CUs that way, one for the few rows of a decoder's step
+template <int IN_DT, int OUT_DT, int U>
 __global__ void __launch_bounds__(256) quant_row_block_kernel(const QuantArgs p) {
-    const uint32_t nbc = (p.cols + 127) / 128;
-    const uint64_t nblocks = (uint64_t)p.rows * nbc;
-    const uint64_t blk = (uint64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
-    if (blk >= nblocks) return;                        // whole half-waves leave together
-    const uint32_t r = (uint32_t)(blk / nbc), jb = (uint32_t)(blk % nbc);
-    const uint32_t c = jb * 128 + (threadIdx.x & 31) * 4;
-    const bool vin = p.ld % 4 == 0 && (uintptr_t)p.x % 16 == 0;
-    const bool vout = p.ldq % 4 == 0 && (uintptr_t)p.q % 4 == 0;
-    const uint32_t valid = c < p.cols ? p.cols - c : 0;
-    const v4f v = load4_as_f32<IN_DT>(p.x, (size_t)r * p.ld + c, vin, valid);
-    float m = 0.0f;
+    typedef Piece<IN_DT> P;
+    constexpr uint32_t G = 256 / P::LANES;                                // blocks per turn of the workgroup
+    const uint32_t row0 = blockIdx.y * p.rows_per_slice;
+    const uint32_t rows = p.rows - row0 < p.rows_per_slice ? p.rows - row0 : p.rows_per_slice, total = rows * p.per_row;
+    const uint32_t lane = threadIdx.x % P::LANES, first = blockIdx.x * G * U + threadIdx.x / P::LANES;
+    v4i v[U];
+    uint32_t r[U], jb[U], valid[U];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) m = __builtin_fmaxf(m, abs_or_zero(v[i]));
-    m = half_wave_max(m);
-    const float s = scale_of(m, p.out_dtype);
-    if ((threadIdx.x & 31) == 0) p.scales[(size_t)r * p.scale_rs + (size_t)jb * p.scale_cs] = s;
-    if (valid) store4(p.q, (size_t)r * p.ldq + c, quant4(v, make_divisor(s), p.out_dtype), vout, valid);
+    for (int u = 0; u < U; ++u) {
+        const uint32_t i = first + u * G;
+        r[u] = row0 + div_by_inv(i, p.per_row, p.inv, jb[u]);
+        const uint32_t c = jb[u] * kScaleBlock + lane * P::VEC;
+        valid[u] = (i < total && c < p.cols) ? p.cols - c : 0;
+        v[u] = v4i{0, 0, 0, 0};
+        if (valid[u]) v[u] = P::load(p.x, (size_t)r[u] * p.ld + c, valid[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t m = lanes_max<P::LANES>(P::max_bits(v[u]));
+        const Divisor dv = block_divisor<IN_DT, OUT_DT>(m, [&] { return lanes_max<P::LANES>(P::max_bits_of_numbers(v[u])); });
+        if (first + u * G >= total) break;                                // (whole groups of lanes leave together)
+        if (lane == 0) p.scales[(size_t)r[u] * p.scale_rs + (size_t)jb[u] * p.scale_cs] = dv.s;
+        if (valid[u])
+            store_piece<IN_DT>(p.q, (size_t)r[u] * p.ldq + jb[u] * kScaleBlock + lane * P::VEC, quant_piece<IN_DT, OUT_DT>(v[u], dv),
+                               valid[u]);
+    }
 }
 
-// ---- 1 x 128 blocks, the common case: whole blocks (cols a multiple of 128), x and q aligned for vector access,
-// fp8 out.  Grid (rows, ceil(blocks per row / 8)): half wave h of workgroup (r, g) takes block 8 g + h of row r, so
-// there is no division to find the block and no bounds check per element.  (The general kernel above spends more
-// instructions on those than on the quantisation: 6144 x 7168 fp32 54 -> 40 us, the same for bf16 input, which
-// says the kernel is bound by instruction issue, not by memory.)
-template <int IN_DT>
-__global__ void __launch_bounds__(256) quant_row_block_whole_kernel(const QuantArgs p) {
-    const uint32_t nbc = p.cols / 128;
-    const uint32_t r = blockIdx.x, jb = blockIdx.y * 8 + (threadIdx.x >> 5);
-    if (jb >= nbc) return;                             // whole half-waves leave together
-    const uint32_t c = jb * 128 + (threadIdx.x & 31) * 4;
-    const v4f v = load4_as_f32<IN_DT>(p.x, (size_t)r * p.ld + c, true, 4);
-    float m = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) m = __builtin_fmaxf(m, abs_or_zero(v[i]));
-    m = half_wave_max(m);
-    const float s = scale_of(m, QGEMM_DT_F8E4M3);
-    if ((threadIdx.x & 31) == 0) p.scales[(size_t)r * p.scale_rs + (size_t)jb * p.scale_cs] = s;
-    *(uint32_t *)((uint8_t *)p.q + (size_t)r * p.ldq + c) = quant4(v, make_divisor(s), QGEMM_DT_F8E4M3);
-}
-
-// ---- 128 x 128 blocks: one workgroup per block; a thread holds 4 columns of 16 rows in registers
-template <int IN_DT>
+// ---- 128 x 128 blocks: one workgroup per block, which it holds in registers
+template <int IN_DT, int OUT_DT>
 __global__ void __launch_bounds__(256) quant_square_block_kernel(const QuantArgs p) {
-    __shared__ float red[4];
+    typedef Piece<IN_DT> P;
+    constexpr int ROWS = 256 / P::LANES, TURNS = 128 / ROWS;
+    __shared__ uint32_t red[4];
     const uint32_t nbc = (p.cols + 127) / 128;
     const uint32_t ib = blockIdx.x / nbc, jb = blockIdx.x % nbc;
-    const uint32_t c = jb * 128 + (threadIdx.x & 31) * 4;
-    const uint32_t r0 = ib * 128 + (threadIdx.x >> 5);            // rows r0, r0 + 8, ...
-    const bool vin = p.ld % 4 == 0 && (uintptr_t)p.x % 16 == 0;
-    const bool vout = p.ldq % 4 == 0 && (uintptr_t)p.q % 4 == 0;
+    const uint32_t c = jb * 128 + (threadIdx.x % P::LANES) * P::VEC;
+    const uint32_t r0 = ib * 128 + threadIdx.x / P::LANES;               // rows r0, r0 + ROWS, ...
     const uint32_t valid = c < p.cols ? p.cols - c : 0;
-    v4f v[16];
-    float m = 0.0f;
+    auto workgroup_max = [&](uint32_t m) {
+        m = lanes_max<64>(m);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+        __syncthreads();
+        const uint32_t a = red[0] > red[1] ? red[0] : red[1], b = red[2] > red[3] ? red[2] : red[3];
+        return a > b ? a : b;
+    };
+    v4i v[TURNS];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const uint32_t r = r0 + i * 8;
-        v[i] = v4f{0, 0, 0, 0};
-        if (r < p.rows && valid) v[i] = load4_as_f32<IN_DT>(p.x, (size_t)r * p.ld + c, vin, valid);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m = __builtin_fmaxf(m, abs_or_zero(v[i][e]));
+    for (int i = 0; i < TURNS; ++i) {
+        const uint32_t r = r0 + i * ROWS;
+        v[i] = v4i{0, 0, 0, 0};
+        if (r < p.rows && valid) v[i] = P::load(p.x, (size_t)r * p.ld + c, valid);
     }
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    const float amax = __builtin_fmaxf(__builtin_fmaxf(red[0], red[1]), __builtin_fmaxf(red[2], red[3]));
-    const float s = scale_of(amax, p.out_dtype);
-    if (threadIdx.x == 0) p.scales[(size_t)ib * p.scale_rs + (size_t)jb * p.scale_cs] = s;
-    const Divisor dv = make_divisor(s);
+    uint32_t m = 0;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const uint32_t r = r0 + i * 8;
-        if (r < p.rows && valid) store4(p.q, (size_t)r * p.ldq + c, quant4(v[i], dv, p.out_dtype), vout, valid);
+    for (int i = 0; i < TURNS; ++i) {
+        const uint32_t b = P::max_bits(v[i]);
+        m = b > m ? b : m;
     }
-}
-
-// ---- 128 x 128 blocks, whole blocks (rows and cols multiples of 128), x and q aligned for vector access, fp8 out:
-// as above without the bounds checks
-template <int IN_DT>
-__global__ void __launch_bounds__(256) quant_square_block_whole_kernel(const QuantArgs p) {
-    __shared__ float red[4];
-    const uint32_t ib = blockIdx.y, jb = blockIdx.x;
-    const uint32_t c = jb * 128 + (threadIdx.x & 31) * 4;
-    const uint32_t r0 = ib * 128 + (threadIdx.x >> 5);            // rows r0, r0 + 8, ...
-    const size_t x0 = (size_t)r0 * p.ld + c, q0 = (size_t)r0 * p.ldq + c;
-    v4f v[16];
-    float m = 0.0f;
+    m = workgroup_max(m);
+    const Divisor dv = block_divisor<IN_DT, OUT_DT>(m, [&] {
+        uint32_t n = 0;
+        for (int i = 0; i < TURNS; ++i) {
+            const uint32_t b = P::max_bits_of_numbers(v[i]);
+            n = b > n ? b : n;
+        }
+        __syncthreads();                                                 // (m is the same in every lane of the workgroup)
+        return workgroup_max(n);
+    });
+    if (threadIdx.x == 0) p.scales[(size_t)ib * p.scale_rs + (size_t)jb * p.scale_cs] = dv.s;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = load4_as_f32<IN_DT>(p.x, x0 + (size_t)i * 8 * p.ld, true, 4);
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m = __builtin_fmaxf(m, abs_or_zero(v[i][e]));
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    const float amax = __builtin_fmaxf(__builtin_fmaxf(red[0], red[1]), __builtin_fmaxf(red[2], red[3]));
-    const float s = scale_of(amax, QGEMM_DT_F8E4M3);
-    if (threadIdx.x == 0) p.scales[(size_t)ib * p.scale_rs + (size_t)jb * p.scale_cs] = s;
-    const Divisor dv = make_divisor(s);
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        *(uint32_t *)((uint8_t *)p.q + q0 + (size_t)i * 8 * p.ldq) = quant4(v[i], dv, QGEMM_DT_F8E4M3);
+    for (int i = 0; i < TURNS; ++i) {
+        const uint32_t r = r0 + i * ROWS;
+        if (r < p.rows && valid) store_piece<IN_DT>(p.q, (size_t)r * p.ldq + c, quant_piece<IN_DT, OUT_DT>(v[i], dv), valid);
+    }
 }
 
 }  // namespace qgemm

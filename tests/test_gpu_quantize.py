@@ -163,3 +163,47 @@ def test_division_by_the_scale_is_the_ieee_division():
         gi, gsi = Q.quantize(dev(part), torch.int8, Q.QUANT_PER_MATRIX)
         assert host(gsi).view(np.uint32)[0] == np.array([si], np.float32).view(np.uint32)[0]
         assert np.array_equal(host(gi), qi), (lo, hi)
+
+
+def _special_rows(rows, cols, seed):
+    """Rows that leave the plain way through the quantisers, each in a block of its own kind: NaNs of either sign beside
+    numbers, infinities, signed zeros, maxima far from 1 (scales beyond 2^+-60 for fp32), single values, subnormals."""
+    x = R.fill_normal((rows, cols), seed)
+    x[0, 1::3] = np.nan
+    x[1 % rows, 5] = -np.inf
+    x[2 % rows] = -0.0
+    x[3 % rows] *= np.float32(1e30)
+    x[4 % rows] *= np.float32(1e-30)
+    x[5 % rows] = 0.0
+    x[5 % rows, cols - 1] = -3.5
+    x[6 % rows, ::2] = np.copysign(np.float32(0), -x[6 % rows, ::2])
+    x[7 % rows] *= np.float32(1e-38)
+    x[8 % rows, 0] = -np.nan
+    return x
+
+
+@pytest.mark.parametrize("source", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("out", ["fp8", "int8"])
+@pytest.mark.parametrize("shape", [(9, 127), (12, 129), (11, 1001), (130, 384), (1100, 520)])
+def test_values_and_edges_bit_exact(shape, out, source):
+    """Every mode on special values, row ends at any element, sources at any address."""
+    say("quantize special values", shape, out, source)
+    x = _special_rows(*shape, seed=51)
+    tdt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[source]
+    with np.errstate(all="ignore"):
+        xt = torch.from_numpy(x).to(tdt)
+        xs = xt.float().numpy()
+        flat = torch.zeros(1 + shape[0] * (shape[1] + 3), dtype=tdt, device="cuda")
+        view = flat[1:].view(shape[0], shape[1] + 3)[:, :shape[1]]            # one element past a boundary, gaps between rows
+        view.copy_(xt)
+        q_dt = torch.float8_e4m3fn if out == "fp8" else torch.int8
+        for rows in (slice(None), slice(5, 7)):                              # (with and without NaNs and infinities per matrix)
+            qm, sm = (R.quantize_fp8 if out == "fp8" else R.quantize_int8)(xs[rows])
+            g, s = Q.quantize(view[rows], q_dt, Q.QUANT_PER_MATRIX)
+            assert np.array_equal(host(s).view(np.uint32), np.array([sm], np.float32).view(np.uint32))
+            assert np.array_equal(_u8(g), qm.view(np.uint8))
+        for mode, br in ((Q.QUANT_BLOCK_1x128, 1), (Q.QUANT_BLOCK_128x128, 128)):
+            qb, sb = (R.quantize_fp8_block if out == "fp8" else R.quantize_int8_block)(xs, br, 128)
+            g, s = Q.quantize(view, q_dt, mode)
+            assert np.array_equal(host(s), sb, equal_nan=True)
+            assert np.array_equal(_u8(g), qb.view(np.uint8))
