@@ -6,8 +6,11 @@
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
+#include <optional>
 #include <stdexcept>
 #include <string>
+#include <tuple>
 
 #include "../../include/qgemm.h"
 
@@ -97,6 +100,86 @@ void bf16_mm(torch::Tensor a, torch::Tensor b, torch::Tensor c) {
           "bf16_mm");
 }
 
+// ---- what qgemm_amd/ops.py calls: its functions with the reading of the tensors, the stream lookup and the call into the
+// library done here (1 x 2048 x 1024, quantise and multiply: 11.6 + 8.4 us of host time through Python and ctypes, 3 of each
+// in torch.cuda.current_stream(), for two kernels of 1.7 and 4.1 us; 4.3 + 3.6 here, most of it the launches).  They answer a status of the library, or kNotPlain, having
+// done nothing, for anything that is not the plain case; ops.py then takes its own way, which raises what there is to raise.
+constexpr int kNotPlain = -1;
+
+// the library's number of a tensor's type, -1 for none; raw_fp8: uint8 means e4m3 codes
+int plain_dtype(const at::Tensor &t, bool raw_fp8) {
+    switch (t.scalar_type()) {
+        case at::kFloat: return QGEMM_DT_F32;
+        case at::kBFloat16: return QGEMM_DT_BF16;
+        case at::kHalf: return QGEMM_DT_F16;
+        case at::kChar: return QGEMM_DT_I8;
+        case at::kInt: return QGEMM_DT_I32;
+        case at::kFloat8_e4m3fn: return QGEMM_DT_F8E4M3;
+        case at::kByte: return raw_fp8 ? QGEMM_DT_F8E4M3 : -1;
+        default: return -1;
+    }
+}
+
+typedef std::optional<int64_t> opt_int;
+
+int ops_gemm(const at::Tensor &A, const at::Tensor &B, const at::Tensor &C, bool kn, opt_int M, opt_int N, opt_int K,
+             opt_int ldA, opt_int ldB, opt_int ldC) {
+    if (!A.is_cuda() || !B.is_cuda() || !C.is_cuda() || A.dim() != 2 || B.dim() != 2 || C.dim() < 1) return kNotPlain;
+    const int in = plain_dtype(A, true), out = plain_dtype(C, false);
+    if (in < 0 || out < 0) return kNotPlain;
+    py::gil_scoped_release no_gil;
+    return qgemm_gemm(in, out, kn ? QGEMM_B_KN : QGEMM_B_NK, A.data_ptr(), ldA ? *ldA : A.stride(0), B.data_ptr(),
+                      ldB ? *ldB : B.stride(0), C.data_ptr(), ldC ? *ldC : C.stride(0), M ? *M : A.size(0),
+                      N ? *N : B.size(kn ? 1 : 0), K ? *K : A.size(1), current_stream());
+}
+
+int ops_scaled_gemm(const at::Tensor &A, const at::Tensor &B, const std::optional<at::Tensor> &a_scale,
+                    const std::optional<at::Tensor> &b_scale, const at::Tensor &C, int64_t M, int64_t N, int64_t K,
+                    int scale_mode, int layout, int split_k, std::optional<int> in_dtype, opt_int ldC) {
+    if (!A.is_cuda() || !B.is_cuda() || !C.is_cuda() || C.dim() < 1 || (a_scale && !a_scale->is_cuda()) ||
+        (b_scale && !b_scale->is_cuda()))
+        return kNotPlain;
+    const int in = in_dtype ? *in_dtype : plain_dtype(A, true), out = plain_dtype(C, false);
+    if (in < 0 || out < 0) return kNotPlain;
+    py::gil_scoped_release no_gil;
+    return qgemm_scaled_gemm(in, out, scale_mode, layout, A.data_ptr(), B.data_ptr(),
+                             a_scale ? (const float *)a_scale->data_ptr() : nullptr,
+                             b_scale ? (const float *)b_scale->data_ptr() : nullptr, C.data_ptr(), ldC ? *ldC : C.stride(0), M,
+                             N, K, split_k, current_stream());
+}
+
+int ops_transpose(const at::Tensor &in, const at::Tensor &out, opt_int M, opt_int N) {
+    if (!in.is_cuda() || !out.is_cuda() || (in.dim() < 2 && (!M || !N))) return kNotPlain;
+    py::gil_scoped_release no_gil;
+    return qgemm_transpose((int)in.element_size(), in.data_ptr(), out.data_ptr(), M ? *M : in.size(0), N ? *N : in.size(1),
+                           current_stream());
+}
+
+// (status, q, scales)
+std::tuple<int, at::Tensor, at::Tensor> ops_quantize(const at::Tensor &x, at::ScalarType out, int mode, bool rows_contiguous_scales) {
+    const std::tuple<int, at::Tensor, at::Tensor> not_plain{kNotPlain, at::Tensor(), at::Tensor()};
+    if (!x.is_cuda() || x.dim() != 2 || x.stride(1) != 1 || (out != at::kChar && out != at::kFloat8_e4m3fn)) return not_plain;
+    const int in = plain_dtype(x, false);
+    if (in < 0) return not_plain;
+    const int64_t rows = x.size(0), cols = x.size(1);
+    at::Tensor q = at::empty({rows, cols}, x.options().dtype(out)), scales;
+    const auto f32 = x.options().dtype(at::kFloat);
+    int64_t rs = 0, cs = 0;
+    if (mode == QGEMM_QUANT_PER_MATRIX) {
+        scales = at::empty({1}, f32);
+    } else {
+        const int64_t nbr = mode == QGEMM_QUANT_BLOCK_1x128 ? rows : (rows + 127) / 128, nbc = (cols + 127) / 128;
+        scales = rows_contiguous_scales ? at::empty({nbc, nbr}, f32) : at::empty({nbr, nbc}, f32);
+        rs = rows_contiguous_scales ? 1 : nbc;
+        cs = rows_contiguous_scales ? nbr : 1;
+    }
+    py::gil_scoped_release no_gil;
+    const int st = qgemm_quantize(in, out == at::kChar ? QGEMM_DT_I8 : QGEMM_DT_F8E4M3, mode, x.data_ptr(),
+                                  rows > 1 ? x.stride(0) : std::max<int64_t>(cols, 1), rows, cols, q.data_ptr(), cols,
+                                  (float *)scales.data_ptr(), rs, cs, current_stream());
+    return {st, q, scales};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -105,4 +188,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("fp8_mm_per_matrix", &fp8_mm_per_matrix, "per-matrix scaled fp8 GEMM, K-contiguous operands");
     m.def("int8_mm", &int8_mm, "per-matrix scaled int8 GEMM, K-contiguous operands");
     m.def("bf16_mm", &bf16_mm, "bf16 / fp16 GEMM, b stored [n, k]");
+    m.def("ops_gemm", &ops_gemm);
+    m.def("ops_scaled_gemm", &ops_scaled_gemm);
+    m.def("ops_transpose", &ops_transpose);
+    m.def("ops_quantize", &ops_quantize);
 }
