@@ -140,9 +140,6 @@ __global__ void __launch_bounds__(256) transpose_kernel(const T *__restrict__ in
     }
 }
 
-typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));       // 16 bytes at any address
-typedef unsigned u32_any __attribute__((aligned(1)));
-
 // ---------------------------------------------------------------------------
 // Byte transpose for shapes with M % 16 == 0, N % 4 == 0 and 16-byte aligned rows (the fp8 / int8
 // operands of the reference layout).  128 x 128 tile, 256 threads.  A thread loads 4 x 4 bytes (four
@@ -382,63 +379,47 @@ struct ReduceArgs {
     const float *as, *bs;
     uint32_t M, N, nsplit;
     uint64_t ldc, plane;   // plane = M*N elements
-    int part_is_i32, out_dtype, per_matrix_scale;
+    int out_dtype, per_matrix_scale;
 };
 
-__global__ void __launch_bounds__(256) splitk_reduce_kernel(const ReduceArgs p) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= p.plane) return;
-    const uint32_t m = (uint32_t)(i / p.N), n = (uint32_t)(i % p.N);
-    const size_t idx = (size_t)m * p.ldc + n;
-    if (p.part_is_i32) {
-        int acc = 0;
-        for (uint32_t z = 0; z < p.nsplit; ++z) acc += ((const int *)p.part)[z * p.plane + i];
-        if (p.out_dtype == QGEMM_DT_I32) {
-            ((int *)p.C)[idx] = acc;
-            return;
-        }
-        const float s = p.per_matrix_scale ? p.as[0] * p.bs[0] : 1.0f;
-        store_out(p.C, idx, (float)acc * s, p.out_dtype);
-        return;
-    }
-    float acc = 0.0f;
-    for (uint32_t z = 0; z < p.nsplit; ++z) acc += ((const float *)p.part)[z * p.plane + i];
-    const float s = p.per_matrix_scale ? p.as[0] * p.bs[0] : 1.0f;
-    store_out(p.C, idx, acc * s, p.out_dtype);
-}
-
-// The same for N a multiple of 4 (the planes are 256-byte aligned, so every group of four elements is 16 bytes,
-// aligned, inside one row): four elements per thread, the loads of up to eight planes in flight together, then the
-// sums in the order of the planes.  The launch is bound by latency, not by the 5 - 30 MB it reads: one element per
-// thread with a dependent chain of loads took 4.2 us for 160 x 2048 in four planes, 11 us for 512 x 4096.
-// c_vec: C and its rows allow a store of the four outputs at once (16 bytes, or 8 for the 2-byte types).
+// Four elements of a row per thread, at any alignment (the last group of a row may be shorter), the loads of up to eight
+// planes in flight together, then the sums in the order of the planes.  The launch is bound by latency, not by the
+// 5 - 30 MB it reads: one element per thread with a dependent chain of loads took 4.2 us for 160 x 2048 in four planes,
+// 11 us for 512 x 4096.
 template <bool IS_I32>
-__global__ void __launch_bounds__(256) splitk_reduce4_kernel(const ReduceArgs p, int c_vec) {
-    typedef int v4i_ __attribute__((ext_vector_type(4)));
-    typedef float v4f_ __attribute__((ext_vector_type(4)));
-    typedef typename std::conditional<IS_I32, v4i_, v4f_>::type vec_t;
-    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i >= p.plane) return;
-    const uint32_t m = (uint32_t)(i / p.N), n = (uint32_t)(i % p.N);
+__global__ void __launch_bounds__(256) splitk_reduce4_kernel(const ReduceArgs p) {
+    typedef typename std::conditional<IS_I32, v4i, v4f>::type vec_t;
+    typedef typename std::conditional<IS_I32, v4i_any, v4f_any>::type vec_any;
+    typedef typename std::conditional<IS_I32, int, float>::type elem_t;
+    const uint32_t per_row = (p.N + 3) / 4;
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (size_t)p.M * per_row) return;
+    const uint32_t m = (uint32_t)(i / per_row), n = (uint32_t)(i % per_row) * 4;
+    const int valid = p.N - n < 4 ? (int)(p.N - n) : 4;
     const size_t idx = (size_t)m * p.ldc + n;
-    const vec_t *src = (const vec_t *)((const char *)p.part + i * 4);
-    const size_t plane_vecs = p.plane / 4;
+    const elem_t *src = (const elem_t *)p.part + (size_t)m * p.N + n;
     vec_t acc = vec_t{0, 0, 0, 0};
-    for (uint32_t z0 = 0; z0 < p.nsplit; z0 += 8) {
-        vec_t t[8];
+    if (valid == 4) {
+        for (uint32_t z0 = 0; z0 < p.nsplit; z0 += 8) {
+            vec_t t[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            if (z0 + j < p.nsplit) t[j] = __builtin_nontemporal_load(src + (size_t)(z0 + j) * plane_vecs);
+            for (int j = 0; j < 8; ++j)
+                if (z0 + j < p.nsplit) t[j] = __builtin_nontemporal_load((const vec_any *)(src + (size_t)(z0 + j) * p.plane));
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            if (z0 + j < p.nsplit) acc += t[j];
+            for (int j = 0; j < 8; ++j)
+                if (z0 + j < p.nsplit) acc += t[j];
+        }
+    } else {
+        for (uint32_t z = 0; z < p.nsplit; ++z)
+            for (int e = 0; e < 3; ++e)
+                if (e < valid) acc[e] += src[z * p.plane + e];
     }
     if constexpr (IS_I32) {
         if (p.out_dtype == QGEMM_DT_I32) {
             int *dst = (int *)p.C + idx;
-            if (c_vec) *(v4i_ *)dst = acc;
+            if (valid == 4) *(v4i_any *)dst = acc;
             else
-                for (int e = 0; e < 4; ++e) dst[e] = acc[e];
+                for (int e = 0; e < valid; ++e) dst[e] = acc[e];
             return;
         }
     }
@@ -446,18 +427,7 @@ __global__ void __launch_bounds__(256) splitk_reduce4_kernel(const ReduceArgs p,
     float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = (float)acc[e] * s;
-    if (p.out_dtype == QGEMM_DT_F32) {
-        float *dst = (float *)p.C + idx;
-        if (c_vec) *(v4f_ *)dst = v4f_{v[0], v[1], v[2], v[3]};
-        else
-            for (int e = 0; e < 4; ++e) dst[e] = v[e];
-    } else {
-        const v2i h = p.out_dtype == QGEMM_DT_BF16 ? pack4_bf16(v[0], v[1], v[2], v[3]) : pack4_f16(v[0], v[1], v[2], v[3]);
-        unsigned short *dst = (unsigned short *)p.C + idx;
-        if (c_vec) *(v2i *)dst = h;
-        else
-            for (int e = 0; e < 4; ++e) dst[e] = pack4_elem(h, e);
-    }
+    store_out4(p.C, idx, v, p.out_dtype, valid);
 }
 
 }  // namespace qgemm

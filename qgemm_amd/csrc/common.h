@@ -14,6 +14,11 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef unsigned short us4 __attribute__((ext_vector_type(4)));
+// loads and stores of several elements at any address of one: the vector memory path takes any byte address
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef int v2i_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef unsigned u32_any __attribute__((aligned(1)));
 
 // Arithmetic families of the MFMA kernels.
 enum Arith : int { AR_I8 = 0, AR_F8 = 1, AR_BF16 = 2, AR_F16 = 3 };
@@ -60,6 +65,24 @@ __device__ inline v2i pack4_f16(float a, float b, float c, float d) {
 }
 // element e (0 .. 3) of such a pack
 __device__ inline unsigned short pack4_elem(v2i p, int e) { return (unsigned short)((unsigned)p[e >> 1] >> ((e & 1) * 16)); }
+
+// Four neighbouring elements of a row of C, the first `valid` of them inside it, at any element address
+__device__ inline void store_out4(void *C, size_t idx, const float *v, int out_dtype, int valid) {
+    if (out_dtype == QGEMM_DT_F32) {
+        float *dst = (float *)C + idx;
+        if (valid >= 4) *(v4f_any *)dst = v4f{v[0], v[1], v[2], v[3]};
+        else
+            for (int e = 0; e < 3; ++e)
+                if (e < valid) dst[e] = v[e];
+        return;
+    }
+    const v2i h = out_dtype == QGEMM_DT_BF16 ? pack4_bf16(v[0], v[1], v[2], v[3]) : pack4_f16(v[0], v[1], v[2], v[3]);
+    unsigned short *dst = (unsigned short *)C + idx;
+    if (valid >= 4) *(v2i_any *)dst = h;
+    else
+        for (int e = 0; e < 3; ++e)
+            if (e < valid) dst[e] = pack4_elem(h, e);
+}
 
 // Linear workgroup id -> (tile_m, tile_n).
 // Step 1 (XCD remap): the dispatcher deals workgroups to the 8 XCDs round

@@ -68,7 +68,6 @@ struct GemmArgs {
                           // every K slice and k_rot a multiple of four steps: the scales travel four K blocks at a time
     int out_dtype;        // qgemm_dtype_t of C
     int per_matrix_scale; // multiply by as[0]*bs[0] in the epilogue
-    int vec_store;        // 0: scalar stores; 1: C and ldc allow 4-element vector stores; 2: also 16-byte row pieces
     int c_plain;          // ordinary instead of non-temporal stores for C (run_nt: launches of at most one round of tiles)
     int b_stream;         // B is read once by the launch (one or two row tiles): its copies carry the streaming hint
     uint32_t k_rot;                  // simple pipeline and skinny-M kernel: the workgroups of column tile i start their K loops (i * k_rot) % nk steps in (0: at 0)
@@ -1306,8 +1305,7 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
     if (p.per_matrix_scale) scale = p.as[0] * p.bs[0];
     char *Cz = p.C + (size_t)z * p.split_stride * dtype_bytes(p.out_dtype);
 
-    // Fast path: the wave tile lies inside C and rows of C are 16-byte aligned.  The accumulator
-    // layout (adjacent lanes = adjacent rows of C) would make every lane of a store its own
+    // The accumulator layout (adjacent lanes = adjacent rows of C) would make every lane of a store its own
     // request; so each 16-row slab goes through this wave's private LDS scratch and leaves as
     // whole 16-byte-per-lane row pieces.  Two scratch slabs per wave: slab a+1 is converted and
     // written while slab a is read back and stored.  The output type is dispatched once, outside
@@ -1344,11 +1342,10 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
     const bool wave_cols_full = col0 + wn * C::WN + C::WN <= p.N;
     const int wave_rows = (int)p.M - (int)(row0 + wm * C::WM);
     // Every accumulator is read in exactly one place (write_slab): the output type is a uniform branch around
-    // the conversion of a slab, and wave tiles that stick out of C sideways or meet unaligned rows take the same way
-    // through the scratch and differ only in how a slab leaves it (element by element, bounds checked).  A wave tile
-    // that sticks out below C (M is whatever the caller's batch is; N and the alignment come with the weights)
-    // keeps the 16-byte stores and leaves out the rows past M; so does one that sticks out sideways when the rows of C
-    // end on a 16-byte boundary (its lanes past N leave their pieces out).
+    // the conversion of a slab, and wave tiles that stick out of C take the same way through the scratch.  The 16-byte
+    // pieces go to any element address (rows of C that are not 16-byte aligned used to leave element by element:
+    // 1531 x 4100 x 3004 int8 to bf16, rows of 8200 bytes, 31.7 -> 23.2 us; 1999 x 3001 x 1000 bf16 28.8 -> 20.7); rows
+    // past M and pieces past N are left out, and the one piece N ends in goes element by element.
     // With the accumulators of a 128 x 128 wave tile pinned in the 256 accumulation registers, several code
     // paths that each name all of them made the register allocator spill two dozen of them to memory here.
     if constexpr (EPI_FITS) {
@@ -1370,9 +1367,11 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
         const int wr_off = (lane & 15) * PITCH + (lane >> 4) * 4 * ES;
         const size_t c_row_bytes = (size_t)p.ldc * ES;
         const uint32_t wrow0 = row0 + wm * C::WM, wcol0 = col0 + wn * C::WN;
-        // 16-byte stores: C and its rows aligned, and every 16-byte piece of a row either inside C or outside
-        const bool fast = p.vec_store == 2 && (wave_cols_full || ((size_t)p.N * ES) % 16 == 0);
-        const bool lane_in_cols = rd_col < ((int)p.N - (int)wcol0) * ES;
+        // What this wave writes of a row: 16-byte pieces at any element address, and, where the row of C ends inside a
+        // piece, the elements of that one piece one by one (16 lanes, a row each)
+        const int wave_cols = wave_cols_full ? C::WN : (wcol0 < p.N ? (int)(p.N - wcol0) : 0);
+        const int whole = wave_cols * ES / 16 * 16, rest = __builtin_amdgcn_readfirstlane(wave_cols - whole / ES);
+        const bool lane_in_cols = rd_col < whole, wave_tile_full = wave_cols_full && wave_rows >= C::WM;
         char *cwave = Cz + ((size_t)wrow0 * p.ldc + wcol0) * ES;
         // Accumulators pinned in the accumulation registers (4-wave solo pipeline) are fetched from there one
         // slab at a time; left to itself the compiler moves all 256 of them into vector registers first.
@@ -1422,32 +1421,35 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
 #pragma unroll
         for (int a = 0; a < C::TM; ++a) {
             const char *slab = scratch + (a & 1) * EPI_BYTES;
-            if (fast) {
-                // read slab a back first (its writes were issued a turn ago; the LDS works in order), convert and
-                // write slab a+1 while those reads are in flight, then store
-                const char *rd = slab + rd_row * PITCH + rd_col;
-                v4i v[PASSES];
+            // read slab a back first (its writes were issued a turn ago; the LDS works in order), convert and
+            // write slab a+1 while those reads are in flight, then store
+            const char *rd = slab + rd_row * PITCH + rd_col;
+            v4i v[PASSES];
 #pragma unroll
-                for (int ps = 0; ps < PASSES; ++ps) v[ps] = *(const v4i *)(rd + ps * RPP * PITCH);
-                if (a + 1 < C::TM) write_slab(a + 1);
+            for (int ps = 0; ps < PASSES; ++ps) v[ps] = *(const v4i *)(rd + ps * RPP * PITCH);
+            if (a + 1 < C::TM) write_slab(a + 1);
+            auto store_piece = [&](int ps) {
+                v4i_any *dst = (v4i_any *)(cwave + rd_col + (size_t)(a * 16 + rd_row + ps * RPP) * c_row_bytes);
+                if constexpr (NT_STORE) __builtin_nontemporal_store(v[ps], dst);
+                else *dst = v[ps];
+            };
+            if (wave_tile_full) {
 #pragma unroll
-                for (int ps = 0; ps < PASSES; ++ps)
-                    if (lane_in_cols && a * 16 + rd_row + ps * RPP < wave_rows) {
-                        v4i *dst = (v4i *)(cwave + rd_col + (size_t)(a * 16 + rd_row + ps * RPP) * c_row_bytes);
-                        if constexpr (NT_STORE) __builtin_nontemporal_store(v[ps], dst);
-                        else *dst = v[ps];
+                for (int ps = 0; ps < PASSES; ++ps) store_piece(ps);
+                continue;
+            }
+#pragma unroll
+            for (int ps = 0; ps < PASSES; ++ps)
+                if (lane_in_cols && a * 16 + rd_row + ps * RPP < wave_rows) store_piece(ps);
+            if (rest != 0) {
+                if (lane < 16 && a * 16 + lane < wave_rows) {
+                    char *dst = cwave + (size_t)(a * 16 + lane) * c_row_bytes + whole;
+                    const char *src = slab + lane * PITCH + whole;
+#pragma clang loop unroll(disable) vectorize(disable)
+                    for (int e = 0; e < rest; ++e) {
+                        if (ES == 2) ((volatile unsigned short *)dst)[e] = ((const unsigned short *)src)[e];
+                        else ((volatile uint32_t *)dst)[e] = ((const uint32_t *)src)[e];
                     }
-            } else {
-                if (a + 1 < C::TM) write_slab(a + 1);
-                // any alignment, any overhang: one element per lane and turn
-                for (int e = lane; e < 16 * C::WN; e += 64) {
-                    const int r = e / C::WN, cidx = e % C::WN;
-                    const uint32_t m = wrow0 + a * 16 + r, n = wcol0 + cidx;
-                    if (m >= p.M || n >= p.N) continue;
-                    char *dst = cwave + (size_t)(a * 16 + r) * c_row_bytes + (size_t)cidx * ES;
-                    const char *src = slab + r * PITCH + cidx * ES;
-                    if (ES == 2) *(unsigned short *)dst = *(const unsigned short *)src;
-                    else *(uint32_t *)dst = *(const uint32_t *)src;
                 }
             }
         }
@@ -1476,34 +1478,21 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
             const uint32_t n = col0 + wn * C::WN + b * 16 + (lane >> 4) * 4;
             if (n >= p.N) continue;
             const size_t idx = (size_t)m * p.ldc + n;
-            const bool full = p.vec_store && n + 3 < p.N;
+            const int valid = p.N - n < 4 ? (int)(p.N - n) : 4;
             if constexpr (C::ARITH == AR_I8 && !C::BLOCK_SCALE) {
                 if (p.out_dtype == QGEMM_DT_I32) {
                     int *dst = (int *)Cz + idx;
-                    if (full) *(v4i *)dst = acc[a][b];
+                    if (valid == 4) *(v4i_any *)dst = acc[a][b];
                     else
-                        for (int r = 0; r < 4; ++r)
-                            if (n + r < p.N) dst[r] = acc[a][b][r];
+                        for (int r = 0; r < 3; ++r)
+                            if (r < valid) dst[r] = acc[a][b][r];
                     continue;
                 }
             }
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = (float)acc[a][b][r] * scale;
-            if (p.out_dtype == QGEMM_DT_F32) {
-                float *dst = (float *)Cz + idx;
-                if (full) *(v4f *)dst = v4f{v[0], v[1], v[2], v[3]};
-                else
-                    for (int r = 0; r < 4; ++r)
-                        if (n + r < p.N) dst[r] = v[r];
-            } else {
-                const v2i h = p.out_dtype == QGEMM_DT_BF16 ? pack4_bf16(v[0], v[1], v[2], v[3]) : pack4_f16(v[0], v[1], v[2], v[3]);
-                unsigned short *dst = (unsigned short *)Cz + idx;
-                if (full) *(v2i *)dst = h;
-                else
-                    for (int r = 0; r < 4; ++r)
-                        if (n + r < p.N) dst[r] = pack4_elem(h, r);
-            }
+            store_out4(Cz, idx, v, p.out_dtype, valid);
         }
     }
     QGEMM_STAMP(3);

@@ -384,34 +384,21 @@ __global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs 
         const uint32_t n = col0 + b * 16 + (lane >> 4) * 4;
         if (m >= p.M || n >= p.N) continue;
         const size_t idx = (size_t)m * p.ldc + n;
-        const bool full = p.vec_store && n + 3 < p.N;
+        const int valid = p.N - n < 4 ? (int)(p.N - n) : 4;
         if constexpr (C::ARITH == AR_I8 && !C::BLOCK_SCALE) {
             if (p.out_dtype == QGEMM_DT_I32) {
                 int *dst = (int *)Cz + idx;
-                if (full) *(v4i *)dst = s;
+                if (valid == 4) *(v4i_any *)dst = s;
                 else
-                    for (int r = 0; r < 4; ++r)
-                        if (n + r < p.N) dst[r] = s[r];
+                    for (int r = 0; r < 3; ++r)
+                        if (r < valid) dst[r] = s[r];
                 continue;
             }
         }
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = (float)s[r] * scale;
-        if (p.out_dtype == QGEMM_DT_F32) {
-            float *dst = (float *)Cz + idx;
-            if (full) *(v4f *)dst = v4f{v[0], v[1], v[2], v[3]};
-            else
-                for (int r = 0; r < 4; ++r)
-                    if (n + r < p.N) dst[r] = v[r];
-        } else {
-            const v2i h = p.out_dtype == QGEMM_DT_BF16 ? pack4_bf16(v[0], v[1], v[2], v[3]) : pack4_f16(v[0], v[1], v[2], v[3]);
-            unsigned short *dst = (unsigned short *)Cz + idx;
-            if (full) *(v2i *)dst = h;
-            else
-                for (int r = 0; r < 4; ++r)
-                    if (n + r < p.N) dst[r] = pack4_elem(h, r);
-        }
+        store_out4(Cz, idx, v, p.out_dtype, valid);
     }
     QGEMM_STAMP(5);
     QGEMM_STAMP_WRITE(p.dbg_cycles, blockIdx.x * C::NW + wave, 6, lane == 0);

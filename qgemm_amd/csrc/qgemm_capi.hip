@@ -830,9 +830,6 @@ int run_nt(const NtProblem &q, Plan &pl, void *split_ws, hipStream_t stream) {
         a.out_dtype = q.out_dtype;
         a.per_matrix_scale = q.per_matrix;
         const int ob = dtype_bytes(q.out_dtype);
-        const int vec = ob == 4 ? 16 : 8;
-        a.vec_store = ((uintptr_t)q.C % vec == 0) && ((q.ldc * ob) % vec == 0);
-        if (a.vec_store && (uintptr_t)q.C % 16 == 0 && (q.ldc * ob) % 16 == 0) a.vec_store = 2;
         // 4-byte C over at least three rounds of 256 x 256 tiles: spread the write bursts (see gemm_nt_kernel)
         // (with fewer than 32 K steps the offsets are too large a part of a tile's time: 7000 x 7168 x 2048 int8 to
         // f32 128 us without, 139 us with)
@@ -859,7 +856,6 @@ int run_nt(const NtProblem &q, Plan &pl, void *split_ws, hipStream_t stream) {
     a.split_stride = plane;
     a.out_dtype = i32_acc ? QGEMM_DT_I32 : QGEMM_DT_F32;
     a.per_matrix_scale = 0;
-    a.vec_store = (q.N % 4 == 0) ? 2 : 0;   // workspace planes are 256-byte aligned, 4-byte elements
     hipError_t e = v.launch(a, (uint32_t)(pl.tiles * a.nsplit), stream);
     if (e != hipSuccess) return QGEMM_ERR_LAUNCH;
 
@@ -874,18 +870,10 @@ int run_nt(const NtProblem &q, Plan &pl, void *split_ws, hipStream_t stream) {
     r.nsplit = a.nsplit;
     r.ldc = q.ldc;
     r.plane = plane;
-    r.part_is_i32 = i32_acc;
     r.out_dtype = q.out_dtype;
     r.per_matrix_scale = q.per_matrix;
-    if (q.N % 4 == 0) {
-        const int ob = dtype_bytes(q.out_dtype), c_align = ob == 4 ? 16 : 8;
-        const int c_vec = (uintptr_t)q.C % c_align == 0 && (q.ldc * ob) % c_align == 0;
-        const dim3 grid((unsigned)((plane / 4 + 255) / 256));
-        if (i32_acc) hipLaunchKernelGGL(splitk_reduce4_kernel<true>, grid, dim3(256), 0, stream, r, c_vec);
-        else hipLaunchKernelGGL(splitk_reduce4_kernel<false>, grid, dim3(256), 0, stream, r, c_vec);
-    } else {
-        hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((plane + 255) / 256)), dim3(256), 0, stream, r);
-    }
+    const dim3 grid((unsigned)((q.M * ((q.N + 3) / 4) + 255) / 256));
+    hipLaunchKernelGGL(i32_acc ? splitk_reduce4_kernel<true> : splitk_reduce4_kernel<false>, grid, dim3(256), 0, stream, r);
     g_ctx.last_config = std::string(v.name) + kmaj_suffix(q.kmaj) + "_splitk" + std::to_string(a.nsplit);
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }

@@ -18,7 +18,6 @@
 // A decoder's 16 x 2048 stays at 2.8: one trip to memory and back.
 #pragma once
 #include "common.h"
-#include "aux_kernels.cuh"
 
 namespace qgemm {
 
@@ -182,7 +181,6 @@ __device__ inline v2i quant_piece(v4i r, const Divisor &dv) {
 
 template <int IN_DT>
 __device__ inline void store_piece(void *q, size_t idx, v2i w, uint32_t valid) {
-    typedef int v2i_any __attribute__((ext_vector_type(2), aligned(1)));
     uint8_t *p = (uint8_t *)q + idx;
     if (valid >= (uint32_t)Piece<IN_DT>::VEC) {
         if constexpr (Piece<IN_DT>::VEC == 8) *(v2i_any *)p = w;
