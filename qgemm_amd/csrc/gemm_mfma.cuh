@@ -64,8 +64,8 @@ struct GemmArgs {
     uint64_t split_stride;
     uint32_t as_ms, as_ks, bs_ns, bs_ks;
     uint32_t nb_max;      // ceil(N/128) - 1
-    uint32_t as_groups;   // rows with two K groups, block scales: a_scale is K-contiguous (as_ks == 1), 16-byte aligned rows,
-                          // every K slice and k_rot a multiple of four steps: the scales travel four K blocks at a time
+    uint32_t as_groups;   // rows with two K groups, block scales: a_scale is K-contiguous (as_ks == 1) and k_rot, where it is not
+                          // zero, as well as every K slice a multiple of four steps: the scales travel four K blocks at a time
     int out_dtype;        // qgemm_dtype_t of C
     int per_matrix_scale; // multiply by as[0]*bs[0] in the epilogue
     int c_plain;          // ordinary instead of non-temporal stores for C (run_nt: launches of at most one round of tiles)
@@ -629,8 +629,7 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
             // Copying waves and K-contiguous a_scale (the twin `_ks` of the row with copying waves): the computing waves
             // fetch no scales themselves.  A copying wave brings the scales of four K blocks of 64 tile rows in one
             // 16-byte-per-lane copy, in front of the A copies of every fourth step, into slot (kt / 4) % 4 of four
-            // behind the operand buffers ([row][4 K blocks]; the host picks this twin only where rows and K slices
-            // start at multiples of four blocks), and a computing wave reads the eight values of its lane for the
+            // behind the operand buffers ([row][4 K blocks]; rows may start at any 4-byte address), and a computing wave reads the eight values of its lane for the
             // next step where the other kernels distribute what they fetched.  That takes the last memory instruction
             // but the b_scale load out of the computing waves, the lane swaps with it, and a row of a_scale costs
             // the fill path one request per four steps instead of one per two from each of the waves that share it.

@@ -813,12 +813,18 @@ int run_nt(const NtProblem &q, Plan &pl, void *split_ws, hipStream_t stream) {
     a.bs_ks = q.bs_ks;
     a.as_groups = 0;
     if (q.block && v.kgroups == 2 && g_ctx.as_groups) {
-        // K-contiguous a_scale on the rows with two K groups: four K blocks of a row per copy (GemmArgs::as_groups) where
-        // rows and K slices start at multiples of four blocks; the rotated start then moves by four steps a column tile
+        // K-contiguous a_scale on the rows with two K groups: four K blocks of a row per copy (GemmArgs::as_groups), at any
+        // 4-byte address (what a row's last group brings beyond the row nobody uses, past the end of the array it is
+        // zeros: probed by qgemm_selftest_layouts).  A rotated start has to move, and to wrap round, by whole groups: it
+        // moves by four steps a column tile where the slices are multiples of four, and is left out where they are
+        // not (rows of B an odd number of K blocks apart do not ask the same memory channels anyway).  One K block per copy
+        // against four, us, B streamed / resident: 500 x 4608 x 7200 53.2 / 41.7 -> 48.0 / 35.7, 512 x 4096 x 4224
+        // 24.2 / 18.0 -> 20.3 / 15.9; up to 256 rows, with the rotation given up for it: 256 x 4608 x 7200 46.2 / 32.8 ->
+        // 40.4 / 27.6, 160 x 7168 x 7200 42.5 / 30.0 -> 39.8 / 25.8, 256 x 7168 x 2176 14.3 / 10.4 -> 12.8 / 10.0.
         const bool slices4 = a.ksteps % 4 == 0 && (a.nsplit == 1 || a.ksteps_per_split % 4 == 0);
-        const bool rows16 = q.as_ks == 1 && q.as_ms % 4 == 0 && ((uintptr_t)q.as & 15u) == 0;
-        if (slices4 && rows16 && g_ctx.k_rot < 0 && a.k_rot) a.k_rot = 4;
-        a.as_groups = slices4 && rows16 && a.k_rot % 4 == 0;
+        const bool k_contiguous = q.as_ks == 1 && ((uintptr_t)q.as & 3u) == 0;
+        if (k_contiguous && g_ctx.k_rot < 0 && a.k_rot) a.k_rot = slices4 ? 4 : 0;
+        a.as_groups = k_contiguous && (a.k_rot == 0 || (slices4 && a.k_rot % 4 == 0));
     }
 #if QGEMM_DEBUG_BUILD
     a.dbg_cycles = (unsigned long long *)g_ctx.dbg_ptr;
@@ -906,8 +912,9 @@ bool settle_scale_layout(const NtProblem &q, Plan &pl) {
     }
     // some other arrangement (K-contiguous, as QGEMM_LAYOUT_K_CONTIGUOUS passes it): fine where every launch of the
     // plan either takes any strides (simple pipeline, skinny-M kernel) or has a twin for it
-    // (a twin fetches the scales of Variant::ks_blocks K blocks of a row per load, two or four: rows aligned to that
-    // many floats, K and every K slice a multiple of that many blocks)
+    // (a twin fetches the scales of Variant::ks_blocks K blocks of a row per load, two or four.  The one that fetches four
+    // used to ask for rows and slices that are whole groups and took a transposed copy of a_scale otherwise: 2048 x 4096 x
+    // 7200, 57 blocks, 66.4 -> 62.7 us, 1536 x 4096 x 4736 39.7 -> 32.3)
     bool as_is = true;
     for (const Plan *p = &pl; as_is && p; p = p->rest.get()) {
         if (p->v->a_scale_any_stride) continue;
@@ -916,14 +923,13 @@ bool settle_scale_layout(const NtProblem &q, Plan &pl) {
             as_is = false;
             break;
         }
+        // (any row length and any slice: loads of 8 bytes and LDS copies of 16 need 4-byte alignment only, what the load of
+        // a row's last blocks brings beyond the row nobody uses, and at the end of the array the range check, which is
+        // per dword, returns zeros for it: probed by qgemm_selftest_layouts.  A row pinned by name whose twin copies
+        // four blocks through LDS takes its twin only where rows and slices are whole groups of them, as its users know it.)
         const uint32_t g = (uint32_t)twin->ks_blocks;
-        // (two K blocks per load, into registers: any row length and any slice.  An 8-byte buffer load needs 4-byte
-        // alignment only, the pair that starts with a row's last block ends with the next row's first, which nobody
-        // uses, and at the end of the array the range check, which is per dword, returns zero for it: probed by
-        // qgemm_selftest_layouts.  Four blocks per copy go through LDS and keep their alignment rules.)
-        as_is = g == 2 ? ((uintptr_t)q.as % 4) == 0
-                       : (g > 0 && q.as_ms % g == 0 && ((uintptr_t)q.as % (4 * g)) == 0 && p->a.ksteps % g == 0 &&
-                          !(p->a.nsplit > 1 && p->a.ksteps_per_split % g != 0));
+        as_is = ((uintptr_t)q.as % 4) == 0 &&
+                !(forced() && g == 4 && (q.as_ms % g != 0 || p->a.ksteps % g != 0 || (p->a.nsplit > 1 && p->a.ksteps_per_split % g != 0)));
     }
     for (Plan *p = &pl; p; p = p->rest.get()) {
         if (p->v->a_scale_any_stride) continue;
@@ -1765,6 +1771,24 @@ QGEMM_EXPORT int qgemm_selftest_layouts(char *buf, size_t buflen) {
             rep += line;
             if (bad) all_ok = false;
         }
+        // 16-byte copies at 4-byte aligned offsets, the last ones across the end of the range: a_scale travels that way,
+        // four K blocks of a row per lane, whatever the number of K blocks in a row
+        for (int l = 0; l < 64; ++l) hoff[l] = (uint32_t)(l < 56 ? 4 * (7 * l % 1000) : nsrc - 4 * (l - 55));
+        HIP_TRY(hipMemcpy(doff, hoff.data(), 256, hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(probe_lds_dma_kernel, dim3(1), dim3(64), 160 * 1024, 0, (const char *)dsrc, (const uint32_t *)doff,
+                           (uint32_t)nsrc, 0u, 0u, (char *)dout);
+        HIP_TRY(hipGetLastError());
+        std::vector<uint8_t> hout(1024);
+        HIP_TRY(hipMemcpy(hout.data(), dout, 1024, hipMemcpyDeviceToHost));
+        int bad = 0;
+        for (int l = 0; l < 64; ++l)
+            for (int j = 0; j < 16; ++j) {
+                const uint32_t off = hoff[l] + j;
+                bad += hout[l * 16 + j] != (off < (uint32_t)nsrc ? hsrc[off] : 0);
+            }
+        std::snprintf(line, sizeof(line), "lds_dma at 4-byte alignment and across the end of the range: mismatched_bytes=%d\n", bad);
+        rep += line;
+        if (bad) all_ok = false;
         (void)hipFree(dsrc);
         (void)hipFree(doff);
         (void)hipFree(dout);

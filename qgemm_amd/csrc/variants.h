@@ -20,9 +20,8 @@ struct Variant {
                                  // it (the others want it rows-contiguous, a_scale[m + kb * ld], or take any strides)
     bool a_scale_any_stride;     // block scales: the kernel reads a_scale[m * ms + kb * ks] for any ms, ks
     // Pair of rows that differ only in the arrangement of a_scale they read (GemmCfg::ASK): index, in the same table,
-    // of the other row of the pair (-1: none), and how many K blocks the K-contiguous one fetches per load (2 or 4:
-    // the caller's a_scale rows, K and every K slice have to be multiples of that many blocks, and rows aligned to
-    // as many floats).
+    // of the other row of the pair (-1: none), and how many K blocks the K-contiguous one fetches per load (2 or 4; any
+    // number of blocks per row and per slice, see settle_scale_layout).
     int twin;
     int ks_blocks;
     hipError_t (*launch)(const GemmArgs &, uint32_t grid, hipStream_t);
