@@ -134,3 +134,24 @@ def test_transpose(shape, dtype):
         Q.matrix_transpose(src, dst)
         assert torch.equal(dst, x.t())
         assert bool((guard[:off] == 99).all()) and bool((guard[off + x.numel():] == 99).all())
+
+
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float16, torch.float32, torch.int32])
+@pytest.mark.parametrize("row", ["256x256_w2x2_solo", "256x256_w2x4_solo8", "256x128_w2x2_cw", "128x128_w2x2_k2", "64x128_w1x4_k2", "128x128_w2x2_dma"])
+def test_rows_of_c_that_end_inside_a_piece(row, out):
+    """The last 16-byte piece of a row of C holds 1 .. 7 elements (1 .. 3 of four bytes): the same numbers, and nothing written
+    beside them.  Small integers: exact in every output type."""
+    M, K = 77, 128
+    Q.force_config(row)
+    try:
+        for N in list(range(257, 265)) + [1, 5, 7]:
+            say("ends of rows", row, out, N)
+            rng = np.random.default_rng(N)
+            a, b = rng.integers(-2, 3, size=(M, K)).astype(np.int8), rng.integers(-1, 2, size=(N, K)).astype(np.int8)
+            c = torch.full((M, N + 9), 7, dtype=out, device="cuda")
+            Q.scaled_gemm(dev(a), dev(b), scalar(1), scalar(1), c[:, :N], M, N, K, Q.SCALE_PER_MATRIX)
+            assert Q.last_config().startswith(row), Q.last_config()
+            assert np.array_equal(c[:, :N].float().cpu().numpy(), R.gemm_i8_i32(a, b).astype(np.float32)), N
+            assert bool((c[:, N:] == 7).all()), N
+    finally:
+        Q.force_config(None)
