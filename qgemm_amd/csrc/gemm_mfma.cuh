@@ -1030,6 +1030,25 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
             // [row][4 K blocks].  Slot i is refilled for stage 4 i + 16, issued in phase 4 i + 17 - NS, after the last
             // read of stage 4 i + 3.  These copies are not counted: a wave that waits until (NS - 2) * NPC copies are
             // left in flight has then waited for one or two operand copies more than it had to.
+            // Rows that are not 128-byte aligned (K bytes not a multiple of 128, or an operand inside a larger buffer): a
+            // K step of a row then lies in two cache lines, every copy asks for both, and the copies, which bound these
+            // tiles, take twice their time (500 x 4608 fp8 with block scales: K = 7168 26.9 us, K = 7200 35.5).  So each
+            // copy fetches one whole line of each row instead: the chunks of a step that lie in the row's second line
+            // travel with the stage behind it (`late` lanes: stage t brings them of step t - 1), the first stage
+            // brings chunks of the last step that nobody reads, and one stage more ends the loop.  A chunk keeps its slot,
+            // only its stage changes, so the fragment reads stay free of bank conflicts; they choose the stage per
+            // lane (the line offset of a row depends on row & 7 alone, as 8 rows are a multiple of 128 bytes).
+            // Phase s needs stages s and s+1, so one stage fewer is in flight.  Old / new, us, one process, in turn: fp8
+            // 500 x 4608 x 7200 33.6 / 24.3 (K = 7168: 24.0), 750 x 4096 x 4112 22.1 / 16.5, 256 x 4608 x 7200 26.8 / 19.1,
+            // bf16 500 x 4608 x 2056 22.2 / 16.7, 130 x 8192 x 3600 24.4 / 19.4; level at 17 steps.  With block scales the
+            // 128 x 128 tile has four stages and two left in flight are fewer than short loops need: 500 x 4608 x 7200
+            // 35.5 / 30.4, x 4112 (33 steps) 23.2 / 19.8, but x 3088 (25 steps) 15.4 / 16.1, so from 32 steps on.  The 64 x 128
+            // tile with block scales, bound by its fold, gained 4 - 12 % from 57 steps on and lost 2 - 4 % on
+            // aligned rows to the longer code, so it keeps its copies as they are.
+            const uint32_t line_a = (uint32_t)((uintptr_t)p.A >> 4) + (lane >> 3) * (p.lda >> 4);    // for row & 7 == lane >> 3
+            const uint32_t line_b = (uint32_t)((uintptr_t)p.B >> 4) + (lane >> 3) * (p.ldb >> 4);
+            constexpr bool LATE_FORM = C::KMAJ == 0 && (!C::BLOCK_SCALE || C::BM >= 128);
+            const bool late = LATE_FORM && nk >= (C::BLOCK_SCALE ? 32 : 1) && (((uint32_t)(uintptr_t)p.A | (uint32_t)(uintptr_t)p.B | p.lda | p.ldb) & 127u) != 0;
             constexpr int NPC = C::NLOAD / C::NPROD;                        // operand copies per stage and copying wave
             constexpr int CPS = NPC + (C::BLOCK_SCALE ? 1 : 0);
             static_assert(C::NPROD == 4 && C::NLOAD % 4 == 0 && C::RBA % 2 == 0 && (NS - 2) * CPS <= 63,
@@ -1046,19 +1065,36 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
                     if (kmajor) return (k * C::KE + (blk % BPP) * 16) * ld + (blk / BPP) * 128;
                     return blk * 16 * ld + k * C::BKB;
                 };
-                auto issue_stage_k2 = [&](int kt, auto nt_tag) {          // (nt_tag: B's copies with the streaming hint)
-                    constexpr bool B_NT = decltype(nt_tag)::value;
+                // `late` rows: per-lane offsets of a stage that opens a turn through K (step 0, and the late chunks of
+                // step nk - 1), of one in the middle (its scalar offset stands one step back) and of the last step
+                const bool late_a = late && (((uint32_t)ld_chunk + (line_a & 7)) & 8), late_b = late && (((uint32_t)ld_chunk + (line_b & 7)) & 8);
+                const uint32_t wrap = (uint32_t)(nk - 1) * C::BKB, tail_one = nk == 1 ? tail_or : 0u;
+                const uint32_t va_first = late_a ? (voff_a + wrap) | tail_or : voff_a | tail_one;
+                const uint32_t vb_first = late_b ? (voff_b + wrap) | tail_or : voff_b | tail_one;
+                const uint32_t va_mid = late_a ? voff_a : voff_a + C::BKB, vb_mid = late_b ? voff_b : voff_b + C::BKB;
+                const uint32_t va_last = late_a ? va_mid : va_mid | tail_or, vb_last = late_b ? vb_mid : vb_mid | tail_or;
+                auto issue_stage_k2 = [&](int kt, auto nt_tag, auto late_tag) {          // (nt_tag: B's copies with the streaming hint)
+                    constexpr bool B_NT = decltype(nt_tag)::value, LATE = decltype(late_tag)::value;
                     char *stage = smem + (kt % NS) * C::STAGE_BYTES + pw * 1024;
-                    const bool tl = kpos(kt) == kt_tail;
-                    const uint32_t va = tl ? voff_a_t : voff_a, vb = tl ? voff_b_t : voff_b;
+                    const int k = kpos(kt);
+                    const bool tl = k == kt_tail;
+                    uint32_t va = tl ? voff_a_t : voff_a, vb = tl ? voff_b_t : voff_b;
+                    uint32_t back = 0;
+                    if constexpr (LATE) {
+                        // (values, not a choice between variables: that kept all of this in scratch memory)
+                        const uint32_t a0 = va_first, a1 = va_last, a2 = va_mid, b0 = vb_first, b1 = vb_last, b2 = vb_mid;
+                        va = k == 0 ? a0 : tl ? a1 : a2;
+                        vb = k == 0 ? b0 : tl ? b1 : b2;
+                        back = k == 0 ? 0 : 128;
+                    }
 #pragma unroll
                     for (int j = 0; j < NPC; ++j) {
                         lds_void *dst = (lds_void *)(stage + j * 4096);
                         const uint32_t blk = (pw >> 1) + 2 * j;
                         if (2 * j < C::RBA)
-                            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, va, soff_k2(C::KMA, blk, p.lda, kt), 0, 0);
+                            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, va, soff_k2(C::KMA, blk, p.lda, kt) - back, 0, 0);
                         else
-                            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst, 16, vb, soff_k2(C::KMB, blk - C::RBA, p.ldb, kt), 0, B_NT ? 2 : 0);
+                            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst, 16, vb, soff_k2(C::KMB, blk - C::RBA, p.ldb, kt) - back, 0, B_NT ? 2 : 0);
                     }
                     if constexpr (C::BLOCK_SCALE) {
                         if (!p.as_groups) {
@@ -1075,32 +1111,46 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
                         }
                     }
                 };
-                // (the loop of a copying wave exists twice, with and without the streaming hint on B's copies: chosen per
-                // copy inside one loop the branch cost these waves 2 - 4 %)
-                auto copy_loop = [&](auto nt_tag) {
+                // (the loop of a copying wave exists once for each form: with and without the streaming hint on B's copies,
+                // with and without late chunks; chosen per copy inside one loop the hint's branch cost these waves 2 - 4 %)
+                auto copy_loop = [&](auto nt_tag, auto late_tag) {
+                    constexpr int LATE = decltype(late_tag)::value ? 1 : 0;
+                    const int stages = nk > 0 ? nk + LATE : 0;
 #pragma unroll
                     for (int j = 0; j < NS - 1; ++j)
-                        if (j < nk) {
-                            issue_scale_group(j);
-                            issue_stage_k2(j, nt_tag);
+                        if (j < stages) {
+                            if (!LATE || j < nk) issue_scale_group(j);
+                            issue_stage_k2(j, nt_tag, late_tag);
                         }
                     const bool counted = !C::BLOCK_SCALE || !p.as_groups;       // the scale copies are among the CPS of a stage
                     for (int ph = 0; ph <= nk; ++ph) {
-                        if (ph + NS - 2 >= nk) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));      // near the end of K fewer are in flight
-                        else if (counted) __builtin_amdgcn_s_waitcnt(waitcnt_vm((NS - 2) * CPS));
-                        else __builtin_amdgcn_s_waitcnt(waitcnt_vm((NS - 2) * NPC));
+                        if (ph + NS - 2 >= stages) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));      // near the end of K fewer are in flight
+                        else if (counted) __builtin_amdgcn_s_waitcnt(waitcnt_vm((NS - 2 - LATE) * CPS));
+                        else __builtin_amdgcn_s_waitcnt(waitcnt_vm((NS - 2 - LATE) * NPC));
                         phase_barrier();
-                        if (ph + NS - 1 < nk) {
-                            issue_scale_group(ph + NS - 1);
-                            issue_stage_k2(ph + NS - 1, nt_tag);
+                        if (ph + NS - 1 < stages) {
+                            if (!LATE || ph + NS - 1 < nk) issue_scale_group(ph + NS - 1);
+                            issue_stage_k2(ph + NS - 1, nt_tag, late_tag);
                         }
                     }
                 };
-                if (p.b_stream) copy_loop(std::integral_constant<bool, true>{});
-                else copy_loop(std::integral_constant<bool, false>{});
+                constexpr std::integral_constant<bool, true> yes{};
+                constexpr std::integral_constant<bool, false> no{};
+                if (LATE_FORM && late) {
+                    if (p.b_stream) copy_loop(yes, std::integral_constant<bool, LATE_FORM>{});
+                    else copy_loop(no, std::integral_constant<bool, LATE_FORM>{});
+                } else {
+                    if (p.b_stream) copy_loop(yes, no);
+                    else copy_loop(no, no);
+                }
             } else {
                 v4i fa[C::TM][2], fb[C::TN][2];
-                auto read_stage = [&](int mine) {
+                // this lane's two chunks of a step: do they come with the stage behind it (row & 7 == fr & 7 here)
+                const uint32_t fa_line = ((uint32_t)((uintptr_t)p.A >> 4) + (fr & 7) * (p.lda >> 4)) & 7;
+                const uint32_t fb_line = ((uint32_t)((uintptr_t)p.B >> 4) + (fr & 7) * (p.ldb >> 4)) & 7;
+                const bool late_a0 = late && fg + fa_line >= 8, late_a1 = late && fg + 4 + fa_line >= 8;
+                const bool late_b0 = late && fg + fb_line >= 8, late_b1 = late && fg + 4 + fb_line >= 8;
+                auto read_stage = [&](int mine, auto late_tag) {
                     if constexpr (C::BLOCK_SCALE) {
                         const int tr = wm * C::WM + (lane & 15);                    // tile row of this lane in row block 0
                         const char *sc = smem + NS * C::STAGE_BYTES +
@@ -1113,16 +1163,23 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
                         for (int j = 0; j < NBS; ++j)
                             bs_cur[j] = p.bs[__builtin_amdgcn_readfirstlane(bs_off[j] + kb * p.bs_ks)];
                     }
-                    const char *st = smem + (mine % NS) * C::STAGE_BYTES;
+                    const char *st = smem + (mine % NS) * C::STAGE_BYTES, *sa0 = st, *sa1 = st, *sb0 = st, *sb1 = st;
+                    if constexpr (decltype(late_tag)::value) {
+                        const char *st1 = smem + ((mine + 1) % NS) * C::STAGE_BYTES;
+                        if (late_a0) sa0 = st1;
+                        if (late_a1) sa1 = st1;
+                        if (late_b0) sb0 = st1;
+                        if (late_b1) sb1 = st1;
+                    }
 #pragma unroll
                     for (int a = 0; a < C::TM; ++a) {
-                        fa[a][0] = frag_a(st, a, 0);
-                        fa[a][1] = frag_a(st, a, 1);
+                        fa[a][0] = frag_a(sa0, a, 0);
+                        fa[a][1] = frag_a(sa1, a, 1);
                     }
 #pragma unroll
                     for (int b = 0; b < C::TN; ++b) {
-                        fb[b][0] = frag_b(st, b, 0);
-                        fb[b][1] = frag_b(st, b, 1);
+                        fb[b][0] = frag_b(sb0, b, 0);
+                        fb[b][1] = frag_b(sb1, b, 1);
                     }
                     __builtin_amdgcn_s_waitcnt(waitcnt_lgkm0());   // reads done before the buffer may be refilled
                 };
@@ -1163,19 +1220,23 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
                                 acc[a][b] = mma128<C::ARITH>(fb[b][0], fb[b][1], fa[a][0], fa[a][1], acc[a][b]);
                     }
                 };
-                int ph = 0;
-                if (kg == 1) {                       // phase 0 of the second set: nothing to multiply yet
-                    phase_barrier();
-                    ph = 1;
-                }
-                for (; ph <= nk; ph += 2) {
-                    phase_barrier();
-                    if (ph < nk) read_stage(ph);
-                    if (ph + 1 <= nk) {
+                auto compute_loop = [&](auto late_tag) {
+                    int ph = 0;
+                    if (kg == 1) {                       // phase 0 of the second set: nothing to multiply yet
                         phase_barrier();
-                        mfma_stage();
+                        ph = 1;
                     }
-                }
+                    for (; ph <= nk; ph += 2) {
+                        phase_barrier();
+                        if (ph < nk) read_stage(ph, late_tag);
+                        if (ph + 1 <= nk) {
+                            phase_barrier();
+                            mfma_stage();
+                        }
+                    }
+                };
+                if (LATE_FORM && late) compute_loop(std::integral_constant<bool, LATE_FORM>{});
+                else compute_loop(std::integral_constant<bool, false>{});
             }
         } else if constexpr (PAIRS) {
 #pragma unroll
