@@ -112,7 +112,11 @@ int qgemm_scaled_gemm(int in_dtype, int out_dtype, int scale_mode, int layout, c
  * QGEMM_LAYOUT_REFERENCE) comes from a static device array of QGEMM_STATIC_SCRATCH_BYTES that every GPU the
  * library runs on holds until the process ends.  The call allocates and frees nothing.  A problem that needs
  * more returns QGEMM_ERR_SCRATCH_TOO_SMALL and launches nothing.  All calls on one GPU share the array: two
- * calls whose kernels overlap in time on one GPU (different streams, or threads) race. */
+ * calls whose kernels overlap in time on one GPU (different streams, or threads) race.
+ * Operands that qgemm_scaled_gemm packs into the workspace first (K not a multiple of 16, unaligned pointers: option
+ * "any_shape") are not packed here: the any-shape kernel reads them as they stand, and such calls take nothing from
+ * the array.  int8 operands with one scale give the same bits either way; block-scaled ones are the same products and
+ * the same folds, summed in another order. */
 #define QGEMM_STATIC_SCRATCH_BYTES ((size_t)32 << 20)
 int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int layout, const void *A, const void *B,
                              const float *a_scale, const float *b_scale, void *C, size_t ldC, size_t M, size_t N,
@@ -125,7 +129,9 @@ int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int la
  * already captured remain valid.  Calls on different streams share the block: each such call waits (on the
  * device, through an event) for the previous user on another stream.  While a stream is being captured into a
  * graph the library neither allocates nor touches that event: a call that would have to grow the block returns
- * QGEMM_ERR_ALLOC, and replays of graphs that use the workspace must not overlap other users of it.
+ * QGEMM_ERR_ALLOC, and replays of graphs that use the workspace must not overlap other users of it.  (Products whose
+ * operands would be packed into the block, see option "any_shape", do not use it while captured: they run the any-shape
+ * kernel, whose fp32 sums have another order than those of an eager call.)
  * qgemm_reserve_workspace makes the block at least `bytes` large ahead of time (it allocates: call it before a
  * capture begins, never during one; a block that has to grow at least doubles); qgemm_workspace_info reports
  * its address and size (NULL / 0 before first use). */
@@ -166,8 +172,9 @@ int qgemm_tile_map(uint32_t wg, uint32_t tiles_m, uint32_t tiles_n, uint32_t gro
 /* Tuning / diagnostics (no reference counterpart: the reference picks its tile at compile time,
  * src/include/gemm_config.h:30-36).
  * qgemm_set_option(key, value): "force_split" (K slices, 0 = heuristic), "group_m", "kmajor", "any_shape" (operands whose K
- *   bytes are no multiple of 16, or whose rows or pointers are unaligned: 0 the scalar kernel, 1 packed into the workspace
- *   for the matrix cores where that is faster, 2 packed wherever possible), "stagger", "k_rot",
+ *   bytes are no multiple of 16, or whose rows or pointers are unaligned: 0 the any-shape kernel, which reads them as they
+ *   stand, 1 packed into the workspace for the other kernels where that is faster, 2 packed wherever possible; captured
+ *   calls and qgemm_scaled_gemm_static always run the any-shape kernel), "stagger", "k_rot",
  *   "stagger_groups", "as_groups", "row_split" (0: one launch always; 1: the rows "a+b" or columns "a|b" of a partly
  *   empty last round of 256 x 256 tiles as a second launch where the estimate gains; 2 / 3: rows / columns wherever
  *   possible), "small_tiles" (0: 17 .. 256 rows against few columns keep a tall tile with a K split instead of several

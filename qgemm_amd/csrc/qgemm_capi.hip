@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "aux_kernels.cuh"
+#include "gemm_any.cuh"
 #include "quant_kernels.cuh"
 #include "selftest.cuh"
 #include "variants.h"
@@ -70,8 +71,8 @@ struct Context {
     long row_split = 1;         // 0: never run the rows (or columns) of a last, mostly empty round of 256 x 256 tiles as a second launch;
                                 // 2 / 3: the rows / the columns always where the geometry allows it, whatever the estimate says
                                 // (for measurements)
-    long any_shape = 1;         // operands no MFMA kernel reads as they stand: 0: the scalar kernel, 1: packed for the MFMA kernels where
-                                // that is faster, 2: packed wherever possible (for measurements and tests)
+    long any_shape = 1;         // operands the MFMA kernels cannot copy as they stand: 0: the any-shape kernel, 1: packed for the others
+                                // where that is faster, 2: packed wherever possible (for measurements and tests)
     long kmajor = 1;            // 0: K-major operands (NN, reference fp8 layout) always go through the transposes; 2: never
                                 // where a K-major kernel fits the shape (for measurements and tests)
     std::string last_config;
@@ -971,23 +972,26 @@ int launch_nt(NtProblem q, hipStream_t stream) {
     return run_nt(q, pl, ws, stream);
 }
 
-// Is a product on the any-shape path large enough for the packing launch and the matrix cores?  The scalar kernel, one
-// thread per element, takes 2 us and 0.07 - 0.09 us per element of K, and no less than a microsecond per 0.8e6 products;
-// packing and the MFMA kernel take 5.5 - 9 us on products this small.  Graph replays, us, scalar / packed: 16 x 1001 bf16
-// K = 33 4.6 / 6.8, 65 6.6 / 7.1, 129 12.2 / 7.4; 1 x 1001 int8 65 6.0 / 7.6, 129 10.0 / 7.7; 256 x 257 bf16 33 6.4 / 8.5,
-// 65 10.5 / 8.8.  Large: 1531 x 4100 x 3004 int8 23 800 / 45 us, bf16 1999 x 1000 x 3001 2 750 / 30.
-bool pack_pays(size_t M, size_t N, size_t K) { return K >= 72 || (double)M * N * K >= 8e6; }
+// Is a product on the any-shape path large enough for the packing launch and the other kernels?  The any-shape kernel
+// takes about a microsecond per 128 bytes of K and round of tiles, packing and the kernel behind it two launches.
+// Eager calls, us (7 of them the host's), any-shape kernel / packed: int8 16 x 1001 K = 401 7.9 / 11.7, 1041 12.9 / 11.8;
+// 256 x 4097 401 9.4 / 14.5, 2001 23.5 / 21.2; 1024 x 2049 201 12.3 / 15.3, 401 16.4 / 15.5; 4096 x 4097 33 32.0 / 24.0,
+// 2001 184 / 54; bf16 16 x 1001 261 8.7 / 11.7, 521 12.6 / 11.6; 1024 x 2049 129 14.1 / 13.5.
+bool pack_pays(size_t M, size_t N, size_t kbytes) { return kbytes > 768 || (double)M * N * kbytes >= 4e8; }
 
 // Operands that no MFMA kernel reads as they stand: pack_kernel writes what has to change into the workspace as rows of
 // whole 128-byte K steps (one launch for both operands), and the K-contiguous kernels take it from there.  a_src / b_src:
 // the operands as the caller has them, ld in bytes between rows, or, k_major, between rows of k.  q: everything else, with
-// the caller's K.  *taken = false, and nothing launched, where the scalar kernel is the one to run:
+// the caller's K.  *taken = false, and nothing launched, where the any-shape kernel is the one to run (launch_any), which
+// needs no memory but the operands:
+//   * calls that are captured and calls on the static scratch: replays of a captured graph, and the calls of several threads
+//     on the scratch, are ordered by nobody, and packed operands in a block that they share would overwrite each other.
+//     (The choice does not depend on how much room there happens to be: a call captured twice gives the same bits.)
 //   * fp8 operands with fp32 output: the matrix core adds the products of an fp8 step with fewer bits than an fp32 sum
 //     keeps (1.5e-5 against 5e-8 of the result at K = 4096: nothing beside a 16-bit output's rounding, all of the error of an
 //     fp32 one), and these shapes have always been summed in fp32;
-//   * no room: the static scratch is too small, a stream capture forbids growing the workspace (the scalar kernel needs
-//     none), or the shape exceeds what the MFMA kernels index;
-//   * a product so small that the scalar kernel is done first (pack_pays).
+//   * the device has no memory left for the workspace, or the shape exceeds what the MFMA kernels index;
+//   * a product so small that the any-shape kernel is done first (pack_pays).
 struct SourceOperand {
     const void *p;
     size_t ld;
@@ -998,7 +1002,8 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
     *taken = false;
     const size_t eb = dtype_bytes(in_dtype);
     if (!g_ctx.any_shape || (in_dtype == QGEMM_DT_F8E4M3 && q.out_dtype == QGEMM_DT_F32)) return QGEMM_OK;
-    if (g_ctx.any_shape == 1 && !pack_pays(q.M, q.N, K)) return QGEMM_OK;
+    if (g_ctx.any_shape == 1 && !pack_pays(q.M, q.N, K * eb)) return QGEMM_OK;
+    if (g_ctx.static_call || stream_is_capturing(stream)) return QGEMM_OK;
     if (q.M >= ((size_t)1 << 31) || q.N >= ((size_t)1 << 31) || K >= ((size_t)1 << 30)) return QGEMM_OK;
     // (a K that ends inside a 16-byte piece has to end in zeros in both operands)
     const bool whole = (K * eb) % 16 == 0;
@@ -1044,7 +1049,7 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
     if (blocks >= ((uint64_t)1 << 31)) return QGEMM_OK;
     void *ws = nullptr;
     int st = ensure_workspace_locked(split_room + as_room + room[0] + room[1], stream, &ws);
-    if (st == QGEMM_ERR_ALLOC || st == QGEMM_ERR_SCRATCH_TOO_SMALL) return QGEMM_OK;
+    if (st == QGEMM_ERR_ALLOC) return QGEMM_OK;
     *taken = true;
     if (st != QGEMM_OK) return st;
     char *at = (char *)ws + split_room + as_room, *bt = at + room[0];
@@ -1063,21 +1068,51 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
     return st;
 }
 
-template <int DT>
-int launch_strided_t(const StridedArgs &s, hipStream_t stream) {
-    dim3 grid((s.N + 15) / 16, (s.M + 15) / 16);
-    hipLaunchKernelGGL(gemm_strided_kernel<DT>, grid, dim3(256), 0, stream, s);
+template <int DT, bool BLOCK>
+int launch_any_t(AnyArgs &a, hipStream_t stream) {
+    // 128 x 128 tiles where they occupy half of the CUs, else 64 x 64
+    constexpr int W = BLOCK && DT == QGEMM_DT_I8 ? 64 : 128;        // (the partial products of int8 blocks would not fit the registers)
+    const bool km = a.a.k_major || a.b.k_major;
+    const uint64_t wide = ((uint64_t)a.a.rows + 127) / 128 * (((uint64_t)a.b.rows + 127) / 128);
+    const int T = wide * 2 >= (uint64_t)g_ctx.num_cus && !(BLOCK && km) ? W : 64;
+    a.tiles_m = (uint32_t)(((uint64_t)a.a.rows + T - 1) / T);
+    a.tiles_n = (uint32_t)(((uint64_t)a.b.rows + T - 1) / T);
+    const uint64_t tiles = (uint64_t)a.tiles_m * a.tiles_n;
+    if (tiles >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;    // grid limit
+    const auto kernel = T == 64 ? (km ? gemm_any_kernel<DT, BLOCK, 64, true> : gemm_any_kernel<DT, BLOCK, 64, false>)
+                                : (km ? gemm_any_kernel<DT, BLOCK, BLOCK ? 64 : W, true> : gemm_any_kernel<DT, BLOCK, W, false>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(256), 0, stream, a);
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }
 
-int launch_strided(int in_dtype, const StridedArgs &s, hipStream_t stream) {
+// The any-shape kernel on the operands as they stand (arguments as for launch_packed; M, N, K below 2^32)
+int launch_any(const NtProblem &q, int in_dtype, const SourceOperand &a_src, const SourceOperand &b_src, size_t K, hipStream_t stream) {
     g_ctx.last_config = "strided_any_shape";
-    if ((s.N + 15) / 16 > 0x7FFFFFFFu || (s.M + 15) / 16 > 65535u) return QGEMM_ERR_TOO_LARGE;    // grid limits
+    const size_t eb = dtype_bytes(in_dtype);
+    AnyArgs a;
+    std::memset(&a, 0, sizeof(a));
+    auto operand = [&](const SourceOperand &s, size_t rows) {
+        const char *p = (const char *)s.p;
+        return AnyOperand{p, p + (s.k_major ? (K - 1) * s.ld + rows * eb : (rows - 1) * s.ld + K * eb), s.ld, (uint32_t)rows, s.k_major};
+    };
+    a.a = operand(a_src, q.M);
+    a.b = operand(b_src, q.N);
+    a.C = q.C;
+    a.as = q.as;
+    a.bs = q.bs;
+    a.K = (uint32_t)K;
+    a.ldc = q.ldc;
+    a.as_ms = q.as_ms;
+    a.as_ks = q.as_ks;
+    a.bs_ns = q.bs_ns;
+    a.bs_ks = q.bs_ks;
+    a.out_dtype = q.out_dtype;
+    a.per_matrix_scale = q.per_matrix;
     switch (in_dtype) {
-        case QGEMM_DT_I8: return launch_strided_t<QGEMM_DT_I8>(s, stream);
-        case QGEMM_DT_F8E4M3: return launch_strided_t<QGEMM_DT_F8E4M3>(s, stream);
-        case QGEMM_DT_BF16: return launch_strided_t<QGEMM_DT_BF16>(s, stream);
-        case QGEMM_DT_F16: return launch_strided_t<QGEMM_DT_F16>(s, stream);
+        case QGEMM_DT_I8: return q.block ? launch_any_t<QGEMM_DT_I8, true>(a, stream) : launch_any_t<QGEMM_DT_I8, false>(a, stream);
+        case QGEMM_DT_F8E4M3: return q.block ? launch_any_t<QGEMM_DT_F8E4M3, true>(a, stream) : launch_any_t<QGEMM_DT_F8E4M3, false>(a, stream);
+        case QGEMM_DT_BF16: return launch_any_t<QGEMM_DT_BF16, false>(a, stream);
+        case QGEMM_DT_F16: return launch_any_t<QGEMM_DT_F16, false>(a, stream);
     }
     return QGEMM_ERR_UNSUPPORTED;
 }
@@ -1446,30 +1481,10 @@ QGEMM_EXPORT int qgemm_gemm(int in_dtype, int out_dtype, int layout_b, const voi
     }
 
     if (M >= ((size_t)1 << 32) || N >= ((size_t)1 << 32) || K >= ((size_t)1 << 32)) return QGEMM_ERR_TOO_LARGE;
+    const SourceOperand a_src{A, ldA * eb, false}, b_src{B, ldB * eb, layout_b == QGEMM_B_KN};
     bool taken = false;
-    st = launch_packed(q, in_dtype, {A, ldA * eb, false}, {B, ldB * eb, layout_b == QGEMM_B_KN}, K, stream, &taken);
-    if (taken) return st;
-    StridedArgs s;
-    std::memset(&s, 0, sizeof(s));
-    s.A = A;
-    s.B = B;
-    s.C = C;
-    s.M = (uint32_t)M;
-    s.N = (uint32_t)N;
-    s.K = (uint32_t)K;
-    s.a_rs = ldA;
-    s.a_cs = 1;
-    if (layout_b == QGEMM_B_NK) {
-        s.b_ns = ldB;
-        s.b_ks = 1;
-    } else {
-        s.b_ns = 1;
-        s.b_ks = ldB;
-    }
-    s.ldc = ldC;
-    s.out_dtype = out_dtype;
-    s.scale_mode = 0;
-    return launch_strided(in_dtype, s, stream);
+    st = launch_packed(q, in_dtype, a_src, b_src, K, stream, &taken);
+    return taken ? st : launch_any(q, in_dtype, a_src, b_src, K, stream);
 }
 
 }  // extern "C"
@@ -1584,31 +1599,10 @@ int scaled_gemm_entry(bool use_static, int in_dtype, int out_dtype, int scale_mo
 
     if (M >= ((size_t)1 << 32) || N >= ((size_t)1 << 32) || K >= ((size_t)1 << 32)) return QGEMM_ERR_TOO_LARGE;
     const bool km = layout == QGEMM_LAYOUT_REFERENCE;
+    const SourceOperand a_src{A, km ? M : K, km}, b_src{B, km ? N : K, km};
     bool taken = false;
-    st = launch_packed(q, in_dtype, {A, km ? M : K, km}, {B, km ? N : K, km}, K, stream, &taken);
-    if (taken) return st;
-    StridedArgs s;
-    std::memset(&s, 0, sizeof(s));
-    s.A = A;
-    s.B = B;
-    s.C = C;
-    s.as = a_scale;
-    s.bs = b_scale;
-    s.M = (uint32_t)M;
-    s.N = (uint32_t)N;
-    s.K = (uint32_t)K;
-    if (layout == QGEMM_LAYOUT_K_CONTIGUOUS) {
-        s.a_rs = K; s.a_cs = 1; s.b_ns = K; s.b_ks = 1;
-    } else {
-        s.a_rs = 1; s.a_cs = M; s.b_ns = 1; s.b_ks = N;
-    }
-    s.ldc = ldC;
-    s.as_ms = q.as_ms; s.as_ks = q.as_ks; s.bs_ns = q.bs_ns; s.bs_ks = q.bs_ks;
-    // partial products per reference K tile: first of {128, 64, 32} dividing K (:442-463)
-    s.bk = K % 128 == 0 ? 128 : (K % 64 == 0 ? 64 : (K % 32 == 0 ? 32 : 128));
-    s.out_dtype = out_dtype;
-    s.scale_mode = raw_acc ? 0 : scale_mode;
-    return launch_strided(in_dtype, s, stream);
+    st = launch_packed(q, in_dtype, a_src, b_src, K, stream, &taken);
+    return taken ? st : launch_any(q, in_dtype, a_src, b_src, K, stream);
 }
 
 }  // namespace
