@@ -84,6 +84,12 @@ __device__ inline void store_out4(void *C, size_t idx, const float *v, int out_d
             if (e < valid) dst[e] = pack4_elem(h, e);
 }
 
+// four e4m3 values -> four bf16 values (exact; NaNs stay NaNs)
+__device__ inline v2i widen_fp8(uint32_t w) {
+    return v2i{__builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, false)),
+               __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true))};
+}
+
 // Linear workgroup id -> (tile_m, tile_n).
 // Step 1 (XCD remap): the dispatcher deals workgroups to the 8 XCDs round
 // robin, so ids {x, x+8, x+16, ..} share an L2.  Renumber so that each XCD

@@ -9,13 +9,15 @@
 // distributed values: fp32 in sequence 7.1e-8, bf16 instructions 7.5e-8, fp8 ones, of 32 or 128 products, 1.4e-5).
 //
 // T x T tile, four waves of T/2 x T/2, two LDS buffers of one K step (128 bytes of K as the matrix cores take it).  The
-// next step's operands are in flight to registers, 16 bytes a lane at whatever address the row has, while a step is
-// computed.  Elements past K are zeroed in registers; rows past M or N repeat the last one and are not stored.
+// operands of the next two steps are in flight to registers, 16 bytes a lane at whatever address the row has, while a step is
+// computed.  A piece that would reach past the end of an operand is fetched from the last 16 bytes of it instead and moved
+// down in registers, elements past K are zeroed there; rows past M or N repeat the last one and are not stored.
 //
-// What bounds it: the loads off 16-byte addresses, each of which asks for two cache lines (300 - 650 TFLOP/s; rows packed to
-// whole lines reach two to four times that, packing included).  One thread per element, which this replaces / this
-// kernel, us: fp8 to fp32 500 x 4608 x 7161 21 495 / 128; graph replays 1 x 1001 x 65 int8 5.5 / 3.9, 16 x 1001 x 33 bf16
-// 4.0 / 3.7, 3 x 3 x 3 1.6 / 3.6 (the tail of the only row, byte by byte).
+// What bounds it: the steps themselves, each with a barrier, fragments out of LDS and MFMAs in turn and two workgroups a CU
+// to overlap them, and loads off cache lines that ask for two lines each.  1531 x 4100 x 3004 int8 42 us (900 TFLOP/s),
+// 4096 x 4096 x 4001 bf16 191 (700), fp8 4096 x 4608 x 7161 357 (760).  (With a branch around the pieces at the end of an
+// operand every load waited for the one before: 94, 473 and 413 us.)  One thread per element took 21 495 us for fp8 to fp32
+// 500 x 4608 x 7161, this kernel 102.
 #pragma once
 #include "gemm_mfma.cuh"
 
@@ -36,46 +38,35 @@ struct AnyArgs {
     int out_dtype, per_matrix_scale;
 };
 
-// BYTES bytes at any address, those from `end` on zeros and not read
-template <int BYTES, int ES>
-__device__ __forceinline__ void load_any(const char *p, const char *end, uint32_t *w) {
-    if (p + BYTES <= end) {
-        if constexpr (BYTES == 16) {
-            const v4i v = *(const v4i_any *)p;
+// BYTES (a power of two up to 16) bytes at any address
+template <int BYTES>
+__device__ __forceinline__ void load_any(const char *p, uint32_t *w) {
+    if constexpr (BYTES == 16) {
+        const v4i v = *(const v4i_any *)p;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) w[i] = (uint32_t)v[i];
-        } else if constexpr (BYTES == 8) {
-            const v2i v = *(const v2i_any *)p;
-            w[0] = (uint32_t)v[0];
-            w[1] = (uint32_t)v[1];
-        } else {
-            w[0] = *(const u32_any *)p;
-        }
-        return;
-    }
-    const int left = (int)(end - p);
-#pragma unroll
-    for (int d = 0; d < BYTES / 4; ++d) {
-        uint32_t x = 0;
-        if (d * 4 < left) {
-            if constexpr (ES == 2) {
-                x = *(const uint16_t *)(p + d * 4);
-                if (d * 4 + 2 < left) x |= (uint32_t) * (const uint16_t *)(p + d * 4 + 2) << 16;
-            } else {
-                x = *(const uint8_t *)(p + d * 4);
-                if (d * 4 + 1 < left) x |= (uint32_t) * (const uint8_t *)(p + d * 4 + 1) << 8;
-                if (d * 4 + 2 < left) x |= (uint32_t) * (const uint8_t *)(p + d * 4 + 2) << 16;
-                if (d * 4 + 3 < left) x |= (uint32_t) * (const uint8_t *)(p + d * 4 + 3) << 24;
-            }
-        }
-        w[d] = x;
+        for (int i = 0; i < 4; ++i) w[i] = (uint32_t)v[i];
+    } else if constexpr (BYTES == 8) {
+        const v2i v = *(const v2i_any *)p;
+        w[0] = (uint32_t)v[0];
+        w[1] = (uint32_t)v[1];
+    } else {
+        w[0] = *(const u32_any *)p;
     }
 }
 
-// four e4m3 values -> four bf16 values (exact; NaNs stay NaNs)
-__device__ inline v2i widen_fp8(uint32_t w) {
-    const f32x2_t lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false), hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
-    return v2i{__builtin_bit_cast(int, __builtin_convertvector(lo, bf16x2_t)), __builtin_bit_cast(int, __builtin_convertvector(hi, bf16x2_t))};
+// W dwords moved down by n bytes (zeros from above)
+template <int W>
+__device__ __forceinline__ void move_down(uint32_t *w, uint32_t n) {
+    uint32_t v[W + 1];
+    const uint32_t q = n >> 2;
+#pragma unroll
+    for (int i = 0; i <= W; ++i) {
+        v[i] = 0;
+#pragma unroll
+        for (int k = i; k < W; ++k) v[i] = q == (uint32_t)(k - i) ? w[k] : v[i];
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i) w[i] = __builtin_amdgcn_alignbyte(v[i + 1], v[i], n & 3);
 }
 
 // One operand of the tile.  LDS: T rows of 128 bytes, chunk c of row r in slot c ^ swz(r): fragment reads (16 rows, one chunk
@@ -104,38 +95,62 @@ struct AnyStage {
         r = ((rest / KQH) * 8 + ((i >> 3) & 7)) * ME;
     }
 
-    __device__ __forceinline__ void load(const AnyOperand &o, uint32_t row0, uint32_t k0, uint32_t K) {
+    // Where piece j of this thread comes from: never past the end of the operand, but moved back from there to the last
+    // whole piece of it (`settle` moves the data down again).
+    template <int BYTES>
+    __device__ static const char *inside(const AnyOperand &o, const char *p) {
+        return p + BYTES <= o.end ? p : o.end - BYTES;
+    }
+    __device__ static const char *row_piece(const AnyOperand &o, uint32_t row0, uint32_t k0, int j) {
+        const int i = threadIdx.x + j * 256, c = i % (RB / 16);
+        const uint32_t r = i / (RB / 16), row = r < o.rows - row0 ? row0 + r : o.rows - 1;
+        return o.p + row * o.ld + (uint64_t)k0 * ES + c * 16;
+    }
+    __device__ static const char *k_piece(const AnyOperand &o, uint32_t row0, uint32_t k0, int j, int e) {
+        int k, r;
+        block_at(j, k, r);
+        return o.p + ((uint64_t)k0 + k + e) * o.ld + ((uint64_t)row0 + r) * ES;
+    }
+
+    // (no branches but uniform ones and nothing that reads what has been loaded: all pieces are in flight together)
+    __device__ __forceinline__ void load(const AnyOperand &o, uint32_t row0, uint32_t k0) {
         if (!KM || !o.k_major) {
 #pragma unroll
-            for (int j = 0; j < NR; ++j) {
-                const int i = threadIdx.x + j * 256, c = i % (RB / 16);
-                const uint32_t r = i / (RB / 16), row = r < o.rows - row0 ? row0 + r : o.rows - 1;
-                const int64_t left = (int64_t)(K - k0) * ES - c * 16;                // bytes of the row from here on
-                uint32_t *v = w + j * 4;
-                if (left > 0) {
-                    load_any<16, ES>(o.p + row * o.ld + (uint64_t)k0 * ES + c * 16, o.end, v);
-                } else {
-                    v[0] = v[1] = v[2] = v[3] = 0;
-                }
-                if (left < 16) {
+            for (int j = 0; j < NR; ++j) load_any<16>(inside<16>(o, row_piece(o, row0, k0, j)), w + j * 4);
+        } else {
 #pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        const int n = (int)left - d * 4;
-                        if (n < 4) v[d] &= n > 0 ? (1u << (8 * n)) - 1 : 0u;
-                    }
-                }
+            for (int j = 0; j < BLOCKS; ++j)
+#pragma unroll
+                for (int e = 0; e < KL; ++e) load_any<LB>(inside<LB>(o, k_piece(o, row0, k0, j, e)), w + (j * KL + e) * (LB / 4));
+        }
+    }
+
+    // What a step that reaches past the end of K, or close to the end of the operand, has loaded: pieces moved back are
+    // moved down again, elements past K become zeros.
+    __device__ __forceinline__ void settle(const AnyOperand &o, uint32_t row0, uint32_t k0, uint32_t K) {
+        if (!KM || !o.k_major) {
+            if (K - k0 >= (uint32_t)KE) return;
+#pragma unroll
+            for (int j = 0; j < NR; ++j) {
+                const char *p = row_piece(o, row0, k0, j);
+                uint32_t *v = w + j * 4;
+                move_down<4>(v, (uint32_t)(p - inside<16>(o, p)));
+                const int left = (int)(K - k0) * ES - (threadIdx.x + j * 256) % (RB / 16) * 16;       // bytes of the row from here on
+#pragma unroll
+                for (int d = 0; d < 4; ++d) v[d] &= left >= 4 * d + 4 ? ~0u : left > 4 * d ? (1u << (8 * (left - 4 * d))) - 1 : 0u;
             }
         } else {
+            if (o.p + ((uint64_t)k0 + KE - 1) * o.ld + ((uint64_t)row0 + T) * ES <= o.end) return;
 #pragma unroll
             for (int j = 0; j < BLOCKS; ++j) {
                 int k, r;
                 block_at(j, k, r);
 #pragma unroll
                 for (int e = 0; e < KL; ++e) {
+                    const char *p = k_piece(o, row0, k0, j, e);
                     uint32_t *v = w + (j * KL + e) * (LB / 4);
-                    if ((uint32_t)r < o.rows - row0 && (uint32_t)(k + e) < K - k0) {
-                        load_any<LB, ES>(o.p + (uint64_t)(k0 + k + e) * o.ld + (uint64_t)(row0 + r) * ES, o.end, v);
-                    } else {
+                    move_down<LB / 4>(v, (uint32_t)(p - inside<LB>(o, p)));
+                    if ((uint32_t)(k + e) >= K - k0) {
 #pragma unroll
                         for (int d = 0; d < LB / 4; ++d) v[d] = 0;
                     }
@@ -210,35 +225,41 @@ __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
             return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, x), __builtin_bit_cast(v8h, y), c, 0, 0, 0);
         else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, x), __builtin_bit_cast(v8bf, y), c, 0, 0, 0);
     };
-    S sa, sb;
     acc_t acc[F][F];
     part_t part[F][F];
 #pragma unroll
     for (int a = 0; a < F; ++a)
 #pragma unroll
-        for (int b = 0; b < F; ++b) {
-            acc[a][b] = acc_t{0, 0, 0, 0};
-            part[a][b] = part_t{0, 0, 0, 0};
-        }
-    sa.load(p.a, row0, 0, p.K);
-    sb.load(p.b, col0, 0, p.K);
-    sa.store(p.a, lds[0][0]);
-    sb.store(p.b, lds[0][1]);
-    for (uint32_t s = 0; s < steps; ++s) {
-        if (s + 1 < steps) {
-            sa.load(p.a, row0, (s + 1) * KE, p.K);
-            sb.load(p.b, col0, (s + 1) * KE, p.K);
-        }
+        for (int b = 0; b < F; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
+    struct Stage {
+        S a, b;
+    } held[2];                                                          // of an even and of an odd step
+    auto load = [&](uint32_t s, Stage &r) {
+        if (s >= steps) return;
+        r.a.load(p.a, row0, s * KE);
+        r.b.load(p.b, col0, s * KE);
+    };
+    auto store = [&](uint32_t s, Stage &r) {
+        if (s >= steps) return;
+        r.a.settle(p.a, row0, s * KE, p.K);
+        r.b.settle(p.b, col0, s * KE, p.K);
+        r.a.store(p.a, lds[s & 1][0]);
+        r.b.store(p.b, lds[s & 1][1]);
+    };
+    // step s: `own` brought it and is free, `next` holds step s + 1
+    auto turn = [&](uint32_t s, auto odd, Stage &own, Stage &next) {
+        load(s + 2, own);
         __syncthreads();                                                // buffer s & 1 is filled, the other one read
-        const char *la = lds[s & 1][0], *lb = lds[s & 1][1];
-        float as[F], bs;
-        if constexpr (BLOCK) {
+        const char *la = lds[odd][0], *lb = lds[odd][1];
+        constexpr bool FIRST = I8 || !odd;                              // of a K block: 128 elements are one step of int8, two of fp8
+        float f[F];
+        if (BLOCK && (I8 || odd || s + 1 == steps)) {
             const uint32_t kb = s * KE / kScaleBlock;
-            bs = p.bs[(size_t)((col0 + wn) / kScaleBlock) * p.bs_ns + (size_t)kb * p.bs_ks];
+            const float bs = p.bs[(size_t)((col0 + wn) / kScaleBlock) * p.bs_ns + (size_t)kb * p.bs_ks];
 #pragma unroll
             for (int a = 0; a < F; ++a) {
                 const uint32_t r = wm + a * 16 + (lane & 15), m = r < p.a.rows - row0 ? row0 + r : p.a.rows - 1;
-                as[a] = p.as[(size_t)m * p.as_ms + (size_t)kb * p.as_ks];
+                f[a] = p.as[(size_t)m * p.as_ms + (size_t)kb * p.as_ks] * bs;
             }
         }
 #pragma unroll
@@ -253,24 +274,26 @@ __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
             for (int a = 0; a < F; ++a)
 #pragma unroll
                 for (int b = 0; b < F; ++b) {
-                    if constexpr (BLOCK) part[a][b] = mma(fb[b], fa[a], part[a][b]);
+                    if constexpr (BLOCK) part[a][b] = mma(fb[b], fa[a], FIRST && h == 0 ? part_t{0, 0, 0, 0} : part[a][b]);
                     else acc[a][b] = mma(fb[b], fa[a], acc[a][b]);
                 }
         }
-        if (BLOCK && (I8 || (s & 1) || s + 1 == steps)) {               // 128 elements of K: one step of int8, two of fp8
+        if (BLOCK && (I8 || odd || s + 1 == steps)) {
 #pragma unroll
             for (int a = 0; a < F; ++a)
 #pragma unroll
-                for (int b = 0; b < F; ++b) {
+                for (int b = 0; b < F; ++b)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[a][b][r] += ((float)part[a][b][r] * as[a]) * bs;
-                    part[a][b] = part_t{0, 0, 0, 0};
-                }
+                    for (int r = 0; r < 4; ++r) acc[a][b][r] += (float)part[a][b][r] * f[a];
         }
-        if (s + 1 < steps) {
-            sa.store(p.a, lds[(s + 1) & 1][0]);
-            sb.store(p.b, lds[(s + 1) & 1][1]);
-        }
+        store(s + 1, next);
+    };
+    load(0, held[0]);
+    load(1, held[1]);
+    store(0, held[0]);
+    for (uint32_t s = 0; s < steps; s += 2) {
+        turn(s, std::integral_constant<int, 0>{}, held[0], held[1]);
+        if (s + 1 < steps) turn(s + 1, std::integral_constant<int, 1>{}, held[1], held[0]);
     }
     const float scale = p.per_matrix_scale ? p.as[0] * p.bs[0] : 1.0f;
 #pragma unroll
@@ -299,6 +322,38 @@ __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
             store_out4(p.C, idx, v, p.out_dtype, valid);
         }
     }
+#endif
+}
+
+// One thread per element of C, for fewer than 16 elements of K: an operand may then be shorter than one load of the kernel
+// above, and where all of it is small a few loads of single elements are done first (graph replays, this / that, us:
+// 3 x 3 x 3 bf16 1.6 / 3.6).  One K block at most, folded as above.
+template <int IN_DT, bool BLOCK>
+__global__ void __launch_bounds__(256) gemm_short_kernel(const AnyArgs p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    const uint32_t n = (uint32_t)(i % p.b.rows);
+    const uint64_t m = i / p.b.rows;
+    if (m >= p.a.rows) return;
+    auto element = [](const AnyOperand &o, uint64_t row, uint32_t k) {
+        constexpr int ES = IN_DT == QGEMM_DT_I8 || IN_DT == QGEMM_DT_F8E4M3 ? 1 : 2;
+        const char *q = o.p + (o.k_major ? k * o.ld + row * ES : row * o.ld + (uint64_t)k * ES);
+        if constexpr (IN_DT == QGEMM_DT_I8) return (int)*(const int8_t *)q;
+        else if constexpr (IN_DT == QGEMM_DT_F8E4M3) return __builtin_amdgcn_cvt_f32_fp8((int)*(const uint8_t *)q, 0);
+        else if constexpr (IN_DT == QGEMM_DT_BF16) return __builtin_bit_cast(float, (uint32_t) * (const uint16_t *)q << 16);
+        else return (float)*(const _Float16 *)q;
+    };
+    std::conditional_t<IN_DT == QGEMM_DT_I8, int, float> sum = 0;
+    for (uint32_t k = 0; k < p.K; ++k) sum += element(p.a, m, k) * element(p.b, n, k);
+    const uint64_t idx = m * p.ldc + n;
+    if (IN_DT == QGEMM_DT_I8 && !BLOCK && p.out_dtype == QGEMM_DT_I32) {
+        ((int *)p.C)[idx] = (int)sum;
+        return;
+    }
+    float f = p.per_matrix_scale ? p.as[0] * p.bs[0] : 1.0f;
+    if (BLOCK) f = p.as[m * p.as_ms] * p.bs[(size_t)(n / kScaleBlock) * p.bs_ns];
+    const float v[4] = {(float)sum * f, 0, 0, 0};
+    store_out4(p.C, idx, v, p.out_dtype, 1);
 #endif
 }
 

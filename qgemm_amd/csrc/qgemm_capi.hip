@@ -973,11 +973,12 @@ int launch_nt(NtProblem q, hipStream_t stream) {
 }
 
 // Is a product on the any-shape path large enough for the packing launch and the other kernels?  The any-shape kernel
-// takes about a microsecond per 128 bytes of K and round of tiles, packing and the kernel behind it two launches.
-// Eager calls, us (7 of them the host's), any-shape kernel / packed: int8 16 x 1001 K = 401 7.9 / 11.7, 1041 12.9 / 11.8;
-// 256 x 4097 401 9.4 / 14.5, 2001 23.5 / 21.2; 1024 x 2049 201 12.3 / 15.3, 401 16.4 / 15.5; 4096 x 4097 33 32.0 / 24.0,
-// 2001 184 / 54; bf16 16 x 1001 261 8.7 / 11.7, 521 12.6 / 11.6; 1024 x 2049 129 14.1 / 13.5.
-bool pack_pays(size_t M, size_t N, size_t kbytes) { return kbytes > 768 || (double)M * N * kbytes >= 4e8; }
+// takes one launch and, per 128 bytes of K and round of tiles, some 1.5 us; twice that where it has to transpose (km).
+// Eager calls, us (7 of them the host's), any-shape kernel / packed: int8 16 x 1001 K = 401 7.1 / 11.2, 2001 10.9 / 12.0;
+// 256 x 4097 1041 11.2 / 18.3, 2001 15.9 / 21.1; 1024 x 2049 401 12.0 / 15.3, 1041 18.1 / 19.2, 2001 26.8 / 23.7;
+// 4096 x 4097 33 28.1 / 24.0, 2001 88.4 / 55.3; bf16 1024 x 2049 401 15.2 / 16.7, 801 21.8 / 20.3, with B stored K x N
+// 261 15.5 / 15.7, 401 18.4 / 16.7; 16 x 1001 401 8.8 / 11.7, 801 13.5 / 11.7.
+bool pack_pays(size_t M, size_t N, size_t kbytes, bool km) { return kbytes > (km ? 512 : 1024) || (double)M * N >= 4e6; }
 
 // Operands that no MFMA kernel reads as they stand: pack_kernel writes what has to change into the workspace as rows of
 // whole 128-byte K steps (one launch for both operands), and the K-contiguous kernels take it from there.  a_src / b_src:
@@ -1002,7 +1003,7 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
     *taken = false;
     const size_t eb = dtype_bytes(in_dtype);
     if (!g_ctx.any_shape || (in_dtype == QGEMM_DT_F8E4M3 && q.out_dtype == QGEMM_DT_F32)) return QGEMM_OK;
-    if (g_ctx.any_shape == 1 && !pack_pays(q.M, q.N, K * eb)) return QGEMM_OK;
+    if (g_ctx.any_shape == 1 && !pack_pays(q.M, q.N, K * eb, a_src.k_major || b_src.k_major)) return QGEMM_OK;
     if (g_ctx.static_call || stream_is_capturing(stream)) return QGEMM_OK;
     if (q.M >= ((size_t)1 << 31) || q.N >= ((size_t)1 << 31) || K >= ((size_t)1 << 30)) return QGEMM_OK;
     // (a K that ends inside a 16-byte piece has to end in zeros in both operands)
@@ -1070,11 +1071,19 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
 
 template <int DT, bool BLOCK>
 int launch_any_t(AnyArgs &a, hipStream_t stream) {
-    // 128 x 128 tiles where they occupy half of the CUs, else 64 x 64
+    const uint64_t elements = (uint64_t)a.a.rows * a.b.rows;
+    if (a.a.end - a.a.p < 16 || a.b.end - a.b.p < 16 || (a.K < 16 && elements * a.K <= 1000000)) {
+        if (elements >= (uint64_t)1 << 39) return QGEMM_ERR_TOO_LARGE;     // grid limit
+        hipLaunchKernelGGL((gemm_short_kernel<DT, BLOCK>), dim3((unsigned)((elements + 255) / 256)), dim3(256), 0, stream, a);
+        return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+    }
+    // 128 x 128 tiles where they make at least one round of the CUs, half of one where operands are transposed on the way:
+    // 64 x 64 / 128 x 128, us, K = 1001 and 3001: int8 512 x 4097 (132 tiles) 15.7 / 16.9 33.3 / 35.8, 1024 x 4097 (264) 22.7 /
+    // 22.5 52.2 / 44.1, 1500 x 4097 30.3 / 23.9 70.7 / 45.6; bf16 with B stored K x N 512 x 4097 33.2 / 30.6 87.8 / 78.1.
     constexpr int W = BLOCK && DT == QGEMM_DT_I8 ? 64 : 128;        // (the partial products of int8 blocks would not fit the registers)
     const bool km = a.a.k_major || a.b.k_major;
     const uint64_t wide = ((uint64_t)a.a.rows + 127) / 128 * (((uint64_t)a.b.rows + 127) / 128);
-    const int T = wide * 2 >= (uint64_t)g_ctx.num_cus && !(BLOCK && km) ? W : 64;
+    const int T = wide * (km ? 2 : 1) >= (uint64_t)g_ctx.num_cus && !(BLOCK && km) ? W : 64;
     a.tiles_m = (uint32_t)(((uint64_t)a.a.rows + T - 1) / T);
     a.tiles_n = (uint32_t)(((uint64_t)a.b.rows + T - 1) / T);
     const uint64_t tiles = (uint64_t)a.tiles_m * a.tiles_n;

@@ -1,0 +1,69 @@
+"""The any-shape kernel (option any_shape = 0) where its loads, tiles and steps end: K up to and around a 16-byte piece, a step
+and two steps, operands shorter than one piece, rows shorter than one, both tile sizes, rows of C with neighbours.  Small
+integers (and block scales that are powers of two) sum exactly, so the results equal the CPU oracle's."""
+import numpy as np
+import pytest
+import torch
+
+import qgemm_amd as Q
+from oracle import cpu_ref as R
+from tests.util import dev, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _any_shape_kernel():
+    Q.set_option("any_shape", 0)
+    yield
+    Q.set_option("any_shape", 1)
+
+
+def _at_the_end(x, dtype):
+    """x as the last elements of a buffer whose length is no multiple of anything."""
+    t = torch.zeros(5 + x.size, dtype=dtype, device="cuda")[5:].view(x.shape)
+    t.copy_(dev(x.astype(np.float32)).to(dtype))
+    return t
+
+
+def _operands(M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    return rng.integers(-4, 5, (M, K)), rng.integers(-4, 5, (N, K))
+
+
+# operands of one to 15 elements, rows of fewer than 16 bytes, K one off a piece, a step, two steps; 128 x 128 tiles
+SHAPES = [(1, 1, 1), (3, 5, 2), (2, 700, 7), (1, 15, 15), (40, 3, 16), (17, 9, 17), (65, 63, 31), (64, 130, 63), (5, 66, 65),
+          (70, 131, 127), (33, 2, 129), (129, 257, 255), (2, 3, 1009), (2100, 2050, 143)]
+
+
+@pytest.mark.parametrize("layout", ["nk", "kn"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.int8, torch.float8_e4m3fn])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_products(shape, dtype, layout):
+    M, N, K = shape
+    say("any-shape kernel", shape, dtype, layout)
+    a, b = _operands(M, N, K)
+    ref = torch.from_numpy(a.astype(np.float32)) @ torch.from_numpy(b.astype(np.float32)).t()
+    c = torch.full((M, N + 3), 7.0, device="cuda")
+    Q.gemm(_at_the_end(a, dtype), _at_the_end(b if layout == "nk" else np.ascontiguousarray(b.T), dtype), c[:, :N], layout)
+    assert Q.last_config() == "strided_any_shape"
+    assert torch.equal(c[:, :N].cpu(), ref)
+    assert bool((c[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.int8, torch.float8_e4m3fn])
+@pytest.mark.parametrize("shape", [(1, 1, 3), (3, 300, 15), (70, 140, 63), (33, 257, 129), (65, 129, 193), (40, 70, 257), (2100, 2050, 191)])
+def test_block_scales(shape, dtype):
+    M, N, K = shape
+    say("any-shape kernel, block scales", shape, dtype)
+    a, b = _operands(M, N, K)
+    KB, rng = (K + 127) // 128, np.random.default_rng(K)
+    as_ = (2.0 ** rng.integers(-1, 2, (M, KB))).astype(np.float32)
+    bs = (2.0 ** rng.integers(-1, 2, ((N + 127) // 128, KB))).astype(np.float32)
+    scaled = lambda x, s: torch.from_numpy(x * np.repeat(s, 128, 1)[:, :K]).float()  # noqa: E731
+    ref = scaled(a, as_) @ scaled(b, np.repeat(bs, 128, 0)[:N]).t()
+    c = torch.zeros(M, N, device="cuda")
+    Q.scaled_gemm(_at_the_end(a, dtype), _at_the_end(b, dtype), dev(as_), dev(bs), c, M, N, K, Q.SCALE_BLOCK128)
+    assert torch.equal(c.cpu(), ref)
+    if dtype == torch.int8 and M < 100:
+        assert torch.equal(c.cpu(), torch.from_numpy(R.gemm_i8_block(a.astype(np.int8), b.astype(np.int8), as_, bs)))
