@@ -21,7 +21,7 @@ typedef int v2i_any __attribute__((ext_vector_type(2), aligned(1)));
 typedef unsigned u32_any __attribute__((aligned(1)));
 
 // Arithmetic families of the MFMA kernels.
-enum Arith : int { AR_I8 = 0, AR_F8 = 1, AR_BF16 = 2, AR_F16 = 3 };
+enum Arith : int { AR_I8 = 0, AR_F8 = 1, AR_BF16 = 2, AR_F16 = 3, AR_F8W = 4 };   // F8W: fp8 operands, multiplied as bf16
 
 constexpr int kWave = 64;          // include/gpu_type.h:23 (WAVE_SIZE)
 constexpr int kXcds = 8;           // include/gpu_type.h:24 (XCD_SWIZZLE)

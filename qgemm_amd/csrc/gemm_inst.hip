@@ -49,6 +49,10 @@ static hipError_t launch_skinny(const GemmArgs &a, uint32_t grid, hipStream_t s)
 
 constexpr int kElemBytes = (INST_ARITH == AR_BF16 || INST_ARITH == AR_F16) ? 2 : 1;
 constexpr bool kBlock = (bool)INST_BLOCK;
+// Widened fp8 keeps the rows whose fragments, twice their size once widened, leave the registers of a wave without spills
+// (128 x 128 with two K groups: 164 bytes of scratch a lane, 308 with block scales; 256 x 256 on eight waves 272 and 676;
+// 256 x 128 with copying waves 148 and 1756; 128 rows of the skinny-M kernel 148 with block scales).
+constexpr bool kWide = INST_ARITH == AR_F8W;
 // A K-major operand needs whole 128-byte panels of its tile side and a multiple of four waves (GemmCfg's
 // static_asserts); tiles that cannot have that are left out of a K-major family.
 constexpr bool kmajor_can(int bm, int bn, int nw) {
@@ -102,7 +106,7 @@ static std::vector<Variant> build_table() {
     // one workgroup per CU; four with block scales, whose a_scale values take 2 KiB behind the ring): for shapes with
     // no more tiles than CUs, where the two-stage row above would sit alone on its CU
     // (K-major families too: the waves that read the tile with the transposing LDS reads have no copies in flight)
-    if constexpr (kmajor_can(128, 128, 4)) add(gemm_row<Simple<128, 128, 2, 2, kBlock ? 4 : 5, 2>>("128x128_w2x2_k2", true));
+    if constexpr (kmajor_can(128, 128, 4) && !kWide) add(gemm_row<Simple<128, 128, 2, 2, kBlock ? 4 : 5, 2>>("128x128_w2x2_k2", true));
     // the same for the 64 x 128 tile, with six stages
     if constexpr (kmajor_can(64, 128, 4)) add(gemm_row<Simple<64, 128, 1, 4, 6, 2>>("64x128_w1x4_k2", true));
     if constexpr (INST_KMAJ == 0) {
@@ -110,8 +114,9 @@ static std::vector<Variant> build_table() {
         // interleaved runs); for int8 and the 16-bit types the table marks the 8-wave one and choose_variant swaps in
         // the 4-wave one where the tiles fill whole rounds of CUs; block scales need the 8-wave form (accumulators in
         // vector registers), which has a twin reading a_scale with the K blocks contiguous, two per load.
-        if constexpr (!kBlock) add(gemm_row<Solo<256, 256, 2, 2>>("256x256_w2x2_solo", INST_ARITH == AR_F8));
-        if constexpr (kBlock)
+        if constexpr (!kBlock && !kWide) add(gemm_row<Solo<256, 256, 2, 2>>("256x256_w2x2_solo", INST_ARITH == AR_F8));
+        if constexpr (kWide) {
+        } else if constexpr (kBlock)
             add_pair(gemm_row<Solo<256, 256, 2, 4>>("256x256_w2x4_solo8", true),
                      gemm_row<Solo<256, 256, 2, 4, true>>("256x256_w2x4_solo8_ks", false), 2);
         else
@@ -128,7 +133,7 @@ static std::vector<Variant> build_table() {
         add(skinny_row<1>("skinny_16x32_k8"));
         add(skinny_row<2>("skinny_32x32_k8"));
         add(skinny_row<4>("skinny_64x32_k8"));
-        add(skinny_row<8>("skinny_128x32_k8"));
+        if constexpr (!kWide || !kBlock) add(skinny_row<8>("skinny_128x32_k8"));
         add(skinny_row<4, 4>("skinny_64x64_k8"));
         add(skinny_row<1, 1>("skinny_16x16_k8"));
         add(skinny_row<2, 1>("skinny_32x16_k8"));
@@ -136,7 +141,8 @@ static std::vector<Variant> build_table() {
     // 256 x 128 on the solo schedule with four computing waves (128 x 64 wave tiles, one per SIMD) and four copying
     // waves (GemmCfg::COPYW): block scales and K-major operands on a large tile; its twin for K-contiguous a_scale
     // takes the scales of four K blocks per copy
-    if constexpr (kBlock && INST_KMAJ == 0)
+    if constexpr (kWide) {
+    } else if constexpr (kBlock && INST_KMAJ == 0)
         add_pair(gemm_row<Solo<256, 128, 2, 2, false, true>>("256x128_w2x2_cw", true),
                  gemm_row<Solo<256, 128, 2, 2, true, true>>("256x128_w2x2_cw_ks", false), 4);
     else

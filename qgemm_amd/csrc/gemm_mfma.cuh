@@ -165,7 +165,7 @@ struct GemmCfg {
                   "K groups: simple pipeline, at least four stages");
     static_assert(BM % (16 * WAVES_M) == 0 && BN % (16 * WAVES_N) == 0, "wave tile must be a multiple of 16");
     static_assert(NLOAD % NW == 0, "load instructions must divide evenly over the waves");
-    static_assert(!BLOCK_SCALE || ARITH == AR_F8 || ARITH == AR_I8, "block scales: fp8 and int8 operands");
+    static_assert(!BLOCK_SCALE || ARITH == AR_F8 || ARITH == AR_F8W || ARITH == AR_I8, "block scales: fp8 and int8 operands");
     static_assert(!BLOCK_SCALE || (128 % WN == 0 || WN % 128 == 0), "wave tile must align with 128-wide scale blocks");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS is 160 KiB per CU");
     static_assert(PIPE != PIPE_SOLO || ((NW == 4 || NW == 8) && TN >= 4 &&
@@ -253,6 +253,16 @@ __device__ inline typename AccT<ARITH>::type mma128(v4i x0, v4i x1, v4i y0, v4i 
         v8i y = {y0[0], y0[1], y0[2], y0[3], y1[0], y1[1], y1[2], y1[3]};
         // cbsz = blgp = 0 selects e4m3 for both operands; zero scale operands select the unscaled form
         return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(x, y, c, 0, 0, 0, 0, 0, 0);
+    } else if constexpr (ARITH == AR_F8W) {
+        // (each lane widens the eight elements of an instruction as it holds them: their order along K is the same in both)
+        auto wide = [](int lo, int hi) {
+            const v2i a = widen_fp8((uint32_t)lo), b = widen_fp8((uint32_t)hi);
+            return __builtin_bit_cast(v8bf, v4i{a[0], a[1], b[0], b[1]});
+        };
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wide(x0[0], x0[1]), wide(y0[0], y0[1]), c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wide(x0[2], x0[3]), wide(y0[2], y0[3]), c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wide(x1[0], x1[1]), wide(y1[0], y1[1]), c, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(wide(x1[2], x1[3]), wide(y1[2], y1[3]), c, 0, 0, 0);
     } else if constexpr (ARITH == AR_I8) {
         c = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0, y0, c, 0, 0, 0);
         return __builtin_amdgcn_mfma_i32_16x16x64_i8(x1, y1, c, 0, 0, 0);
@@ -271,6 +281,7 @@ __device__ inline typename AccT<ARITH>::type mma128(v4i x0, v4i x1, v4i y0, v4i 
 // 16-byte MFMAs are issued by the caller a row apart (`half`), so no dependent pair is back to back.
 template <int ARITH>
 __device__ inline void mma128_inplace(v4i x0, v4i x1, v4i y0, v4i y1, typename AccT<ARITH>::type &c, int half) {
+    static_assert(ARITH != AR_F8W, "widened fp8 has no row with pinned accumulators");
     if constexpr (ARITH == AR_F8) {
         v8i x = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
         v8i y = {y0[0], y0[1], y0[2], y0[3], y1[0], y1[1], y1[2], y1[3]};

@@ -35,7 +35,7 @@ struct SkinnyCfg {
     // an MFMA tile picked out of that with ds_bpermute); the scales of a round are requested in front of the round's
     // copies, so they have arrived wherever the copies they precede have.
     static constexpr bool BLOCK_SCALE = BLOCK_SCALE_;
-    static_assert(!BLOCK_SCALE_ || ARITH_ == AR_F8 || ARITH_ == AR_I8, "block scales: fp8 and int8 operands");
+    static_assert(!BLOCK_SCALE_ || ARITH_ == AR_F8 || ARITH_ == AR_F8W || ARITH_ == AR_I8, "block scales: fp8 and int8 operands");
     // TN = 4 (with TM = 4: a 64 x 64 tile): half the strips, so A is fetched half as often; for shapes with several
     // row tiles, where a CU's load path, not the stream of B from HBM, is what bounds a 32-column strip.
     static constexpr int TM = TM_, TN = TN_;                // 16 x 16 MFMA tiles of the workgroup's tile

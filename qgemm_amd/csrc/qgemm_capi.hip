@@ -194,10 +194,12 @@ const Variant *table_for(int arith, bool block, int kmaj, int *count) {
     if (kmaj == 3) return (block && arith == AR_F8) ? variants_f8_block_tn(count) : nullptr;
     if (kmaj == 2) return block ? nullptr : (arith == AR_BF16 ? variants_bf16_nn(count) : (arith == AR_F16 ? variants_f16_nn(count) : nullptr));
     if (kmaj != 0) return nullptr;
+    if (block && arith == AR_F8W) return variants_f8w_block(count);
     if (block) return arith == AR_F8 ? variants_f8_block(count) : (arith == AR_I8 ? variants_i8_block(count) : nullptr);
     switch (arith) {
         case AR_I8: return variants_i8(count);
         case AR_F8: return variants_f8(count);
+        case AR_F8W: return variants_f8w(count);
         case AR_BF16: return variants_bf16(count);
         case AR_F16: return variants_f16(count);
     }
@@ -988,11 +990,14 @@ bool pack_pays(size_t M, size_t N, size_t kbytes, bool km) { return kbytes > (km
 //   * calls that are captured and calls on the static scratch: replays of a captured graph, and the calls of several threads
 //     on the scratch, are ordered by nobody, and packed operands in a block that they share would overwrite each other.
 //     (The choice does not depend on how much room there happens to be: a call captured twice gives the same bits.)
-//   * fp8 operands with fp32 output: the matrix core adds the products of an fp8 step with fewer bits than an fp32 sum
-//     keeps (1.5e-5 against 5e-8 of the result at K = 4096: nothing beside a 16-bit output's rounding, all of the error of an
-//     fp32 one), and these shapes have always been summed in fp32;
 //   * the device has no memory left for the workspace, or the shape exceeds what the MFMA kernels index;
 //   * a product so small that the any-shape kernel is done first (pack_pays).
+// fp8 operands run on the family that widens them to bf16 in front of the matrix core (AR_F8W), which adds in fp32 as these
+// shapes have always been summed: the fp8 instructions keep some 18 bits of the largest product of a step.  Relative error
+// against 64 bits, 301 x 100 x 4001 to fp32, one scale / block scales: in sequence 9.0e-8 / 1.1e-7, any-shape kernel 8.9e-8 /
+// 1.1e-7, packed 6.9e-8 / 7.5e-8, packed on the fp8 instructions 1.4e-5.  It costs, us, fp8 instructions / widened: 500 x 4608 x
+// 7161 41.8 / 61.1, block scales 44.9 / 65.3; 4096 x 4608 x 7161 125.5 / 239.9 and 148.7 / 267.7 (fp32 output, one thread per
+// element before: 500 x 4608 x 7161 21 500 / 61).
 struct SourceOperand {
     const void *p;
     size_t ld;
@@ -1002,7 +1007,8 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
                   bool *taken) {
     *taken = false;
     const size_t eb = dtype_bytes(in_dtype);
-    if (!g_ctx.any_shape || (in_dtype == QGEMM_DT_F8E4M3 && q.out_dtype == QGEMM_DT_F32)) return QGEMM_OK;
+    if (!g_ctx.any_shape) return QGEMM_OK;
+    if (q.arith == AR_F8) q.arith = AR_F8W;
     if (g_ctx.any_shape == 1 && !pack_pays(q.M, q.N, K * eb, a_src.k_major || b_src.k_major)) return QGEMM_OK;
     if (g_ctx.static_call || stream_is_capturing(stream)) return QGEMM_OK;
     if (q.M >= ((size_t)1 << 31) || q.N >= ((size_t)1 << 31) || K >= ((size_t)1 << 30)) return QGEMM_OK;

@@ -34,6 +34,9 @@ const Variant *variants_f8_block(int *count);
 const Variant *variants_i8_block(int *count);
 const Variant *variants_bf16(int *count);
 const Variant *variants_f16(int *count);
+// fp8 operands multiplied as bf16 (packed operands: see launch_packed)
+const Variant *variants_f8w(int *count);
+const Variant *variants_f8w_block(int *count);
 // K-major operand storage (GemmCfg::KMAJ): the reference's fp8 layout (A is K x M, B is K x N) and "NN" 16-bit GEMMs
 const Variant *variants_f8_block_tn(int *count);
 const Variant *variants_bf16_nn(int *count);
