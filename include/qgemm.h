@@ -198,7 +198,8 @@ int qgemm_last_config(char *buf, size_t buflen);
 
 /* Which kernel configuration the library would run for a problem with dense, 16-byte aligned operands: the name
  * qgemm_last_config would report after the call ("256x256_w2x2_solo", "128x128_w2x2_dma_tn_splitk2", ...;
- * "strided_any_shape" for both forms of what option "any_shape" chooses between;
+ * "strided_any_shape" for operands that option "any_shape" decides about, whichever way it sends them: after such a call
+ * qgemm_last_config says "pack+<name>" where they were packed and "strided_any_shape" where the any-shape kernel ran;
  * "transpose+<name>" when operands stored K-major go through the transpose kernels first).  Nothing is launched
  * and no device is needed (256 CUs are assumed before qgemm_init).  No reference counterpart: the reference picks
  * its tile at compile time (src/include/gemm_config.h:30-36).

@@ -1071,7 +1071,7 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
         if (st != QGEMM_OK) return st;
     }
     st = run_nt(q, pl, ws, stream);
-    g_ctx.last_config = "strided_any_shape";        // (one name for both forms of the any-shape path, as qgemm_plan gives it)
+    g_ctx.last_config = "pack+" + g_ctx.last_config;
     return st;
 }
 

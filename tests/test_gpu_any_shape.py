@@ -1,5 +1,5 @@
-"""Operands no MFMA kernel reads as they stand (K bytes not a multiple of 16, unaligned rows or pointers): packed for the
-MFMA kernels (any_shape = 2) and on the scalar kernel (any_shape = 0).  Inputs are small integers, every product and sum
+"""Operands the MFMA kernels cannot copy as they stand (K bytes not a multiple of 16, unaligned rows or pointers): packed for
+those kernels (any_shape = 2) and on the any-shape kernel (any_shape = 0).  Inputs are small integers, every product and sum
 of which is exact in every type the kernels sum in, so both forms give the oracle's numbers exactly."""
 import numpy as np
 import pytest
@@ -17,6 +17,11 @@ def _reset_options():
     yield
     Q.set_option("any_shape", 1)
     Q.set_option("force_split", 0)
+
+
+def _ran(any_shape):
+    """Did the way that was asked for run?  (Both give the same numbers here.)"""
+    return Q.last_config().startswith("pack+") if any_shape == 2 else Q.last_config() == "strided_any_shape"
 
 
 def _ints(rng, shape):
@@ -50,6 +55,7 @@ def test_product(shape, dtype, layout, any_shape):
     Q.set_option("any_shape", any_shape)
     c = torch.full((M, N), 7.0, dtype=out, device="cuda")
     Q.gemm(_tensor(a, dtype), _tensor(b if layout == "nk" else np.ascontiguousarray(b.T), dtype), c, layout)
+    assert _ran(any_shape), Q.last_config()
     assert torch.equal(c.cpu(), torch.from_numpy(ref).to(out))
 
 
@@ -67,6 +73,8 @@ def test_leading_dimensions_and_pointers(K, dtype, layout):
         say("any shape, strides", dtype, layout, pads, offs)
         c = torch.full((M, N + 3), 7.0, dtype=torch.float32, device="cuda")[:, :N]
         Q.gemm(_tensor(a, dtype, pads[0], offs[0]), _tensor(bt, dtype, pads[1], offs[1]), c, layout)
+        if layout == "nk" or K % 16 or pads != (0, 0):        # (else B goes through the transpose kernel alone)
+            assert _ran(2), Q.last_config()
         assert torch.equal(c.cpu(), ref)
 
 
@@ -86,6 +94,7 @@ def test_block_scales(shape, dtype):
             Q.set_option("force_split", split)
             c = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
             Q.scaled_gemm(_tensor(a, dtype), _tensor(b, dtype), dev(as_), dev(bs), c, M, N, K, Q.SCALE_BLOCK128)
+            assert _ran(any_shape), Q.last_config()
             assert torch.equal(c.cpu(), ref.to(torch.bfloat16)), (any_shape, split)
 
 
@@ -98,11 +107,12 @@ def test_int8_accumulators_and_one_scale():
     for dtype, want in ((torch.int32, acc), (torch.float32, R.scale_i32_to_f32(acc, np.float32(0.5), np.float32(3.0)))):
         c = torch.zeros((M, N), dtype=dtype, device="cuda")
         Q.int8_mm(dev(a), dev(b), scalar(0.5), scalar(3.0), c)
+        assert _ran(2), Q.last_config()
         assert np.array_equal(host(c), want)
 
 
 def test_capture_without_room_uses_no_workspace():
-    """While a stream is captured the workspace may not grow: the scalar kernel, which needs none, takes over."""
+    """While a stream is captured nothing is packed: the any-shape kernel, which needs no workspace, runs."""
     Q.load_library().qgemm_shutdown()       # (gives the workspace back: it is empty when the capture begins)
     a, b = (torch.randint(-3, 4, (r, 9001), device="cuda").to(torch.int8) for r in (64, 96))
     c, want = (torch.zeros(64, 96, dtype=torch.int32, device="cuda") for _ in range(2))
@@ -114,6 +124,7 @@ def test_capture_without_room_uses_no_workspace():
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
         Q.int8_mm(a, b, one, one, c)
+    assert _ran(0), Q.last_config()
     for _ in range(3):
         c.zero_()
         g.replay()

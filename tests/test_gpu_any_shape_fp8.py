@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(params=[0, 2], ids=["any_shape_kernel", "packed"], autouse=True)
 def _way(request):
     Q.set_option("any_shape", request.param)
-    yield
+    yield request.param
     Q.set_option("any_shape", 1)
     Q.set_option("force_split", 0)
     Q.force_config(None)
@@ -38,7 +38,7 @@ def _cancelling(M, N, K):
 
 @pytest.mark.parametrize("out", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("shape", [(5, 70, 129), (16, 200, 1001), (64, 700, 4097), (130, 300, 2001), (700, 520, 1025), (1100, 1030, 777)])
-def test_no_bits_are_lost(shape, out):
+def test_no_bits_are_lost(shape, out, _way):
     M, N, K = shape
     say("fp8 any shape, cancelling products", shape, out)
     a, b, ref = _cancelling(M, N, K)
@@ -47,6 +47,7 @@ def test_no_bits_are_lost(shape, out):
         for split in (1, 0):
             c = torch.full((M, N), 7.0, dtype=out, device="cuda")
             Q.scaled_gemm(a, b, sa, sb, c, M, N, K, mode, split_k=split)
+            assert Q.last_config().startswith("pack+") == (_way == 2), Q.last_config()
             assert torch.equal(c.cpu(), ref.to(out)), (mode, split, Q.last_config())
 
 

@@ -199,8 +199,7 @@ def test_values_next_to_the_tail_never_count():
 
 
 def test_what_is_left_for_the_any_shape_kernel():
-    """K bytes not a multiple of 16, or operands that are not 16-byte aligned: the one-thread-per-element kernel, and
-    qgemm_plan says so."""
+    """K bytes not a multiple of 16, or operands that are not 16-byte aligned: the any-shape path, and qgemm_plan says so."""
     assert Q.plan(Q.DT_F8E4M3, Q.SCALE_PER_MATRIX, 0, 64, 64, 100) == "strided_any_shape"
     assert Q.plan(Q.DT_BF16, 0, 0, 64, 64, 100) == "strided_any_shape"           # 200 bytes
     assert Q.plan(Q.DT_F8E4M3, Q.SCALE_PER_MATRIX, 0, 64, 64, 96) != "strided_any_shape"
