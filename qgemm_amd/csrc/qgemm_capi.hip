@@ -61,7 +61,8 @@ struct Context {
 #if QGEMM_DEBUG_BUILD
     long dbg_ptr = 0;           // measurement builds: device buffer for the kernels' time stamps (GemmArgs::dbg_cycles)
 #endif
-    long as_groups = 1;         // 0: a_scale always one K block per copy on the rows with two K groups (see run_nt)
+    long as_groups = 1;         // 0: no copies of four K blocks of a_scale: one block per copy on the rows with two K groups (see run_nt), a
+                                // transposed copy of a_scale for the row with copying waves (see settle_scale_layout)
     long small_tiles = 1;       // 0: 17 .. 256 rows never go to several row tiles of the skinny-M kernel in place of a K split
     long k_rot = -1;            // -1: rotated K start for at most 256 rows (see plan_nt), 0: never, n: steps per column tile
     long stagger = -1;          // -1: staggered start where it pays (4-byte C, three or more rounds), else microseconds per group
@@ -928,11 +929,8 @@ bool settle_scale_layout(const NtProblem &q, Plan &pl) {
         }
         // (any row length and any slice: loads of 8 bytes and LDS copies of 16 need 4-byte alignment only, what the load of
         // a row's last blocks brings beyond the row nobody uses, and at the end of the array the range check, which is
-        // per dword, returns zeros for it: probed by qgemm_selftest_layouts.  A row pinned by name whose twin copies
-        // four blocks through LDS takes its twin only where rows and slices are whole groups of them, as its users know it.)
-        const uint32_t g = (uint32_t)twin->ks_blocks;
-        as_is = ((uintptr_t)q.as % 4) == 0 &&
-                !(forced() && g == 4 && (q.as_ms % g != 0 || p->a.ksteps % g != 0 || (p->a.nsplit > 1 && p->a.ksteps_per_split % g != 0)));
+        // per dword, returns zeros for it: probed by qgemm_selftest_layouts.)
+        as_is = (uintptr_t)q.as % 4 == 0 && (twin->ks_blocks != 4 || g_ctx.as_groups);
     }
     for (Plan *p = &pl; p; p = p->rest.get()) {
         if (p->v->a_scale_any_stride) continue;

@@ -57,7 +57,7 @@ def test_every_number_of_k_steps(fam):
                 else:
                     as_ = (2.0 ** rng.integers(-3, 4, size=(M, ksteps))).astype(np.float32)
                     bs = (2.0 ** rng.integers(-3, 4, size=((N + 127) // 128, ksteps))).astype(np.float32)
-                    if fam == "f8_block":                    # (even K block counts take the twin that reads a_scale as given)
+                    if fam == "f8_block":                    # (more than one K block: the twin that reads a_scale as given)
                         Q.scaled_gemm(fp8_tensor(R.encode_fp8(a)), fp8_tensor(R.encode_fp8(b)), dev(as_), dev(bs), c, M, N, K,
                                       Q.SCALE_BLOCK128)
                     else:

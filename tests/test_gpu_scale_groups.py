@@ -17,6 +17,7 @@ def _reset_options():
     Q.force_config(None)
     Q.set_option("force_split", 0)
     Q.set_option("k_rot", -1)
+    Q.set_option("as_groups", 1)
 
 
 def _problem(M, N, K, seed):
@@ -63,3 +64,22 @@ def test_copying_waves(M, N, K):
     assert Q.last_config() == "256x128_w2x2_cw_ks"
     rows = np.r_[0:70, M - 70:M]                         # (the oracle on the first and last rows)
     assert np.array_equal(got[rows], R.gemm_fp8_block(p[0][rows], p[1], p[2][rows], p[3]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("K", [128 * 5, 128 * 9 + 16, 128 * 14, 128 * 19 + 96])
+def test_copying_waves_pinned(K, dtype):
+    """A row pinned by name reads the scales as the planner's choice does, also where K slices begin between groups of four
+    blocks; as_groups = 0 takes the other row of the pair, on a transposed copy of a_scale."""
+    M, N = 300, 200
+    p = _problem(M, N, K, seed=K)
+    ref = R.gemm_fp8_block(*p)
+    for groups, name in ((1, "256x128_w2x2_cw_ks"), (0, "256x128_w2x2_cw")):
+        for split in (1, 2, 3):
+            for off in (0, 1):
+                say("scale groups, copying waves, pinned", (M, N, K), dtype, groups, split, off)
+                Q.force_config("256x128_w2x2_cw")
+                Q.set_option("as_groups", groups)
+                Q.set_option("force_split", split)
+                assert np.array_equal(_run(*p, dtype, off), ref)
+                assert Q.last_config() == name + (f"_splitk{split}" if split > 1 else "")
