@@ -81,22 +81,25 @@ _torch_ext = None
 def load_torch_extension():
     """The module `qgemm_python` (qgemm_amd/qgemm_python*.so, built by csrc/build_torch_ext.py): the
     torch-facing entry points fp8_mm / int8_mm / bf16_mm the reference's packaging names (setup.py:73).
-    Raises ImportError when it has not been built."""
+    Raises ImportError when it has not been built for the running Python."""
     global _torch_ext
     if _torch_ext is None:
-        import glob
+        import importlib.machinery
         import importlib.util
 
         import torch  # noqa: F401  (its libraries must be loaded first)
 
         load_library()
-        found = glob.glob(os.path.join(_HERE, "qgemm_python*.so"))
+        # (the endings this Python loads, its own before the general ones: modules built for others may lie beside it)
+        paths = [os.path.join(_HERE, "qgemm_python" + ending) for ending in importlib.machinery.EXTENSION_SUFFIXES]
+        found = [path for path in paths if os.path.exists(path)]
         if not found:
-            raise ImportError(f"{_HERE}/qgemm_python*.so is missing: run `python qgemm_amd/csrc/build_torch_ext.py` "
+            raise ImportError(f"{paths[0]} is missing: run `python qgemm_amd/csrc/build_torch_ext.py` "
                               "(or __graft_entry__.build())")
         spec = importlib.util.spec_from_file_location("qgemm_python", found[0])
-        _torch_ext = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(_torch_ext)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _torch_ext = module                  # (only once it has loaded)
     return _torch_ext
 
 

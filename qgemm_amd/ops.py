@@ -11,6 +11,7 @@ Tensors are torch CUDA(HIP) tensors; only their data pointers and the current
 stream cross the boundary."""
 import ctypes as C
 import os
+import warnings
 
 import torch
 
@@ -32,16 +33,23 @@ _native_module = None
 
 
 def _native():
-    """The extension module that reads the tensors and calls the library in one step, or False: it has not been built, or
-    QGEMM_LIBRARY names a library it is not linked to.  The functions below then go through ctypes, to the same entries.
+    """The extension module that reads the tensors and calls the library in one step, or False: QGEMM_LIBRARY names a library
+    it is not linked to, or it cannot be used (not built for this Python, or built before it had what is called here), which
+    is said once.  The functions below then go through ctypes, to the same entries.
     (Host time of quantise and multiply, 1 x 2048 x 1024: 11.6 + 8.4 us through ctypes, 4.3 + 3.6 us through the module.)"""
     global _native_module
     if _native_module is None:
-        try:
-            _native_module = False if os.environ.get("QGEMM_LIBRARY") else load_torch_extension()
-        except ImportError:
+        _native_module = False
+        if not os.environ.get("QGEMM_LIBRARY"):
             load_library()                      # (its absence is an error, not a reason to go another way)
-            _native_module = False
+            try:
+                module = load_torch_extension()
+                missing = [f for f in ("ops_gemm", "ops_scaled_gemm", "ops_transpose", "ops_quantize") if not hasattr(module, f)]
+                if missing:
+                    raise ImportError(f"{getattr(module, '__file__', 'qgemm_python')} has no {', '.join(missing)}: build it again")
+                _native_module = module
+            except ImportError as e:
+                warnings.warn(f"calls go through ctypes, at twice the host time: {e}", RuntimeWarning, stacklevel=3)
     return _native_module
 
 
