@@ -6,41 +6,33 @@
 namespace qgemm {
 
 // ---------------------------------------------------------------------------
-// Transpose: out[n*M + m] = in[m*N + n]   (src/transpose/transpose.cu:11-58).
-// 64 x 64 element tile through LDS, 256 threads.  The LDS tile is stored with
-// its 4-byte words XOR-swizzled by the row, so both the row-wise fill and the
-// column-wise drain touch 32 distinct banks; no padding column.  Any M, N.
+// Transpose of 4-byte elements: out[n*M + m] = in[m*N + n]   (src/transpose/transpose.cu:11-58).
+// 64 x 64 element tile through LDS, 256 threads.  The columns of the LDS tile are XOR-swizzled by
+// the row, so both the row-wise fill and the column-wise drain touch all banks; no padding column.
+// Any M, N.
 // ---------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(256) transpose_kernel(const T *__restrict__ in, T *__restrict__ out, uint32_t M,
-                                                        uint32_t N) {
+__global__ void __launch_bounds__(256) transpose_u32_kernel(const uint32_t *__restrict__ in, uint32_t *__restrict__ out, uint32_t M,
+                                                            uint32_t N) {
     constexpr int TILE = 64;
-    __shared__ T tile[TILE][TILE];
+    __shared__ uint32_t tile[TILE][TILE];
     const uint32_t m0 = blockIdx.y * TILE, n0 = blockIdx.x * TILE;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;   // 64 x 4
-    constexpr int PER_WORD = sizeof(T) >= 4 ? 1 : 4 / sizeof(T);
 #pragma unroll
     for (int r = ty; r < TILE; r += 4) {
         const uint32_t m = m0 + r, n = n0 + tx;
-        if (m < M && n < N) {
-            const int word = (tx / PER_WORD) ^ (r & (TILE / PER_WORD - 1));
-            tile[r][word * PER_WORD + tx % PER_WORD] = in[(size_t)m * N + n];
-        }
+        if (m < M && n < N) tile[r][tx ^ r] = in[(size_t)m * N + n];
     }
     __syncthreads();
 #pragma unroll
     for (int r = ty; r < TILE; r += 4) {
         const uint32_t n = n0 + r, m = m0 + tx;   // output row n, column m
-        if (n < N && m < M) {
-            const int word = (r / PER_WORD) ^ (tx & (TILE / PER_WORD - 1));
-            out[(size_t)n * M + m] = tile[tx][word * PER_WORD + r % PER_WORD];
-        }
+        if (n < N && m < M) out[(size_t)n * M + m] = tile[tx][r ^ tx];
     }
 }
 
 // ---------------------------------------------------------------------------
-// Byte transpose for shapes with M % 16 == 0, N % 4 == 0 and 16-byte aligned rows (the fp8 / int8
-// operands of the reference layout).  128 x 128 tile, 256 threads.  A thread loads 4 x 4 bytes (four
+// Byte transpose (the fp8 / int8 operands of the reference layout, packed operands, matrix_transpose).
+// 128 x 128 tile, 256 threads.  A thread loads 4 x 4 bytes (four
 // rows, one dword each: a wave reads whole 128-byte row pieces), transposes the 4 x 4 block in
 // registers with byte permutes, and writes the four resulting dwords (4 consecutive m of one n)
 // into the LDS tile [n][m]; the tile leaves as 16-byte pieces of output rows, 128 bytes per row.
@@ -128,8 +120,8 @@ __global__ void __launch_bounds__(256) transpose_bytes2_kernel(const Transpose2A
 }
 
 // ---------------------------------------------------------------------------
-// 2-byte transpose.  Written for shapes with M % 8 == 0, N % 8 == 0 and 16-byte aligned rows (what
-// matrix_transpose<bf16 / fp16> of the reference is called with, src/transpose/transpose.cu:60-74).
+// 2-byte transpose (matrix_transpose<bf16 / fp16>, src/transpose/transpose.cu:60-74; 16-bit operands
+// stored K x N; packed operands).
 // No LDS: a lane owns an 8 x 8 block.  It loads eight 16-byte row pieces, interleaves the 16-bit halves
 // of vertically adjacent dwords (one v_perm each: 32 per block), and the rest of the transposition is
 // which register goes into which output dword.  Lanes 8g..8g+7 hold eight neighbouring column blocks,

@@ -1148,7 +1148,7 @@ int launch_transpose(int elem_bytes, const void *in, void *out, size_t M, size_t
         const auto kernel = aligned ? transpose_u16_kernel<true> : transpose_u16_kernel<false>;
         hipLaunchKernelGGL(kernel, g, dim3(256), 0, stream, (const uint16_t *)in, (uint16_t *)out, (uint32_t)M, (uint32_t)N);
     } else if (elem_bytes == 4) {
-        hipLaunchKernelGGL(transpose_kernel<uint32_t>, grid, dim3(256), 0, stream, (const uint32_t *)in, (uint32_t *)out,
+        hipLaunchKernelGGL(transpose_u32_kernel, grid, dim3(256), 0, stream, (const uint32_t *)in, (uint32_t *)out,
                            (uint32_t)M, (uint32_t)N);
     } else {
         return QGEMM_ERR_UNSUPPORTED;
