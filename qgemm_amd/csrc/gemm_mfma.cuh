@@ -1035,8 +1035,8 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
             // two waves, so that all of them count alike) to the stage's 512 bytes behind the ring.
             // That is one request per row and stage, as many again as the operands' own when the caller's a_scale is
             // K-contiguous (every lane another cache line: 2048 x 2048 x 8192 took 46 us where the same copies at
-            // contiguous addresses take 37).  Where the host finds such an a_scale aligned for it (GemmArgs::as_groups)
-            // a lane fetches the scales of four K blocks of its row at once, 16 bytes, in front of every fourth stage
+            // contiguous addresses take 37).  With such an a_scale (GemmArgs::as_groups) a lane fetches the scales of four K
+            // blocks of its row at once, 16 bytes at any 4-byte address, in front of every fourth stage
             // (waves 0 and 1 of the copying four, 64 rows each), into slot (kt / 4) % 4 of four behind the ring:
             // [row][4 K blocks].  Slot i is refilled for stage 4 i + 16, issued in phase 4 i + 17 - NS, after the last
             // read of stage 4 i + 3.  These copies are not counted: a wave that waits until (NS - 2) * NPC copies are
@@ -1414,12 +1414,10 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
     const int wave_rows = (int)p.M - (int)(row0 + wm * C::WM);
     // Every accumulator is read in exactly one place (write_slab): the output type is a uniform branch around
     // the conversion of a slab, and wave tiles that stick out of C take the same way through the scratch.  The 16-byte
-    // pieces go to any element address (rows of C that are not 16-byte aligned used to leave element by element:
-    // 1531 x 4100 x 3004 int8 to bf16, rows of 8200 bytes, 31.7 -> 23.2 us; 1999 x 3001 x 1000 bf16 28.8 -> 20.7); rows
-    // past M and pieces past N are left out, and the one piece N ends in goes in parts of 8, 4 and 2 bytes out of the
-    // registers that hold it.  (It used to go through a loop over volatile elements, each of which waited for the one before
-    // to reach memory: the workgroups of the last columns took 5 - 11 us longer than the others.  Quantise and multiply
-    // 1531 x 4100 x 3004 int8 58.8 -> 47.8 us, training step 1999 x 3001 x 1000 bf16 94.0 -> 90.8.)
+    // pieces go to any element address, rows past M and pieces past N are left out, and the one piece N ends in goes in parts
+    // of 8, 4 and 2 bytes out of the registers that hold it.  (Element by element where rows of C are not 16-byte aligned or
+    // N ends inside a piece / so, us, one process, in turn: int8 to bf16 1531 x 4100 x 3004, rows of 8200 bytes, packing and
+    // product 43.9 / 35.3; bf16 1999 x 3001 x 1000 forward 27.5 / 19.3, with its backward 97.1 / 89.4.)
     // With the accumulators of a 128 x 128 wave tile pinned in the 256 accumulation registers, several code
     // paths that each name all of them made the register allocator spill two dozen of them to memory here.
     if constexpr (EPI_FITS) {
