@@ -315,6 +315,21 @@ const TileModel kTileModels[] = {{256, 256, 1, 1.25, 1.25, 4.0, false, 1, 1.40, 
                                  {128, 128, 1, 0.43, 0.43, 4.5, true, 1, 0.50, 0.50},  {64, 128, 1, 0.52, 0.52, 1.5, false, 3, 1.21, 0.83},
                                  {64, 128, 1, 0.27, 0.27, 4.5, true, 1, 0.34, 0.34},   {128, 32, 1, 0.39, 0.39, 1.0, false, 2, 0.74, 0.60},
                                  {256, 128, 1, 0.71, 0.58, 6.0, false, 1, 0.93, 0.76}, {192, 256, 1, 1.03, 0.97, 6.0, false, 1, 1.27, 1.18}};
+// Widened fp8 (AR_F8W: packed operands): twice the matrix instructions of a 16-bit step and the conversions in front of them, on
+// the rows that family has.  Fitted on 56 ragged shapes of 1 .. 4096 rows x 1024 .. 7168 columns x 777 .. 7161, every row forced
+// (within 5 % of the measured time on average).  Priced as fp8 before, us in a kernel trace: 512 x 4608 x 7161 58.5 (128 x 128) ->
+// 44.4 (192 x 256, four slices), 1024 x 4608 x 7161 88.6 -> 69.8, block scales 512 x 5000 x 3004 41.7 (64 x 128 with K groups) ->
+// 30.3 (128 x 32).
+const TileModel kWideTileModels[] = {{128, 128, 2, 1.55, 0.96, 3.5, false, 2, 1.95, 1.19}, {64, 128, 1, 0.70, 0.72, 3.0, false, 3, 1.49, 0.87},
+                                     {64, 128, 1, 0.41, 0.44, 4.5, true, 1, 0.68, 0.72},   {128, 32, 1, 0.43, 0.47, 2.0, false, 3, 0.99, 0.71},
+                                     {192, 256, 1, 1.99, 1.70, 5.5, false, 1, 2.36, 2.01}};
+// `wgs` workgroups of `steps` K steps, `slots` of them on the chip at a time
+double rounds_cost(size_t wgs, size_t slots, size_t cus, size_t steps, double shared, double alone, double fixed) {
+    const size_t full = wgs / slots, rem = wgs % slots;
+    double t = (double)full * (steps * shared + fixed);
+    if (rem) t += steps * (rem <= cus ? alone : shared) + fixed;
+    return t;
+}
 // rows with two K groups: two sets of computing waves on a tile that otherwise has one (one workgroup per CU)
 bool is_kgroup_row(const Variant &v) { return v.kgroups == 2; }
 
@@ -322,7 +337,10 @@ int choose_by_cost(const Variant *tab, int count, size_t M, size_t N, size_t kst
                    uint32_t *nsplit_out, double *cost_out = nullptr) {
     int best = -1;
     double best_t = 0;
-    for (const TileModel &tm : kTileModels) {
+    const bool wide = tab[0].arith == AR_F8W;
+    const TileModel *models = wide ? kWideTileModels : kTileModels;
+    for (size_t mi = 0; mi < (wide ? std::size(kWideTileModels) : std::size(kTileModels)); ++mi) {
+        const TileModel &tm = models[mi];
         int vi = -1;
         for (int i = 0; i < count; ++i)
             if (tab[i].auto_ok && tab[i].bm == tm.bm && tab[i].bn == tm.bn && is_kgroup_row(tab[i]) == tm.kgroups) vi = i;
@@ -331,10 +349,7 @@ int choose_by_cost(const Variant *tab, int count, size_t M, size_t N, size_t kst
         for (uint32_t ns = 1; ns <= 8; ns *= 2) {
             if (ns > 1 && (!may_split || ksteps / ns < 4)) break;
             const size_t wgs = tiles * ns, slots = (size_t)cus * (block ? tm.blk_per_cu : tm.per_cu), steps = (ksteps + ns - 1) / ns;
-            const size_t full = wgs / slots, rem = wgs % slots;
-            const double shared = block ? tm.blk_shared : tm.step_shared, alone = block ? tm.blk_alone : tm.step_alone;
-            double t = (double)full * (steps * shared + tm.fixed);
-            if (rem) t += steps * (rem <= (size_t)cus ? alone : shared) + tm.fixed;
+            double t = rounds_cost(wgs, slots, cus, steps, block ? tm.blk_shared : tm.step_shared, block ? tm.blk_alone : tm.step_alone, tm.fixed);
             if (ns > 1) t += 4.0 + (double)M * N * 4.0 * (ns + 1) / 3.0e6;
             if (best < 0 || t < best_t) {
                 best = vi;
@@ -972,13 +987,51 @@ int launch_nt(NtProblem q, hipStream_t stream) {
     return run_nt(q, pl, ws, stream);
 }
 
-// Is a product on the any-shape path large enough for the packing launch and the other kernels?  The any-shape kernel
-// takes one launch and, per 128 bytes of K and round of tiles, some 1.5 us; twice that where it has to transpose (km).
-// Eager calls, us (7 of them the host's), any-shape kernel / packed: int8 16 x 1001 K = 401 7.1 / 11.2, 2001 10.9 / 12.0;
-// 256 x 4097 1041 11.2 / 18.3, 2001 15.9 / 21.1; 1024 x 2049 401 12.0 / 15.3, 1041 18.1 / 19.2, 2001 26.8 / 23.7;
-// 4096 x 4097 33 28.1 / 24.0, 2001 88.4 / 55.3; bf16 1024 x 2049 401 15.2 / 16.7, 801 21.8 / 20.3, with B stored K x N
-// 261 15.5 / 15.7, 401 18.4 / 16.7; 16 x 1001 401 8.8 / 11.7, 801 13.5 / 11.7.
-bool pack_pays(size_t M, size_t N, size_t kbytes, bool km) { return kbytes > (km ? 512 : 1024) || (double)M * N >= 4e6; }
+// Tile side of the any-shape kernel (block: with block scales; km: an operand is transposed on the way): 128 x 128 tiles where
+// they make at least one round of the CUs, half of one where operands are transposed: 64 x 64 / 128 x 128, us, K = 1001 and
+// 3001: int8 512 x 4097 (132 tiles) 15.7 / 16.9 33.3 / 35.8, 1024 x 4097 (264) 22.7 / 22.5 52.2 / 44.1, 1500 x 4097 30.3 / 23.9
+// 70.7 / 45.6; bf16 with B stored K x N 512 x 4097 33.2 / 30.6 87.8 / 78.1.
+int any_tile(int in_dtype, bool block, bool km, size_t M, size_t N) {
+    if (block && (km || in_dtype == QGEMM_DT_I8)) return 64;        // (the partial products of int8 blocks would not fit the registers)
+    const uint64_t wide = ((uint64_t)M + 127) / 128 * (((uint64_t)N + 127) / 128);
+    return wide * (km ? 2 : 1) >= (uint64_t)g_ctx.num_cus ? 128 : 64;
+}
+
+// Is a product on the any-shape path faster packed?  Estimates of both, in microseconds, fitted on 240 ragged shapes (1 .. 4096
+// rows x 1024 .. 7168 columns x K = 777 .. 7161; fp8 and int8 with one scale and with block scales, bf16), eager calls: the way
+// chosen is 0.7 % behind the faster one on average, 33 % at worst (int8 block scales 200 x 5000 x 3004 20.4 / 27.1).  Two
+// thresholds on the sizes, K and M N, were 21 % behind on average.  Any-shape kernel / packed: int8 1 x 2048 x 1032 8.2 / 13.3,
+// 512 x 3000 x 1500 11.1 / 21.2, 1024 x 4096 x 2001 28.4 / 26.9, 4096 x 4096 x 2001 68.4 / 45.5, fp8 64 x 7168 x 2056 17.5 / 22.1,
+// 512 x 2048 x 1032 11.2 / 17.8, 4096 x 4608 x 7161 356 / 234, bf16 512 x 2048 x 1036 11.4 / 17.7, 2048 x 3000 x 1500 40.4 / 33.6.
+// Operands that are transposed on the way (km) make the any-shape kernel twice as slow: thresholds do there (bf16 with B stored
+// K x N 1024 x 2049 x 261 15.5 / 15.7, x 401 18.4 / 16.7).
+bool pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
+    const size_t kbytes = K * dtype_bytes(in_dtype), cus = g_ctx.num_cus;
+    if (km) return kbytes > 512 || (double)q.M * q.N >= 4e6;
+    // any-shape kernel: 64 x 64 tiles, three on a CU, and 128 x 128, two on a CU
+    struct AnyModel {
+        double shared64, alone64, fixed64, shared128, alone128, fixed128;
+    };
+    static const AnyModel kAny16{0.68, 0.45, 3.6, 1.29, 0.90, 10.4}, kAnyF8{0.63, 0.43, 3.2, 1.11, 0.72, 8.6},
+        kAnyF8Block{0.72, 0.48, 2.7, 1.37, 0.99, 6.6}, kAnyI8{0.81, 0.47, 3.4, 1.37, 0.94, 8.9}, kAnyI8Block{1.18, 0.67, 1.6, 0, 0, 0};
+    const AnyModel &m = in_dtype == QGEMM_DT_F8E4M3 ? (q.block ? kAnyF8Block : kAnyF8) : (in_dtype == QGEMM_DT_I8 ? (q.block ? kAnyI8Block : kAnyI8) : kAny16);
+    const size_t tile = any_tile(in_dtype, q.block, false, q.M, q.N), any_steps = (K - 1) / (in_dtype == QGEMM_DT_I8 ? 128 : 64) + 1;
+    const size_t tiles = ((q.M + tile - 1) / tile) * ((q.N + tile - 1) / tile);
+    const double t_any = tile == 64 ? rounds_cost(tiles, 3 * cus, cus, any_steps, m.shared64, m.alone64, m.fixed64)
+                                    : rounds_cost(tiles, 2 * cus, cus, any_steps, m.shared128, m.alone128, m.fixed128);
+    // packed: two launches and the packing, then the tiles' estimate or the skinny-M kernel's (see choose_variant)
+    int count = 0;
+    const Variant *tab = table_for(q.arith, q.block, 0, &count);
+    uint32_t nsplit = 0;
+    double t_rows = 0;
+    const size_t steps = (kbytes + 127) / 128;
+    if (!tab || choose_by_cost(tab, count, q.M, q.N, steps, q.block, (int)cus, true, &nsplit, &t_rows) < 0) return false;
+    if (q.M <= 256) {
+        const size_t bm = q.M <= 16 ? 16 : (q.M <= 32 ? 32 : 64), strips = ((q.M + 63) / 64) * ((q.N + 31) / 32);
+        t_rows = std::min(t_rows, std::max(4.0, (bm + 32) * steps * 128.0 / 50.0e3) * std::max(1.0, (double)strips / cus));
+    }
+    return 12.0 + 0.2e-6 * (double)(q.M + q.N) * kbytes + t_rows < t_any;
+}
 
 // Operands that no MFMA kernel reads as they stand: pack_kernel writes what has to change into the workspace as rows of
 // whole 128-byte K steps (one launch for both operands), and the K-contiguous kernels take it from there.  a_src / b_src:
@@ -1007,7 +1060,7 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
     const size_t eb = dtype_bytes(in_dtype);
     if (!g_ctx.any_shape) return QGEMM_OK;
     if (q.arith == AR_F8) q.arith = AR_F8W;
-    if (g_ctx.any_shape == 1 && !pack_pays(q.M, q.N, K * eb, a_src.k_major || b_src.k_major)) return QGEMM_OK;
+    if (g_ctx.any_shape == 1 && !pack_pays(q, in_dtype, K, a_src.k_major || b_src.k_major)) return QGEMM_OK;
     if (g_ctx.static_call || stream_is_capturing(stream)) return QGEMM_OK;
     if (q.M >= ((size_t)1 << 31) || q.N >= ((size_t)1 << 31) || K >= ((size_t)1 << 30)) return QGEMM_OK;
     // (a K that ends inside a 16-byte piece has to end in zeros in both operands)
@@ -1081,13 +1134,9 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
         hipLaunchKernelGGL((gemm_short_kernel<DT, BLOCK>), dim3((unsigned)((elements + 255) / 256)), dim3(256), 0, stream, a);
         return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
     }
-    // 128 x 128 tiles where they make at least one round of the CUs, half of one where operands are transposed on the way:
-    // 64 x 64 / 128 x 128, us, K = 1001 and 3001: int8 512 x 4097 (132 tiles) 15.7 / 16.9 33.3 / 35.8, 1024 x 4097 (264) 22.7 /
-    // 22.5 52.2 / 44.1, 1500 x 4097 30.3 / 23.9 70.7 / 45.6; bf16 with B stored K x N 512 x 4097 33.2 / 30.6 87.8 / 78.1.
-    constexpr int W = BLOCK && DT == QGEMM_DT_I8 ? 64 : 128;        // (the partial products of int8 blocks would not fit the registers)
+    constexpr int W = BLOCK && DT == QGEMM_DT_I8 ? 64 : 128;
     const bool km = a.a.k_major || a.b.k_major;
-    const uint64_t wide = ((uint64_t)a.a.rows + 127) / 128 * (((uint64_t)a.b.rows + 127) / 128);
-    const int T = wide * (km ? 2 : 1) >= (uint64_t)g_ctx.num_cus && !(BLOCK && km) ? W : 64;
+    const int T = any_tile(DT, BLOCK, km, a.a.rows, a.b.rows);
     a.tiles_m = (uint32_t)(((uint64_t)a.a.rows + T - 1) / T);
     a.tiles_n = (uint32_t)(((uint64_t)a.b.rows + T - 1) / T);
     const uint64_t tiles = (uint64_t)a.tiles_m * a.tiles_n;

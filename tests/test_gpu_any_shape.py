@@ -71,11 +71,13 @@ def test_leading_dimensions_and_pointers(K, dtype, layout):
     Q.set_option("any_shape", 2)
     for pads, offs in (((3, 0), (0, 0)), ((0, 5), (1, 0)), ((7, 1), (3, 5)), ((0, 0), (0, 1))):
         say("any shape, strides", dtype, layout, pads, offs)
-        c = torch.full((M, N + 3), 7.0, dtype=torch.float32, device="cuda")[:, :N]
+        wide = torch.full((M, N + 3), 7.0, dtype=torch.float32, device="cuda")
+        c = wide[:, :N]
         Q.gemm(_tensor(a, dtype, pads[0], offs[0]), _tensor(bt, dtype, pads[1], offs[1]), c, layout)
         if layout == "nk" or K % 16 or pads != (0, 0):        # (else B goes through the transpose kernel alone)
             assert _ran(2), Q.last_config()
         assert torch.equal(c.cpu(), ref)
+        assert bool((wide[:, N:] == 7).all())            # (what lies between the rows of C)
 
 
 @pytest.mark.parametrize("dtype", [torch.int8, torch.float8_e4m3fn])
@@ -166,3 +168,16 @@ def test_rows_of_c_that_end_inside_a_piece(row, out):
             assert bool((c[:, N:] == 7).all()), N
     finally:
         Q.force_config(None)
+
+
+@pytest.mark.parametrize("dtype", [torch.float8_e4m3fn, torch.int8, torch.bfloat16])
+@pytest.mark.parametrize("shape, packed", [((16, 2048, 1036), False), ((2048, 2048, 4001), True)])
+def test_the_way_that_is_estimated_faster(shape, packed, dtype):
+    M, N, K = shape
+    say("any shape, by the estimate", shape, dtype)
+    rng = np.random.default_rng(K)
+    a, b = _ints(rng, (M, K)), _ints(rng, (N, K))
+    c = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    Q.gemm(_tensor(a, dtype), _tensor(b, dtype), c)
+    assert _ran(2 if packed else 0), Q.last_config()
+    assert torch.equal(c.cpu(), torch.from_numpy(a) @ torch.from_numpy(b).t())
