@@ -126,3 +126,31 @@ def test_two_streams_share_the_workspace_in_order():
     for r in range(rounds):
         assert torch.equal(ci[r], ci_ref), f"int8 round {r}"
         assert torch.equal(cf[r].view(torch.int16), cf_ref.view(torch.int16)), f"fp8 round {r}"
+
+
+def test_packed_operands_on_two_streams():
+    """Eager products whose operands are packed into the workspace first, on two streams with no host synchronisation in
+    between: each waits for the other's use of the block, so every result is the oracle's."""
+    say("two streams, packed operands")
+    M, N, K, rounds = 300, 520, 2003, 12
+    jobs = []
+    Q.set_option("any_shape", 2)
+    try:
+        for seed in (91, 92):
+            rng = np.random.default_rng(seed)
+            a, b = (rng.integers(-127, 128, (r, K)).astype(np.int8) for r in (M, N))
+            jobs.append((dev(a), dev(b), R.gemm_i8_i32(a, b), torch.cuda.Stream(),
+                         [torch.zeros((M, N), dtype=torch.int32, device="cuda") for _ in range(rounds)]))
+        one = scalar(1)
+        torch.cuda.synchronize()
+        for r in range(rounds):
+            for a8, b8, _, stream, c in jobs:
+                with torch.cuda.stream(stream):
+                    Q.int8_mm(a8, b8, one, one, c[r])
+                assert Q.last_config().startswith("pack+"), Q.last_config()
+        torch.cuda.synchronize()
+    finally:
+        Q.set_option("any_shape", 1)
+    for _, _, ref, _, c in jobs:
+        for r in range(rounds):
+            assert np.array_equal(host(c[r]), ref), r
