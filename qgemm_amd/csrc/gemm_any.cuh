@@ -205,9 +205,20 @@ struct AnyStage {
     }
 };
 
-template <int IN_DT, bool BLOCK, int T, bool KM>
+// How the products of K are added up: in one chain of matrix instructions; in blocks of 128 elements of K from zero, folded into
+// fp32 sums with their scales; or a step at a time from zero, added to fp32 sums.  The matrix instructions do not round to
+// nearest, so a chain's error grows with its length, where the rows for few rows, which share K among waves, have eight short
+// ones.  So 16-bit operands with fp32 output are folded on 64 x 64 tiles, into two sums in turn (relative error, bf16 to fp32,
+// eight chains / one chain / one sum / two: 16 x 2048 x 1036 8.4e-8 / 18.4e-8 / 9.1e-8 / 7.8e-8, 64 x 7168 x 2060 10.4e-8 /
+// 27.3e-8 / 11.7e-8 / 9.4e-8); on 128 x 128 tiles, where the other kernels have one chain too and more sums do not fit the
+// registers, they are not.  A 16-bit output hides the difference.  Blocks of int8 alternate too (512 x 5000 x 3004 to fp32,
+// other kernels / one sum / two: 7.5e-8 / 9.4e-8 / 7.4e-8).
+enum AnySum : int { ANY_CHAIN = 0, ANY_SCALED = 1, ANY_FOLDED = 2 };
+
+template <int IN_DT, int SUM, int T, bool KM>
 __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
+    constexpr bool BLOCK = SUM == ANY_SCALED;
     typedef AnyStage<IN_DT, T, KM> S;
     constexpr int KE = S::KE, W = T / 2, F = W / 16;                    // wave tile W x W, F x F MFMA tiles
     constexpr bool I8 = IN_DT == QGEMM_DT_I8;
@@ -225,12 +236,16 @@ __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
             return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, x), __builtin_bit_cast(v8h, y), c, 0, 0, 0);
         else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, x), __builtin_bit_cast(v8bf, y), c, 0, 0, 0);
     };
-    acc_t acc[F][F];
+    constexpr int SUMS = SUM == ANY_FOLDED || (BLOCK && I8) ? 2 : 1;    // one of the even and one of the odd steps
+    acc_t sums[SUMS][F][F];
+    auto &acc = sums[0];
     part_t part[F][F];
 #pragma unroll
-    for (int a = 0; a < F; ++a)
+    for (int i = 0; i < SUMS; ++i)
 #pragma unroll
-        for (int b = 0; b < F; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
+        for (int a = 0; a < F; ++a)
+#pragma unroll
+            for (int b = 0; b < F; ++b) sums[i][a][b] = acc_t{0, 0, 0, 0};
     struct Stage {
         S a, b;
     } held[2];                                                          // of an even and of an odd step
@@ -262,21 +277,43 @@ __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
                 f[a] = p.as[(size_t)m * p.as_ms + (size_t)kb * p.as_ks] * bs;
             }
         }
+        auto frag = [&](const char *l, int r, int h) { return *(const v4i *)(l + S::slot(r + (lane & 15), h * 4 + (lane >> 4))); };
+        if constexpr (SUM == ANY_FOLDED) {
+            v4i fb[2][F];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            v4i fa[F], fb[F];
+            for (int i = 0; i < F; ++i)
 #pragma unroll
-            for (int i = 0; i < F; ++i) {
-                fa[i] = *(const v4i *)(la + S::slot(wm + i * 16 + (lane & 15), h * 4 + (lane >> 4)));
-                fb[i] = *(const v4i *)(lb + S::slot(wn + i * 16 + (lane & 15), h * 4 + (lane >> 4)));
+                for (int h = 0; h < 2; ++h) fb[h][i] = frag(lb, wn + i * 16, h);
+#pragma unroll
+            for (int a = 0; a < F; ++a) {
+                const v4i fa0 = frag(la, wm + a * 16, 0), fa1 = frag(la, wm + a * 16, 1);
+                part_t q[F];
+#pragma unroll
+                for (int b = 0; b < F; ++b) q[b] = mma(fb[0][b], fa0, part_t{0, 0, 0, 0});
+#pragma unroll
+                for (int b = 0; b < F; ++b) q[b] = mma(fb[1][b], fa1, q[b]);
+#pragma unroll
+                for (int b = 0; b < F; ++b)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sums[odd][a][b][r] += q[b][r];
             }
+        } else {
 #pragma unroll
-            for (int a = 0; a < F; ++a)
+            for (int h = 0; h < 2; ++h) {
+                v4i fa[F], fb[F];
 #pragma unroll
-                for (int b = 0; b < F; ++b) {
-                    if constexpr (BLOCK) part[a][b] = mma(fb[b], fa[a], FIRST && h == 0 ? part_t{0, 0, 0, 0} : part[a][b]);
-                    else acc[a][b] = mma(fb[b], fa[a], acc[a][b]);
+                for (int i = 0; i < F; ++i) {
+                    fa[i] = frag(la, wm + i * 16, h);
+                    fb[i] = frag(lb, wn + i * 16, h);
                 }
+#pragma unroll
+                for (int a = 0; a < F; ++a)
+#pragma unroll
+                    for (int b = 0; b < F; ++b) {
+                        if constexpr (BLOCK) part[a][b] = mma(fb[b], fa[a], FIRST && h == 0 ? part_t{0, 0, 0, 0} : part[a][b]);
+                        else acc[a][b] = mma(fb[b], fa[a], acc[a][b]);
+                    }
+            }
         }
         if (BLOCK && (I8 || odd || s + 1 == steps)) {
 #pragma unroll
@@ -284,7 +321,7 @@ __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
 #pragma unroll
                 for (int b = 0; b < F; ++b)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[a][b][r] += (float)part[a][b][r] * f[a];
+                    for (int r = 0; r < 4; ++r) sums[SUMS == 2 && odd][a][b][r] += (float)part[a][b][r] * f[a];
         }
         store(s + 1, next);
     };
@@ -318,7 +355,7 @@ __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
             }
             float v[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = (float)acc[a][b][r] * scale;
+            for (int r = 0; r < 4; ++r) v[r] = (float)(SUMS == 2 ? acc[a][b][r] + sums[SUMS - 1][a][b][r] : acc[a][b][r]) * scale;
             store_out4(p.C, idx, v, p.out_dtype, valid);
         }
     }

@@ -990,11 +990,13 @@ int launch_nt(NtProblem q, hipStream_t stream) {
 // Tile side of the any-shape kernel (block: with block scales; km: an operand is transposed on the way): 128 x 128 tiles where
 // they make at least one round of the CUs, half of one where operands are transposed: 64 x 64 / 128 x 128, us, K = 1001 and
 // 3001: int8 512 x 4097 (132 tiles) 15.7 / 16.9 33.3 / 35.8, 1024 x 4097 (264) 22.7 / 22.5 52.2 / 44.1, 1500 x 4097 30.3 / 23.9
-// 70.7 / 45.6; bf16 with B stored K x N 512 x 4097 33.2 / 30.6 87.8 / 78.1.
-int any_tile(int in_dtype, bool block, bool km, size_t M, size_t N) {
+// 70.7 / 45.6; bf16 with B stored K x N 512 x 4097 33.2 / 30.6 87.8 / 78.1 (with fp32 output the smaller tiles, which add up more
+// exactly: any_folded).
+bool any_folded(int in_dtype, int out_dtype) { return dtype_bytes(in_dtype) == 2 && out_dtype == QGEMM_DT_F32; }
+int any_tile(int in_dtype, int out_dtype, bool block, bool km, size_t M, size_t N) {
     if (block && (km || in_dtype == QGEMM_DT_I8)) return 64;        // (the partial products of int8 blocks would not fit the registers)
     const uint64_t wide = ((uint64_t)M + 127) / 128 * (((uint64_t)N + 127) / 128);
-    return wide * (km ? 2 : 1) >= (uint64_t)g_ctx.num_cus ? 128 : 64;
+    return wide * (km && !any_folded(in_dtype, out_dtype) ? 2 : 1) >= (uint64_t)g_ctx.num_cus ? 128 : 64;
 }
 
 // Is a product on the any-shape path faster packed?  Estimates of both, in microseconds, fitted on 240 ragged shapes (1 .. 4096
@@ -1015,7 +1017,7 @@ bool pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
     static const AnyModel kAny16{0.68, 0.45, 3.6, 1.29, 0.90, 10.4}, kAnyF8{0.63, 0.43, 3.2, 1.11, 0.72, 8.6},
         kAnyF8Block{0.72, 0.48, 2.7, 1.37, 0.99, 6.6}, kAnyI8{0.81, 0.47, 3.4, 1.37, 0.94, 8.9}, kAnyI8Block{1.18, 0.67, 1.6, 0, 0, 0};
     const AnyModel &m = in_dtype == QGEMM_DT_F8E4M3 ? (q.block ? kAnyF8Block : kAnyF8) : (in_dtype == QGEMM_DT_I8 ? (q.block ? kAnyI8Block : kAnyI8) : kAny16);
-    const size_t tile = any_tile(in_dtype, q.block, false, q.M, q.N), any_steps = (K - 1) / (in_dtype == QGEMM_DT_I8 ? 128 : 64) + 1;
+    const size_t tile = any_tile(in_dtype, q.out_dtype, q.block, false, q.M, q.N), any_steps = (K - 1) / (in_dtype == QGEMM_DT_I8 ? 128 : 64) + 1;
     const size_t tiles = ((q.M + tile - 1) / tile) * ((q.N + tile - 1) / tile);
     const double t_any = tile == 64 ? rounds_cost(tiles, 3 * cus, cus, any_steps, m.shared64, m.alone64, m.fixed64)
                                     : rounds_cost(tiles, 2 * cus, cus, any_steps, m.shared128, m.alone128, m.fixed128);
@@ -1136,13 +1138,16 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
     }
     constexpr int W = BLOCK && DT == QGEMM_DT_I8 ? 64 : 128;
     const bool km = a.a.k_major || a.b.k_major;
-    const int T = any_tile(DT, BLOCK, km, a.a.rows, a.b.rows);
+    const int T = any_tile(DT, a.out_dtype, BLOCK, km, a.a.rows, a.b.rows);
     a.tiles_m = (uint32_t)(((uint64_t)a.a.rows + T - 1) / T);
     a.tiles_n = (uint32_t)(((uint64_t)a.b.rows + T - 1) / T);
     const uint64_t tiles = (uint64_t)a.tiles_m * a.tiles_n;
     if (tiles >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;    // grid limit
-    const auto kernel = T == 64 ? (km ? gemm_any_kernel<DT, BLOCK, 64, true> : gemm_any_kernel<DT, BLOCK, 64, false>)
-                                : (km ? gemm_any_kernel<DT, BLOCK, BLOCK ? 64 : W, true> : gemm_any_kernel<DT, BLOCK, W, false>);
+    constexpr int SUM = BLOCK ? ANY_SCALED : ANY_CHAIN;
+    auto kernel = T == 64 ? (km ? gemm_any_kernel<DT, SUM, 64, true> : gemm_any_kernel<DT, SUM, 64, false>)
+                          : (km ? gemm_any_kernel<DT, SUM, BLOCK ? 64 : W, true> : gemm_any_kernel<DT, SUM, W, false>);
+    if constexpr (DT == QGEMM_DT_BF16 || DT == QGEMM_DT_F16)
+        if (T == 64 && any_folded(DT, a.out_dtype)) kernel = km ? gemm_any_kernel<DT, ANY_FOLDED, 64, true> : gemm_any_kernel<DT, ANY_FOLDED, 64, false>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(256), 0, stream, a);
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }

@@ -67,3 +67,21 @@ def test_block_scales(shape, dtype):
     assert torch.equal(c.cpu(), ref)
     if dtype == torch.int8 and M < 100:
         assert torch.equal(c.cpu(), torch.from_numpy(R.gemm_i8_block(a.astype(np.int8), b.astype(np.int8), as_, bs)))
+
+
+@pytest.mark.parametrize("layout", ["nk", "kn"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_sums_of_16_bit_operands(dtype, layout):
+    """fp32 output: steps of 64 products are added to two fp32 sums in turn.  The 33 / 2 additions into a sum that grows like their
+    square root, each rounded to half of 2^-23 and uniform, leave 2^-24 / sqrt(3) * sqrt(33 / 4) = 9.9e-8 of the result; a chain of
+    matrix instructions over the same K leaves 2.7e-7."""
+    M, N, K = 64, 300, 2060
+    say("any-shape kernel, 16-bit operands to fp32", dtype, layout)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    a, b = (torch.randn(r, K, generator=g, device="cuda").to(dtype) for r in (M, N))
+    c = torch.zeros(M, N, device="cuda")
+    Q.gemm(a, b if layout == "nk" else b.t().contiguous(), c, layout)
+    assert Q.last_config() == "strided_any_shape"
+    ref = a.double().cpu() @ b.double().cpu().t()
+    assert float((c.double().cpu() - ref).norm() / ref.norm()) < 1.4e-7
