@@ -263,61 +263,64 @@ __global__ void __launch_bounds__(256) pack_kernel(const PackArgs a) {
 // Split-K second pass: C[m,n] = cast(scale * sum_z part[z][m,n]), z ascending
 // (a fixed order, so results do not depend on scheduling; int32 stays exact).
 // ---------------------------------------------------------------------------
-struct ReduceArgs {
-    const void *part;      // [nsplit][M][N] f32 or i32
-    void *C;
-    const float *as, *bs;
-    uint32_t M, N, nsplit;
-    uint64_t ldc, plane;   // plane = M*N elements
-    int out_dtype, per_matrix_scale;
-};
-
 // Four elements of a row per thread, at any alignment (the last group of a row may be shorter), the loads of up to eight
 // planes in flight together, then the sums in the order of the planes.  The launch is bound by latency, not by the
 // 5 - 30 MB it reads: one element per thread with a dependent chain of loads took 4.2 us for 160 x 2048 in four planes,
 // 11 us for 512 x 4096.
+// part: [nsplit][M][N] f32 or i32; inv: inverse_of(groups of four in a row); scaled: the two scales are applied here.
+// (Arguments of their own, not a struct: they arrive in scalar registers with the wave, see LaunchHead.)
 template <bool IS_I32>
-__global__ void __launch_bounds__(256) splitk_reduce4_kernel(const ReduceArgs p) {
+__global__ void __launch_bounds__(256)
+splitk_reduce4_kernel(const void *part, void *C, const float *as, const float *bs, uint32_t M, uint32_t N, uint32_t nsplit,
+                      uint32_t ldc, uint32_t inv, uint32_t out_dtype, uint32_t scaled) {
     typedef typename std::conditional<IS_I32, v4i, v4f>::type vec_t;
     typedef typename std::conditional<IS_I32, v4i_any, v4f_any>::type vec_any;
     typedef typename std::conditional<IS_I32, int, float>::type elem_t;
-    const uint32_t per_row = (p.N + 3) / 4;
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (size_t)p.M * per_row) return;
-    const uint32_t m = (uint32_t)(i / per_row), n = (uint32_t)(i % per_row) * 4;
-    const int valid = p.N - n < 4 ? (int)(p.N - n) : 4;
-    const size_t idx = (size_t)m * p.ldc + n;
-    const elem_t *src = (const elem_t *)p.part + (size_t)m * p.N + n;
+    const uint32_t per_row = (N + 3) / 4;
+    const size_t plane = (size_t)M * N, total = (size_t)M * per_row, i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    const float sa = scaled ? as[0] : 1.0f, sb = scaled ? bs[0] : 1.0f;
+    uint32_t m, n;
+    if (total >> 32) {
+        m = (uint32_t)(i / per_row);
+        n = (uint32_t)(i % per_row);
+    } else {
+        m = div_by_inv((uint32_t)i, per_row, inv, n);
+    }
+    n *= 4;
+    const int valid = N - n < 4 ? (int)(N - n) : 4;
+    const size_t idx = (size_t)m * ldc + n;
+    const elem_t *src = (const elem_t *)part + (size_t)m * N + n;
     vec_t acc = vec_t{0, 0, 0, 0};
     if (valid == 4) {
-        for (uint32_t z0 = 0; z0 < p.nsplit; z0 += 8) {
+        for (uint32_t z0 = 0; z0 < nsplit; z0 += 8) {
             vec_t t[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                if (z0 + j < p.nsplit) t[j] = __builtin_nontemporal_load((const vec_any *)(src + (size_t)(z0 + j) * p.plane));
+                if (z0 + j < nsplit) t[j] = __builtin_nontemporal_load((const vec_any *)(src + (size_t)(z0 + j) * plane));
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                if (z0 + j < p.nsplit) acc += t[j];
+                if (z0 + j < nsplit) acc += t[j];
         }
     } else {
-        for (uint32_t z = 0; z < p.nsplit; ++z)
+        for (uint32_t z = 0; z < nsplit; ++z)
             for (int e = 0; e < 3; ++e)
-                if (e < valid) acc[e] += src[z * p.plane + e];
+                if (e < valid) acc[e] += src[z * plane + e];
     }
     if constexpr (IS_I32) {
-        if (p.out_dtype == QGEMM_DT_I32) {
-            int *dst = (int *)p.C + idx;
+        if (out_dtype == (uint32_t)QGEMM_DT_I32) {
+            int *dst = (int *)C + idx;
             if (valid == 4) *(v4i_any *)dst = acc;
             else
                 for (int e = 0; e < valid; ++e) dst[e] = acc[e];
             return;
         }
     }
-    const float s = p.per_matrix_scale ? p.as[0] * p.bs[0] : 1.0f;
+    const float s = sa * sb;
     float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = (float)acc[e] * s;
-    store_out4(p.C, idx, v, p.out_dtype, valid);
+    store_out4(C, idx, v, (int)out_dtype, valid);
 }
 
 }  // namespace qgemm

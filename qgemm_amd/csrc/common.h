@@ -36,6 +36,9 @@ __host__ __device__ inline int dtype_bytes(int dt) {
     }
 }
 
+// bytes of an element of C (fp32, int32, or one of the 16-bit types)
+__device__ inline uint32_t c_elem_bytes(int dt) { return dt == QGEMM_DT_F32 || dt == QGEMM_DT_I32 ? 4 : 2; }
+
 // float -> bf16 bits, round to nearest even with a NaN guard: the intent of
 // src/include/fast_quat.h:4-12 (which has no guard).  The compiler lowers the
 // cast to v_cvt_pk_bf16_f32 on gfx950.
@@ -90,6 +93,21 @@ __device__ inline v2i widen_fp8(uint32_t w) {
                __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true))};
 }
 
+// i / d and i % d with inv = inverse_of(d): the estimate is at most one too small.  Four scalar instructions where the values are
+// uniform; the compiler's own division by a variable is two dozen, half of them on the vector ALU.
+__host__ __device__ inline uint32_t inverse_of(uint32_t d) {
+    return d <= 1 ? 0xFFFFFFFFu : (uint32_t)(((uint64_t)1 << 32) / d);
+}
+__host__ __device__ inline uint32_t div_by_inv(uint32_t i, uint32_t d, uint32_t inv, uint32_t &rem) {
+    uint32_t q = (uint32_t)(((uint64_t)i * inv) >> 32);
+    rem = i - q * d;
+    if (rem >= d) {
+        rem -= d;
+        ++q;
+    }
+    return q;
+}
+
 // Linear workgroup id -> (tile_m, tile_n).
 // Step 1 (XCD remap): the dispatcher deals workgroups to the 8 XCDs round
 // robin, so ids {x, x+8, x+16, ..} share an L2.  Renumber so that each XCD
@@ -98,9 +116,17 @@ __device__ inline v2i widen_fp8(uint32_t w) {
 // tile rows column by column, so that concurrently resident tiles share A
 // panels and B panels.  The group-size clamp uses the tile count (the
 // reference clamps with M in rows).
-__host__ __device__ inline void tile_map(uint32_t wg, uint32_t tiles_m, uint32_t tiles_n, uint32_t group_m,
-                                         uint32_t &tm, uint32_t &tn) {
-    const uint32_t total = tiles_m * tiles_n;
+// The divisors come with their inverses from the host: every workgroup starts with this map, in front of its first copy.
+struct TileMap {
+    uint32_t tiles_m, tiles_n, group_m;
+    uint32_t inv_group, inv_gm, inv_last;      // of a group's tiles, of group_m, of the rows in the last, shorter group
+};
+__host__ __device__ inline TileMap make_tile_map(uint32_t tiles_m, uint32_t tiles_n, uint32_t group_m) {
+    const uint32_t g = group_m > 1 ? (group_m < tiles_m ? group_m : tiles_m) : 1;
+    return TileMap{tiles_m, tiles_n, g, inverse_of(g * tiles_n), inverse_of(g), inverse_of(tiles_m % g)};
+}
+__host__ __device__ inline void tile_map(uint32_t wg, const TileMap &t, uint32_t &tm, uint32_t &tn) {
+    const uint32_t total = t.tiles_m * t.tiles_n;
     uint32_t id = wg;
     if (total >= (uint32_t)kXcds * 2) {
         const uint32_t per = (total + kXcds - 1) / kXcds;           // ids owned by a "tall" XCD
@@ -108,18 +134,11 @@ __host__ __device__ inline void tile_map(uint32_t wg, uint32_t tiles_m, uint32_t
         const uint32_t xcd = wg % kXcds, local = wg / kXcds;
         id = xcd < tall ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
     }
-    if (group_m <= 1) {
-        tm = id / tiles_n;
-        tn = id % tiles_n;
-        return;
-    }
-    const uint32_t per_group = group_m * tiles_n;
-    const uint32_t g = id / per_group;
-    const uint32_t start_m = g * group_m;
-    const uint32_t gsize = tiles_m - start_m < group_m ? tiles_m - start_m : group_m;
-    const uint32_t in_group = id % per_group;
-    tm = start_m + in_group % gsize;
-    tn = in_group / gsize;
+    uint32_t in_group, row;
+    const uint32_t start_m = div_by_inv(id, t.group_m * t.tiles_n, t.inv_group, in_group) * t.group_m;
+    const uint32_t left = t.tiles_m - start_m;
+    tn = div_by_inv(in_group, left < t.group_m ? left : t.group_m, left < t.group_m ? t.inv_last : t.inv_gm, row);
+    tm = start_m + row;
 }
 
 }  // namespace qgemm

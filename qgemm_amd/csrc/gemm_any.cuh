@@ -32,7 +32,8 @@ struct AnyArgs {
     AnyOperand a, b;
     void *C;
     const float *as, *bs;
-    uint32_t K, tiles_m, tiles_n;
+    uint32_t K;
+    TileMap map;
     uint64_t ldc;
     uint32_t as_ms, as_ks, bs_ns, bs_ks;
     int out_dtype, per_matrix_scale;
@@ -227,8 +228,8 @@ __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
     __shared__ __attribute__((aligned(1024))) char lds[2][2][T * 128];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = (wave >> 1) * W, wn = (wave & 1) * W;
     uint32_t tm, tn;
-    tile_map(blockIdx.x, p.tiles_m, p.tiles_n, 8, tm, tn);
-    const uint32_t row0 = __builtin_amdgcn_readfirstlane(tm) * T, col0 = __builtin_amdgcn_readfirstlane(tn) * T;
+    tile_map(blockIdx.x, p.map, tm, tn);
+    const uint32_t row0 = tm * T, col0 = tn * T;
     const uint32_t steps = (p.K - 1) / KE + 1;
     auto mma = [](v4i x, v4i y, part_t c) {
         if constexpr (I8) return __builtin_amdgcn_mfma_i32_16x16x64_i8(x, y, c, 0, 0, 0);

@@ -59,8 +59,9 @@ struct GemmArgs {
     uint32_t k_tail;      // bytes of K in the last step when it is partial (a multiple of 16), 0 when it is whole
     uint32_t lda, ldb;    // bytes
     uint32_t ldc;         // elements
-    uint32_t tiles_m, tiles_n, group_m;
+    TileMap map;          // tiles of the launch
     uint32_t nsplit, ksteps_per_split;
+    uint32_t inv_nsplit, inv_tiles_m, inv_nk, inv_nk_last;      // inverse_of: K slices, rows of tiles, K steps of a slice and of the last slice
     uint64_t split_stride;
     uint32_t as_ms, as_ks, bs_ns, bs_ks;
     uint32_t nb_max;      // ceil(N/128) - 1
@@ -294,8 +295,29 @@ __device__ inline void mma128_inplace(v4i x0, v4i x1, v4i y0, v4i y1, typename A
     }
 }
 
+// What a wave needs for its first copies travels in front of GemmArgs as arguments of its own: such arguments arrive in scalar
+// registers with the wave (kernarg preloading, at most 14 dwords: -amdgpu-kernarg-preload-count in the Makefile), while a field
+// of a struct is a scalar load, a trip to memory that every launch starts with.  The divisions are multiplications with inverses
+// from the host, and whatever is not needed for the first copies is located behind them.  us, as fields of the struct / so,
+// graph replays with B streamed: fp8 1 x 2048 x 1024 3.82 / 3.22 (one scale), 3.75 / 3.34 (block scales), 16 x 7168 x 2048 5.59 /
+// 5.10 and 5.77 / 5.39, 128 x 7168 x 2048 9.0 / 8.4, fp16 1024^3 7.28 / 6.94; tiles with longer loops gain 0 - 0.2.
+// Besides pointers, strides and sizes:
+constexpr uint32_t kHeadSplit = 1, kHeadStream = 2, kHeadStagger = 4;      // K split across workgroups; GemmArgs::b_stream; GemmArgs::stagger
+constexpr int kHeadRotShift = 3, kHeadGroupShift = 16;                     // GemmArgs::k_rot; TileMap::group_m
+constexpr uint32_t kHeadRotMax = 0x1FFF, kHeadGroupMax = 0xFFFF;
+struct LaunchHead {
+    uint32_t k_bytes, flags;
+    explicit LaunchHead(const GemmArgs &a)
+        : k_bytes(a.k_tail ? (a.ksteps - 1) * 128 + a.k_tail : a.ksteps * 128),
+          flags((a.nsplit > 1 ? kHeadSplit : 0) | (a.b_stream ? kHeadStream : 0) | (a.stagger ? kHeadStagger : 0) |
+                (a.k_rot < kHeadRotMax ? a.k_rot : kHeadRotMax) << kHeadRotShift |
+                (a.map.group_m < kHeadGroupMax ? a.map.group_m : kHeadGroupMax) << kHeadGroupShift) {}
+};
+
 template <class C>
-__global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
+__global__ void __launch_bounds__(C::THREADS)
+gemm_nt_kernel(const char *A, const char *B, uint32_t lda, uint32_t ldb, uint32_t M, uint32_t N, uint32_t k_bytes, uint32_t flags,
+               uint32_t inv_group, uint32_t inv_gm, uint32_t inv_last, uint32_t inv_nk, const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the launch stub
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     // part_t: what one MFMA step of 128 bytes of K delivers (int32 for int8 operands, else fp32); acc_t: the running
@@ -314,7 +336,7 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
     // and the bursts interleave with other CUs' K loops.  int8 8192^3 to f32, interleaved in one process, us: none
     // 381.0, four groups 2 us apart 374.2, eight groups 1 us apart 367.9 (what the host asks for), 8 x 2 371.7,
     // 16 x 1 383.6, 32 x 1 412.3; the same product with bf16 output 359.9.  8192 x 8192 x 4096: 226.4 / 216.2 / 213.2.
-    if (p.stagger > 0 && blockIdx.x < p.stagger_wgs) {
+    if ((flags & kHeadStagger) && blockIdx.x < p.stagger_wgs) {
         const int g = (blockIdx.x >> 3) % p.stagger_groups;            // (workgroup i runs on XCD i % 8: whole rows of XCDs per group)
         for (int i = 0; i < g * (int)p.stagger; ++i) __builtin_amdgcn_s_sleep(32);
     }
@@ -326,47 +348,44 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
     const int wm = wave_q / C::WAVES_N, wn = wave_q % C::WAVES_N;
 
     // ---- which tile, which K slice
-    uint32_t wg = blockIdx.x, z = 0;
-    if (p.nsplit > 1) {
-        z = __builtin_amdgcn_readfirstlane(wg % p.nsplit);
-        wg = __builtin_amdgcn_readfirstlane(wg / p.nsplit);
+    const uint32_t ksteps = (k_bytes + C::BKB - 1) / C::BKB, k_tail = k_bytes % C::BKB;
+    uint32_t wg = blockIdx.x, z = 0, kbeg = 0, kend = ksteps;
+    if (flags & kHeadSplit) {
+        wg = div_by_inv(wg, p.nsplit, p.inv_nsplit, z);
+        kbeg = z * p.ksteps_per_split;
+        if (kbeg + p.ksteps_per_split < ksteps) kend = kbeg + p.ksteps_per_split;
+        else inv_nk = p.inv_nk_last;
     }
     uint32_t tm, tn;
-    tile_map(wg, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
-    // the divisions of tile_map run on the vector ALU: bring the (uniform) result back to scalar registers so
-    // that everything derived from it (buffer descriptors, scalar offsets) stays there
-    tm = __builtin_amdgcn_readfirstlane(tm);
-    tn = __builtin_amdgcn_readfirstlane(tn);
+    tile_map(wg, TileMap{(M + C::BM - 1) / C::BM, (N + C::BN - 1) / C::BN, flags >> kHeadGroupShift, inv_group, inv_gm, inv_last}, tm, tn);
     const uint32_t row0 = tm * C::BM, col0 = tn * C::BN;
-    const uint32_t kbeg = z * p.ksteps_per_split;
-    const uint32_t kend = kbeg + p.ksteps_per_split < p.ksteps ? kbeg + p.ksteps_per_split : p.ksteps;
     const int nk = (int)(kend - kbeg);
 
     // ---- buffer resources: base at this tile's first row and first K byte; the
     // range ends with the last valid row, so rows past M / N read as out of
     // range (never a fault; the DMA then writes zeros) and only ever feed outputs
     // that are not stored.
-    const uint32_t a_rows = p.M - row0 < (uint32_t)C::BM ? p.M - row0 : C::BM;
-    const uint32_t b_rows = p.N - col0 < (uint32_t)C::BN ? p.N - col0 : C::BN;
+    const uint32_t a_rows = M - row0 < (uint32_t)C::BM ? M - row0 : C::BM;
+    const uint32_t b_rows = N - col0 < (uint32_t)C::BN ? N - col0 : C::BN;
     // A partial last K step (K bytes not a multiple of 128; the slice that ends with the last step has it): the
     // ranges end with the last byte of K, and in that one step the lanes whose 16-byte chunk of a K-contiguous row
     // lies past the end of the row present an offset that is out of range (bit 31; the host keeps every valid
     // offset below 2^31 for such shapes), so the DMA writes zeros where the next row's bytes would have landed.
     // A K-major operand needs nothing: its k rows past the end of K lie past the end of the range.
-    const bool has_tail = p.k_tail != 0 && kend == p.ksteps && nk > 0;
-    const uint32_t kbytes = has_tail ? (uint32_t)(nk - 1) * C::BKB + p.k_tail : (uint32_t)nk * C::BKB;
+    const bool has_tail = k_tail != 0 && kend == ksteps && nk > 0;
+    const uint32_t kbytes = has_tail ? (uint32_t)(nk - 1) * C::BKB + k_tail : (uint32_t)nk * C::BKB;
     // K-major operand: rows are k (stride lda / ldb bytes), the tile starts at column row0 / col0; the range ends
     // with the last column of the last k row of this K slice.  Columns past M / N inside an earlier row read
     // the neighbouring row instead (valid memory) and, as above, only feed outputs that are not stored.
     const uint32_t krows = nk > 0 ? kbytes / C::ES : 1;
     const __amdgpu_buffer_rsrc_t ra =
-        C::KMA ? make_rsrc(p.A + (size_t)kbeg * C::KE * p.lda + (size_t)row0 * C::ES,
-                           (krows - 1) * p.lda + (p.M - row0) * C::ES)
-               : make_rsrc(p.A + (size_t)row0 * p.lda + (size_t)kbeg * C::BKB, (a_rows - 1) * p.lda + kbytes);
+        C::KMA ? make_rsrc(A + (size_t)kbeg * C::KE * lda + (size_t)row0 * C::ES,
+                           (krows - 1) * lda + (M - row0) * C::ES)
+               : make_rsrc(A + (size_t)row0 * lda + (size_t)kbeg * C::BKB, (a_rows - 1) * lda + kbytes);
     const __amdgpu_buffer_rsrc_t rb =
-        C::KMB ? make_rsrc(p.B + (size_t)kbeg * C::KE * p.ldb + (size_t)col0 * C::ES,
-                           (krows - 1) * p.ldb + (p.N - col0) * C::ES)
-               : make_rsrc(p.B + (size_t)col0 * p.ldb + (size_t)kbeg * C::BKB, (b_rows - 1) * p.ldb + kbytes);
+        C::KMB ? make_rsrc(B + (size_t)kbeg * C::KE * ldb + (size_t)col0 * C::ES,
+                           (krows - 1) * ldb + (N - col0) * C::ES)
+               : make_rsrc(B + (size_t)col0 * ldb + (size_t)kbeg * C::BKB, (b_rows - 1) * ldb + kbytes);
 
     // ---- the LPT load instructions of this wave.  Instruction q = wave + i*NW (0 .. NLOAD-1) covers
     // rows 8*(q & 1) .. +7 of row block q >> 1 and lands at stage + 1024*q.  With NW even, q & 1 =
@@ -383,16 +402,18 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
     // bytes of m or n).  Bit 4 of k is bit 0 of blk = bit 1 of the wave number for every instruction of the wave
     // (NW / 2 and KE / 16 are even), so the swizzled chunk is one VGPR here too.
     const int ld_chunk_km = (lane & 7) ^ kmajor_swz<C::ES>(ld_r + 16 * ((lw >> 1) & 1));
-    const uint32_t voff_a = ld_r * p.lda + (C::KMA ? ld_chunk_km : ld_chunk) * 16;
-    const uint32_t voff_b = ld_r * p.ldb + (C::KMB ? ld_chunk_km : ld_chunk) * 16;
+    const uint32_t voff_a = ld_r * lda + (C::KMA ? ld_chunk_km : ld_chunk) * 16;
+    const uint32_t voff_b = ld_r * ldb + (C::KMB ? ld_chunk_km : ld_chunk) * 16;
     // (the chunk of a lane is the same in every copy instruction of every pipeline: (lane & 7) - (lane >> 3) mod 8)
-    const uint32_t tail_or = (has_tail && (uint32_t)ld_chunk * 16 >= p.k_tail) ? 0x80000000u : 0u;
+    const uint32_t tail_or = (has_tail && (uint32_t)ld_chunk * 16 >= k_tail) ? 0x80000000u : 0u;
     const uint32_t voff_a_t = C::KMA ? voff_a : (voff_a | tail_or), voff_b_t = C::KMB ? voff_b : (voff_b | tail_or);
     const int kt_tail = has_tail ? nk - 1 : -1;              // the step (of this slice) that is partial
     // K step the loop's step kt stands for (rotated start, simple pipeline only: the pipelined kernels run
     // compute-bound shapes, whose workgroups share panels and should stay in step)
     constexpr bool K_ROT = C::PIPE == PIPE_SIMPLE;
-    const int k_first = K_ROT && p.k_rot && nk > 0 ? (int)((tn * p.k_rot) % (uint32_t)nk) : 0;    // by column tile: the row tiles of a panel of B stay in step
+    uint32_t k_first_ = 0;                                    // by column tile: the row tiles of a panel of B stay in step
+    if (K_ROT && nk > 0) (void)div_by_inv(tn * ((flags >> kHeadRotShift) & kHeadRotMax), (uint32_t)nk, inv_nk, k_first_);
+    const int k_first = (int)k_first_;
     auto kpos = [&](int kt) -> int {
         if constexpr (K_ROT) {
             const int k = kt + k_first;
@@ -405,7 +426,7 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
         const int kt = kpos(kt_loop);
         const bool is_a = i < LPT_A0;
         const uint32_t blk = (lw >> 1) + (is_a ? i : i - LPT_A0) * (C::NW / 2);
-        const uint32_t ld = is_a ? p.lda : p.ldb;
+        const uint32_t ld = is_a ? lda : ldb;
         if (is_a ? C::KMA : C::KMB) {
             constexpr uint32_t BPP = C::KE / 16;                        // row blocks per panel
             return ((uint32_t)kt * C::KE + (blk % BPP) * 16) * ld + (blk / BPP) * 128;
@@ -423,7 +444,7 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
             // (B read once by the launch, i.e. streamed out of memory: its copies carry the streaming hint)
             if (i < LPT_A0)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, va, load_soff(i, kt), 0, 0);
-            else if (p.b_stream)
+            else if ((flags & kHeadStream))
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst, 16, vb, load_soff(i, kt), 0, 2);
             else
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst, 16, vb, load_soff(i, kt), 0, 0);
@@ -447,10 +468,10 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
     const int bp0 = (lane & 15) * 4;
     __amdgpu_buffer_rsrc_t ras = make_rsrc(p.as, 0);
     if constexpr (C::BLOCK_SCALE) {
-        // rows contiguous (as_ms == 1), p.as_ks floats from one K block to the next (p.as_ks > p.M when the rows
+        // rows contiguous (as_ms == 1), p.as_ks floats from one K block to the next (p.as_ks > M when the rows
         // are part of a taller matrix); or, solo pipeline only, K blocks contiguous (as_ks == 1), as_ms floats from
         // one row to the next
-        ras = make_rsrc(p.as, ((p.ksteps - 1) * p.as_ks + (p.M - 1) * p.as_ms + 1) * 4);
+        ras = make_rsrc(p.as, ((ksteps - 1) * p.as_ks + (M - 1) * p.as_ms + 1) * 4);
         as_voff = (row0 + wm * C::WM + lane) * p.as_ms * 4;
 #pragma unroll
         for (int j = 0; j < NBS; ++j) {
@@ -466,7 +487,7 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
             for (int j = 0; j < NLD; ++j)
                 as_raw[j] = __builtin_amdgcn_raw_buffer_load_b32(ras, as_voff, (64 * j * p.as_ms + kb * p.as_ks) * 4, 0);
             // (the solo pipeline fetches one step past the end of K: keep that read inside the array)
-            const uint32_t kbc = kb < p.ksteps ? kb : p.ksteps - 1;
+            const uint32_t kbc = kb < ksteps ? kb : ksteps - 1;
 #pragma unroll
             for (int j = 0; j < NBS; ++j) bs_raw[j] = p.bs[bs_off[j] + kbc * p.bs_ks];
         }
@@ -549,10 +570,10 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
         uint32_t vo_copy[VOFF_PER_COPY ? C::LPT : 1];
         __amdgpu_buffer_rsrc_t ra_g = ra, rb_g = rb;
         if constexpr (VOFF_PER_COPY) {
-            const uint32_t a_rows_ = p.M - row0 < (uint32_t)C::BM ? p.M - row0 : C::BM;
-            const uint32_t b_rows_ = p.N - col0 < (uint32_t)C::BN ? p.N - col0 : C::BN;
-            ra_g = make_rsrc(p.A + (size_t)row0 * p.lda + (size_t)kbeg * C::BKB - GROUP_SPAN, (a_rows_ - 1) * p.lda + kbytes + GROUP_SPAN);
-            rb_g = make_rsrc(p.B + (size_t)col0 * p.ldb + (size_t)kbeg * C::BKB - GROUP_SPAN, (b_rows_ - 1) * p.ldb + kbytes + GROUP_SPAN);
+            const uint32_t a_rows_ = M - row0 < (uint32_t)C::BM ? M - row0 : C::BM;
+            const uint32_t b_rows_ = N - col0 < (uint32_t)C::BN ? N - col0 : C::BN;
+            ra_g = make_rsrc(A + (size_t)row0 * lda + (size_t)kbeg * C::BKB - GROUP_SPAN, (a_rows_ - 1) * lda + kbytes + GROUP_SPAN);
+            rb_g = make_rsrc(B + (size_t)col0 * ldb + (size_t)kbeg * C::BKB - GROUP_SPAN, (b_rows_ - 1) * ldb + kbytes + GROUP_SPAN);
             const uint32_t chunk = (((lane & 7) - (lane >> 3)) & 7) * 16;          // rotation: see lds_slot
 #pragma unroll
             for (int i = 0; i < C::LPT; ++i) {
@@ -560,7 +581,7 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
                 const int il = is_a ? i : i - LPT_A;
                 const uint32_t q = lw * (is_a ? LPT_A : LPT_B) + il;
                 const uint32_t row = (q >> 1) * 16 + (q & 1) * 8 + (lane >> 3);
-                vo_copy[i] = row * (is_a ? p.lda : p.ldb) + chunk + GROUP_SPAN - (il & 3) * 1024;
+                vo_copy[i] = row * (is_a ? lda : ldb) + chunk + GROUP_SPAN - (il & 3) * 1024;
             }
         }
         // one LDS-DMA instruction with the immediate offset 1024 * k (a literal: the builtin wants a constant)
@@ -666,7 +687,7 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
             auto fetch_b_scales = [&](int kt) {
                 if constexpr (C::BLOCK_SCALE) {
                     // (one step past the end of K is fetched like the others: keep that read inside the array)
-                    const uint32_t kb = kbeg + kt, kbc = kb < p.ksteps ? kb : p.ksteps - 1;
+                    const uint32_t kb = kbeg + kt, kbc = kb < ksteps ? kb : ksteps - 1;
 #pragma unroll
                     for (int j = 0; j < NBS; ++j) bs_raw[j] = p.bs[bs_off[j] + kbc * p.bs_ks];
                 }
@@ -1056,10 +1077,10 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
             // 35.5 / 30.4, x 4112 (33 steps) 23.2 / 19.8, but x 3088 (25 steps) 15.4 / 16.1, so from 32 steps on.  The 64 x 128
             // tile with block scales, bound by its fold, gained 4 - 12 % from 57 steps on and lost 2 - 4 % on
             // aligned rows to the longer code, so it keeps its copies as they are.
-            const uint32_t line_a = (uint32_t)((uintptr_t)p.A >> 4) + (lane >> 3) * (p.lda >> 4);    // for row & 7 == lane >> 3
-            const uint32_t line_b = (uint32_t)((uintptr_t)p.B >> 4) + (lane >> 3) * (p.ldb >> 4);
+            const uint32_t line_a = (uint32_t)((uintptr_t)A >> 4) + (lane >> 3) * (lda >> 4);    // for row & 7 == lane >> 3
+            const uint32_t line_b = (uint32_t)((uintptr_t)B >> 4) + (lane >> 3) * (ldb >> 4);
             constexpr bool LATE_FORM = C::KMAJ == 0 && (!C::BLOCK_SCALE || C::BM >= 128);
-            const bool late = LATE_FORM && nk >= (C::BLOCK_SCALE ? 32 : 1) && (((uint32_t)(uintptr_t)p.A | (uint32_t)(uintptr_t)p.B | p.lda | p.ldb) & 127u) != 0;
+            const bool late = LATE_FORM && nk >= (C::BLOCK_SCALE ? 32 : 1) && (((uint32_t)(uintptr_t)A | (uint32_t)(uintptr_t)B | lda | ldb) & 127u) != 0;
             constexpr int NPC = C::NLOAD / C::NPROD;                        // operand copies per stage and copying wave
             constexpr int CPS = NPC + (C::BLOCK_SCALE ? 1 : 0);
             static_assert(C::NPROD == 4 && C::NLOAD % 4 == 0 && C::RBA % 2 == 0 && (NS - 2) * CPS <= 63,
@@ -1103,9 +1124,9 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
                         lds_void *dst = (lds_void *)(stage + j * 4096);
                         const uint32_t blk = (pw >> 1) + 2 * j;
                         if (2 * j < C::RBA)
-                            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, va, soff_k2(C::KMA, blk, p.lda, kt) - back, 0, 0);
+                            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, va, soff_k2(C::KMA, blk, lda, kt) - back, 0, 0);
                         else
-                            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst, 16, vb, soff_k2(C::KMB, blk - C::RBA, p.ldb, kt) - back, 0, B_NT ? 2 : 0);
+                            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst, 16, vb, soff_k2(C::KMB, blk - C::RBA, ldb, kt) - back, 0, B_NT ? 2 : 0);
                     }
                     if constexpr (C::BLOCK_SCALE) {
                         if (!p.as_groups) {
@@ -1148,17 +1169,17 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
                 constexpr std::integral_constant<bool, true> yes{};
                 constexpr std::integral_constant<bool, false> no{};
                 if (LATE_FORM && late) {
-                    if (p.b_stream) copy_loop(yes, std::integral_constant<bool, LATE_FORM>{});
+                    if ((flags & kHeadStream)) copy_loop(yes, std::integral_constant<bool, LATE_FORM>{});
                     else copy_loop(no, std::integral_constant<bool, LATE_FORM>{});
                 } else {
-                    if (p.b_stream) copy_loop(yes, no);
+                    if ((flags & kHeadStream)) copy_loop(yes, no);
                     else copy_loop(no, no);
                 }
             } else {
                 v4i fa[C::TM][2], fb[C::TN][2];
                 // this lane's two chunks of a step: do they come with the stage behind it (row & 7 == fr & 7 here)
-                const uint32_t fa_line = ((uint32_t)((uintptr_t)p.A >> 4) + (fr & 7) * (p.lda >> 4)) & 7;
-                const uint32_t fb_line = ((uint32_t)((uintptr_t)p.B >> 4) + (fr & 7) * (p.ldb >> 4)) & 7;
+                const uint32_t fa_line = ((uint32_t)((uintptr_t)A >> 4) + (fr & 7) * (lda >> 4)) & 7;
+                const uint32_t fb_line = ((uint32_t)((uintptr_t)B >> 4) + (fr & 7) * (ldb >> 4)) & 7;
                 const bool late_a0 = late && fg + fa_line >= 8, late_a1 = late && fg + 4 + fa_line >= 8;
                 const bool late_b0 = late && fg + fb_line >= 8, late_b1 = late && fg + 4 + fb_line >= 8;
                 auto read_stage = [&](int mine, auto late_tag) {
@@ -1374,7 +1395,8 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
     // ---- epilogue: lane holds C[m][n0 .. n0+3] of every 16x16 tile
     float scale = 1.0f;
     if (p.per_matrix_scale) scale = p.as[0] * p.bs[0];
-    char *Cz = p.C + (size_t)z * p.split_stride * dtype_bytes(p.out_dtype);
+    char *Cz = p.C;
+    if (z) Cz += (size_t)z * p.split_stride * c_elem_bytes(p.out_dtype);
 
     // The accumulator layout (adjacent lanes = adjacent rows of C) would make every lane of a store its own
     // request; so each 16-row slab goes through this wave's private LDS scratch and leaves as
@@ -1410,8 +1432,8 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
         __syncthreads();
     }
     // columns of the wave tile inside C; rows of it inside C (at most WM; none or fewer where the tile sticks out below)
-    const bool wave_cols_full = col0 + wn * C::WN + C::WN <= p.N;
-    const int wave_rows = (int)p.M - (int)(row0 + wm * C::WM);
+    const bool wave_cols_full = col0 + wn * C::WN + C::WN <= N;
+    const int wave_rows = (int)M - (int)(row0 + wm * C::WM);
     // Every accumulator is read in exactly one place (write_slab): the output type is a uniform branch around
     // the conversion of a slab, and wave tiles that stick out of C take the same way through the scratch.  The 16-byte
     // pieces go to any element address, rows past M and pieces past N are left out, and the one piece N ends in goes in parts
@@ -1441,7 +1463,7 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
         const uint32_t wrow0 = row0 + wm * C::WM, wcol0 = col0 + wn * C::WN;
         // What this wave writes of a row: 16-byte pieces at any element address, and, where the row of C ends inside a
         // piece, the part of that one piece inside it
-        const int wave_cols = wave_cols_full ? C::WN : (wcol0 < p.N ? (int)(p.N - wcol0) : 0);
+        const int wave_cols = wave_cols_full ? C::WN : (wcol0 < N ? (int)(N - wcol0) : 0);
         const int whole = wave_cols * ES / 16 * 16, rest = __builtin_amdgcn_readfirstlane(wave_cols - whole / ES);
         const bool lane_in_cols = rd_col < whole, wave_tile_full = wave_cols_full && wave_rows >= C::WM;
         char *cwave = Cz + ((size_t)wrow0 * p.ldc + wcol0) * ES;
@@ -1554,13 +1576,13 @@ __global__ void __launch_bounds__(C::THREADS) gemm_nt_kernel(const GemmArgs p) {
 #pragma unroll
     for (int a = 0; a < C::TM; ++a) {
         const uint32_t m = row0 + wm * C::WM + a * 16 + (lane & 15);
-        if (m >= p.M) continue;
+        if (m >= M) continue;
 #pragma unroll
         for (int b = 0; b < C::TN; ++b) {
             const uint32_t n = col0 + wn * C::WN + b * 16 + (lane >> 4) * 4;
-            if (n >= p.N) continue;
+            if (n >= N) continue;
             const size_t idx = (size_t)m * p.ldc + n;
-            const int valid = p.N - n < 4 ? (int)(p.N - n) : 4;
+            const int valid = N - n < 4 ? (int)(N - n) : 4;
             if constexpr (C::ARITH == AR_I8 && !C::BLOCK_SCALE) {
                 if (p.out_dtype == QGEMM_DT_I32) {
                     int *dst = (int *)Cz + idx;

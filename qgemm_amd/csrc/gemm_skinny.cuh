@@ -32,7 +32,7 @@ struct SkinnyCfg {
     // 128-block scales (fp8): every MFMA starts from zero and its product of one K block is folded into the running
     // sum with a_scale[row, kb] * b_scale[strip, kb], as in gemm_nt_kernel.  The strip of 32 (or 64) columns lies inside
     // one 128-column block of b_scale.  a_scale is read with the caller's strides (lane l: row l of the tile, the rows of
-    // an MFMA tile picked out of that with ds_bpermute); the scales of a round are requested in front of the round's
+    // an MFMA tile picked out of that with ds_bpermute); the scales of a round are requested among the round's
     // copies, so they have arrived wherever the copies they precede have.
     static constexpr bool BLOCK_SCALE = BLOCK_SCALE_;
     static_assert(!BLOCK_SCALE_ || ARITH_ == AR_F8 || ARITH_ == AR_F8W || ARITH_ == AR_I8, "block scales: fp8 and int8 operands");
@@ -61,8 +61,11 @@ __device__ inline void wait_landed() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// (arguments in front of `p`: see LaunchHead; inv0 .. inv2: of the row tiles, or, 64 x 64 form, the three of TileMap)
 template <class C>
-__global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs p) {
+__global__ void __launch_bounds__(C::THREADS)
+gemm_skinny_kernel(const char *A, const char *B, uint32_t lda, uint32_t ldb, uint32_t M, uint32_t N, uint32_t k_bytes, uint32_t flags,
+                   uint32_t inv_nk, uint32_t inv0, uint32_t inv1, uint32_t inv2, const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     typedef typename AccT<C::ARITH>::type part_t;                       // one MFMA step: int32 for int8 operands, else fp32
@@ -72,44 +75,41 @@ __global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs 
     QGEMM_STAMP_DECL(6);
     QGEMM_STAMP(0);
 
-    uint32_t wg = blockIdx.x, z = 0;
-    if (p.nsplit > 1) {
-        z = __builtin_amdgcn_readfirstlane(wg % p.nsplit);
-        wg = __builtin_amdgcn_readfirstlane(wg / p.nsplit);
+    const bool split = flags & kHeadSplit;
+    const uint32_t k_rot = (flags >> kHeadRotShift) & kHeadRotMax;
+    const uint32_t tiles_m = (M + C::BM - 1) / C::BM, ksteps = (k_bytes + 127) / 128, k_tail = k_bytes % 128;
+    uint32_t wg = blockIdx.x, z = 0, kbeg = 0, kend = ksteps;
+    if (split) {
+        wg = div_by_inv(wg, p.nsplit, p.inv_nsplit, z);
+        kbeg = z * p.ksteps_per_split;
+        if (kbeg + p.ksteps_per_split < ksteps) kend = kbeg + p.ksteps_per_split;
+        else inv_nk = p.inv_nk_last;
     }
     // column strips side by side (the few row tiles of one strip are neighbours: they share the strip of B in L2)
     // (the 64 x 64 form has many row tiles: there the tiles an XCD holds at one time form a compact block, as in
     // gemm_nt_kernel, so that its L2 fetches each panel of A and B once)
     uint32_t tm, tn;
-    if constexpr (C::TN == 4) {
-        tile_map(wg, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
-        tm = __builtin_amdgcn_readfirstlane(tm);
-        tn = __builtin_amdgcn_readfirstlane(tn);
-    } else {
-        tm = __builtin_amdgcn_readfirstlane(wg % p.tiles_m);
-        tn = __builtin_amdgcn_readfirstlane(wg / p.tiles_m);
-    }
+    if constexpr (C::TN == 4) tile_map(wg, TileMap{tiles_m, (N + C::BN - 1) / C::BN, flags >> kHeadGroupShift, inv0, inv1, inv2}, tm, tn);
+    else tn = div_by_inv(wg, tiles_m, inv0, tm);
     const uint32_t row0 = tm * C::BM, col0 = tn * C::BN;
-    const uint32_t kbeg = z * p.ksteps_per_split;
-    const uint32_t kend = kbeg + p.ksteps_per_split < p.ksteps ? kbeg + p.ksteps_per_split : p.ksteps;
     const int nk = (int)(kend - kbeg);
 
     // Buffer resources end with the last valid row of the tile and the last byte of the K slice: rows past M / N and
     // steps past the end of K read as zeros.
-    const uint32_t a_rows = p.M - row0 < (uint32_t)C::BM ? p.M - row0 : C::BM;
-    const uint32_t b_rows = p.N - col0 < (uint32_t)C::BN ? p.N - col0 : C::BN;
+    const uint32_t a_rows = M - row0 < (uint32_t)C::BM ? M - row0 : C::BM;
+    const uint32_t b_rows = N - col0 < (uint32_t)C::BN ? N - col0 : C::BN;
     // (a partial last K step: the ranges end with the last byte of K, and in that step the lanes whose 16-byte chunk
     // lies past the end of a row present an offset that is out of range, as in gemm_nt_kernel)
-    const bool has_tail = p.k_tail != 0 && kend == p.ksteps && nk > 0;
-    const uint32_t kbytes = has_tail ? (uint32_t)(nk - 1) * 128 + p.k_tail : (uint32_t)nk * 128;
+    const bool has_tail = k_tail != 0 && kend == ksteps && nk > 0;
+    const uint32_t kbytes = has_tail ? (uint32_t)(nk - 1) * 128 + k_tail : (uint32_t)nk * 128;
     const int kt_tail = has_tail ? nk - 1 : -1;
-    const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A + (size_t)row0 * p.lda + (size_t)kbeg * 128, (a_rows - 1) * p.lda + kbytes);
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.B + (size_t)col0 * p.ldb + (size_t)kbeg * 128, (b_rows - 1) * p.ldb + kbytes);
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(A + (size_t)row0 * lda + (size_t)kbeg * 128, (a_rows - 1) * lda + kbytes);
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(B + (size_t)col0 * ldb + (size_t)kbeg * 128, (b_rows - 1) * ldb + kbytes);
     // a copy moves 8 rows x 128 bytes; lane l fetches the chunk of row l >> 3 that belongs in 16-byte slot l of
     // the kilobyte (rotation by the row: see lds_slot)
     const uint32_t rot = (((lane & 7) - (lane >> 3)) & 7) * 16;
-    const uint32_t voff_a = (lane >> 3) * p.lda + rot, voff_b = (lane >> 3) * p.ldb + rot;
-    const uint32_t tail_or = (has_tail && rot >= p.k_tail) ? 0x80000000u : 0u;
+    const uint32_t voff_a = (lane >> 3) * lda + rot, voff_b = (lane >> 3) * ldb + rot;
+    const uint32_t tail_or = (has_tail && rot >= k_tail) ? 0x80000000u : 0u;
     char *ring = smem + wave * C::RING_BYTES;
     const int fr = lane & 15, fg = lane >> 4;
     const int off0 = lds_slot(fr, fg) * 16, off1 = lds_slot(fr, 4 + fg) * 16;
@@ -117,7 +117,9 @@ __global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs 
     // K step the loop's step kt stands for: the workgroups of a column strip start k_first steps in and wrap round
     // (GemmArgs::k_rot);
     // steps past the end stay past the end (they read zeros)
-    const int k_first = p.k_rot && nk > 0 ? (int)((tn * p.k_rot) % (uint32_t)nk) : 0;
+    uint32_t k_first_ = 0;
+    if (nk > 0) (void)div_by_inv(tn * k_rot, (uint32_t)nk, inv_nk, k_first_);
+    const int k_first = (int)k_first_;
     auto kpos = [&](int kt) -> int {
         const int k = kt + k_first;
         return kt >= nk ? kt : (k >= nk ? k - nk : k);
@@ -129,23 +131,23 @@ __global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs 
 #pragma unroll
         for (int i = 0; i < n; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void *)(ring + (slot + i) * 1024), 16, va,
-                                                     (first + i) * 8 * p.lda + (uint32_t)kt * 128, 0, 0);
+                                                     (first + i) * 8 * lda + (uint32_t)kt * 128, 0, 0);
     };
     auto copy_b_part = [&](int kt_loop, int first, int n, int slot) {
         const int kt = kpos(kt_loop);
         const uint32_t vb = kt == kt_tail ? (voff_b | tail_or) : voff_b;
         // B streamed out of memory and read once: the copies carry the streaming hint (nt).  Config 5 with B in rotation
         // through 352 MB: M = 16 5.65 -> 5.40 us, M = 64 6.96 -> 6.82, M = 128 8.35 -> 8.22; level with B resident.
-        if (p.b_stream) {
+        if (flags & kHeadStream) {
 #pragma unroll
             for (int i = 0; i < n; ++i)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void *)(ring + (slot + i) * 1024), 16, vb,
-                                                         (first + i) * 8 * p.ldb + (uint32_t)kt * 128, 0, 2);
+                                                         (first + i) * 8 * ldb + (uint32_t)kt * 128, 0, 2);
         } else {
 #pragma unroll
             for (int i = 0; i < n; ++i)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void *)(ring + (slot + i) * 1024), 16, vb,
-                                                         (first + i) * 8 * p.ldb + (uint32_t)kt * 128, 0, 0);
+                                                         (first + i) * 8 * ldb + (uint32_t)kt * 128, 0, 0);
         }
     };
     auto copy_b = [&](int kt, int slot) { copy_b_part(kt, 0, C::SB, slot); };
@@ -184,20 +186,22 @@ __global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs 
     float bs_cur[2], bs_nxt[2];
     __amdgpu_buffer_rsrc_t ras = make_rsrc(p.as, 0);
     uint32_t as_voff = 0, bs_base = 0;
-    if constexpr (C::BLOCK_SCALE) {
-        ras = make_rsrc(p.as, ((p.ksteps - 1) * p.as_ks + (p.M - 1) * p.as_ms + 1) * 4);
-        as_voff = (row0 + lane) * p.as_ms * 4;
-        uint32_t nb = col0 / 128;
-        nb = nb < p.nb_max ? nb : p.nb_max;
-        bs_base = nb * p.bs_ns;
-    }
-    auto fetch_scales = [&](int k) {            // for steps k and k + 8 of this wave (called in front of their copies)
+    auto locate_scales = [&]() {
+        if constexpr (C::BLOCK_SCALE) {
+            ras = make_rsrc(p.as, ((ksteps - 1) * p.as_ks + (M - 1) * p.as_ms + 1) * 4);
+            as_voff = (row0 + lane) * p.as_ms * 4;
+            uint32_t nb = col0 / 128;
+            nb = nb < p.nb_max ? nb : p.nb_max;
+            bs_base = nb * p.bs_ns;
+        }
+    };
+    auto fetch_scales = [&](int k) {            // for steps k and k + 8 of this wave
         if constexpr (C::BLOCK_SCALE) {
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 const uint32_t kb = kbeg + (uint32_t)kpos(k + s * C::NW);
                 // (a step past the end of K multiplies zeros: any finite scale will do, so keep the reads inside)
-                const uint32_t kbc = kb < p.ksteps ? kb : p.ksteps - 1;
+                const uint32_t kbc = kb < ksteps ? kb : ksteps - 1;
 #pragma unroll
                 for (int j = 0; j < NLD; ++j)
                     as_nxt[s][j] = __builtin_amdgcn_raw_buffer_load_b32(ras, as_voff, (64 * j * p.as_ms + kbc * p.as_ks) * 4, 0);
@@ -256,25 +260,34 @@ __global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs 
     // A goes in front of B where the ring cannot take the round at once: the wait for it then does not include
     // the trip to HBM, and its slots turn over while B is still on its way.
     constexpr int SA = C::SA, SB = C::SB;
-    auto start_round = [&](int k) {
-        fetch_scales(k);
-        __builtin_amdgcn_sched_barrier(0);          // (the scale loads stay in front of the copies)
+    // (The scales of a round are requested behind its first copies, whose wait they share, and in front of the others.)
+    auto start_round = [&](int k, auto first_tag) {
+        auto scales = [&]() {
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (decltype(first_tag)::value) locate_scales();
+            fetch_scales(k);
+            __builtin_amdgcn_sched_barrier(0);
+        };
         if constexpr (C::TN == 4) {                   // 64 x 64: A0 B0 B1[0..4) fill the ring
             copy_a(k, 0, 8, 0);
+            scales();
             copy_b(k, 8);
             copy_b_part(k + C::NW, 0, 4, 16);
         } else if constexpr (C::ALL_AT_ONCE) {
             copy_b(k, 0);
             copy_b(k + C::NW, SB);
+            scales();
             copy_a(k, 0, SA, 2 * SB);
             copy_a(k + C::NW, 0, SA, 2 * SB + SA);
         } else if constexpr (C::TM == 4) {
             copy_a(k, 0, 8, 0);
+            scales();
             copy_b(k, 8);
             copy_b(k + C::NW, 12);
             copy_a(k + C::NW, 0, 4, 16);
         } else {
             copy_a(k, 0, 12, 0);
+            scales();
             copy_b(k, 12);
             copy_b(k + C::NW, 16);
         }
@@ -342,12 +355,18 @@ __global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs 
             drain_a(1, 4, 4, 12);
         }
         drained();
-        if (next) start_round(k + 2 * C::NW);
+        if (next) start_round(k + 2 * C::NW, std::integral_constant<bool, false>{});
         if (two) compute(1);
     };
     int k = wave;
-    start_round(k);
+    start_round(k, std::integral_constant<bool, true>{});
     QGEMM_STAMP(1);
+    // (the scales of a matrix, fetched here: behind the barrier at the end they were a trip to memory of their own)
+    float scale_a = 1.0f, scale_b = 1.0f;
+    if (!C::BLOCK_SCALE && p.per_matrix_scale) {
+        scale_a = p.as[0];
+        scale_b = p.bs[0];
+    }
     for (; k < nk; k += 2 * C::NW) finish_round(k, k + 2 * C::NW < nk, k + C::NW < nk);
     // (a wave without a step has copies of zeros on their way into its ring, which now takes the partial sums)
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0) & 0xF0FF);
@@ -364,9 +383,9 @@ __global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs 
     __syncthreads();
     QGEMM_STAMP(4);
 
-    float scale = 1.0f;
-    if (p.per_matrix_scale) scale = p.as[0] * p.bs[0];
-    char *Cz = p.C + (size_t)z * p.split_stride * dtype_bytes(p.out_dtype);
+    const float scale = scale_a * scale_b;
+    char *Cz = p.C;
+    if (z) Cz += (size_t)z * p.split_stride * c_elem_bytes(p.out_dtype);
     // wave w finishes tiles w, w + 8, ...
 #pragma unroll
     for (int i = 0; i < (T + C::NW - 1) / C::NW; ++i) {
@@ -382,9 +401,9 @@ __global__ void __launch_bounds__(C::THREADS) gemm_skinny_kernel(const GemmArgs 
         const int a = t / C::TN, b = t % C::TN;
         const uint32_t m = row0 + a * 16 + (lane & 15);
         const uint32_t n = col0 + b * 16 + (lane >> 4) * 4;
-        if (m >= p.M || n >= p.N) continue;
+        if (m >= M || n >= N) continue;
         const size_t idx = (size_t)m * p.ldc + n;
-        const int valid = p.N - n < 4 ? (int)(p.N - n) : 4;
+        const int valid = N - n < 4 ? (int)(N - n) : 4;
         if constexpr (C::ARITH == AR_I8 && !C::BLOCK_SCALE) {
             if (p.out_dtype == QGEMM_DT_I32) {
                 int *dst = (int *)Cz + idx;

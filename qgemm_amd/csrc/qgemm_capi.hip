@@ -745,9 +745,9 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     a.k_tail = (uint32_t)(q.Kbytes % 128);
     a.lda = (uint32_t)q.lda_bytes;
     a.ldb = (uint32_t)q.ldb_bytes;
-    a.tiles_m = (uint32_t)((q.M + v.bm - 1) / v.bm);
-    a.tiles_n = (uint32_t)((q.N + v.bn - 1) / v.bn);
-    a.group_m = g_ctx.force_group_m > 0 ? (uint32_t)g_ctx.force_group_m : 8;
+    const uint32_t tiles_m = (uint32_t)((q.M + v.bm - 1) / v.bm), tiles_n = (uint32_t)((q.N + v.bn - 1) / v.bn);
+    a.map = make_tile_map(tiles_m, tiles_n, g_ctx.force_group_m > 0 ? (uint32_t)g_ctx.force_group_m : 8);
+    a.inv_tiles_m = inverse_of(tiles_m);
     // Few rows (every workgroup streams a strip of B of its own out of memory, all of them at the same k): the workgroups
     // of column tile i (which share that strip of B and stay in step) start their K loops k_rot * i steps in and wrap
     // round, so that at any time the column tiles read at different offsets
@@ -767,9 +767,9 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     // a caller who loops over one small B that sits in that cache loses 14 - 30 % with it (the same shapes with one B:
     // 3.56 / 5.04 -> 4.61 / 5.73), and with two row tiles sharing a strip of B it costs up to 8 %.  Option b_stream = 1
     // puts it on for every launch with one row tile: for callers whose weights do not stay in the cache between calls.
-    a.b_stream = g_ctx.b_stream >= 0 ? (int)(g_ctx.b_stream && a.tiles_m == 1)
-                                     : (a.tiles_m == 1 && q.N * q.Kbytes >= ((size_t)32 << 20));
-    pl.tiles = (size_t)a.tiles_m * a.tiles_n;
+    a.b_stream = g_ctx.b_stream >= 0 ? (int)(g_ctx.b_stream && tiles_m == 1)
+                                     : (tiles_m == 1 && q.N * q.Kbytes >= ((size_t)32 << 20));
+    pl.tiles = (size_t)tiles_m * tiles_n;
     if (pl.tiles * 64 >= ((size_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
 
     uint32_t nsplit = 1;
@@ -787,6 +787,9 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     a.ksteps_per_split = (a.ksteps + nsplit - 1) / nsplit;
     nsplit = (a.ksteps + a.ksteps_per_split - 1) / a.ksteps_per_split;   // no empty slices
     a.nsplit = nsplit;
+    a.inv_nsplit = inverse_of(nsplit);
+    a.inv_nk = inverse_of(a.ksteps_per_split);
+    a.inv_nk_last = inverse_of(a.ksteps - (nsplit - 1) * a.ksteps_per_split);
     pl.split_bytes = nsplit > 1 ? q.M * q.N * 4 * (size_t)nsplit : 0;
     return QGEMM_OK;
 }
@@ -884,21 +887,11 @@ int run_nt(const NtProblem &q, Plan &pl, void *split_ws, hipStream_t stream) {
     hipError_t e = v.launch(a, (uint32_t)(pl.tiles * a.nsplit), stream);
     if (e != hipSuccess) return QGEMM_ERR_LAUNCH;
 
-    ReduceArgs r;
-    std::memset(&r, 0, sizeof(r));
-    r.part = split_ws;
-    r.C = q.C;
-    r.as = q.as;
-    r.bs = q.bs;
-    r.M = (uint32_t)q.M;
-    r.N = (uint32_t)q.N;
-    r.nsplit = a.nsplit;
-    r.ldc = q.ldc;
-    r.plane = plane;
-    r.out_dtype = q.out_dtype;
-    r.per_matrix_scale = q.per_matrix;
-    const dim3 grid((unsigned)((q.M * ((q.N + 3) / 4) + 255) / 256));
-    hipLaunchKernelGGL(i32_acc ? splitk_reduce4_kernel<true> : splitk_reduce4_kernel<false>, grid, dim3(256), 0, stream, r);
+    const uint32_t per_row = (uint32_t)((q.N + 3) / 4);
+    const dim3 grid((unsigned)((q.M * per_row + 255) / 256));
+    hipLaunchKernelGGL(i32_acc ? splitk_reduce4_kernel<true> : splitk_reduce4_kernel<false>, grid, dim3(256), 0, stream, split_ws, q.C, q.as,
+                       q.bs, (uint32_t)q.M, (uint32_t)q.N, a.nsplit, (uint32_t)q.ldc, inverse_of(per_row), (uint32_t)q.out_dtype,
+                       (uint32_t)(q.per_matrix != 0));
     g_ctx.last_config = std::string(v.name) + kmaj_suffix(q.kmaj) + "_splitk" + std::to_string(a.nsplit);
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }
@@ -1139,10 +1132,9 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
     constexpr int W = BLOCK && DT == QGEMM_DT_I8 ? 64 : 128;
     const bool km = a.a.k_major || a.b.k_major;
     const int T = any_tile(DT, a.out_dtype, BLOCK, km, a.a.rows, a.b.rows);
-    a.tiles_m = (uint32_t)(((uint64_t)a.a.rows + T - 1) / T);
-    a.tiles_n = (uint32_t)(((uint64_t)a.b.rows + T - 1) / T);
-    const uint64_t tiles = (uint64_t)a.tiles_m * a.tiles_n;
+    const uint64_t tiles_m = ((uint64_t)a.a.rows + T - 1) / T, tiles_n = ((uint64_t)a.b.rows + T - 1) / T, tiles = tiles_m * tiles_n;
     if (tiles >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;    // grid limit
+    a.map = make_tile_map((uint32_t)tiles_m, (uint32_t)tiles_n, 8);
     constexpr int SUM = BLOCK ? ANY_SCALED : ANY_CHAIN;
     auto kernel = T == 64 ? (km ? gemm_any_kernel<DT, SUM, 64, true> : gemm_any_kernel<DT, SUM, 64, false>)
                           : (km ? gemm_any_kernel<DT, SUM, BLOCK ? 64 : W, true> : gemm_any_kernel<DT, SUM, W, false>);
@@ -1215,7 +1207,7 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
     typedef Piece<IN_DT> P;
     auto number = [&](uint32_t per_row) {       // see QuantArgs::per_row
         a.per_row = std::max<uint32_t>(1, per_row);
-        a.inv = (uint32_t)std::min<uint64_t>(((uint64_t)1 << 32) / a.per_row, 0xFFFFFFFFu);
+        a.inv = inverse_of(a.per_row);
         a.rows_per_slice = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(a.rows, ((uint64_t)1 << 31) / a.per_row));
     };
     if (mode == QGEMM_QUANT_PER_MATRIX) {
@@ -1303,7 +1295,7 @@ QGEMM_EXPORT int qgemm_tile_map(uint32_t wg, uint32_t tiles_m, uint32_t tiles_n,
                    uint32_t *tile_n) {
     if (!tile_m || !tile_n || tiles_m == 0 || tiles_n == 0) return QGEMM_ERR_INVALID_ARG;
     if ((uint64_t)wg >= (uint64_t)tiles_m * tiles_n) return QGEMM_ERR_INVALID_ARG;
-    tile_map(wg, tiles_m, tiles_n, group_m, *tile_m, *tile_n);
+    tile_map(wg, make_tile_map(tiles_m, tiles_n, group_m), *tile_m, *tile_n);
     return QGEMM_OK;
 }
 

@@ -29,20 +29,9 @@ struct QuantArgs {
     uint32_t rows, cols, npartial;
     uint64_t ld, ldq, scale_rs, scale_cs;
     // Work is numbered along rows in units of a piece (per matrix) or of a 1 x 128 block: `per_row` of them in a row,
-    // inv = floor(2^32 / per_row).  blockIdx.y counts slices of rows_per_slice rows, so that a number fits 32 bits.
+    // inv = inverse_of(per_row).  blockIdx.y counts slices of rows_per_slice rows, so that a number fits 32 bits.
     uint32_t per_row, inv, rows_per_slice;
 };
-
-// i / d and i % d with inv = min(floor(2^32 / d), 2^32 - 1): the estimate is at most one too small
-__device__ inline uint32_t div_by_inv(uint32_t i, uint32_t d, uint32_t inv, uint32_t &rem) {
-    uint32_t q = __umulhi(i, inv);
-    rem = i - q * d;
-    if (rem >= d) {
-        rem -= d;
-        ++q;
-    }
-    return q;
-}
 
 // ---- 16 bytes of input
 template <int IN_DT>
