@@ -1227,17 +1227,16 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
     } else if (mode == QGEMM_QUANT_BLOCK_1x128) {
         number((a.cols + 127) / 128);
         const uint64_t blocks = (uint64_t)a.rows_per_slice * a.per_row;
-        const uint32_t slices = (a.rows + a.rows_per_slice - 1) / a.rows_per_slice, per_turn = 256 / P::LANES;
-        if (blocks >= (uint64_t)4096 * per_turn)
-            hipLaunchKernelGGL((quant_row_block_kernel<IN_DT, OUT_DT, 4>), dim3((unsigned)((blocks + 4 * per_turn - 1) / (4 * per_turn)), slices),
-                               dim3(256), 0, stream, a);
+        const uint32_t slices = (a.rows + a.rows_per_slice - 1) / a.rows_per_slice, per_group = 256 / P::LANES;
+        const dim3 grid((unsigned)((blocks + per_group - 1) / per_group), slices);
+        if (blocks >= (uint64_t)kQuantManyGroups * per_group)
+            hipLaunchKernelGGL((quant_row_block_kernel<IN_DT, OUT_DT>), grid, dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
         else
-            hipLaunchKernelGGL((quant_row_block_kernel<IN_DT, OUT_DT, 1>), dim3((unsigned)((blocks + per_turn - 1) / per_turn), slices),
-                               dim3(256), 0, stream, a);
+            hipLaunchKernelGGL((quant_few_blocks_kernel<IN_DT, OUT_DT>), grid, dim3(256), 0, stream, a);
     } else {
         const uint64_t nblocks = (uint64_t)((a.rows + 127) / 128) * ((a.cols + 127) / 128);
         if (nblocks >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
-        hipLaunchKernelGGL((quant_square_block_kernel<IN_DT, OUT_DT>), dim3((unsigned)nblocks), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((quant_square_block_kernel<IN_DT, OUT_DT>), dim3((unsigned)nblocks), dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
     }
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }

@@ -13,8 +13,8 @@
 //     with infinities and NaNs on top, so that one look at a block's maximum tells whether the plain form below will do;
 //   * plain form (a finite maximum: no element is NaN or infinite, no quotient exceeds the type's largest value): the
 //     quotient of |x| without special cases, the sign moved over afterwards; anything else takes the careful form.
-// Before and now, us (to fp8 unless said): 1 x 128 6144 x 7168 bf16 45.7 -> 28.4 (4.7 TB/s, what a copy reaches), 500 x 7200
-// 7.3 -> 5.7; 128 x 128 7168 x 6144 fp32 43.4 -> 39.6 (5.6 TB/s); per matrix 1531 x 3004 bf16 to int8 4.9 + 8.5 -> 4.2 + 6.6.
+// Before and now, us (to fp8 unless said): 1 x 128 6144 x 7168 bf16 45.7 -> 25.7 (5.1 TB/s, what a copy reaches), 500 x 7200
+// 7.3 -> 4.5; 128 x 128 7168 x 6144 fp32 43.4 -> 39.6 (5.6 TB/s); per matrix 1531 x 3004 bf16 to int8 4.9 + 8.5 -> 4.2 + 6.6.
 // A decoder's 16 x 2048 stays at 2.8: one trip to memory and back.
 #pragma once
 #include "common.h"
@@ -32,6 +32,13 @@ struct QuantArgs {
     // inv = inverse_of(per_row).  blockIdx.y counts slices of rows_per_slice rows, so that a number fits 32 bits.
     uint32_t per_row, inv, rows_per_slice;
 };
+
+// What the kernels start with, in front of QuantArgs: arguments of their own arrive in scalar registers with the wave (kernarg
+// preloading, see LaunchHead), fields of a struct are a trip to memory in front of the first load.
+#define QGEMM_QUANT_HEAD                                                                                                  \
+    const void *x, void *q, float *scales, uint64_t ld, uint32_t rows_all, uint32_t cols, uint32_t per_row, uint32_t inv, \
+        uint32_t rows_per_slice
+#define QGEMM_QUANT_HEAD_OF(a) (a).x, (a).q, (a).scales, (a).ld, (a).rows, (a).cols, (a).per_row, (a).inv, (a).rows_per_slice, a
 
 // ---- 16 bytes of input
 template <int IN_DT>
@@ -307,49 +314,51 @@ __device__ inline Divisor block_divisor(uint32_t m, F numbers) {
     return make_divisor(scale_of<OUT_DT>(Piece<IN_DT>::element(m)), finite);
 }
 
-// ---- 1 x 128 blocks: Piece::LANES lanes (16 or 32) per block and turn, U turns in flight per lane: four where there are
-// enough blocks to fill the CUs that way, one for the few rows of a decoder's step
-template <int IN_DT, int OUT_DT, int U>
-__global__ void __launch_bounds__(256) quant_row_block_kernel(const QuantArgs p) {
+// ---- 1 x 128 blocks: Piece::LANES lanes (16 or 32) per block, one piece a lane.  What keeps memory busy is waves: with four
+// pieces in flight per lane and a quarter of the waves, as it was from 65536 blocks on, 1500 x 7168 bf16 took 10.9 us and takes
+// 7.8, 6144 x 7168 29.5 and 25.7 (5.1 TB/s, what a copy reaches).
+template <int IN_DT, int OUT_DT>
+__device__ __forceinline__ void quant_row_block(QGEMM_QUANT_HEAD, const QuantArgs &p) {
     typedef Piece<IN_DT> P;
-    constexpr uint32_t G = 256 / P::LANES;                                // blocks per turn of the workgroup
-    const uint32_t row0 = blockIdx.y * p.rows_per_slice;
-    const uint32_t rows = p.rows - row0 < p.rows_per_slice ? p.rows - row0 : p.rows_per_slice, total = rows * p.per_row;
-    const uint32_t lane = threadIdx.x % P::LANES, first = blockIdx.x * G * U + threadIdx.x / P::LANES;
-    v4i v[U];
-    uint32_t r[U], jb[U], valid[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const uint32_t i = first + u * G;
-        r[u] = row0 + div_by_inv(i, p.per_row, p.inv, jb[u]);
-        const uint32_t c = jb[u] * kScaleBlock + lane * P::VEC;
-        valid[u] = (i < total && c < p.cols) ? p.cols - c : 0;
-        v[u] = v4i{0, 0, 0, 0};
-        if (valid[u]) v[u] = P::load(p.x, (size_t)r[u] * p.ld + c, valid[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const uint32_t m = lanes_max<P::LANES>(P::max_bits(v[u]));
-        const Divisor dv = block_divisor<IN_DT, OUT_DT>(m, [&] { return lanes_max<P::LANES>(P::max_bits_of_numbers(v[u])); });
-        if (first + u * G >= total) break;                                // (whole groups of lanes leave together)
-        if (lane == 0) p.scales[(size_t)r[u] * p.scale_rs + (size_t)jb[u] * p.scale_cs] = dv.s;
-        if (valid[u])
-            store_piece<IN_DT>(p.q, (size_t)r[u] * p.ldq + jb[u] * kScaleBlock + lane * P::VEC, quant_piece<IN_DT, OUT_DT>(v[u], dv),
-                               valid[u]);
-    }
+    const uint32_t row0 = blockIdx.y * rows_per_slice;
+    const uint32_t rows = rows_all - row0 < rows_per_slice ? rows_all - row0 : rows_per_slice, total = rows * per_row;
+    const uint32_t lane = threadIdx.x % P::LANES, i = blockIdx.x * (256 / P::LANES) + threadIdx.x / P::LANES;
+    uint32_t jb;
+    const uint32_t r = row0 + div_by_inv(i, per_row, inv, jb), c = jb * kScaleBlock + lane * P::VEC;
+    const uint32_t valid = (i < total && c < cols) ? cols - c : 0;
+    v4i v = v4i{0, 0, 0, 0};
+    if (valid) v = P::load(x, (size_t)r * ld + c, valid);
+    uint64_t ldq = p.ldq, scale_rs = p.scale_rs, scale_cs = p.scale_cs;
+    asm volatile("" : "+s"(ldq), "+s"(scale_rs), "+s"(scale_cs));          // (fetched here, while the load flies, not where they are used)
+    const uint32_t m = lanes_max<P::LANES>(P::max_bits(v));
+    const Divisor dv = block_divisor<IN_DT, OUT_DT>(m, [&] { return lanes_max<P::LANES>(P::max_bits_of_numbers(v)); });
+    if (i >= total) return;                                                // (whole groups of lanes leave together)
+    if (lane == 0) scales[(size_t)r * scale_rs + (size_t)jb * scale_cs] = dv.s;
+    if (valid) store_piece<IN_DT>(q, (size_t)r * ldq + c, quant_piece<IN_DT, OUT_DT>(v, dv), valid);
+}
+// The arguments of a launch with preloaded ones cost it 0.07 us, which more than a few hundred workgroups gain back (256 x 7168
+// 3.69 -> 3.52 us, 500 x 7200 4.81 -> 4.51; 128 x 4096 2.90 against 2.96): kQuantManyGroups.
+constexpr uint32_t kQuantManyGroups = 640;
+template <int IN_DT, int OUT_DT>
+__global__ void __launch_bounds__(256) quant_row_block_kernel(QGEMM_QUANT_HEAD, const QuantArgs p) {
+    quant_row_block<IN_DT, OUT_DT>(x, q, scales, ld, rows_all, cols, per_row, inv, rows_per_slice, p);
+}
+template <int IN_DT, int OUT_DT>
+__global__ void __launch_bounds__(256) quant_few_blocks_kernel(const QuantArgs p) {
+    quant_row_block<IN_DT, OUT_DT>(QGEMM_QUANT_HEAD_OF(p));
 }
 
 // ---- 128 x 128 blocks: one workgroup per block, which it holds in registers
 template <int IN_DT, int OUT_DT>
-__global__ void __launch_bounds__(256) quant_square_block_kernel(const QuantArgs p) {
+__global__ void __launch_bounds__(256) quant_square_block_kernel(QGEMM_QUANT_HEAD, const QuantArgs p) {
     typedef Piece<IN_DT> P;
     constexpr int ROWS = 256 / P::LANES, TURNS = 128 / ROWS;
     __shared__ uint32_t red[4];
-    const uint32_t nbc = (p.cols + 127) / 128;
+    const uint32_t nbc = (cols + 127) / 128;
     const uint32_t ib = blockIdx.x / nbc, jb = blockIdx.x % nbc;
     const uint32_t c = jb * 128 + (threadIdx.x % P::LANES) * P::VEC;
     const uint32_t r0 = ib * 128 + threadIdx.x / P::LANES;               // rows r0, r0 + ROWS, ...
-    const uint32_t valid = c < p.cols ? p.cols - c : 0;
+    const uint32_t valid = c < cols ? cols - c : 0;
     auto workgroup_max = [&](uint32_t m) {
         m = lanes_max<64>(m);
         if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -362,8 +371,10 @@ __global__ void __launch_bounds__(256) quant_square_block_kernel(const QuantArgs
     for (int i = 0; i < TURNS; ++i) {
         const uint32_t r = r0 + i * ROWS;
         v[i] = v4i{0, 0, 0, 0};
-        if (r < p.rows && valid) v[i] = P::load(p.x, (size_t)r * p.ld + c, valid);
+        if (r < rows_all && valid) v[i] = P::load(x, (size_t)r * ld + c, valid);
     }
+    uint64_t ldq = p.ldq, scale_rs = p.scale_rs, scale_cs = p.scale_cs;
+    asm volatile("" : "+s"(ldq), "+s"(scale_rs), "+s"(scale_cs));
     uint32_t m = 0;
 #pragma unroll
     for (int i = 0; i < TURNS; ++i) {
@@ -380,11 +391,11 @@ __global__ void __launch_bounds__(256) quant_square_block_kernel(const QuantArgs
         __syncthreads();                                                 // (m is the same in every lane of the workgroup)
         return workgroup_max(n);
     });
-    if (threadIdx.x == 0) p.scales[(size_t)ib * p.scale_rs + (size_t)jb * p.scale_cs] = dv.s;
+    if (threadIdx.x == 0) scales[(size_t)ib * scale_rs + (size_t)jb * scale_cs] = dv.s;
 #pragma unroll
     for (int i = 0; i < TURNS; ++i) {
         const uint32_t r = r0 + i * ROWS;
-        if (r < p.rows && valid) store_piece<IN_DT>(p.q, (size_t)r * p.ldq + c, quant_piece<IN_DT, OUT_DT>(v[i], dv), valid);
+        if (r < rows_all && valid) store_piece<IN_DT>(q, (size_t)r * ldq + c, quant_piece<IN_DT, OUT_DT>(v[i], dv), valid);
     }
 }
 
