@@ -19,6 +19,7 @@ typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
 typedef float v4f_any __attribute__((ext_vector_type(4), aligned(1)));
 typedef int v2i_any __attribute__((ext_vector_type(2), aligned(1)));
 typedef unsigned u32_any __attribute__((aligned(1)));
+typedef unsigned short u16_any __attribute__((aligned(1)));
 
 // Arithmetic families of the MFMA kernels.
 enum Arith : int { AR_I8 = 0, AR_F8 = 1, AR_BF16 = 2, AR_F16 = 3, AR_F8W = 4 };   // F8W: fp8 operands, multiplied as bf16
@@ -85,6 +86,21 @@ __device__ inline void store_out4(void *C, size_t idx, const float *v, int out_d
     else
         for (int e = 0; e < 3; ++e)
             if (e < valid) dst[e] = pack4_elem(h, e);
+}
+
+// W dwords moved down by n bytes (zeros from above); DWORDS: n is a multiple of 4
+template <int W, bool DWORDS = false>
+__device__ __forceinline__ void move_down(uint32_t *w, uint32_t n) {
+    uint32_t v[W + 1];
+    const uint32_t q = n >> 2;
+#pragma unroll
+    for (int i = 0; i <= W; ++i) {
+        v[i] = 0;
+#pragma unroll
+        for (int k = i; k < W; ++k) v[i] = q == (uint32_t)(k - i) ? w[k] : v[i];
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i) w[i] = DWORDS ? v[i] : __builtin_amdgcn_alignbyte(v[i + 1], v[i], n & 3);
 }
 
 // four e4m3 values -> four bf16 values (exact; NaNs stay NaNs)

@@ -55,21 +55,6 @@ __device__ __forceinline__ void load_any(const char *p, uint32_t *w) {
     }
 }
 
-// W dwords moved down by n bytes (zeros from above)
-template <int W>
-__device__ __forceinline__ void move_down(uint32_t *w, uint32_t n) {
-    uint32_t v[W + 1];
-    const uint32_t q = n >> 2;
-#pragma unroll
-    for (int i = 0; i <= W; ++i) {
-        v[i] = 0;
-#pragma unroll
-        for (int k = i; k < W; ++k) v[i] = q == (uint32_t)(k - i) ? w[k] : v[i];
-    }
-#pragma unroll
-    for (int i = 0; i < W; ++i) w[i] = __builtin_amdgcn_alignbyte(v[i + 1], v[i], n & 3);
-}
-
 // One operand of the tile.  LDS: T rows of 128 bytes, chunk c of row r in slot c ^ swz(r): fragment reads (16 rows, one chunk
 // each) and the writes of a transposed block (rows 8 apart) both spread over the banks.
 // KM: the operand may be K-major (AnyOperand::k_major says so); without, the code that transposes is left out.

@@ -1210,9 +1210,20 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         a.inv = inverse_of(a.per_row);
         a.rows_per_slice = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(a.rows, ((uint64_t)1 << 31) / a.per_row));
     };
+    const bool ragged = a.cols % P::VEC != 0;           // rows end inside a piece
     if (mode == QGEMM_QUANT_PER_MATRIX) {
-        // two passes: partial maxima (one per workgroup) into the workspace, then scale and cast
+        if (a.ld == a.cols && a.ldq == a.cols && (uint64_t)a.rows * a.cols < ((uint64_t)1 << 31)) {      // no gaps: one row
+            a.cols *= a.rows;
+            a.rows = a.rows ? 1 : 0;
+        }
         number((a.cols + P::VEC - 1) / P::VEC);
+        const uint64_t pieces = (uint64_t)a.rows * a.per_row;
+        if (pieces * 16 <= kQuantSmallBytes) {
+            hipLaunchKernelGGL((a.rows == 1 ? quant_small_matrix_kernel<IN_DT, OUT_DT, true> : quant_small_matrix_kernel<IN_DT, OUT_DT, false>), dim3((unsigned)std::max<uint64_t>(1, (pieces + 1023) / 1024)), dim3(1024), 0,
+                               stream, a);
+            return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+        }
+        // two passes: partial maxima (one per workgroup) into the workspace, then scale and cast
         const uint32_t slices = std::max<uint32_t>(1, (a.rows + a.rows_per_slice - 1) / a.rows_per_slice);
         const uint64_t turns = ((uint64_t)a.rows_per_slice * a.per_row + 256 * kQuantTurn - 1) / (256 * kQuantTurn);
         const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(1024, turns));
@@ -1221,22 +1232,22 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         int st = ensure_workspace_locked((size_t)a.npartial * sizeof(uint32_t), stream, &ws);
         if (st != QGEMM_OK) return st;
         a.partial = (uint32_t *)ws;
-        hipLaunchKernelGGL(quant_amax_kernel<IN_DT>, dim3(nblk, slices), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((a.rows == 1 ? quant_amax_kernel<IN_DT, true> : quant_amax_kernel<IN_DT, false>), dim3(nblk, slices), dim3(256), 0, stream, a);
         const uint32_t nq = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(2048, turns));
-        hipLaunchKernelGGL((quant_matrix_kernel<IN_DT, OUT_DT>), dim3(nq, slices), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((a.rows == 1 ? quant_matrix_kernel<IN_DT, OUT_DT, true> : quant_matrix_kernel<IN_DT, OUT_DT, false>), dim3(nq, slices), dim3(256), 0, stream, a);
     } else if (mode == QGEMM_QUANT_BLOCK_1x128) {
         number((a.cols + 127) / 128);
         const uint64_t blocks = (uint64_t)a.rows_per_slice * a.per_row;
         const uint32_t slices = (a.rows + a.rows_per_slice - 1) / a.rows_per_slice, per_group = 256 / P::LANES;
         const dim3 grid((unsigned)((blocks + per_group - 1) / per_group), slices);
         if (blocks >= (uint64_t)kQuantManyGroups * per_group)
-            hipLaunchKernelGGL((quant_row_block_kernel<IN_DT, OUT_DT>), grid, dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
+            hipLaunchKernelGGL((ragged ? quant_row_block_kernel<IN_DT, OUT_DT, true> : quant_row_block_kernel<IN_DT, OUT_DT, false>), grid, dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
         else
-            hipLaunchKernelGGL((quant_few_blocks_kernel<IN_DT, OUT_DT>), grid, dim3(256), 0, stream, a);
+            hipLaunchKernelGGL((ragged ? quant_few_blocks_kernel<IN_DT, OUT_DT, true> : quant_few_blocks_kernel<IN_DT, OUT_DT, false>), grid, dim3(256), 0, stream, a);
     } else {
         const uint64_t nblocks = (uint64_t)((a.rows + 127) / 128) * ((a.cols + 127) / 128);
         if (nblocks >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
-        hipLaunchKernelGGL((quant_square_block_kernel<IN_DT, OUT_DT>), dim3((unsigned)nblocks), dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
+        hipLaunchKernelGGL((ragged ? quant_square_block_kernel<IN_DT, OUT_DT, true> : quant_square_block_kernel<IN_DT, OUT_DT, false>), dim3((unsigned)nblocks), dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
     }
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }

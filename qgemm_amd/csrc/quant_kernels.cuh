@@ -52,18 +52,45 @@ struct Piece {
         else if constexpr (IN_DT == QGEMM_DT_BF16) return __builtin_bit_cast(float, bits << 16);
         else return (float)__builtin_bit_cast(_Float16, (unsigned short)bits);
     }
-    // elements idx .. idx + VEC - 1; those from `valid` on are zeros and not read
-    __device__ static v4i load(const void *base, size_t idx, uint32_t valid) {
+    // Elements idx .. idx + VEC - 1 of a row that has `valid` of them left.  Where the row ends inside the piece load_whole fetches
+    // the last whole piece of the row instead, and `settle` moves its end down and leaves zeros behind it: nothing waits and
+    // nothing branches between the loads of a lane.  (Element by element behind a branch each, every load waited for the one
+    // before: 128 x 128 blocks of 500 x 7195 bf16 11.3 us, 7.0 so, 1 x 128 5.3 and 4.7, per matrix 9.9 and 8.3.)  Rows of fewer than VEC elements: load_elements.
+    __device__ static v4i load_whole(const void *base, size_t idx, uint32_t valid) {
+        return *(const v4i_any *)((const char *)base + idx * ES - (valid ? missing(valid) * ES : 0));
+    }
+    __device__ static v4i load_elements(const void *base, size_t idx, uint32_t valid) {          // (valid: 1 or more)
         const char *p = (const char *)base + idx * ES;
-        if (valid >= (uint32_t)VEC) return *(const v4i_any *)p;
         uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll 1
+        for (uint32_t e = valid; e-- > 0;) {
 #pragma unroll
-        for (int e = 0; e < VEC - 1; ++e)
-            if ((uint32_t)e < valid) {
-                if constexpr (ES == 4) w[e] = ((const uint32_t *)p)[e];
-                else w[e >> 1] |= (uint32_t)((const uint16_t *)p)[e] << (16 * (e & 1));
-            }
+            for (int i = 3; i > 0; --i) w[i] = ES == 4 ? w[i - 1] : (w[i] << 16 | w[i - 1] >> 16);
+            if constexpr (ES == 4) w[0] = ((const uint32_t *)p)[e];
+            else w[0] = w[0] << 16 | ((const uint16_t *)p)[e];
+        }
         return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+    }
+    // RAGGED: the row may end inside a piece
+    template <bool RAGGED>
+    __device__ static v4i load(const void *base, size_t idx, uint32_t valid, bool wide) {
+        if constexpr (!RAGGED) return *(const v4i_any *)((const char *)base + idx * ES);
+        else return wide ? load_whole(base, idx, valid) : load_elements(base, idx, valid);
+    }
+    // element e + 1 to where element e is
+    __device__ static void next_element(v4i &r) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t up = i < 3 ? (uint32_t)r[i < 3 ? i + 1 : 3] : 0u, at = (uint32_t)r[i];
+            r[i] = (int)(ES == 4 ? up : (at >> 16 | up << 16));
+        }
+    }
+    __device__ static uint32_t missing(uint32_t valid) { return valid < (uint32_t)VEC ? VEC - valid : 0; }
+    __device__ static void settle(v4i &r, uint32_t valid) {
+        if (!__any(valid != 0 && valid < (uint32_t)VEC)) return;
+        uint32_t w[4] = {(uint32_t)r[0], (uint32_t)r[1], (uint32_t)r[2], (uint32_t)r[3]};
+        move_down<4, ES == 4>(w, valid ? missing(valid) * ES : 0);
+        r = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     }
     __device__ static uint32_t bits(v4i r, int e) {
         if constexpr (ES == 4) return (uint32_t)r[e];
@@ -83,12 +110,31 @@ struct Piece {
             return hi > lo ? hi : lo;
         }
     }
-    // the same over the elements that are numbers
+    // acc = the larger |x| of acc and r, element by element; max_bits(acc) is the maximum in the end
+    __device__ static void fold_max(v4i &acc, v4i r) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (ES == 4) {
+                const uint32_t b = (uint32_t)r[i] & 0x7FFFFFFFu;
+                acc[i] = (int)(b > (uint32_t)acc[i] ? b : (uint32_t)acc[i]);
+            } else {
+                typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+                const uint32_t old = (uint32_t)acc[i], bits = (uint32_t)r[i] & 0x7FFF7FFFu;
+                acc[i] = __builtin_bit_cast(int, __builtin_elementwise_max(__builtin_bit_cast(us2, old), __builtin_bit_cast(us2, bits)));
+            }
+        }
+    }
+    // max_bits over the elements that are numbers
     __device__ static uint32_t max_bits_of_numbers(v4i r) {
+        // (rolled, an element a turn out of the low bits: unrolled and hoisted out of its rare branch it took up to 235 registers of
+        // the kernels that hold several pieces, and with them the waves that keep memory busy: 128 x 128 blocks of 6144 x 7168
+        // fp16 95.7 us, 27.8 with this and the loads of quant_square_block_kernel)
         uint32_t m = 0;
+#pragma unroll 1
         for (int e = 0; e < VEC; ++e) {
-            const uint32_t b = bits(r, e) & (ES == 4 ? 0x7FFFFFFFu : 0x7FFFu);
+            const uint32_t b = (uint32_t)r[0] & (ES == 4 ? 0x7FFFFFFFu : 0x7FFFu);
             if (b <= INF && b > m) m = b;
+            next_element(r);
         }
         return m;
     }
@@ -138,6 +184,7 @@ template <int IN_DT, int OUT_DT>
 __device__ inline v2i quant_piece(v4i r, const Divisor &dv) {
     typedef Piece<IN_DT> P;
     uint32_t w[2] = {0, 0};
+    asm volatile("" : "+v"(r));             // (a piece at a time: nothing of the next pieces' conversions moves in front of this one)
     if (dv.plain) {
 #pragma unroll
         for (int h = 0; h < P::VEC / 4; ++h) {
@@ -167,9 +214,18 @@ __device__ inline v2i quant_piece(v4i r, const Divisor &dv) {
             }
         }
     } else {
+        // (an element a turn out of the low bits)
+#pragma unroll 1
         for (int e = 0; e < P::VEC; ++e) {
-            const float v = P::element(P::bits(r, e)) / dv.s;
-            w[e >> 2] |= (OUT_DT == QGEMM_DT_F8E4M3 ? f32_to_fp8_careful(v) : f32_to_i8_careful(v)) << (8 * (e & 3));
+            const float v = P::element(P::ES == 4 ? (uint32_t)r[0] : (uint32_t)r[0] & 0xFFFFu) / dv.s;
+            const uint32_t q = OUT_DT == QGEMM_DT_F8E4M3 ? f32_to_fp8_careful(v) : f32_to_i8_careful(v);
+            if constexpr (P::ES == 4) {
+                w[0] = w[0] >> 8 | q << 24;
+            } else {
+                w[0] = w[0] >> 8 | w[1] << 24;
+                w[1] = w[1] >> 8 | q << 24;
+            }
+            P::next_element(r);
         }
     }
     return v2i{(int)w[0], (int)w[1]};
@@ -183,7 +239,18 @@ __device__ inline void store_piece(void *q, size_t idx, v2i w, uint32_t valid) {
         else *(u32_any *)p = (uint32_t)w[0];
         return;
     }
-    for (uint32_t e = 0; e < valid; ++e) p[e] = (uint8_t)((uint32_t)w[e >> 2] >> (8 * (e & 3)));
+    uint32_t b = (uint32_t)w[0];                                  // the parts of 4, 2 and 1 bytes that the row still has
+    if (valid & 4) {
+        *(u32_any *)p = b;
+        p += 4;
+        b = (uint32_t)w[1];
+    }
+    if (valid & 2) {
+        *(u16_any *)p = (uint16_t)b;
+        p += 2;
+        b >>= 16;
+    }
+    if (valid & 1) *p = (uint8_t)b;
 }
 
 // maximum over groups of 16, 32 or 64 neighbouring lanes, in every lane, on the vector ALU alone: lane exchanges inside a
@@ -218,91 +285,141 @@ __device__ inline float scale_of(float amax) {
 constexpr uint32_t kQuantNan = 0x80000000u;
 constexpr int kQuantTurn = 4;                    // pieces a lane has in flight (per-matrix passes)
 
-// ---- per matrix, pass 1: one partial maximum per workgroup
-template <int IN_DT>
-__global__ void __launch_bounds__(256) quant_amax_kernel(const QuantArgs p) {
+// ---- per matrix.  The host hands over a matrix without gaps as a single row (QuantArgs::per_row pieces), which saves the
+// divisions and all row ends but one.
+// Where piece i of `total` lies, loads and stores of it
+template <int IN_DT, bool ONE_ROW>
+struct MatrixPieces {
     typedef Piece<IN_DT> P;
-    __shared__ uint32_t red[4];
-    const uint32_t row0 = blockIdx.y * p.rows_per_slice;
-    const uint32_t rows = p.rows - row0 < p.rows_per_slice ? p.rows - row0 : p.rows_per_slice, total = rows * p.per_row;
-    uint32_t m = 0, nan = 0;
-    for (uint32_t first = blockIdx.x * 256 * kQuantTurn; first < total; first += gridDim.x * 256 * kQuantTurn) {
-        v4i v[kQuantTurn];
+    const QuantArgs &p;
+    uint32_t row0, total;
+    bool wide;
+    __device__ MatrixPieces(const QuantArgs &a, uint32_t slice) : p(a) {
+        row0 = slice * a.rows_per_slice;
+        total = (a.rows - row0 < a.rows_per_slice ? a.rows - row0 : a.rows_per_slice) * a.per_row;
+        wide = a.cols >= (uint32_t)P::VEC;
+    }
+    // element c of its row
+    __device__ void at(uint32_t i, size_t &r, uint32_t &c) const {
+        r = 0;
+        c = i;
+        if constexpr (!ONE_ROW) r = row0 + div_by_inv(i, p.per_row, p.inv, c);
+        c *= P::VEC;
+    }
+    // N pieces, `stride` apart: requested together, zeros past the end
+    template <int N>
+    __device__ void load(v4i (&v)[N], uint32_t first, uint32_t stride) const {
+        uint32_t valid[N];
+        size_t idx[N];
 #pragma unroll
-        for (int j = 0; j < kQuantTurn; ++j) {
-            const uint32_t i = first + j * 256 + threadIdx.x;
-            v[j] = v4i{0, 0, 0, 0};
-            if (i < total) {
-                uint32_t c;
-                const uint32_t r = div_by_inv(i, p.per_row, p.inv, c);
-                v[j] = P::load(p.x, (size_t)(row0 + r) * p.ld + c * P::VEC, p.cols - c * P::VEC);
-            }
+        for (int j = 0; j < N; ++j) {
+            const uint32_t i = first + j * stride;
+            size_t r;
+            uint32_t c;
+            at(i < total ? i : 0, r, c);
+            idx[j] = ONE_ROW ? c : r * p.ld + c;
+            valid[j] = i < total ? p.cols - c : 0;
         }
+        if (wide) {
 #pragma unroll
-        for (int j = 0; j < kQuantTurn; ++j) {
-            uint32_t b = P::max_bits(v[j]);
-            if (b > P::INF) {
-                nan = kQuantNan;
-                b = P::max_bits_of_numbers(v[j]);
-            }
-            m = b > m ? b : m;
+            for (int j = 0; j < N; ++j) v[j] = P::load_whole(p.x, idx[j], valid[j]);
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+                if (!valid[j]) v[j] = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < N; ++j) P::settle(v[j], valid[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < N; ++j) v[j] = valid[j] ? P::load_elements(p.x, idx[j], valid[j]) : v4i{0, 0, 0, 0};
         }
     }
-    m = lanes_max<64>(m) | (__any(nan != 0) ? kQuantNan : 0u);
+    __device__ void store(uint32_t i, v2i w) const {
+        if (i >= total) return;
+        size_t r;
+        uint32_t c;
+        at(i, r, c);
+        store_piece<IN_DT>(p.q, r * p.ldq + c, w, p.cols - c);
+    }
+    // bits of the largest |x| that is a number, bit 31 set where there is something else, of N pieces, `stride` apart, from
+    // `first` on, N from first + `turn` on, ...
+    template <int N>
+    __device__ uint32_t maximum(uint32_t first, uint32_t stride, uint32_t turn) const {
+        v4i acc = v4i{0, 0, 0, 0}, v[N];
+        for (uint32_t i = first; i < total; i += turn) {
+            load<N>(v, i, stride);
+#pragma unroll
+            for (int j = 0; j < N; ++j) P::fold_max(acc, v[j]);
+        }
+        uint32_t m = P::max_bits(acc);
+        if (m <= P::INF) return m;
+        m = 0;
+        for (uint32_t i = first; i < total; i += turn)
+            for (int j = 0; j < N; ++j) {
+                v4i one[1];
+                load<1>(one, i + j * stride, 0);
+                const uint32_t b = P::max_bits_of_numbers(one[0]);
+                m = b > m ? b : m;
+            }
+        return m | kQuantNan;
+    }
+};
+// the same over the workgroup's waves; bit 31 as above
+template <int WAVES>
+__device__ inline uint32_t workgroup_maximum(uint32_t m) {
+    __shared__ uint32_t red[WAVES];
+    m = lanes_max<64>(m & ~kQuantNan) | (__any((m & kQuantNan) != 0) ? kQuantNan : 0u);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t best = 0, any = 0;
-        for (int w = 0; w < 4; ++w) {
-            any |= red[w] & kQuantNan;
-            best = (red[w] & ~kQuantNan) > best ? (red[w] & ~kQuantNan) : best;
-        }
-        p.partial[blockIdx.y * gridDim.x + blockIdx.x] = best | any;
-    }
+    m = red[threadIdx.x % WAVES];                                   // (the 16 lanes of a row hold all of them)
+    return lanes_max<16>(m & ~kQuantNan) | (__any((m & kQuantNan) != 0) ? kQuantNan : 0u);
+}
+template <int IN_DT, int OUT_DT>
+__device__ inline Divisor matrix_divisor(uint32_t m) {
+    const uint32_t b = m & ~kQuantNan;
+    return make_divisor(scale_of<OUT_DT>(Piece<IN_DT>::element(b)), m < Piece<IN_DT>::INF);
 }
 
-// ---- per matrix, pass 2: every workgroup reduces the partial maxima again (a few KB, L2 resident), then
+// Small: one launch, no workspace.  Every workgroup takes the maximum of the whole matrix, then quantises its own 1024 pieces.
+// A workgroup reads some 100 GB/s, so this ends where that takes as long as a second launch: against the two passes below, us,
+// graph replays, bf16 16 x 2048 (64 KiB) 4.8 / 6.5, 64 x 2048 (256 KiB) 6.1 / 6.5, 64 x 3000 (375 KiB) 7.6 / 6.6.
+constexpr uint64_t kQuantSmallBytes = 256 << 10;
+template <int IN_DT, int OUT_DT, bool ONE_ROW>
+__global__ void __launch_bounds__(1024) quant_small_matrix_kernel(const QuantArgs p) {
+    const MatrixPieces<IN_DT, ONE_ROW> x(p, 0);
+    const uint32_t mine = blockIdx.x * 1024 + threadIdx.x;
+    v4i own[1];
+    x.template load<1>(own, mine, 1);
+    const Divisor dv = matrix_divisor<IN_DT, OUT_DT>(workgroup_maximum<16>(x.template maximum<8>(threadIdx.x, 1024, 8 * 1024)));
+    if (mine == 0) p.scales[0] = dv.s;
+    x.store(mine, quant_piece<IN_DT, OUT_DT>(own[0], dv));
+}
+
+// pass 1: one partial maximum per workgroup
+template <int IN_DT, bool ONE_ROW>
+__global__ void __launch_bounds__(256) quant_amax_kernel(const QuantArgs p) {
+    const MatrixPieces<IN_DT, ONE_ROW> x(p, blockIdx.y);
+    const uint32_t m = workgroup_maximum<4>(x.template maximum<kQuantTurn>(blockIdx.x * 256 * kQuantTurn + threadIdx.x, 256, gridDim.x * 256 * kQuantTurn));
+    if (threadIdx.x == 0) p.partial[blockIdx.y * gridDim.x + blockIdx.x] = m;
+}
+
+// pass 2: every workgroup reduces the partial maxima again (a few KB, L2 resident), then
 // quantises its share; workgroup 0 writes the scale
-template <int IN_DT, int OUT_DT>
+template <int IN_DT, int OUT_DT, bool ONE_ROW>
 __global__ void __launch_bounds__(256) quant_matrix_kernel(const QuantArgs p) {
-    typedef Piece<IN_DT> P;
-    __shared__ uint32_t red[4];
+    const MatrixPieces<IN_DT, ONE_ROW> x(p, blockIdx.y);
     uint32_t m = 0, nan = 0;
     for (uint32_t i = threadIdx.x; i < p.npartial; i += 256) {
         const uint32_t b = p.partial[i];
         nan |= b & kQuantNan;
         m = (b & ~kQuantNan) > m ? (b & ~kQuantNan) : m;
     }
-    m = lanes_max<64>(m) | (__any(nan != 0) ? kQuantNan : 0u);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    m = 0;
-    nan = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        nan |= red[w] & kQuantNan;
-        m = (red[w] & ~kQuantNan) > m ? (red[w] & ~kQuantNan) : m;
-    }
-    const float s = scale_of<OUT_DT>(P::element(m));
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.scales[0] = s;
-    const Divisor dv = make_divisor(s, m < P::INF && !nan);
-    const uint32_t row0 = blockIdx.y * p.rows_per_slice;
-    const uint32_t rows = p.rows - row0 < p.rows_per_slice ? p.rows - row0 : p.rows_per_slice, total = rows * p.per_row;
-    for (uint32_t first = blockIdx.x * 256 * kQuantTurn; first < total; first += gridDim.x * 256 * kQuantTurn) {
+    const Divisor dv = matrix_divisor<IN_DT, OUT_DT>(workgroup_maximum<4>(m | nan));
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.scales[0] = dv.s;
+    for (uint32_t first = blockIdx.x * 256 * kQuantTurn; first < x.total; first += gridDim.x * 256 * kQuantTurn) {
         v4i v[kQuantTurn];
-        uint32_t r[kQuantTurn], c[kQuantTurn];
+        x.template load<kQuantTurn>(v, first + threadIdx.x, 256);
 #pragma unroll
-        for (int j = 0; j < kQuantTurn; ++j) {
-            const uint32_t i = first + j * 256 + threadIdx.x;
-            r[j] = div_by_inv(i, p.per_row, p.inv, c[j]);
-            v[j] = v4i{0, 0, 0, 0};
-            if (i < total) v[j] = P::load(p.x, (size_t)(row0 + r[j]) * p.ld + c[j] * P::VEC, p.cols - c[j] * P::VEC);
-        }
-#pragma unroll
-        for (int j = 0; j < kQuantTurn; ++j)
-            if (first + j * 256 + threadIdx.x < total)
-                store_piece<IN_DT>(p.q, (size_t)(row0 + r[j]) * p.ldq + c[j] * P::VEC, quant_piece<IN_DT, OUT_DT>(v[j], dv),
-                                   p.cols - c[j] * P::VEC);
+        for (int j = 0; j < kQuantTurn; ++j) x.store(first + threadIdx.x + j * 256, quant_piece<IN_DT, OUT_DT>(v[j], dv));
     }
 }
 
@@ -317,7 +434,7 @@ __device__ inline Divisor block_divisor(uint32_t m, F numbers) {
 // ---- 1 x 128 blocks: Piece::LANES lanes (16 or 32) per block, one piece a lane.  What keeps memory busy is waves: with four
 // pieces in flight per lane and a quarter of the waves, as it was from 65536 blocks on, 1500 x 7168 bf16 took 10.9 us and takes
 // 7.8, 6144 x 7168 29.5 and 25.7 (5.1 TB/s, what a copy reaches).
-template <int IN_DT, int OUT_DT>
+template <int IN_DT, int OUT_DT, bool RAGGED>
 __device__ __forceinline__ void quant_row_block(QGEMM_QUANT_HEAD, const QuantArgs &p) {
     typedef Piece<IN_DT> P;
     const uint32_t row0 = blockIdx.y * rows_per_slice;
@@ -327,9 +444,11 @@ __device__ __forceinline__ void quant_row_block(QGEMM_QUANT_HEAD, const QuantArg
     const uint32_t r = row0 + div_by_inv(i, per_row, inv, jb), c = jb * kScaleBlock + lane * P::VEC;
     const uint32_t valid = (i < total && c < cols) ? cols - c : 0;
     v4i v = v4i{0, 0, 0, 0};
-    if (valid) v = P::load(x, (size_t)r * ld + c, valid);
+    const bool wide = cols >= (uint32_t)P::VEC;
+    if (valid) v = P::template load<RAGGED>(x, (size_t)r * ld + c, valid, wide);
     uint64_t ldq = p.ldq, scale_rs = p.scale_rs, scale_cs = p.scale_cs;
     asm volatile("" : "+s"(ldq), "+s"(scale_rs), "+s"(scale_cs));          // (fetched here, while the load flies, not where they are used)
+    if (RAGGED && wide) P::settle(v, valid);
     const uint32_t m = lanes_max<P::LANES>(P::max_bits(v));
     const Divisor dv = block_divisor<IN_DT, OUT_DT>(m, [&] { return lanes_max<P::LANES>(P::max_bits_of_numbers(v)); });
     if (i >= total) return;                                                // (whole groups of lanes leave together)
@@ -339,17 +458,17 @@ __device__ __forceinline__ void quant_row_block(QGEMM_QUANT_HEAD, const QuantArg
 // The arguments of a launch with preloaded ones cost it 0.07 us, which more than a few hundred workgroups gain back (256 x 7168
 // 3.69 -> 3.52 us, 500 x 7200 4.81 -> 4.51; 128 x 4096 2.90 against 2.96): kQuantManyGroups.
 constexpr uint32_t kQuantManyGroups = 640;
-template <int IN_DT, int OUT_DT>
+template <int IN_DT, int OUT_DT, bool RAGGED>
 __global__ void __launch_bounds__(256) quant_row_block_kernel(QGEMM_QUANT_HEAD, const QuantArgs p) {
-    quant_row_block<IN_DT, OUT_DT>(x, q, scales, ld, rows_all, cols, per_row, inv, rows_per_slice, p);
+    quant_row_block<IN_DT, OUT_DT, RAGGED>(x, q, scales, ld, rows_all, cols, per_row, inv, rows_per_slice, p);
 }
-template <int IN_DT, int OUT_DT>
+template <int IN_DT, int OUT_DT, bool RAGGED>
 __global__ void __launch_bounds__(256) quant_few_blocks_kernel(const QuantArgs p) {
-    quant_row_block<IN_DT, OUT_DT>(QGEMM_QUANT_HEAD_OF(p));
+    quant_row_block<IN_DT, OUT_DT, RAGGED>(QGEMM_QUANT_HEAD_OF(p));
 }
 
 // ---- 128 x 128 blocks: one workgroup per block, which it holds in registers
-template <int IN_DT, int OUT_DT>
+template <int IN_DT, int OUT_DT, bool RAGGED>
 __global__ void __launch_bounds__(256) quant_square_block_kernel(QGEMM_QUANT_HEAD, const QuantArgs p) {
     typedef Piece<IN_DT> P;
     constexpr int ROWS = 256 / P::LANES, TURNS = 128 / ROWS;
@@ -367,11 +486,28 @@ __global__ void __launch_bounds__(256) quant_square_block_kernel(QGEMM_QUANT_HEA
         return a > b ? a : b;
     };
     v4i v[TURNS];
+    if (!RAGGED || cols >= (uint32_t)P::VEC) {
+        // (every lane loads, those outside from the nearest row or the start of a row: with a branch around each load the compiler
+        // copied the array at each of them, up to 235 registers, and the waves that keep memory busy were gone: 6144 x 7168 fp16 95.7 us, 27.8 so)
+        const uint32_t from = valid ? c : 0;
 #pragma unroll
-    for (int i = 0; i < TURNS; ++i) {
-        const uint32_t r = r0 + i * ROWS;
-        v[i] = v4i{0, 0, 0, 0};
-        if (r < rows_all && valid) v[i] = P::load(x, (size_t)r * ld + c, valid);
+        for (int i = 0; i < TURNS; ++i) {
+            const uint32_t r = r0 + i * ROWS;
+            v[i] = P::template load<RAGGED>(x, (size_t)(r < rows_all ? r : rows_all - 1) * ld + from, valid, true);
+        }
+#pragma unroll
+        for (int i = 0; i < TURNS; ++i) {
+            const bool in = r0 + i * ROWS < rows_all && valid;
+            if (RAGGED && jb + 1 == nbc) P::settle(v[i], in ? valid : 0);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[i][k] = in ? v[i][k] : 0;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < TURNS; ++i) {
+            const uint32_t r = r0 + i * ROWS;
+            v[i] = r < rows_all && valid ? P::load_elements(x, (size_t)r * ld + c, valid) : v4i{0, 0, 0, 0};
+        }
     }
     uint64_t ldq = p.ldq, scale_rs = p.scale_rs, scale_cs = p.scale_cs;
     asm volatile("" : "+s"(ldq), "+s"(scale_rs), "+s"(scale_cs));

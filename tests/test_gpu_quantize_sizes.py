@@ -29,3 +29,48 @@ def test_row_blocks_either_side_of_the_many_groups_rule(rows, cols, dt):
     q, s = R.quantize_fp8_block(xf, 1, 128)
     g, gs = Q.quantize(x, torch.float8_e4m3fn, Q.QUANT_BLOCK_1x128)
     assert np.array_equal(host(gs), s) and np.array_equal(_u8(g), q)
+
+
+def _strided(x, gap):
+    base = torch.zeros((x.shape[0], x.shape[1] + gap), dtype=x.dtype, device="cuda")
+    base[:, gap:] = x
+    return base[:, gap:]
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (3, 7), (129, 5), (2, 8), (16, 2045), (64, 2048), (64, 2049), (33, 1985), (260, 1027), (70, 4100)])
+def test_every_mode_at_row_ends_and_either_side_of_the_small_matrix(rows, cols, dt):
+    """64 x 2048 16-bit elements are the last small matrix; rows that end 1 .. 7 elements into a piece, shorter than one, with and
+    without a gap between them; the largest element last."""
+    say("quantize sizes", rows, cols, dt)
+    x, xf = _input(rows, cols, dt, 33)
+    x[-1, -1] = 9.0
+    xf = x.float().cpu().numpy()
+    for t in (x, _strided(x, 1), _strided(x, 3)):
+        for qt, ref, block in ((torch.int8, R.quantize_int8, R.quantize_int8_block), (torch.float8_e4m3fn, R.quantize_fp8, R.quantize_fp8_block)):
+            q, s = ref(xf)
+            g, gs = Q.quantize(t, qt, Q.QUANT_PER_MATRIX)
+            assert host(gs)[0] == s and np.array_equal(_u8(g), q.view(np.uint8)), (rows, cols, qt)
+            for mode, br in ((Q.QUANT_BLOCK_1x128, 1), (Q.QUANT_BLOCK_128x128, 128)):
+                q, s = block(xf, br, 128)
+                g, gs = Q.quantize(t, qt, mode)
+                assert np.array_equal(host(gs), s) and np.array_equal(_u8(g), q.view(np.uint8)), (rows, cols, qt, mode)
+
+
+@pytest.mark.parametrize("rows,cols", [(9, 517), (300, 1031)])
+@pytest.mark.parametrize("special", [float("nan"), float("inf"), -float("inf")])
+def test_special_values_wherever_they_stand(rows, cols, special):
+    """One NaN or infinity, in the last piece of a row and in the middle of one: the maximum is that of the numbers (infinity
+    counts as one), every other element keeps its bytes, for the single launch as for the two passes."""
+    x, _ = _input(rows, cols, torch.bfloat16, 35)
+    for at in ((rows - 1, cols - 1), (rows // 2, 128), (0, 3)):
+        say("quantize special", rows, cols, special, at)
+        y = x.clone()
+        y[at] = special
+        yf = y.float().cpu().numpy()
+        q, s = R.quantize_fp8(yf)
+        g, gs = Q.quantize(y, torch.float8_e4m3fn, Q.QUANT_PER_MATRIX)
+        assert np.array_equal(host(gs).view(np.uint32), np.array([s]).view(np.uint32)) and np.array_equal(_u8(g), q), at
+        q, s = R.quantize_fp8_block(yf, 128, 128)
+        g, gs = Q.quantize(y, torch.float8_e4m3fn, Q.QUANT_BLOCK_128x128)
+        assert np.array_equal(host(gs).view(np.uint32), s.view(np.uint32)) and np.array_equal(_u8(g), q), at
