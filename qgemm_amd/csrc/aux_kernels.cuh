@@ -30,6 +30,29 @@ __global__ void __launch_bounds__(256) transpose_u32_kernel(const uint32_t *__re
     }
 }
 
+// the first `bytes` (below 16) of v at any address, in parts of 8, 4, 2 and 1 bytes
+__device__ inline void store_part(void *p, v4i v, uint32_t bytes) {
+    char *dst = (char *)p;
+    uint32_t e0 = (uint32_t)v[0], e1 = (uint32_t)v[1];
+    if (bytes & 8) {
+        *(v2i_any *)dst = v2i{v[0], v[1]};
+        dst += 8;
+        e0 = (uint32_t)v[2];
+        e1 = (uint32_t)v[3];
+    }
+    if (bytes & 4) {
+        *(u32_any *)dst = e0;
+        dst += 4;
+        e0 = e1;
+    }
+    if (bytes & 2) {
+        *(u16_any *)dst = (uint16_t)e0;
+        dst += 2;
+        e0 >>= 16;
+    }
+    if (bytes & 1) *(uint8_t *)dst = (uint8_t)e0;
+}
+
 // ---------------------------------------------------------------------------
 // Byte transpose (the fp8 / int8 operands of the reference layout, packed operands, matrix_transpose).
 // 128 x 128 tile, 256 threads.  A thread loads 4 x 4 bytes (four
@@ -51,25 +74,37 @@ __device__ inline void transpose_bytes_tile(const uint8_t *__restrict__ in, size
     const uint32_t m0 = tile_m * T, n0 = tile_n * T;
     const int cg = threadIdx.x & 31, rg = threadIdx.x >> 5;      // 32 column groups of 4 bytes x 8 row groups of 16
     const uint32_t n = n0 + cg * 4;
-    auto load4 = [&](const uint8_t *src, bool row_in) -> uint32_t {        // four bytes of one row, zeros outside
-        if constexpr (ALIGNED) return *(const word_t *)src;
-        if (!row_in) return 0;
-        if (n + 4 <= N) return *(const word_t *)src;
+    // Four bytes of one row, zeros outside.  Ragged: every lane loads, from the nearest row and, where its row ends inside the four
+    // bytes, from the row's last four, and moves them down (no branch, in which each load would wait for the one before).
+    const bool wide = N >= 4;
+    const uint32_t from = n + 4 <= N ? n : (wide ? N - 4 : 0), down = (n - from) < 4 ? (n - from) * 8 : 32;
+    auto load4 = [&](uint32_t m) -> uint32_t {
+        const uint8_t *src = in + (size_t)(m < M ? m : M - 1) * ld + from;
         uint32_t w = 0;
-        for (int e = 0; e < 3; ++e)
-            if (n + e < N) w |= (uint32_t)src[e] << (8 * e);
-        return w;
+        if (wide) {
+            w = *(const word_t *)src;
+        } else {
+            for (uint32_t e = 0; e < N; ++e) w |= (uint32_t)src[e] << (8 * e);
+        }
+        return m < M && down < 32 ? w >> down : 0;
     };
 #pragma unroll
     for (int ch = 0; ch < 4; ++ch) {
         const uint32_t m = m0 + rg * 16 + ch * 4;
         uint32_t a = 0, b = 0, c = 0, d = 0;
-        if (n < N && m < M) {                     // (aligned: M % 4 == 0, the four rows are all inside or all outside)
-            const uint8_t *src = in + (size_t)m * ld + n;
-            a = load4(src, true);
-            b = load4(src + ld, m + 1 < M);
-            c = load4(src + 2 * ld, m + 2 < M);
-            d = load4(src + 3 * ld, m + 3 < M);
+        if constexpr (ALIGNED) {
+            if (n < N && m < M) {                 // (M % 4 == 0, the four rows are all inside or all outside)
+                const uint8_t *src = in + (size_t)m * ld + n;
+                a = *(const word_t *)src;
+                b = *(const word_t *)(src + ld);
+                c = *(const word_t *)(src + 2 * ld);
+                d = *(const word_t *)(src + 3 * ld);
+            }
+        } else {
+            a = load4(m);
+            b = load4(m + 1);
+            c = load4(m + 2);
+            d = load4(m + 3);
         }
         // v_perm_b32: selector byte k picks byte k of the result out of {src1 bytes 0-3, src0 bytes 4-7}
         const uint32_t ab_lo = __builtin_amdgcn_perm(b, a, 0x05010400), ab_hi = __builtin_amdgcn_perm(b, a, 0x07030602);
@@ -94,7 +129,7 @@ __device__ inline void transpose_bytes_tile(const uint8_t *__restrict__ in, size
         if (ALIGNED || om + 16 <= Mout) {
             *(vec_t *)dst = *(const v4i *)src;
         } else {
-            for (uint32_t e = 0; om + e < Mout; ++e) dst[e] = src[e];
+            store_part(dst, *(const v4i *)src, Mout - om);
         }
     }
 #endif
@@ -130,7 +165,8 @@ __global__ void __launch_bounds__(256) transpose_bytes2_kernel(const Transpose2A
 // elements, a workgroup of four waves 64 rows x 256 columns.
 // ---------------------------------------------------------------------------
 // ALIGNED: M and N multiples of 8, 16-byte aligned rows, Mout == M.  Otherwise any M, N, ld, pitch and element-aligned
-// pointers (through LDS one element per lane before: 1999 x 3001 11.4 -> 9.6 us): pieces that stick out go element by
+// pointers (1999 x 3001, us: through LDS one element per lane 11.4; so, with a branch around every
+// element of a row end 11.3, without 9.7): pieces that stick out go element by
 // element, the columns M .. Mout - 1 of the output are filled with zeros.
 template <bool ALIGNED>
 __device__ inline void transpose_u16_tile(const uint16_t *__restrict__ in, size_t ld, uint16_t *__restrict__ out, size_t pitch,
@@ -143,18 +179,33 @@ __device__ inline void transpose_u16_tile(const uint16_t *__restrict__ in, size_
     if (m >= Mout || n >= N) return;                                        // (aligned: blocks are wholly in or out)
     const bool cols = ALIGNED || n + 8 <= N, rows = ALIGNED || m + 8 <= Mout;
     v4i row[8];
-    const uint16_t *src = in + (size_t)m * ld + n;
+    if constexpr (ALIGNED) {
+        const uint16_t *src = in + (size_t)m * ld + n;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        if (!ALIGNED && m + j >= M) {
-            row[j] = v4i{0, 0, 0, 0};
-        } else if (cols) {
-            row[j] = *(const vec_t *)(src + (size_t)j * ld);
-        } else {
+        for (int j = 0; j < 8; ++j) row[j] = *(const vec_t *)(src + (size_t)j * ld);
+    } else if (N >= 8) {
+        // (every lane loads, from the nearest row and, where its row ends inside the piece, the row's last eight elements, which it
+        // moves down: no branch, in which each load would wait for the one before.)
+        const uint16_t *src = in + (cols ? n : N - 8);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) row[j] = *(const vec_t *)(src + (size_t)(m + j < M ? m + j : M - 1) * ld);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (__any(!cols)) {
+                uint32_t w[4] = {(uint32_t)row[j][0], (uint32_t)row[j][1], (uint32_t)row[j][2], (uint32_t)row[j][3]};
+                move_down<4>(w, cols ? 0 : (n + 8 - N) * 2);
+                row[j] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) row[j][k] = m + j < M ? row[j][k] : 0;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
             uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
             for (int e = 0; e < 7; ++e)
-                if (n + e < N) w[e >> 1] |= (uint32_t)src[(size_t)j * ld + e] << (16 * (e & 1));
+                if (m + j < M && n + e < N) w[e >> 1] |= (uint32_t)in[(size_t)(m + j) * ld + n + e] << (16 * (e & 1));
             row[j] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
         }
     }
@@ -177,9 +228,7 @@ __device__ inline void transpose_u16_tile(const uint16_t *__restrict__ in, size_
         if (rows) {
             *(vec_t *)(dst + (size_t)k * pitch) = v;
         } else {
-#pragma unroll
-            for (int e = 0; e < 7; ++e)
-                if (m + e < Mout) dst[(size_t)k * pitch + e] = (uint16_t)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
+            store_part(dst + (size_t)k * pitch, v, (Mout - m) * 2);
         }
     }
 #endif
@@ -206,32 +255,47 @@ struct PackOperand {
     uint32_t pitch;       // bytes between rows of dst, a multiple of 128
     uint32_t k_major;     // the source is K x rows
     uint32_t blocks, tiles_k;      // workgroups of this operand; k_major: tiles along k (the slower index is the tile of rows)
+    uint32_t inv;                  // inverse_of: k_major: tiles_k, else 16-byte pieces in a row of dst
 };
 struct PackArgs {
     PackOperand op[2];
 };
 
-// rows of the operand as they are: 16 bytes of dst per lane and turn, four turns per workgroup
+// rows of the operand as they are: 16 bytes of dst per lane and turn, four turns per workgroup.  Every lane loads: a piece that
+// reaches past the end of its row fetches the row's last 16 bytes and moves them down, one behind the end leaves zeros (rows of
+// fewer than 16 bytes go element by element).  (Element by element behind branches, each load waited for the one before; with product,
+// us: int8 2611 x 2104 x 3960 40.5 -> 36.2, 1531 x 4100 x 3004 36.2 -> 33.8, bf16 3001 x 1000 x 1999 with B stored K x N 34.4 -> 31.1.)
 template <int ES>
 __device__ inline void pack_rows(const PackOperand &o, uint32_t block) {
     const uint32_t per_row = o.pitch / 16, kbytes = o.k * ES;
     const uint32_t total = o.rows * per_row, first = block * 1024 + threadIdx.x;       // (the host keeps these below 2^32)
     v4i v[4];
+    uint32_t at[4];
+    const char *row[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const uint32_t i = first + j * 256;
-        v[j] = v4i{0, 0, 0, 0};
-        if (i >= total) continue;
-        const uint32_t r = i / per_row, at = (i - r * per_row) * 16;
-        const char *src = o.src + r * o.ld + at;
-        if (at + 16 <= kbytes) {
-            v[j] = *(const v4i_any *)src;
-        } else if (at < kbytes) {
+        const uint32_t i = first + j * 256, r = div_by_inv(i < total ? i : total - 1, per_row, o.inv, at[j]);
+        at[j] *= 16;
+        row[j] = o.src + r * o.ld;
+    }
+    if (kbytes >= 16) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = *(const v4i_any *)(row[j] + (at[j] + 16 <= kbytes ? at[j] : kbytes - 16));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (!__any(at[j] + 16 > kbytes)) continue;
+            uint32_t w[4] = {(uint32_t)v[j][0], (uint32_t)v[j][1], (uint32_t)v[j][2], (uint32_t)v[j][3]};
+            move_down<4>(w, at[j] + 16 <= kbytes ? 0 : (at[j] < kbytes ? at[j] + 16 - kbytes : 16));
+            v[j] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
             uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
             for (int e = 0; e < 16 / ES; ++e)
-                if (at + e * ES < kbytes) {
-                    const uint32_t x = ES == 2 ? (uint32_t)((const uint16_t *)src)[e] : (uint32_t)((const uint8_t *)src)[e];
+                if (at[j] + e * ES < kbytes) {
+                    const uint32_t x = ES == 2 ? (uint32_t)((const uint16_t *)row[j])[e] : (uint32_t)((const uint8_t *)row[j])[e];
                     w[e * ES / 4] |= x << (8 * (e * ES % 4));
                 }
             v[j] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
@@ -252,7 +316,8 @@ __global__ void __launch_bounds__(256) pack_kernel(const PackArgs a) {
         pack_rows<ES>(o, block);
         return;
     }
-    const uint32_t tk = block % o.tiles_k, tr = block / o.tiles_k;
+    uint32_t tk;
+    const uint32_t tr = div_by_inv(block, o.tiles_k, o.inv, tk);
     if constexpr (ES == 2)
         transpose_u16_tile<false>((const uint16_t *)o.src, o.ld / 2, (uint16_t *)o.dst, o.pitch / 2, o.k, o.pitch / 2, o.rows, tk, tr);
     else

@@ -1096,6 +1096,7 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
             n = ((uint64_t)rows[i] * (pitch / 16) + 1023) / 1024;
             if (n >= ((uint64_t)1 << 22)) return QGEMM_OK;          // (32-bit piece numbers in pack_rows)
         }
+        o.inv = inverse_of(o.k_major ? o.tiles_k : o.pitch / 16);
         o.blocks = (uint32_t)n;
         blocks += n;
     }
