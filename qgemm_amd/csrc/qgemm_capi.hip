@@ -385,7 +385,7 @@ size_t cols_for_full_rounds(const Variant *tab, int count, size_t M, size_t N, s
 // bf16 53.7 / 37.2; 64 x 2048 x 8192 15.2 / 11.3 (four slices), bf16 26.8 / 14.7; no split for 16 x 4096 x 4096 (7.6
 // against 9.5 with two slices) and none where the strips fill the CUs (16 x 8192 x 8192 15.2 against 18.8).
 // kmaj: the table is a K-major family, which has no narrow tiles: the estimate then serves every M
-int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
+int choose_by_rules(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
                    bool may_split, uint32_t *nsplit_out) {
     const int vi = choose_tile(tab, count, M, N, ksteps, block, kmaj, cus, may_split, nsplit_out);
     // The same kernel on 64 x 64 tiles: shapes with several row tiles whose 64 x 64 tiles fit one
@@ -504,6 +504,99 @@ int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t kst
             return i;
         }
     return vi;
+}
+
+// Up to 400 rows: an estimate of every row worth having there, fitted on 980 shapes (1 .. 400 rows x 512 .. 14336 columns x 512 ..
+// 8192 elements of K; fp8, int8 and bf16, and fp8 with block scales), every row forced, as the geometric mean of weights streamed
+// out of memory and weights resident.  The rules above were made on a few dozen shapes around 32 K steps, and with kernels that
+// started later; measured against the fastest row they are 15 % behind on average, at worst twice its time: 48 x 1200 x 1024 int8
+// 6.34 (two K slices) -> 4.05 us (16 x 16 tiles), 24 x 4432 x 1152 with block scales 7.52 -> 5.00, 136 x 7072 x 7088 38.4 -> 29.5,
+// 108 x 2048 x 3968 8.1 -> 6.4.  What the estimate takes is 2.5 % behind (on the third of the shapes that it was not fitted on 2.9).
+// A row costs `fixed`, and every round of `slots` workgroups per CU `round` plus its K steps at `alone` (few workgroups) .. `full`
+// (all CUs at work) us each, or, where that is longer, `late` and B at `stream` us/MB.  (The eight waves of the skinny-M kernel
+// take the steps in turn: halfway between the steps and the next multiple of eight.)
+struct FewRowsModel {
+    int slots;
+    double fixed, round, alone, full, late, stream;
+};
+struct FewRowsTile {
+    int bm, bn, kgroups;
+    FewRowsModel plain, block;
+};
+const FewRowsTile kFewRows[] = {
+    {16, 16, 8, {1, 1.51, 0.92, 0.0322, 0.0701, 2.91, 0.080}, {1, 1.60, 1.08, 0.0379, 0.0726, 1.23, 0.142}},
+    {32, 16, 8, {1, 1.57, 1.20, 0.0405, 0.0760, 0.47, 0.279}, {1, 1.47, 1.39, 0.0571, 0.0861, 2.70, 0.201}},
+    {16, 32, 8, {1, 1.37, 0.87, 0.0580, 0.1362, 3.22, 0.082}, {1, 1.11, 1.25, 0.0704, 0.1325, 3.30, 0.084}},
+    {32, 32, 8, {1, 1.64, 1.27, 0.0619, 0.1399, 1.40, 0.231}, {1, 1.65, 1.38, 0.0742, 0.1468, 2.68, 0.118}},
+    {64, 32, 8, {1, 1.54, 1.92, 0.0918, 0.1658, 0.00, 0.369}, {1, 1.98, 1.62, 0.1140, 0.1946, 1.52, 0.287}},
+    {128, 32, 8, {1, 1.16, 3.28, 0.1514, 0.2366, 3.00, 0.250}, {1, 1.89, 2.83, 0.2255, 0.2790, 3.00, 0.250}},
+    {64, 64, 8, {1, 1.04, 3.41, 0.1437, 0.1852, 2.72, 0.274}, {1, 1.89, 2.73, 0.1700, 0.2182, 3.17, 0.353}},
+    {16, 32, 1, {5, 2.44, 0.00, 0.1888, 0.5637, 2.90, 0.186}, {8, 0.33, 1.73, 0.3657, 0.9489, 0.94, 0.503}},
+    {64, 32, 1, {1, 1.51, 1.17, 0.2213, 0.2290, 3.64, 0.216}, {5, 1.74, 0.29, 0.3816, 1.1589, 2.88, 0.382}},
+    {128, 32, 1, {1, 1.62, 1.46, 0.3006, 0.3251, 3.00, 0.250}, {4, 2.09, 0.00, 0.4505, 1.4063, 3.00, 0.250}},
+    {64, 128, 1, {1, 1.47, 1.64, 0.5108, 0.5546, 3.00, 0.250}, {3, 2.03, 0.45, 0.6274, 1.4203, 3.00, 0.250}},
+    {64, 128, 2, {1, 1.42, 2.72, 0.2736, 0.3462, 4.01, 0.312}, {1, 2.64, 1.61, 0.3269, 0.5024, 3.00, 0.250}},
+    {128, 128, 2, {1, 1.97, 2.90, 0.3409, 0.5439, 3.00, 0.250}, {1, 2.50, 2.25, 0.4247, 0.6367, 3.00, 0.250}}};
+
+// slices of K a launch has where the choice of a row has no opinion (see plan_nt)
+uint32_t slices_for_few_tiles(size_t tiles, uint32_t ksteps, int cus) {
+    if (tiles * 2 > (size_t)cus || ksteps < 8) return 1;
+    // enough slices to cover the CUs about twice, at least 4 K steps each
+    const uint32_t want = (uint32_t)((2 * (size_t)cus + tiles - 1) / tiles);
+    return std::min<uint32_t>(want, ksteps / 4);
+}
+
+// us; 0: the estimate does not know the row
+double few_rows_estimate(const Variant &v, size_t M, size_t N, size_t ksteps, bool block, int cus, uint32_t nsplit) {
+    for (const FewRowsTile &t : kFewRows) {
+        if (t.bm != v.bm || t.bn != v.bn || t.kgroups != v.kgroups) continue;
+        const FewRowsModel &m = block ? t.block : t.plain;
+        const size_t steps = (ksteps + nsplit - 1) / nsplit, slices = (ksteps + steps - 1) / steps;
+        const size_t wgs = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * slices, slots = (size_t)cus * m.slots;
+        const double load = std::min(1.0, (double)wgs / slots), n = t.kgroups == 8 ? (steps + (steps + 7) / 8 * 8) * 0.5 : (double)steps;
+        const double rounds = (double)((wgs + slots - 1) / slots);
+        double us = std::max(m.fixed + rounds * (m.round + n * (m.alone + (m.full - m.alone) * load)),
+                             m.late + (double)N * ksteps * 128e-6 * m.stream);
+        if (slices > 1) us += 2.6 + (double)M * N * 4e-6 * (slices + 1) / 4.5;
+        return us;
+    }
+    return 0;
+}
+
+// The row of the rules, or where the estimate puts another one 3 % ahead of it that one, with no more K slices than the rules asked
+// for (so that no call needs a workspace that did not need one).  Below 32 K steps, and with block scales up to 128 rows; from 32
+// K steps on the rules above are 7 - 8 % behind, and their choice, which was measured with streamed weights, stays.  With 8 K steps
+// and one scale the waves of the skinny-M kernel have a single step each and the estimate is less sure of them: 13 %.
+// (whole: not the rows or columns beside a first launch, whose estimate the split of the two was made with)
+int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
+                   bool may_split, bool whole, uint32_t *nsplit_out) {
+    const int vi = choose_by_rules(tab, count, M, N, ksteps, block, kmaj, cus, may_split, nsplit_out);
+    if (vi < 0 || kmaj || !whole || M > 400 || tab[vi].arith == AR_F8W || !g_ctx.small_tiles || !(ksteps < 32 || (block && M <= 128))) return vi;
+    uint32_t asked = std::max<uint32_t>(1, *nsplit_out);
+    if (*nsplit_out == 0 && may_split)
+        asked = std::max<uint32_t>(1, slices_for_few_tiles(((M + tab[vi].bm - 1) / tab[vi].bm) * ((N + tab[vi].bn - 1) / tab[vi].bn), (uint32_t)ksteps, cus));
+    const double t_rules = few_rows_estimate(tab[vi], M, N, ksteps, block, cus, asked);
+    if (t_rules == 0) return vi;
+    int best = vi;
+    uint32_t best_ns = *nsplit_out;
+    double best_t = t_rules * (ksteps == 8 && !block ? 0.87 : 0.97);
+    for (int i = 0; i < count; ++i) {
+        const Variant &v = tab[i];
+        if ((v.bm > 32 && (size_t)v.bm > 2 * M) || M > 12 * (size_t)v.bm) continue;
+        const size_t tiles = ((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn);
+        if (tiles > 1400) continue;
+        for (uint32_t ns = 1; ns <= 8 && ns <= asked; ns *= 2) {
+            if (ns > 1 && (ksteps / ns < 6 || tiles * ns > 300)) break;
+            const double t = few_rows_estimate(v, M, N, ksteps, block, cus, ns);
+            if (t > 0 && t < best_t) {
+                best = i;
+                best_ns = ns;
+                best_t = t;
+            }
+        }
+    }
+    *nsplit_out = best_ns;
+    return best;
 }
 
 int choose_tile(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
@@ -683,7 +776,7 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     const Variant *tab = table_for(q.arith, q.block, q.kmaj, &count);
     if (!tab) return QGEMM_ERR_UNSUPPORTED;
     uint32_t model_split = 0;
-    int vi = choose_variant(tab, count, q.M, q.N, ksteps_of(q), q.block, q.kmaj, g_ctx.num_cus, q.split_k == 0, &model_split);
+    int vi = choose_variant(tab, count, q.M, q.N, ksteps_of(q), q.block, q.kmaj, g_ctx.num_cus, q.split_k == 0, may_split_rows, &model_split);
     if (may_split_rows && vi >= 0 && !forced() && g_ctx.force_split <= 0 && q.split_k == 0 && model_split <= 1 &&
         q.M > 128 && q.kmaj == 0) {
         uint32_t ns = 0;
@@ -777,11 +870,7 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     else if (q.split_k == 0) {
         if (g_ctx.force_split > 0) nsplit = (uint32_t)g_ctx.force_split;
         else if (model_split > 0) nsplit = model_split;
-        else if (pl.tiles * 2 <= (size_t)g_ctx.num_cus && a.ksteps >= 8) {
-            // enough slices to cover the CUs about twice, at least 4 K steps each
-            uint32_t want = (uint32_t)((2 * (size_t)g_ctx.num_cus + pl.tiles - 1) / pl.tiles);
-            nsplit = std::min<uint32_t>(want, a.ksteps / 4);
-        }
+        else nsplit = slices_for_few_tiles(pl.tiles, a.ksteps, g_ctx.num_cus);
     }
     nsplit = std::max<uint32_t>(1, std::min<uint32_t>(nsplit, a.ksteps));
     a.ksteps_per_split = (a.ksteps + nsplit - 1) / nsplit;
