@@ -348,6 +348,155 @@ __global__ void __launch_bounds__(256, 2) gemm_any_kernel(const AnyArgs p) {
 #endif
 }
 
+// Few rows: the plan of the skinny-M kernel (gemm_skinny.cuh) on operands at any address.  16 TM rows x 32 columns a workgroup,
+// the K steps of 128 bytes dealt to its eight waves in turn, two in flight a wave; nothing is shared until the eight partial sums
+// meet in LDS, added in wave order.  The pieces travel through registers, where the last step's are moved and cut (as in
+// AnyStage), to the wave's own corner of LDS and from there to the fragments: no barrier in the loop.
+// Bound by latency, hence by bytes in flight: 12 KiB a wave and 96 a workgroup, where the kernel above has 16 KiB a workgroup and
+// half as many of them.  Up to 16 rows two workgroups share a CU (128 registers a lane; widened blocks of fp8 need more).  us, graph
+// replays, kernel above / this: fp8 block scales 16 x 1152 x 4475 39.2 / 9.2, 16 x 7168 x 8001 82.0 / 21.4 (2.7 TB/s), 48 x 4096 x 2001
+// 21.6 / 8.6; int8 17 x 1152 x 4475 21.9 / 9.5, bf16 1 x 1176 x 2561 23.8 / 7.1.
+template <int ARITH, bool BLOCK, int TM>
+__global__ void __launch_bounds__(512, TM == 1 && !(BLOCK && ARITH == AR_F8W) ? 4 : 2) gemm_few_kernel(const AnyArgs p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int TN = 2, NW = 8, PA = 2 * TM, PB = 2 * TN, ES = ARITH == AR_BF16 || ARITH == AR_F16 ? 2 : 1;
+    constexpr int AREA = (PA + PB) * 1024;                               // of one step, a wave's own
+    static_assert(TM * TN * 1024 <= AREA && NW * AREA <= 65536, "");
+    __shared__ __attribute__((aligned(1024))) char lds[NW * AREA];
+    typedef typename AccT<ARITH>::type part_t;
+    typedef std::conditional_t<BLOCK, v4f, part_t> acc_t;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t row0 = blockIdx.y * (16 * TM), col0 = blockIdx.x * (16 * TN);
+    const uint32_t kbytes = p.K * ES, steps = (kbytes + 127) / 128;
+    // piece j of a step: rows 8 j .. 8 j + 7, lane l's 16 bytes of row l >> 3 in slot l (rotated by the row: lds_slot)
+    const uint32_t chunk = (((lane & 7) - (lane >> 3)) & 7) * 16;
+    const char *pa[PA], *pb[PB];
+    auto first = [&](const AnyOperand &o, uint32_t r) { return o.p + (r < o.rows ? r : o.rows - 1) * o.ld + chunk; };
+#pragma unroll
+    for (int j = 0; j < PA; ++j) pa[j] = first(p.a, row0 + 8 * j + (lane >> 3));
+#pragma unroll
+    for (int j = 0; j < PB; ++j) pb[j] = first(p.b, col0 + 8 * j + (lane >> 3));
+    auto inside = [](const AnyOperand &o, const char *q) { return q + 16 <= o.end ? q : o.end - 16; };
+    v4i ra[2][PA], rb[2][PB];
+    float as[2][TM], bs[2];
+    auto load = [&](uint32_t k) {                                        // steps k and k + 8
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const uint32_t kt = k + s * NW;
+            if (kt >= steps) return;
+#pragma unroll
+            for (int j = 0; j < PB; ++j) rb[s][j] = *(const v4i_any *)inside(p.b, pb[j] + (size_t)kt * 128);
+#pragma unroll
+            for (int j = 0; j < PA; ++j) ra[s][j] = *(const v4i_any *)inside(p.a, pa[j] + (size_t)kt * 128);
+            if constexpr (BLOCK) {
+#pragma unroll
+                for (int a = 0; a < TM; ++a) {
+                    const uint32_t m = row0 + a * 16 + (lane & 15);
+                    as[s][a] = p.as[(size_t)(m < p.a.rows ? m : p.a.rows - 1) * p.as_ms + (size_t)kt * p.as_ks];
+                }
+                bs[s] = p.bs[(size_t)(col0 / kScaleBlock) * p.bs_ns + (size_t)kt * p.bs_ks];
+            }
+        }
+    };
+    auto settle = [&](const AnyOperand &o, const char *q, uint32_t kt, v4i &r) {
+        uint32_t w[4] = {(uint32_t)r[0], (uint32_t)r[1], (uint32_t)r[2], (uint32_t)r[3]};
+        q += (size_t)kt * 128;
+        move_down<4>(w, (uint32_t)(q - inside(o, q)));
+        const int left = (int)(kbytes - kt * 128) - (int)chunk;          // bytes of the row from here on
+#pragma unroll
+        for (int d = 0; d < 4; ++d) w[d] &= left >= 4 * d + 4 ? ~0u : left > 4 * d ? (1u << (8 * (left - 4 * d))) - 1 : 0u;
+        r = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+    };
+    char *mine = lds + wave * AREA;
+    const int off0 = lds_slot(lane & 15, lane >> 4) * 16, off1 = lds_slot(lane & 15, 4 + (lane >> 4)) * 16;
+    acc_t acc[TM][TN];
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
+    v4i fa[TM][2], fb[TN][2];
+    float f[TM];
+    auto turn = [&](int s, uint32_t kt) {                                // the pieces of step kt to fragments
+        if ((kt + 1) * 128 > kbytes) {
+#pragma unroll
+            for (int j = 0; j < PA; ++j) settle(p.a, pa[j], kt, ra[s][j]);
+#pragma unroll
+            for (int j = 0; j < PB; ++j) settle(p.b, pb[j], kt, rb[s][j]);
+        }
+#pragma unroll
+        for (int j = 0; j < PA; ++j) *(v4i *)(mine + j * 1024 + lane * 16) = ra[s][j];
+#pragma unroll
+        for (int j = 0; j < PB; ++j) *(v4i *)(mine + (PA + j) * 1024 + lane * 16) = rb[s][j];
+#pragma unroll
+        for (int a = 0; a < TM; ++a) {
+            fa[a][0] = *(const v4i *)(mine + a * 2048 + off0);
+            fa[a][1] = *(const v4i *)(mine + a * 2048 + off1);
+            if constexpr (BLOCK) f[a] = as[s][a] * bs[s];
+        }
+#pragma unroll
+        for (int b = 0; b < TN; ++b) {
+            fb[b][0] = *(const v4i *)(mine + (TM + b) * 2048 + off0);
+            fb[b][1] = *(const v4i *)(mine + (TM + b) * 2048 + off1);
+        }
+    };
+    auto compute = [&]() {
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+            for (int b = 0; b < TN; ++b) {
+                if constexpr (BLOCK) {
+                    const part_t q = mma128<ARITH>(fb[b][0], fb[b][1], fa[a][0], fa[a][1], part_t{0, 0, 0, 0});
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[a][b][r] += (float)q[r] * f[a];
+                } else {
+                    acc[a][b] = mma128<ARITH>(fb[b][0], fb[b][1], fa[a][0], fa[a][1], acc[a][b]);
+                }
+            }
+    };
+    load(wave);
+    const float scale = !BLOCK && p.per_matrix_scale ? p.as[0] * p.bs[0] : 1.0f;
+    for (uint32_t k = wave; k < steps; k += 2 * NW) {
+        const bool two = k + NW < steps;
+        turn(0, k);
+        compute();
+        if (two) turn(1, k + NW);
+        if (k + 2 * NW < steps) load(k + 2 * NW);
+        if (two) compute();
+    }
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) *(acc_t *)(mine + (a * TN + b) * 1024 + lane * 16) = acc[a][b];
+    __syncthreads();
+    if (wave >= TM * TN) return;
+    acc_t sum = *(const acc_t *)(lds + wave * 1024 + lane * 16);
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+        const acc_t o = *(const acc_t *)(lds + w * AREA + wave * 1024 + lane * 16);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[r] += o[r];
+    }
+    const uint32_t m = row0 + wave / TN * 16 + (lane & 15), n = col0 + wave % TN * 16 + (lane >> 4) * 4;
+    if (m >= p.a.rows || n >= p.b.rows) return;
+    const size_t idx = (size_t)m * p.ldc + n;
+    const int valid = p.b.rows - n < 4 ? (int)(p.b.rows - n) : 4;
+    if constexpr (ARITH == AR_I8 && !BLOCK) {
+        if (p.out_dtype == QGEMM_DT_I32) {
+            int *dst = (int *)p.C + idx;
+            if (valid == 4) *(v4i_any *)dst = sum;
+            else
+                for (int r = 0; r < 3; ++r)
+                    if (r < valid) dst[r] = sum[r];
+            return;
+        }
+    }
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = (float)sum[r] * scale;
+    store_out4(p.C, idx, v, p.out_dtype, valid);
+#endif
+}
+
 // One thread per element of C, for fewer than 16 elements of K: an operand may then be shorter than one load of the kernel
 // above, and where all of it is small a few loads of single elements are done first (graph replays, this / that, us:
 // 3 x 3 x 3 bf16 1.6 / 3.6).  One K block at most, folded as above.

@@ -1081,6 +1081,44 @@ int any_tile(int in_dtype, int out_dtype, bool block, bool km, size_t M, size_t 
     return wide * (km && !any_folded(in_dtype, out_dtype) ? 2 : 1) >= (uint64_t)g_ctx.num_cus ? 128 : 64;
 }
 
+// Time of the any-shape kernel on operands that are not transposed on the way, us: 64 x 64 tiles, three on a CU, and 128 x 128, two
+// on a CU.  (fitted as pack_pays says)
+double any_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N, size_t K) {
+    struct AnyModel {
+        double shared64, alone64, fixed64, shared128, alone128, fixed128;
+    };
+    static const AnyModel kAny16{0.68, 0.45, 3.6, 1.29, 0.90, 10.4}, kAnyF8{0.63, 0.43, 3.2, 1.11, 0.72, 8.6},
+        kAnyF8Block{0.72, 0.48, 2.7, 1.37, 0.99, 6.6}, kAnyI8{0.81, 0.47, 3.4, 1.37, 0.94, 8.9}, kAnyI8Block{1.18, 0.67, 1.6, 0, 0, 0};
+    const AnyModel &m = in_dtype == QGEMM_DT_F8E4M3 ? (block ? kAnyF8Block : kAnyF8) : (in_dtype == QGEMM_DT_I8 ? (block ? kAnyI8Block : kAnyI8) : kAny16);
+    const size_t cus = g_ctx.num_cus, tile = any_tile(in_dtype, out_dtype, block, false, M, N), steps = (K - 1) / (in_dtype == QGEMM_DT_I8 ? 128 : 64) + 1;
+    const size_t tiles = ((M + tile - 1) / tile) * ((N + tile - 1) / tile);
+    return tile == 64 ? rounds_cost(tiles, 3 * cus, cus, steps, m.shared64, m.alone64, m.fixed64)
+                      : rounds_cost(tiles, 2 * cus, cus, steps, m.shared128, m.alone128, m.fixed128);
+}
+
+// ... and of the kernel for few rows (gemm_few_kernel), on 16 x 32 tiles up to 16 rows, else 32 x 32: every round of
+// per_cu workgroups a CU costs `round` and its steps of 128 bytes at `alone` .. `full` (all CUs at work).  Fitted on 500 ragged shapes of 1 .. 128 rows x 512 ..
+// 14336 columns x K = 301 .. 8191, graph replays: the faster of the two kernels by these estimates is 1 % behind the faster one
+// measured, the any-shape kernel alone 78 %.  On average this kernel takes 1 / 2.18 of its time up to 16 rows, 1 / 1.96 up to 32,
+// 1 / 1.55 up to 64 and 1 / 1.45 up to 128 (where it is behind on many columns: 64 x 8272 x 1109 bf16 13.8 against 17.1 us).
+// 16-bit operands with fp32 output stay with the sums that any_folded says, and block scales with fp32 output below 3000 elements:
+// a wave's few blocks are rounded once more where the partial sums meet (relative error, tiles / few rows, int8 16 x 300 x 1031
+// 5.3e-8 / 6.4e-8, x 2051 6.8e-8 / 6.9e-8, but x 4001 8.4e-8 / 7.3e-8, fp8 x 7999 14.8e-8 / 8.3e-8; a 16-bit output hides it).
+double few_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N, size_t K) {
+    if (M > 128 || K >= ((size_t)1 << 30) || any_folded(in_dtype, out_dtype) || (block && out_dtype == QGEMM_DT_F32 && K < 3000)) return 1e30;
+    struct FewModel {
+        double fixed, round, alone, full;
+        size_t per_cu;
+    };
+    static const FewModel k16[2] = {{1.39, 1.38, 0.098, 0.391, 2}, {2.28, 0.98, 0.154, 0.203, 1}}, kF8[2] = {{1.27, 1.27, 0.151, 0.446, 2}, {1.55, 1.41, 0.211, 0.268, 1}},
+        kF8Block[2] = {{2.29, 0.32, 0.164, 0.252, 1}, {2.46, 0.53, 0.217, 0.285, 1}}, kI8[2] = {{1.19, 1.14, 0.136, 0.495, 2}, {2.11, 0.86, 0.183, 0.235, 1}},
+        kI8Block[2] = {{1.22, 1.22, 0.133, 0.537, 2}, {2.12, 0.80, 0.199, 0.279, 1}};
+    const FewModel &m = (in_dtype == QGEMM_DT_F8E4M3 ? (block ? kF8Block : kF8) : (in_dtype == QGEMM_DT_I8 ? (block ? kI8Block : kI8) : k16))[M > 16];
+    const size_t slots = g_ctx.num_cus * m.per_cu, steps = (K * dtype_bytes(in_dtype) + 127) / 128, wgs = ((N + 31) / 32) * (M > 16 ? (M + 31) / 32 : 1);
+    const double load = std::min(1.0, (double)wgs / slots), n = (steps + (steps + 7) / 8 * 8) * 0.5;
+    return m.fixed + (double)((wgs + slots - 1) / slots) * (m.round + n * (m.alone + (m.full - m.alone) * load));
+}
+
 // Is a product on the any-shape path faster packed?  Estimates of both, in microseconds, fitted on 240 ragged shapes (1 .. 4096
 // rows x 1024 .. 7168 columns x K = 777 .. 7161; fp8 and int8 with one scale and with block scales, bf16), eager calls: the way
 // chosen is 0.7 % behind the faster one on average, 33 % at worst (int8 block scales 200 x 5000 x 3004 20.4 / 27.1).  Two
@@ -1092,17 +1130,7 @@ int any_tile(int in_dtype, int out_dtype, bool block, bool km, size_t M, size_t 
 bool pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
     const size_t kbytes = K * dtype_bytes(in_dtype), cus = g_ctx.num_cus;
     if (km) return kbytes > 512 || (double)q.M * q.N >= 4e6;
-    // any-shape kernel: 64 x 64 tiles, three on a CU, and 128 x 128, two on a CU
-    struct AnyModel {
-        double shared64, alone64, fixed64, shared128, alone128, fixed128;
-    };
-    static const AnyModel kAny16{0.68, 0.45, 3.6, 1.29, 0.90, 10.4}, kAnyF8{0.63, 0.43, 3.2, 1.11, 0.72, 8.6},
-        kAnyF8Block{0.72, 0.48, 2.7, 1.37, 0.99, 6.6}, kAnyI8{0.81, 0.47, 3.4, 1.37, 0.94, 8.9}, kAnyI8Block{1.18, 0.67, 1.6, 0, 0, 0};
-    const AnyModel &m = in_dtype == QGEMM_DT_F8E4M3 ? (q.block ? kAnyF8Block : kAnyF8) : (in_dtype == QGEMM_DT_I8 ? (q.block ? kAnyI8Block : kAnyI8) : kAny16);
-    const size_t tile = any_tile(in_dtype, q.out_dtype, q.block, false, q.M, q.N), any_steps = (K - 1) / (in_dtype == QGEMM_DT_I8 ? 128 : 64) + 1;
-    const size_t tiles = ((q.M + tile - 1) / tile) * ((q.N + tile - 1) / tile);
-    const double t_any = tile == 64 ? rounds_cost(tiles, 3 * cus, cus, any_steps, m.shared64, m.alone64, m.fixed64)
-                                    : rounds_cost(tiles, 2 * cus, cus, any_steps, m.shared128, m.alone128, m.fixed128);
+    const double t_any = std::min(any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K), few_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K));
     // packed: two launches and the packing, then the tiles' estimate or the skinny-M kernel's (see choose_variant)
     int count = 0;
     const Variant *tab = table_for(q.arith, q.block, 0, &count);
@@ -1221,6 +1249,13 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
     }
     constexpr int W = BLOCK && DT == QGEMM_DT_I8 ? 64 : 128;
     const bool km = a.a.k_major || a.b.k_major;
+    if (!km && few_estimate(DT, a.out_dtype, BLOCK, a.a.rows, a.b.rows, a.K) < any_estimate(DT, a.out_dtype, BLOCK, a.a.rows, a.b.rows, a.K)) {
+        constexpr int ARITH = DT == QGEMM_DT_I8 ? AR_I8 : DT == QGEMM_DT_F8E4M3 ? AR_F8W : DT == QGEMM_DT_BF16 ? AR_BF16 : AR_F16;
+        const bool one = a.a.rows <= 16;
+        hipLaunchKernelGGL((one ? gemm_few_kernel<ARITH, BLOCK, 1> : gemm_few_kernel<ARITH, BLOCK, 2>),
+                           dim3((a.b.rows + 31) / 32, one ? 1 : (a.a.rows + 31) / 32), dim3(512), 0, stream, a);
+        return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+    }
     const int T = any_tile(DT, a.out_dtype, BLOCK, km, a.a.rows, a.b.rows);
     const uint64_t tiles_m = ((uint64_t)a.a.rows + T - 1) / T, tiles_n = ((uint64_t)a.b.rows + T - 1) / T, tiles = tiles_m * tiles_n;
     if (tiles >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;    // grid limit
