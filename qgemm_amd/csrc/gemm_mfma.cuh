@@ -305,20 +305,33 @@ __device__ inline void mma128_inplace(v4i x0, v4i x1, v4i y0, v4i y1, typename A
 constexpr uint32_t kHeadSplit = 1, kHeadStream = 2, kHeadStagger = 4;      // K split across workgroups; GemmArgs::b_stream; GemmArgs::stagger
 constexpr int kHeadRotShift = 3, kHeadGroupShift = 16;                     // GemmArgs::k_rot; TileMap::group_m
 constexpr uint32_t kHeadRotMax = 0x1FFF, kHeadGroupMax = 0xFFFF;
+// (Seven 64-bit numbers: the runtime looks up what every pointer among the arguments points into and sets them one by one; as two
+// pointers and ten 32-bit numbers they cost a launch 0.3 us of host time more.)
 struct LaunchHead {
-    uint32_t k_bytes, flags;
-    explicit LaunchHead(const GemmArgs &a)
-        : k_bytes(a.k_tail ? (a.ksteps - 1) * 128 + a.k_tail : a.ksteps * 128),
-          flags((a.nsplit > 1 ? kHeadSplit : 0) | (a.b_stream ? kHeadStream : 0) | (a.stagger ? kHeadStagger : 0) |
-                (a.k_rot < kHeadRotMax ? a.k_rot : kHeadRotMax) << kHeadRotShift |
-                (a.map.group_m < kHeadGroupMax ? a.map.group_m : kHeadGroupMax) << kHeadGroupShift) {}
+    uint64_t A, B, ld, mn, kf, inv01, inv23;
+    LaunchHead(const GemmArgs &a, uint32_t inv0, uint32_t inv1, uint32_t inv2, uint32_t inv3)
+        : A((uint64_t)(uintptr_t)a.A), B((uint64_t)(uintptr_t)a.B), ld(two(a.lda, a.ldb)), mn(two(a.M, a.N)),
+          kf(two(a.k_tail ? (a.ksteps - 1) * 128 + a.k_tail : a.ksteps * 128,
+                 (a.nsplit > 1 ? kHeadSplit : 0) | (a.b_stream ? kHeadStream : 0) | (a.stagger ? kHeadStagger : 0) |
+                     (a.k_rot < kHeadRotMax ? a.k_rot : kHeadRotMax) << kHeadRotShift |
+                     (a.map.group_m < kHeadGroupMax ? a.map.group_m : kHeadGroupMax) << kHeadGroupShift)),
+          inv01(two(inv0, inv1)), inv23(two(inv2, inv3)) {}
+    static uint64_t two(uint32_t lo, uint32_t hi) { return lo | (uint64_t)hi << 32; }
 };
+#define QGEMM_HEAD uint64_t A_, uint64_t B_, uint64_t ld_, uint64_t mn_, uint64_t kf_, uint64_t inv01_, uint64_t inv23_
+#define QGEMM_HEAD_OF(h) (h).A, (h).B, (h).ld, (h).mn, (h).kf, (h).inv01, (h).inv23
+#define QGEMM_HEAD_NAMES                                                                                                  \
+    const char *A = (const char *)A_, *B = (const char *)B_;                                                              \
+    const uint32_t lda = (uint32_t)ld_, ldb = (uint32_t)(ld_ >> 32), M = (uint32_t)mn_, N = (uint32_t)(mn_ >> 32),        \
+                   k_bytes = (uint32_t)kf_, flags = (uint32_t)(kf_ >> 32), inv0 = (uint32_t)inv01_, inv1 = (uint32_t)(inv01_ >> 32), \
+                   inv2 = (uint32_t)inv23_
 
 template <class C>
 __global__ void __launch_bounds__(C::THREADS)
-gemm_nt_kernel(const char *A, const char *B, uint32_t lda, uint32_t ldb, uint32_t M, uint32_t N, uint32_t k_bytes, uint32_t flags,
-               uint32_t inv_group, uint32_t inv_gm, uint32_t inv_last, uint32_t inv_nk, const GemmArgs p) {
+gemm_nt_kernel(QGEMM_HEAD, const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the launch stub
+    QGEMM_HEAD_NAMES;                  // (inv0 .. inv2: the three of TileMap, then of the K steps)
+    uint32_t inv_nk = (uint32_t)(inv23_ >> 32);
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     // part_t: what one MFMA step of 128 bytes of K delivers (int32 for int8 operands, else fp32); acc_t: the running
     // sums.  With block scales the sums are fp32 whatever the operands: an int8 partial product of one K block is an
@@ -357,7 +370,7 @@ gemm_nt_kernel(const char *A, const char *B, uint32_t lda, uint32_t ldb, uint32_
         else inv_nk = p.inv_nk_last;
     }
     uint32_t tm, tn;
-    tile_map(wg, TileMap{(M + C::BM - 1) / C::BM, (N + C::BN - 1) / C::BN, flags >> kHeadGroupShift, inv_group, inv_gm, inv_last}, tm, tn);
+    tile_map(wg, TileMap{(M + C::BM - 1) / C::BM, (N + C::BN - 1) / C::BN, flags >> kHeadGroupShift, inv0, inv1, inv2}, tm, tn);
     const uint32_t row0 = tm * C::BM, col0 = tn * C::BN;
     const int nk = (int)(kend - kbeg);
 

@@ -61,12 +61,13 @@ __device__ inline void wait_landed() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// (arguments in front of `p`: see LaunchHead; inv0 .. inv2: of the row tiles, or, 64 x 64 form, the three of TileMap)
+// (arguments in front of `p`: see LaunchHead; inverses of the row tiles, or, 64 x 64 form, the three of TileMap, then of the K steps)
 template <class C>
 __global__ void __launch_bounds__(C::THREADS)
-gemm_skinny_kernel(const char *A, const char *B, uint32_t lda, uint32_t ldb, uint32_t M, uint32_t N, uint32_t k_bytes, uint32_t flags,
-                   uint32_t inv_nk, uint32_t inv0, uint32_t inv1, uint32_t inv2, const GemmArgs p) {
+gemm_skinny_kernel(QGEMM_HEAD, const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
+    QGEMM_HEAD_NAMES;
+    uint32_t inv_nk = (uint32_t)(inv23_ >> 32);
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     typedef typename AccT<C::ARITH>::type part_t;                       // one MFMA step: int32 for int8 operands, else fp32
     typedef std::conditional_t<C::BLOCK_SCALE, v4f, part_t> acc_t;      // the running sums: fp32 with block scales
