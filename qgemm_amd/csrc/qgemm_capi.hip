@@ -577,9 +577,13 @@ int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t kst
         asked = std::max<uint32_t>(1, slices_for_few_tiles(((M + tab[vi].bm - 1) / tab[vi].bm) * ((N + tab[vi].bn - 1) / tab[vi].bn), (uint32_t)ksteps, cus));
     const double t_rules = few_rows_estimate(tab[vi], M, N, ksteps, block, cus, asked);
     if (t_rules == 0) return vi;
+    // (with streamed weights tiles of a second round, rows without a K split inside the workgroup where they stand several on a CU, and
+    // those rows behind long loops with block scales cost more than the estimate says, which is a mean of streamed and resident
+    // weights: 32 x 14336 x 4096 with block scales 14.7 us on 224 tiles of 64 x 64, 16.2 on 448 of 32 x 32)
+    const bool one_round = ((M + tab[vi].bm - 1) / tab[vi].bm) * ((N + tab[vi].bn - 1) / tab[vi].bn) * asked <= (size_t)cus;
     int best = vi;
     uint32_t best_ns = *nsplit_out;
-    double best_t = t_rules * (ksteps == 8 && !block ? 0.87 : 0.97);
+    double best_t = t_rules * (ksteps == 8 && !block ? 0.87 : ksteps >= 32 ? 0.93 : 0.97);
     for (int i = 0; i < count; ++i) {
         const Variant &v = tab[i];
         if ((v.bm > 32 && (size_t)v.bm > 2 * M) || M > 12 * (size_t)v.bm) continue;
@@ -587,7 +591,9 @@ int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t kst
         if (tiles > 1400) continue;
         for (uint32_t ns = 1; ns <= 8 && ns <= asked; ns *= 2) {
             if (ns > 1 && (ksteps / ns < 6 || tiles * ns > 300)) break;
-            const double t = few_rows_estimate(v, M, N, ksteps, block, cus, ns);
+            double t = few_rows_estimate(v, M, N, ksteps, block, cus, ns);
+            if (tiles * ns > (size_t)cus && (one_round || v.kgroups == 1)) t *= 1.12;
+            if (ksteps >= 32 && v.kgroups != 8) t *= 1.15;
             if (t > 0 && t < best_t) {
                 best = i;
                 best_ns = ns;
