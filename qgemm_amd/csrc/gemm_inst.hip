@@ -36,8 +36,7 @@ static hipError_t launch_variant(const GemmArgs &a, uint32_t grid, hipStream_t s
     hipError_t e = allow_lds(gemm_nt_kernel<C>, C::LDS_BYTES);
     if (e != hipSuccess) return e;
     const LaunchHead h(a, a.map.inv_group, a.map.inv_gm, a.map.inv_last, a.inv_nk);
-    hipLaunchKernelGGL(gemm_nt_kernel<C>, dim3(grid), dim3(C::THREADS), C::LDS_BYTES, s, QGEMM_HEAD_OF(h), a);
-    return hipGetLastError();
+    return launch_kernel(gemm_nt_kernel<C>, dim3(grid), dim3(C::THREADS), C::LDS_BYTES, s, QGEMM_HEAD_OF(h), a);
 }
 
 template <class C>
@@ -45,8 +44,7 @@ static hipError_t launch_skinny(const GemmArgs &a, uint32_t grid, hipStream_t s)
     hipError_t e = allow_lds(gemm_skinny_kernel<C>, C::LDS_BYTES);
     if (e != hipSuccess) return e;
     const LaunchHead h(a, C::TN == 4 ? a.map.inv_group : a.inv_tiles_m, a.map.inv_gm, a.map.inv_last, a.inv_nk);
-    hipLaunchKernelGGL(gemm_skinny_kernel<C>, dim3(grid), dim3(C::THREADS), C::LDS_BYTES, s, QGEMM_HEAD_OF(h), a);
-    return hipGetLastError();
+    return launch_kernel(gemm_skinny_kernel<C>, dim3(grid), dim3(C::THREADS), C::LDS_BYTES, s, QGEMM_HEAD_OF(h), a);
 }
 
 constexpr int kElemBytes = (INST_ARITH == AR_BF16 || INST_ARITH == AR_F16) ? 2 : 1;

@@ -984,11 +984,11 @@ int run_nt(const NtProblem &q, Plan &pl, void *split_ws, hipStream_t stream) {
 
     const uint32_t per_row = (uint32_t)((q.N + 3) / 4);
     const dim3 grid((unsigned)((q.M * per_row + 255) / 256));
-    hipLaunchKernelGGL(i32_acc ? splitk_reduce4_kernel<true> : splitk_reduce4_kernel<false>, grid, dim3(256), 0, stream, split_ws, q.C, q.as,
+    e = launch_kernel(i32_acc ? splitk_reduce4_kernel<true> : splitk_reduce4_kernel<false>, grid, dim3(256), 0, stream, split_ws, q.C, q.as,
                        q.bs, (uint32_t)q.M, (uint32_t)q.N, a.nsplit, (uint32_t)q.ldc, inverse_of(per_row), (uint32_t)q.out_dtype,
                        (uint32_t)(q.per_matrix != 0));
     g_ctx.last_config = std::string(v.name) + kmaj_suffix(q.kmaj) + "_splitk" + std::to_string(a.nsplit);
-    return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+    return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }
 
 // plan, get the split workspace (plus `extra` bytes behind it for transposed operands), run
@@ -1258,9 +1258,9 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
     if (!km && few_estimate(DT, a.out_dtype, BLOCK, a.a.rows, a.b.rows, a.K) < any_estimate(DT, a.out_dtype, BLOCK, a.a.rows, a.b.rows, a.K)) {
         constexpr int ARITH = DT == QGEMM_DT_I8 ? AR_I8 : DT == QGEMM_DT_F8E4M3 ? AR_F8W : DT == QGEMM_DT_BF16 ? AR_BF16 : AR_F16;
         const bool one = a.a.rows <= 16;
-        hipLaunchKernelGGL((one ? gemm_few_kernel<ARITH, BLOCK, 1> : gemm_few_kernel<ARITH, BLOCK, 2>),
-                           dim3((a.b.rows + 31) / 32, one ? 1 : (a.a.rows + 31) / 32), dim3(512), 0, stream, a);
-        return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+        const hipError_t e = launch_kernel(one ? gemm_few_kernel<ARITH, BLOCK, 1> : gemm_few_kernel<ARITH, BLOCK, 2>,
+                                           dim3((a.b.rows + 31) / 32, one ? 1 : (a.a.rows + 31) / 32), dim3(512), 0, stream, a);
+        return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
     }
     const int T = any_tile(DT, a.out_dtype, BLOCK, km, a.a.rows, a.b.rows);
     const uint64_t tiles_m = ((uint64_t)a.a.rows + T - 1) / T, tiles_n = ((uint64_t)a.b.rows + T - 1) / T, tiles = tiles_m * tiles_n;
@@ -1341,6 +1341,7 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         a.inv = inverse_of(a.per_row);
         a.rows_per_slice = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(a.rows, ((uint64_t)1 << 31) / a.per_row));
     };
+    hipError_t e;
     const bool ragged = a.cols % P::VEC != 0;           // rows end inside a piece
     if (mode == QGEMM_QUANT_PER_MATRIX) {
         if (a.ld == a.cols && a.ldq == a.cols && (uint64_t)a.rows * a.cols < ((uint64_t)1 << 31)) {      // no gaps: one row
@@ -1350,9 +1351,9 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         number((a.cols + P::VEC - 1) / P::VEC);
         const uint64_t pieces = (uint64_t)a.rows * a.per_row;
         if (pieces * 16 <= kQuantSmallBytes) {
-            hipLaunchKernelGGL((a.rows == 1 ? quant_small_matrix_kernel<IN_DT, OUT_DT, true> : quant_small_matrix_kernel<IN_DT, OUT_DT, false>), dim3((unsigned)std::max<uint64_t>(1, (pieces + 1023) / 1024)), dim3(1024), 0,
-                               stream, a);
-            return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+            e = launch_kernel(a.rows == 1 ? quant_small_matrix_kernel<IN_DT, OUT_DT, true> : quant_small_matrix_kernel<IN_DT, OUT_DT, false>,
+                              dim3((unsigned)std::max<uint64_t>(1, (pieces + 1023) / 1024)), dim3(1024), 0, stream, a);
+            return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
         }
         // two passes: partial maxima (one per workgroup) into the workspace, then scale and cast
         const uint32_t slices = std::max<uint32_t>(1, (a.rows + a.rows_per_slice - 1) / a.rows_per_slice);
@@ -1363,24 +1364,25 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         int st = ensure_workspace_locked((size_t)a.npartial * sizeof(uint32_t), stream, &ws);
         if (st != QGEMM_OK) return st;
         a.partial = (uint32_t *)ws;
-        hipLaunchKernelGGL((a.rows == 1 ? quant_amax_kernel<IN_DT, true> : quant_amax_kernel<IN_DT, false>), dim3(nblk, slices), dim3(256), 0, stream, a);
+        e = launch_kernel(a.rows == 1 ? quant_amax_kernel<IN_DT, true> : quant_amax_kernel<IN_DT, false>, dim3(nblk, slices), dim3(256), 0, stream, a);
+        if (e != hipSuccess) return QGEMM_ERR_LAUNCH;
         const uint32_t nq = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(2048, turns));
-        hipLaunchKernelGGL((a.rows == 1 ? quant_matrix_kernel<IN_DT, OUT_DT, true> : quant_matrix_kernel<IN_DT, OUT_DT, false>), dim3(nq, slices), dim3(256), 0, stream, a);
+        e = launch_kernel(a.rows == 1 ? quant_matrix_kernel<IN_DT, OUT_DT, true> : quant_matrix_kernel<IN_DT, OUT_DT, false>, dim3(nq, slices), dim3(256), 0, stream, a);
     } else if (mode == QGEMM_QUANT_BLOCK_1x128) {
         number((a.cols + 127) / 128);
         const uint64_t blocks = (uint64_t)a.rows_per_slice * a.per_row;
         const uint32_t slices = (a.rows + a.rows_per_slice - 1) / a.rows_per_slice, per_group = 256 / P::LANES;
         const dim3 grid((unsigned)((blocks + per_group - 1) / per_group), slices);
         if (blocks >= (uint64_t)kQuantManyGroups * per_group)
-            hipLaunchKernelGGL((ragged ? quant_row_block_kernel<IN_DT, OUT_DT, true> : quant_row_block_kernel<IN_DT, OUT_DT, false>), grid, dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
+            e = launch_kernel(ragged ? quant_row_block_kernel<IN_DT, OUT_DT, true> : quant_row_block_kernel<IN_DT, OUT_DT, false>, grid, dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
         else
-            hipLaunchKernelGGL((ragged ? quant_few_blocks_kernel<IN_DT, OUT_DT, true> : quant_few_blocks_kernel<IN_DT, OUT_DT, false>), grid, dim3(256), 0, stream, a);
+            e = launch_kernel(ragged ? quant_few_blocks_kernel<IN_DT, OUT_DT, true> : quant_few_blocks_kernel<IN_DT, OUT_DT, false>, grid, dim3(256), 0, stream, a);
     } else {
         const uint64_t nblocks = (uint64_t)((a.rows + 127) / 128) * ((a.cols + 127) / 128);
         if (nblocks >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
-        hipLaunchKernelGGL((ragged ? quant_square_block_kernel<IN_DT, OUT_DT, true> : quant_square_block_kernel<IN_DT, OUT_DT, false>), dim3((unsigned)nblocks), dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
+        e = launch_kernel(ragged ? quant_square_block_kernel<IN_DT, OUT_DT, true> : quant_square_block_kernel<IN_DT, OUT_DT, false>, dim3((unsigned)nblocks), dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
     }
-    return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+    return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }
 
 }  // namespace
