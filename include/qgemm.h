@@ -123,8 +123,8 @@ int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int la
                              size_t K, int split_k, void *stream);
 
 /* Library workspace (no reference counterpart: the reference's entries take none).  Calls that split K, that
- * take operands or scales in an arrangement the kernels do not read directly, and the per-matrix quantiser keep
- * their intermediate data in one device block owned by the library and grown on demand.  A block that is
+ * take operands or scales in an arrangement the kernels do not read directly, and the per-matrix quantiser (of
+ * more than 256 KiB) keep their intermediate data in one device block owned by the library and grown on demand.  A block that is
  * outgrown is replaced but stays allocated until qgemm_shutdown, so launches already enqueued and graphs
  * already captured remain valid.  Calls on different streams share the block: each such call waits (on the
  * device, through an event) for the previous user on another stream.  While a stream is being captured into a
@@ -178,7 +178,8 @@ int qgemm_tile_map(uint32_t wg, uint32_t tiles_m, uint32_t tiles_n, uint32_t gro
  *   "stagger_groups", "as_groups", "row_split" (0: one launch always; 1: the rows "a+b" or columns "a|b" of a partly
  *   empty last round of 256 x 256 tiles as a second launch where the estimate gains; 2 / 3: rows / columns wherever
  *   possible), "small_tiles" (0: 17 .. 256 rows against few columns keep a tall tile with a K split instead of several
- *   row tiles of the skinny-M kernel), "c_plain" (0 / 1: non-temporal / ordinary stores for C; -1: the library's
+ *   row tiles of the skinny-M kernel, and up to 400 rows follow the general rules instead of the estimate of every row that
+ *   serves them below 32 K steps and, block scales, up to 128 rows), "c_plain" (0 / 1: non-temporal / ordinary stores for C; -1: the library's
  *   choice), "b_stream" (0 / 1: copies of B without / with the streaming hint; -1: the library's choice); "force_config" accepts only -1 (back to the heuristic).
  *   "k_rot": with at most 256 rows the workgroups of column tile i start their K loops 3 i steps in and wrap round
  *   (memory channels), so the order of an fp32 sum depends on the column tile: results are the same from run to

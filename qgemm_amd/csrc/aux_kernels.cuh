@@ -61,7 +61,8 @@ __device__ inline void store_part(void *p, v4i v, uint32_t bytes) {
 // into the LDS tile [n][m]; the tile leaves as 16-byte pieces of output rows, 128 bytes per row.
 // ---------------------------------------------------------------------------
 // One 128 x 128 tile of the byte transpose (tile_m, tile_n in tiles).  ALIGNED: M a multiple of 16, N of 4, aligned rows,
-// Mout == M.  Otherwise any M, N, ld, pitch and pointers: pieces that stick out go byte by byte, and the columns
+// Mout == M.  Otherwise any M, N, ld, pitch and pointers: at a row's end the last whole piece is loaded and moved down, what
+// sticks out of the output is stored in parts, and the columns
 // M .. Mout - 1 of the output are filled with zeros.
 template <bool ALIGNED>
 __device__ inline void transpose_bytes_tile(const uint8_t *__restrict__ in, size_t ld, uint8_t *__restrict__ out, size_t pitch,
@@ -166,8 +167,8 @@ __global__ void __launch_bounds__(256) transpose_bytes2_kernel(const Transpose2A
 // ---------------------------------------------------------------------------
 // ALIGNED: M and N multiples of 8, 16-byte aligned rows, Mout == M.  Otherwise any M, N, ld, pitch and element-aligned
 // pointers (1999 x 3001, us: through LDS one element per lane 11.4; so, with a branch around every
-// element of a row end 11.3, without 9.7): pieces that stick out go element by
-// element, the columns M .. Mout - 1 of the output are filled with zeros.
+// element of a row end 11.3, without 9.7): at a row's end the last whole piece is loaded and moved
+// down, what sticks out of the output is stored in parts, the columns M .. Mout - 1 of the output are filled with zeros.
 template <bool ALIGNED>
 __device__ inline void transpose_u16_tile(const uint16_t *__restrict__ in, size_t ld, uint16_t *__restrict__ out, size_t pitch,
                                           uint32_t M, uint32_t Mout, uint32_t N, uint32_t tile_m, uint32_t tile_n) {
@@ -245,7 +246,7 @@ __global__ void __launch_bounds__(256) transpose_u16_kernel(const uint16_t *__re
 // 16-byte aligned, B stored K x N with such rows): one launch brings one or both of them to rows of `pitch` bytes, K
 // contiguous, zeros behind the last element up to the pitch (a multiple of 128), so that the whole of K is whole K steps.
 // Bound by memory: every element is read and written once.  Loads are 16 bytes a lane at whatever address the row has
-// (the vector memory path takes any byte address; only the pieces that reach past a row's end go element by element).
+// (the vector memory path takes any byte address).
 // ---------------------------------------------------------------------------
 struct PackOperand {
     const char *src;

@@ -510,8 +510,8 @@ int choose_by_rules(const Variant *tab, int count, size_t M, size_t N, size_t ks
 // 8192 elements of K; fp8, int8 and bf16, and fp8 with block scales), every row forced, as the geometric mean of weights streamed
 // out of memory and weights resident.  The rules above were made on a few dozen shapes around 32 K steps, and with kernels that
 // started later; measured against the fastest row they are 15 % behind on average, at worst twice its time: 48 x 1200 x 1024 int8
-// 6.34 (two K slices) -> 4.05 us (16 x 16 tiles), 24 x 4432 x 1152 with block scales 7.52 -> 5.00, 136 x 7072 x 7088 38.4 -> 29.5,
-// 108 x 2048 x 3968 8.1 -> 6.4.  What the estimate takes is 2.5 % behind (on the third of the shapes that it was not fitted on 2.9).
+// 6.34 (two K slices) -> 4.05 us (16 x 16 tiles), 24 x 4432 x 1152 with block scales 7.52 -> 5.00, 110 x 1024 x 1280
+// 7.90 -> 3.97, 124 x 3072 x 1792 8.97 -> 5.87.  What the estimate takes is 2.5 % behind (on the third of the shapes that it was not fitted on 2.9).
 // A row costs `fixed`, and every round of `slots` workgroups per CU `round` plus its K steps at `alone` (few workgroups) .. `full`
 // (all CUs at work) us each, or, where that is longer, `late` and B at `stream` us/MB.  (The eight waves of the skinny-M kernel
 // take the steps in turn: halfway between the steps and the next multiple of eight.)
@@ -1126,11 +1126,13 @@ double few_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N,
 }
 
 // Is a product on the any-shape path faster packed?  Estimates of both, in microseconds, fitted on 240 ragged shapes (1 .. 4096
-// rows x 1024 .. 7168 columns x K = 777 .. 7161; fp8 and int8 with one scale and with block scales, bf16), eager calls: the way
-// chosen is 0.7 % behind the faster one on average, 33 % at worst (int8 block scales 200 x 5000 x 3004 20.4 / 27.1).  Two
-// thresholds on the sizes, K and M N, were 21 % behind on average.  Any-shape kernel / packed: int8 1 x 2048 x 1032 8.2 / 13.3,
-// 512 x 3000 x 1500 11.1 / 21.2, 1024 x 4096 x 2001 28.4 / 26.9, 4096 x 4096 x 2001 68.4 / 45.5, fp8 64 x 7168 x 2056 17.5 / 22.1,
-// 512 x 2048 x 1032 11.2 / 17.8, 4096 x 4608 x 7161 356 / 234, bf16 512 x 2048 x 1036 11.4 / 17.7, 2048 x 3000 x 1500 40.4 / 33.6.
+// rows x 1024 .. 7168 columns x K = 777 .. 7161; fp8 and int8 with one scale and with block scales, bf16), eager calls, before
+// gemm_few_kernel and faster row ends in pack_kernel; on 150 other shapes with both the way chosen is 1.1 % behind the faster one
+// on average, 59 % at worst (bf16 657 x 4159 x 4585 79.2 / 49.7), and a smaller constant part (7 .. 10.5 for 12) is level with it
+// (0.9 - 1.3 %).  Two thresholds on the sizes, K and M N, were 21 % behind on average.  Unpacked / packed: int8 1 x 2048 x 1032
+// 7.9 / 11.5, 512 x 3000 x 1500 11.3 / 18.5, 1024 x 4096 x 2001 26.5 / 23.7, 4096 x 4096 x 2001 74.9 / 42.0, fp8 64 x 7168 x 2056
+// 10.3 / 19.1, 512 x 2048 x 1032 11.2 / 14.7, 4096 x 4608 x 7161 357 / 229, bf16 512 x 2048 x 1036 11.5 / 15.8, 2048 x 3000 x 1500
+// 39.7 / 31.6.
 // Operands that are transposed on the way (km) make the any-shape kernel twice as slow: thresholds do there (bf16 with B stored
 // K x N 1024 x 2049 x 261 15.5 / 15.7, x 401 18.4 / 16.7).
 bool pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
@@ -1312,8 +1314,8 @@ int launch_transpose(int elem_bytes, const void *in, void *out, size_t M, size_t
     if (M >= ((size_t)1 << 31) || N >= ((size_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
     dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
     if (grid.y > 65535u * 1024u) return QGEMM_ERR_TOO_LARGE;
-    // Sizes or addresses that rule out aligned 16-byte pieces take the same tiles with pieces at any address, the ones on
-    // the edges element by element.
+    // Sizes or addresses that rule out aligned 16-byte pieces take the same tiles with pieces at any address, stored in
+    // parts on the edges.
     if (elem_bytes == 1) {
         const bool aligned = M % 16 == 0 && N % 4 == 0 && (uintptr_t)in % 4 == 0 && (uintptr_t)out % 16 == 0;
         const dim3 g((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128));

@@ -8,14 +8,14 @@
 // What bounds them: memory, once the instructions per element are few.  16-bit input leaves 1.2 ns per element and CU at
 // the rate a copy reaches, a dozen vector instructions; element by element, with a test for NaN, infinity and zero and a
 // clamp around every quotient, it took 25 and the 1 x 128 quantiser of bf16 ran at 2.9 TB/s.  So:
-//   * a lane works on pieces of 16 bytes (8 16-bit or 4 fp32 elements), at any address, the row ends element by element;
+//   * a lane works on pieces of 16 bytes (8 16-bit or 4 fp32 elements), at any address, a row's end out of its last whole piece;
 //   * maxima are integer maxima of the bits without the sign (two at a time for 16-bit input): the order of the numbers,
 //     with infinities and NaNs on top, so that one look at a block's maximum tells whether the plain form below will do;
 //   * plain form (a finite maximum: no element is NaN or infinite, no quotient exceeds the type's largest value): the
 //     quotient of |x| without special cases, the sign moved over afterwards; anything else takes the careful form.
 // Before and now, us (to fp8 unless said): 1 x 128 6144 x 7168 bf16 45.7 -> 25.7 (5.1 TB/s, what a copy reaches), 500 x 7200
-// 7.3 -> 4.5; 128 x 128 7168 x 6144 fp32 43.4 -> 39.6 (5.6 TB/s); per matrix 1531 x 3004 bf16 to int8 4.9 + 8.5 -> 4.2 + 6.6.
-// A decoder's 16 x 2048 stays at 2.8: one trip to memory and back.
+// 7.3 -> 4.5; 128 x 128 7168 x 6144 fp32 43.4 -> 39.6 (5.6 TB/s); per matrix 1531 x 3004 bf16 to int8 4.9 + 8.5 -> 4.2 + 4.6
+// (a trace's times of the two passes).  A decoder's one row of 2048 1.98 -> 1.85: one trip to memory and back.
 #pragma once
 #include "common.h"
 

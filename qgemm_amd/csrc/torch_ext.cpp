@@ -102,7 +102,7 @@ void bf16_mm(torch::Tensor a, torch::Tensor b, torch::Tensor c) {
 
 // ---- what qgemm_amd/ops.py calls: its functions with the reading of the tensors, the stream lookup and the call into the
 // library done here (1 x 2048 x 1024, quantise and multiply: 11.6 + 8.4 us of host time through Python and ctypes, 3 of each
-// in torch.cuda.current_stream(), for two kernels of 1.7 and 4.1 us; 4.3 + 3.6 here, most of it the launches).  They answer a status of the library, or kNotPlain, having
+// in torch.cuda.current_stream(), for two kernels of 1.9 and 3.3 us; 4.1 + 3.8 here, most of it the launches).  They answer a status of the library, or kNotPlain, having
 // done nothing, for anything that is not the plain case; ops.py then takes its own way, which raises what there is to raise.
 constexpr int kNotPlain = -1;
 
