@@ -304,7 +304,7 @@ __device__ inline void mma128_inplace(v4i x0, v4i x1, v4i y0, v4i y1, typename A
 // Besides pointers, strides and sizes:
 constexpr uint32_t kHeadSplit = 1, kHeadStream = 2, kHeadStagger = 4;      // K split across workgroups; GemmArgs::b_stream; GemmArgs::stagger
 constexpr int kHeadRotShift = 3, kHeadGroupShift = 16;                     // GemmArgs::k_rot; TileMap::group_m
-constexpr uint32_t kHeadRotMax = 0x1FFF, kHeadGroupMax = 0xFFFF;
+constexpr uint32_t kHeadRotMax = 0x1FFF, kHeadGroupMax = 0xFFFF;         // (what fits: plan_nt keeps to it, everything else derives from the same numbers)
 // (Seven 64-bit numbers: the runtime looks up what every pointer among the arguments points into and sets them one by one; as two
 // pointers and ten 32-bit numbers they cost a launch 0.3 us of host time more.)
 struct LaunchHead {
@@ -313,8 +313,7 @@ struct LaunchHead {
         : A((uint64_t)(uintptr_t)a.A), B((uint64_t)(uintptr_t)a.B), ld(two(a.lda, a.ldb)), mn(two(a.M, a.N)),
           kf(two(a.k_tail ? (a.ksteps - 1) * 128 + a.k_tail : a.ksteps * 128,
                  (a.nsplit > 1 ? kHeadSplit : 0) | (a.b_stream ? kHeadStream : 0) | (a.stagger ? kHeadStagger : 0) |
-                     (a.k_rot < kHeadRotMax ? a.k_rot : kHeadRotMax) << kHeadRotShift |
-                     (a.map.group_m < kHeadGroupMax ? a.map.group_m : kHeadGroupMax) << kHeadGroupShift)),
+                     a.k_rot << kHeadRotShift | a.map.group_m << kHeadGroupShift)),
           inv01(two(inv0, inv1)), inv23(two(inv2, inv3)) {}
     static uint64_t two(uint32_t lo, uint32_t hi) { return lo | (uint64_t)hi << 32; }
 };

@@ -845,7 +845,7 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     a.lda = (uint32_t)q.lda_bytes;
     a.ldb = (uint32_t)q.ldb_bytes;
     const uint32_t tiles_m = (uint32_t)((q.M + v.bm - 1) / v.bm), tiles_n = (uint32_t)((q.N + v.bn - 1) / v.bn);
-    a.map = make_tile_map(tiles_m, tiles_n, g_ctx.force_group_m > 0 ? (uint32_t)g_ctx.force_group_m : 8);
+    a.map = make_tile_map(tiles_m, tiles_n, g_ctx.force_group_m > 0 ? (uint32_t)std::min<long>(g_ctx.force_group_m, kHeadGroupMax) : 8);
     a.inv_tiles_m = inverse_of(tiles_m);
     // Few rows (every workgroup streams a strip of B of its own out of memory, all of them at the same k): the workgroups
     // of column tile i (which share that strip of B and stay in step) start their K loops k_rot * i steps in and wrap
@@ -885,6 +885,9 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     a.inv_nsplit = inverse_of(nsplit);
     a.inv_nk = inverse_of(a.ksteps_per_split);
     a.inv_nk_last = inverse_of(a.ksteps - (nsplit - 1) * a.ksteps_per_split);
+    // (a start further in than the launch head holds: the same start in a whole slice, and still a multiple of four where it and the
+    // slices are, which run_nt asks about)
+    if (a.k_rot > kHeadRotMax) a.k_rot = std::min(a.k_rot % a.ksteps_per_split, kHeadRotMax & ~3u);
     pl.split_bytes = nsplit > 1 ? q.M * q.N * 4 * (size_t)nsplit : 0;
     return QGEMM_OK;
 }
