@@ -63,7 +63,9 @@ struct Context {
 #endif
     long as_groups = 1;         // 0: no copies of four K blocks of a_scale: one block per copy on the rows with two K groups (see run_nt), a
                                 // transposed copy of a_scale for the row with copying waves (see settle_scale_layout)
-    long small_tiles = 1;       // 0: 17 .. 256 rows never go to several row tiles of the skinny-M kernel in place of a K split
+    long small_tiles = 1;       // 0: 17 .. 256 rows never go to several row tiles of the skinny-M kernel in place of a K split (and up to 400
+                                // rows follow the rules, as the estimate likes such tiles)
+    long row_estimate = 1;      // 0: up to 400 rows follow the rules (choose_by_rules) instead of the estimate of every row (choose_variant)
     long k_rot = -1;            // -1: rotated K start for at most 256 rows (see plan_nt), 0: never, n: steps per column tile
     long stagger = -1;          // -1: staggered start where it pays (4-byte C, three or more rounds), else microseconds per group
     long stagger_groups = 8;    // groups the workgroups of the first round start in
@@ -571,7 +573,7 @@ double few_rows_estimate(const Variant &v, size_t M, size_t N, size_t ksteps, bo
 int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
                    bool may_split, bool whole, uint32_t *nsplit_out) {
     const int vi = choose_by_rules(tab, count, M, N, ksteps, block, kmaj, cus, may_split, nsplit_out);
-    if (vi < 0 || kmaj || !whole || M > 400 || tab[vi].arith == AR_F8W || !g_ctx.small_tiles || !(ksteps < 32 || (block && M <= 128))) return vi;
+    if (vi < 0 || kmaj || !whole || M > 400 || tab[vi].arith == AR_F8W || !g_ctx.row_estimate || !g_ctx.small_tiles || !(ksteps < 32 || (block && M <= 128))) return vi;
     uint32_t asked = std::max<uint32_t>(1, *nsplit_out);
     if (*nsplit_out == 0 && may_split)
         asked = std::max<uint32_t>(1, slices_for_few_tiles(((M + tab[vi].bm - 1) / tab[vi].bm) * ((N + tab[vi].bn - 1) / tab[vi].bn), (uint32_t)ksteps, cus));
@@ -1464,6 +1466,7 @@ QGEMM_EXPORT int qgemm_set_option(const char *key, long value) {
     else if (!std::strcmp(key, "k_rot")) g_ctx.k_rot = value;
     else if (!std::strcmp(key, "as_groups")) g_ctx.as_groups = value;
     else if (!std::strcmp(key, "small_tiles")) g_ctx.small_tiles = value;
+    else if (!std::strcmp(key, "row_estimate")) g_ctx.row_estimate = value;
 #if QGEMM_DEBUG_BUILD
     else if (!std::strcmp(key, "dbg_ptr")) g_ctx.dbg_ptr = value;
 #endif

@@ -1,0 +1,50 @@
+"""The choice of a row for up to 400 rows (the estimate of every row against the general rules), through qgemm_plan: no device needed."""
+import re
+
+import pytest
+
+import qgemm_amd as Q
+
+FAMILIES = [(Q.DT_BF16, 0), (Q.DT_F16, 0), (Q.DT_F8E4M3, Q.SCALE_PER_MATRIX), (Q.DT_I8, Q.SCALE_PER_MATRIX),
+            (Q.DT_F8E4M3, Q.SCALE_BLOCK128), (Q.DT_I8, Q.SCALE_BLOCK128)]
+SHAPES = [(M, N, K) for M in (1, 2, 8, 16, 17, 32, 40, 56, 64, 72, 109, 128, 130, 200, 300, 400)
+          for N in (256, 816, 1024, 2048, 3072, 4432, 8336, 12720) for K in (512, 576, 1024, 1040, 1648, 1824, 2048, 3072, 4096, 7536)]
+
+
+@pytest.fixture(autouse=True)
+def _reset_options():
+    yield
+    Q.set_option("row_estimate", 1)
+    Q.set_option("small_tiles", 1)
+
+
+def _plans(family, shapes, **options):
+    for key, value in options.items():
+        Q.set_option(key, value)
+    try:
+        return [Q.plan(*family, 0, *shape) for shape in shapes]
+    finally:
+        Q.set_option("row_estimate", 1)
+        Q.set_option("small_tiles", 1)
+
+
+def _slices(name):
+    m = re.search(r"_splitk(\d+)", name)
+    return int(m.group(1)) if m else 1
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+def test_never_more_k_slices_than_the_rules_ask_for(family):
+    """K slices are what a call needs workspace for: none may need more than by the rules."""
+    rules, chosen = _plans(family, SHAPES, row_estimate=0), _plans(family, SHAPES)
+    assert sum(a != b for a, b in zip(rules, chosen)) > 100           # (the option does something)
+    for shape, a, b in zip(SHAPES, rules, chosen):
+        assert _slices(b) <= _slices(a), (family, shape, a, b)
+
+
+def test_options_of_the_estimate_and_of_small_tiles():
+    """row_estimate = 0 is the rules with their small tiles, small_tiles = 0 neither."""
+    family, estimated, small = (Q.DT_F8E4M3, Q.SCALE_PER_MATRIX), (110, 1024, 1280), (128, 1024, 4096)
+    assert _plans(family, [estimated, small]) == ["skinny_32x16_k8", "skinny_32x32_k8"]
+    assert _plans(family, [estimated, small], row_estimate=0) == ["128x32_w4x1_dma", "skinny_32x32_k8"]
+    assert _plans(family, [estimated, small], small_tiles=0) == ["128x32_w4x1_dma", "skinny_128x32_k8_splitk4"]
