@@ -207,6 +207,9 @@ int qgemm_last_config(char *buf, size_t buflen);
  *   scale_mode 0 = plain GEMM (qgemm_gemm), else as for qgemm_scaled_gemm
  *   k_major    bit 0: A is stored K x M, bit 1: B is stored K x N (2 = QGEMM_B_KN, 3 = QGEMM_LAYOUT_REFERENCE) */
 int qgemm_plan(int in_dtype, int scale_mode, int k_major, size_t M, size_t N, size_t K, char *buf, size_t buflen);
+/* The same for an output type (qgemm_plan answers for a 16-bit one): up to 400 rows fp32 output of 16-bit operands and of int8 with
+ * block scales keeps to rows that sum as exactly as those of the general rules. */
+int qgemm_plan_out(int in_dtype, int out_dtype, int scale_mode, int k_major, size_t M, size_t N, size_t K, char *buf, size_t buflen);
 
 /* Self-check of the MFMA / LDS-DMA lane layouts the kernels assume, run on the
  * current device.  Writes a short report into buf; returns QGEMM_OK when every

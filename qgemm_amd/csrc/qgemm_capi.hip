@@ -565,13 +565,31 @@ double few_rows_estimate(const Variant &v, size_t M, size_t N, size_t ksteps, bo
     return 0;
 }
 
+// How many partial sums an element of C is made of: K groups of the row times K slices.
+struct PartialSums {
+    uint32_t groups, slices;
+};
+// Are sums in parts `b` no further from 64 bits than in parts `a`, as far as the output shows it?  Only fp32 does, and not where the
+// sums are exact (int8 with one scale) or the matrix instruction's own rounding covers them (fp8: 1.5e-5 of the result in any order).
+// 16-bit operands: the more parts the shorter the chains.  Relative error, 1e-8, bf16 at 8 / 16 / 31 K steps: one chain 12.3 / 18.2 /
+// 26.5, two groups 8.9 / 12.8 / 18.2, two groups in four slices - / 7.7 / 9.8, eight groups 7.0 / 8.2 / 10.1, in two slices 6.5 / 7.6 / 8.6.
+// int8 blocks: no such order (eight groups add few blocks each and round once more where they meet; one chain 5.9 / 7.8 / 10.4, two
+// groups 5.5 / 6.6 / 8.1, eight 6.6 / 6.9 / 7.4), so only the same parts.
+bool sums_as_exact(int arith, bool block, int out_dtype, PartialSums a, PartialSums b) {
+    if (out_dtype != QGEMM_DT_F32 || arith == AR_F8 || (arith == AR_I8 && !block)) return true;
+    if (a.groups == b.groups && a.slices == b.slices) return true;
+    return !block && b.groups * b.slices > a.groups * a.slices;
+}
+
 // The row of the rules, or where the estimate puts another one 3 % ahead of it that one, with no more K slices than the rules asked
 // for (so that no call needs a workspace that did not need one).  Below 32 K steps, and with block scales up to 128 rows; from 32
 // K steps on the rules above are 7 - 8 % behind, and their choice, which was measured with streamed weights, stays.  With 8 K steps
 // and one scale the waves of the skinny-M kernel have a single step each and the estimate is less sure of them: 13 %.
 // (whole: not the rows or columns beside a first launch, whose estimate the split of the two was made with)
+// Where an fp32 output would show it, only rows whose sums are as exact as those of the rules' row (sums_as_exact): bf16 8 x 8788 x 544
+// is 7.4e-8 of the result off on eight groups, which the rules ask for, 13.0e-8 in the one chain that the estimate likes.
 int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
-                   bool may_split, bool whole, uint32_t *nsplit_out) {
+                   bool may_split, bool whole, int out_dtype, uint32_t *nsplit_out) {
     const int vi = choose_by_rules(tab, count, M, N, ksteps, block, kmaj, cus, may_split, nsplit_out);
     if (vi < 0 || kmaj || !whole || M > 400 || tab[vi].arith == AR_F8W || !g_ctx.row_estimate || !g_ctx.small_tiles || !(ksteps < 32 || (block && M <= 128))) return vi;
     uint32_t asked = std::max<uint32_t>(1, *nsplit_out);
@@ -593,6 +611,7 @@ int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t kst
         if (tiles > 1400) continue;
         for (uint32_t ns = 1; ns <= 8 && ns <= asked; ns *= 2) {
             if (ns > 1 && (ksteps / ns < 6 || tiles * ns > 300)) break;
+            if (!sums_as_exact(v.arith, block, out_dtype, {(uint32_t)tab[vi].kgroups, asked}, {(uint32_t)v.kgroups, ns})) continue;
             double t = few_rows_estimate(v, M, N, ksteps, block, cus, ns);
             if (tiles * ns > (size_t)cus && (one_round || v.kgroups == 1)) t *= 1.12;
             if (ksteps >= 32 && v.kgroups != 8) t *= 1.15;
@@ -784,7 +803,8 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     const Variant *tab = table_for(q.arith, q.block, q.kmaj, &count);
     if (!tab) return QGEMM_ERR_UNSUPPORTED;
     uint32_t model_split = 0;
-    int vi = choose_variant(tab, count, q.M, q.N, ksteps_of(q), q.block, q.kmaj, g_ctx.num_cus, q.split_k == 0, may_split_rows, &model_split);
+    int vi = choose_variant(tab, count, q.M, q.N, ksteps_of(q), q.block, q.kmaj, g_ctx.num_cus, q.split_k == 0, may_split_rows, q.out_dtype,
+                            &model_split);
     if (may_split_rows && vi >= 0 && !forced() && g_ctx.force_split <= 0 && q.split_k == 0 && model_split <= 1 &&
         q.M > 128 && q.kmaj == 0) {
         uint32_t ns = 0;
@@ -1522,12 +1542,18 @@ QGEMM_EXPORT int qgemm_last_config(char *buf, size_t buflen) {
 
 QGEMM_EXPORT int qgemm_plan(int in_dtype, int scale_mode, int k_major, size_t M, size_t N, size_t K, char *buf,
                             size_t buflen) {
+    return qgemm_plan_out(in_dtype, QGEMM_DT_BF16, scale_mode, k_major, M, N, K, buf, buflen);
+}
+
+QGEMM_EXPORT int qgemm_plan_out(int in_dtype, int out_dtype, int scale_mode, int k_major, size_t M, size_t N, size_t K, char *buf,
+                                size_t buflen) {
     if (!buf || buflen == 0 || M == 0 || N == 0 || K == 0 || k_major < 0 || k_major > 3) return QGEMM_ERR_INVALID_ARG;
     const int arith = arith_of(in_dtype);
     if (arith < 0) return QGEMM_ERR_UNSUPPORTED;
     if (scale_mode != 0 && scale_mode != QGEMM_SCALE_PER_MATRIX && scale_mode != QGEMM_SCALE_BLOCK128)
         return QGEMM_ERR_INVALID_ARG;
     if (scale_mode == QGEMM_SCALE_BLOCK128 && arith != AR_F8 && arith != AR_I8) return QGEMM_ERR_UNSUPPORTED;
+    if (!out_dtype_ok(in_dtype, out_dtype) || (scale_mode == QGEMM_SCALE_BLOCK128 && out_dtype == QGEMM_DT_I32)) return QGEMM_ERR_UNSUPPORTED;
     std::lock_guard<std::mutex> lock(g_ctx.mu);          // no device call below: 256 CUs are assumed before qgemm_init
     const size_t eb = (arith == AR_BF16 || arith == AR_F16) ? 2 : 1;
     NtProblem q;
@@ -1539,6 +1565,7 @@ QGEMM_EXPORT int qgemm_plan(int in_dtype, int scale_mode, int k_major, size_t M,
     q.Kbytes = K * eb;
     q.lda_bytes = q.ldb_bytes = K * eb;
     q.ldc = N;
+    q.out_dtype = out_dtype;
     std::string name;
     if (k_major) {
         const size_t lda = (k_major & 1) ? M * eb : K * eb, ldb = (k_major & 2) ? N * eb : K * eb;

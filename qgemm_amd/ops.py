@@ -92,10 +92,10 @@ def variant_names(in_dtype, scale_mode=0, k_major=0):
     return out
 
 
-def plan(in_dtype, scale_mode, k_major, M, N, K):
+def plan(in_dtype, scale_mode, k_major, M, N, K, out_dtype=DT_BF16):
     """Name of the kernel configuration the library would choose (no launch, no device needed)."""
     buf = C.create_string_buffer(128)
-    check(load_library().qgemm_plan(in_dtype, scale_mode, k_major, M, N, K, buf, 128))
+    check(load_library().qgemm_plan_out(in_dtype, out_dtype, scale_mode, k_major, M, N, K, buf, 128))
     return buf.value.decode()
 
 

@@ -48,3 +48,31 @@ def test_options_of_the_estimate_and_of_small_tiles():
     assert _plans(family, [estimated, small]) == ["skinny_32x16_k8", "skinny_32x32_k8"]
     assert _plans(family, [estimated, small], row_estimate=0) == ["128x32_w4x1_dma", "skinny_32x32_k8"]
     assert _plans(family, [estimated, small], small_tiles=0) == ["128x32_w4x1_dma", "skinny_128x32_k8_splitk4"]
+
+
+def _parts(name):
+    """(K groups of the row, K slices)"""
+    return 8 if name.startswith("skinny") else 2 if "_k2" in name else 1, _slices(name)
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+def test_fp32_sums_in_no_fewer_parts_than_by_the_rules(family):
+    """An fp32 output shows how often a sum was rounded.  16-bit operands: as many partial sums as by the rules (the same, or more);
+    int8 blocks, where more are not always closer to 64 bits: the same; fp8 and exact int32 sums: whatever is fastest."""
+    def plans(out):
+        return [Q.plan(*family, 0, *shape, out) for shape in SHAPES]
+
+    free = plans(Q.DT_BF16)
+    fp32 = plans(Q.DT_F32)
+    Q.set_option("row_estimate", 0)
+    rules = plans(Q.DT_F32)
+    assert rules == plans(Q.DT_BF16)
+    if family[0] == Q.DT_F8E4M3 or family == (Q.DT_I8, Q.SCALE_PER_MATRIX):
+        assert fp32 == free
+        return
+    kept = 0
+    for shape, a, b, f in zip(SHAPES, rules, fp32, free):
+        (ga, sa), (gb, sb) = _parts(a), _parts(b)
+        assert (ga, sa) == (gb, sb) or (family[1] == 0 and gb * sb > ga * sa), (family, shape, a, b)
+        kept += b != f
+    assert kept > 10 and fp32 != rules
