@@ -575,8 +575,11 @@ struct PartialSums {
 // 26.5, two groups 8.9 / 12.8 / 18.2, two groups in four slices - / 7.7 / 9.8, eight groups 7.0 / 8.2 / 10.1, in two slices 6.5 / 7.6 / 8.6.
 // int8 blocks: no such order (eight groups add few blocks each and round once more where they meet; one chain 5.9 / 7.8 / 10.4, two
 // groups 5.5 / 6.6 / 8.1, eight 6.6 / 6.9 / 7.4), so only the same parts.
+bool output_shows_sums(int arith, bool block, int out_dtype) {
+    return out_dtype == QGEMM_DT_F32 && arith != AR_F8 && (arith != AR_I8 || block);
+}
 bool sums_as_exact(int arith, bool block, int out_dtype, PartialSums a, PartialSums b) {
-    if (out_dtype != QGEMM_DT_F32 || arith == AR_F8 || (arith == AR_I8 && !block)) return true;
+    if (!output_shows_sums(arith, block, out_dtype)) return true;
     if (a.groups == b.groups && a.slices == b.slices) return true;
     return !block && b.groups * b.slices > a.groups * a.slices;
 }
@@ -1160,22 +1163,24 @@ double few_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N,
 // 39.7 / 31.6.
 // Operands that are transposed on the way (km) make the any-shape kernel twice as slow: thresholds do there (bf16 with B stored
 // K x N 1024 x 2049 x 261 15.5 / 15.7, x 401 18.4 / 16.7).
-bool pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
+enum class Packing { NO, YES, UNLESS_FEW_ROWS };        // UNLESS_FEW_ROWS: gemm_few_kernel is faster still
+Packing pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
     const size_t kbytes = K * dtype_bytes(in_dtype), cus = g_ctx.num_cus;
-    if (km) return kbytes > 512 || (double)q.M * q.N >= 4e6;
-    const double t_any = std::min(any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K), few_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K));
+    if (km) return kbytes > 512 || (double)q.M * q.N >= 4e6 ? Packing::YES : Packing::NO;
     // packed: two launches and the packing, then the tiles' estimate or the skinny-M kernel's (see choose_variant)
     int count = 0;
     const Variant *tab = table_for(q.arith, q.block, 0, &count);
     uint32_t nsplit = 0;
     double t_rows = 0;
     const size_t steps = (kbytes + 127) / 128;
-    if (!tab || choose_by_cost(tab, count, q.M, q.N, steps, q.block, (int)cus, true, &nsplit, &t_rows) < 0) return false;
+    if (!tab || choose_by_cost(tab, count, q.M, q.N, steps, q.block, (int)cus, true, &nsplit, &t_rows) < 0) return Packing::NO;
     if (q.M <= 256) {
         const size_t bm = q.M <= 16 ? 16 : (q.M <= 32 ? 32 : 64), strips = ((q.M + 63) / 64) * ((q.N + 31) / 32);
         t_rows = std::min(t_rows, std::max(4.0, (bm + 32) * steps * 128.0 / 50.0e3) * std::max(1.0, (double)strips / cus));
     }
-    return 12.0 + 0.2e-6 * (double)(q.M + q.N) * kbytes + t_rows < t_any;
+    const double t_packed = 12.0 + 0.2e-6 * (double)(q.M + q.N) * kbytes + t_rows;
+    if (t_packed >= any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K)) return Packing::NO;
+    return t_packed >= few_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K) ? Packing::UNLESS_FEW_ROWS : Packing::YES;
 }
 
 // Operands that no MFMA kernel reads as they stand: pack_kernel writes what has to change into the workspace as rows of
@@ -1187,7 +1192,9 @@ bool pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
 //     on the scratch, are ordered by nobody, and packed operands in a block that they share would overwrite each other.
 //     (The choice does not depend on how much room there happens to be: a call captured twice gives the same bits.)
 //   * the device has no memory left for the workspace, or the shape exceeds what the MFMA kernels index;
-//   * a product so small that the any-shape kernel is done first (pack_pays).
+//   * a product so small that the any-shape kernel is done first (pack_pays), or gemm_few_kernel, unless an fp32 output would show
+//     that the packed rows sum more exactly than its eight parts (fp8 51 x 616 x 7907, seven slices: 6.3e-8 of the result off, in eight
+//     parts 6.8e-8).
 // fp8 operands run on the family that widens them to bf16 in front of the matrix core (AR_F8W), which adds in fp32 as these
 // shapes have always been summed: the fp8 instructions keep some 18 bits of the largest product of a step.  Relative error
 // against 64 bits, 301 x 100 x 4001 to fp32, one scale / block scales: in sequence 9.0e-8 / 1.1e-7, any-shape kernel 8.9e-8 /
@@ -1205,7 +1212,8 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
     const size_t eb = dtype_bytes(in_dtype);
     if (!g_ctx.any_shape) return QGEMM_OK;
     if (q.arith == AR_F8) q.arith = AR_F8W;
-    if (g_ctx.any_shape == 1 && !pack_pays(q, in_dtype, K, a_src.k_major || b_src.k_major)) return QGEMM_OK;
+    const Packing pays = g_ctx.any_shape == 1 ? pack_pays(q, in_dtype, K, a_src.k_major || b_src.k_major) : Packing::YES;
+    if (pays == Packing::NO || (pays == Packing::UNLESS_FEW_ROWS && !output_shows_sums(q.arith, q.block, q.out_dtype))) return QGEMM_OK;
     if (g_ctx.static_call || stream_is_capturing(stream)) return QGEMM_OK;
     if (q.M >= ((size_t)1 << 31) || q.N >= ((size_t)1 << 31) || K >= ((size_t)1 << 30)) return QGEMM_OK;
     // (a K that ends inside a 16-byte piece has to end in zeros in both operands)
@@ -1224,6 +1232,8 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
     if (!mfma_shape_ok(q)) return QGEMM_OK;
     Plan pl;
     if (plan_nt(q, pl) != QGEMM_OK) return QGEMM_OK;
+    if (pays == Packing::UNLESS_FEW_ROWS &&
+        sums_as_exact(q.arith, q.block, q.out_dtype, {(uint32_t)pl.v->kgroups, pl.a.nsplit}, {8, 1})) return QGEMM_OK;
     const size_t split_room = (pl.split_bytes + 255) / 256 * 256;
     const size_t as_room = settle_scale_layout(q, pl) ? 0 : scales_room(q);
     PackArgs pa;

@@ -29,3 +29,32 @@ def test_sums_in_eight_parts_or_more(shape, dtype):
     err = float((c.double().cpu() - ref).norm() / ref.norm())
     print(Q.last_config(), err)
     assert err < 1.25 * 2.0 ** -24 / math.sqrt(3) * math.sqrt(K / 128 / 2 + 7 / 2), (Q.last_config(), err)
+
+
+@pytest.mark.parametrize("shape", [(51, 616, 7907), (47, 344, 6287), (40, 480, 7001)])
+@pytest.mark.parametrize("block", [False, True])
+def test_ragged_fp8_sums_as_it_does_packed(shape, block):
+    """Packed rows with a K split sum in more parts than the kernel for few rows, which an fp32 output shows: the faster kernel is for
+    outputs that hide it."""
+    M, N, K = shape
+    say("ragged fp8 to fp32", shape, "block scales" if block else "one scale")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(N)
+    a, b = ((60 * torch.randn(r, K, generator=g, device="cuda")).to(torch.float8_e4m3fn) for r in (M, N))
+    kb = (K + 127) // 128 if block else 1
+    sa, sb = torch.rand(M if block else 1, kb, generator=g, device="cuda"), torch.rand((N + 127) // 128 if block else 1, kb, generator=g, device="cuda")
+
+    def run(dtype, any_shape):
+        Q.set_option("any_shape", any_shape)
+        try:
+            c = torch.zeros(M, N, device="cuda", dtype=dtype)
+            Q.scaled_gemm(a, b, sa, sb, c, M, N, K, Q.SCALE_BLOCK128 if block else Q.SCALE_PER_MATRIX)
+            return c, Q.last_config()
+        finally:
+            Q.set_option("any_shape", 1)
+
+    packed, row = run(torch.float32, 2)
+    assert row.startswith("pack+") and "_splitk" in row, row
+    c, name = run(torch.float32, 1)
+    assert name == row and torch.equal(c, packed)
+    assert run(torch.bfloat16, 1)[1] == "strided_any_shape"
