@@ -169,6 +169,11 @@ int qgemm_quantize(int in_dtype, int out_dtype, int mode, const void *x, size_t 
 int qgemm_tile_map(uint32_t wg, uint32_t tiles_m, uint32_t tiles_n, uint32_t group_m, uint32_t *tile_m,
                    uint32_t *tile_n);
 
+/* Launch of the 1 x 128 quantiser for a matrix: rows of a slice, slices (the y extent of the grid) and workgroups of 256 threads in
+ * one (the x extent).  Host-callable so tests can check that every block is covered and that a launch stays below the
+ * runtime's 2^32 threads along x. */
+int qgemm_quantize_grid(int in_dtype, size_t rows, size_t cols, uint32_t *rows_per_slice, uint32_t *slices, uint32_t *groups);
+
 /* Tuning / diagnostics (no reference counterpart: the reference picks its tile at compile time,
  * src/include/gemm_config.h:30-36).
  * qgemm_set_option(key, value): "force_split" (K slices, 0 = heuristic), "group_m", "kmajor", "any_shape" (operands whose K

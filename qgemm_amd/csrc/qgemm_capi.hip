@@ -31,6 +31,7 @@ namespace {
 constexpr size_t kStaticScratchBytes = QGEMM_STATIC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 constexpr int kMaxDevices = 64;
+constexpr uint32_t kMaxGridY = 65535;
 
 struct WsBlock {
     void *p = nullptr;
@@ -1370,6 +1371,21 @@ int launch_transpose(int elem_bytes, const void *in, void *out, size_t M, size_t
     return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }
 
+// Slices of rows of the 1 x 128 quantiser (QuantArgs::rows_per_slice; blockIdx.y) and workgroups of one slice.  A launch takes fewer
+// than 2^32 threads along x, 256 for `per_group` blocks (a 64 GiB matrix of fp32 is past that, or 8 GiB of rows of 16), and block
+// numbers are 32-bit.
+struct RowBlockGrid {
+    uint32_t rows_per_slice, slices, groups;
+};
+RowBlockGrid row_block_grid(uint32_t rows, uint32_t per_row, uint32_t per_group) {
+    const uint64_t most = std::min<uint64_t>((uint64_t)1 << 31, (uint64_t)per_group * ((1 << 24) - 1));        // blocks of a slice
+    RowBlockGrid g;
+    g.rows_per_slice = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(rows, most / per_row));
+    g.slices = (uint32_t)(((uint64_t)rows + g.rows_per_slice - 1) / g.rows_per_slice);
+    g.groups = (uint32_t)(((uint64_t)g.rows_per_slice * per_row + per_group - 1) / per_group);
+    return g;
+}
+
 template <int IN_DT, int OUT_DT>
 int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
     typedef Piece<IN_DT> P;
@@ -1407,10 +1423,11 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         e = launch_kernel(a.rows == 1 ? quant_matrix_kernel<IN_DT, OUT_DT, true> : quant_matrix_kernel<IN_DT, OUT_DT, false>, dim3(nq, slices), dim3(256), 0, stream, a);
     } else if (mode == QGEMM_QUANT_BLOCK_1x128) {
         number((a.cols + 127) / 128);
-        const uint64_t blocks = (uint64_t)a.rows_per_slice * a.per_row;
-        const uint32_t slices = (a.rows + a.rows_per_slice - 1) / a.rows_per_slice, per_group = 256 / P::LANES;
-        const dim3 grid((unsigned)((blocks + per_group - 1) / per_group), slices);
-        if (blocks >= (uint64_t)kQuantManyGroups * per_group)
+        const RowBlockGrid g = row_block_grid(a.rows, a.per_row, 256 / P::LANES);
+        a.rows_per_slice = g.rows_per_slice;
+        if (g.slices > kMaxGridY) return QGEMM_ERR_TOO_LARGE;
+        const dim3 grid(g.groups, g.slices);
+        if ((uint64_t)g.rows_per_slice * a.per_row >= (uint64_t)kQuantManyGroups * (256 / P::LANES))
             e = launch_kernel(ragged ? quant_row_block_kernel<IN_DT, OUT_DT, true> : quant_row_block_kernel<IN_DT, OUT_DT, false>, grid, dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
         else
             e = launch_kernel(ragged ? quant_few_blocks_kernel<IN_DT, OUT_DT, true> : quant_few_blocks_kernel<IN_DT, OUT_DT, false>, grid, dim3(256), 0, stream, a);
@@ -1477,6 +1494,17 @@ QGEMM_EXPORT int qgemm_tile_map(uint32_t wg, uint32_t tiles_m, uint32_t tiles_n,
     if ((uint64_t)wg >= (uint64_t)tiles_m * tiles_n) return QGEMM_ERR_INVALID_ARG;
     tile_map(wg, make_tile_map(tiles_m, tiles_n, group_m), *tile_m, *tile_n);
     return QGEMM_OK;
+}
+
+QGEMM_EXPORT int qgemm_quantize_grid(int in_dtype, size_t rows, size_t cols, uint32_t *rows_per_slice, uint32_t *slices, uint32_t *groups) {
+    if (in_dtype != QGEMM_DT_F32 && in_dtype != QGEMM_DT_BF16 && in_dtype != QGEMM_DT_F16) return QGEMM_ERR_UNSUPPORTED;
+    if (!rows_per_slice || !slices || !groups || rows == 0 || cols == 0) return QGEMM_ERR_INVALID_ARG;
+    if (rows >= ((size_t)1 << 31) || cols >= ((size_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
+    const RowBlockGrid g = row_block_grid((uint32_t)rows, (uint32_t)((cols + 127) / 128), 256 / (in_dtype == QGEMM_DT_F32 ? Piece<QGEMM_DT_F32>::LANES : Piece<QGEMM_DT_BF16>::LANES));
+    *rows_per_slice = g.rows_per_slice;
+    *slices = g.slices;
+    *groups = g.groups;
+    return g.slices > kMaxGridY ? QGEMM_ERR_TOO_LARGE : QGEMM_OK;
 }
 
 QGEMM_EXPORT int qgemm_set_option(const char *key, long value) {

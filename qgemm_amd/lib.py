@@ -46,6 +46,7 @@ SIGNATURES = {
     "qgemm_quantize": (_i, [_i, _i, _i, _vp, _sz, _sz, _sz, _vp, _sz, _vp, _sz, _sz, _vp]),
     "qgemm_tile_map": (_i, [C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32, C.POINTER(C.c_uint32),
                             C.POINTER(C.c_uint32)]),
+    "qgemm_quantize_grid": (_i, [_i, _sz, _sz, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32), C.POINTER(C.c_uint32)]),
     "qgemm_set_option": (_i, [C.c_char_p, C.c_long]),
     "qgemm_force_config": (_i, [C.c_char_p]),
     "qgemm_variant_count": (_i, [_i, _i, _i]),

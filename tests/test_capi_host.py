@@ -347,3 +347,23 @@ def test_bench_has_traffic_counters_for_the_headline_kernel():
     cited = [w for w in source.replace(",", " ").split() if w.startswith("profiles/")]
     assert cited and all(os.path.exists(os.path.join(root, f)) for f in cited), source
     assert bench.measured_traffic("no_such_kernel", 8192)[0] is None
+
+
+@pytest.mark.parametrize("dt,per_group", [(Q.DT_F32, 8), (Q.DT_BF16, 16), (Q.DT_F16, 16)])
+def test_1x128_quantiser_launches_stay_below_the_threads_of_a_launch(dt, per_group):
+    """Every block in exactly one slice, block numbers in 32 bits, and fewer than 2^32 threads along x, also for matrices of
+    more blocks than that many threads cover (8 GiB of fp32 in rows of 16)."""
+    lib, out = L.load_library(), [C.c_uint32() for _ in range(3)]
+    most = 2 ** 24 * per_group                                       # blocks whose threads are 2^32
+    shapes = [(1, 1), (1, 128), (500, 7200), (6144, 7168), (most - per_group, 16), (most - per_group + 1, 16), (most, 16), (2 ** 31 - 1, 1),
+              (most // 56, 7168), (most // 56 + 1, 7168), (33, 2 ** 31 - 1), (2 ** 20, 2 ** 17 - 5)]
+    for rows, cols in shapes:
+        assert lib.qgemm_quantize_grid(dt, rows, cols, *[C.byref(v) for v in out]) == 0
+        per_slice, slices, groups = (v.value for v in out)
+        per_row = (cols + 127) // 128
+        assert (slices - 1) * per_slice < rows <= slices * per_slice and slices <= 65535
+        assert groups == (per_slice * per_row + per_group - 1) // per_group and groups * 256 < 2 ** 32
+        assert per_slice == rows or (per_slice + 1) * per_row > most - per_group      # (no more slices than it takes)
+    assert lib.qgemm_quantize_grid(99, 1, 1, *[C.byref(v) for v in out]) == 2
+    assert lib.qgemm_quantize_grid(dt, 0, 1, *[C.byref(v) for v in out]) == 1
+    assert lib.qgemm_quantize_grid(dt, 2 ** 31, 1, *[C.byref(v) for v in out]) == 9

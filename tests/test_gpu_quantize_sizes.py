@@ -74,3 +74,19 @@ def test_special_values_wherever_they_stand(rows, cols, special):
         q, s = R.quantize_fp8_block(yf, 128, 128)
         g, gs = Q.quantize(y, torch.float8_e4m3fn, Q.QUANT_BLOCK_128x128)
         assert np.array_equal(host(gs).view(np.uint32), s.view(np.uint32)) and np.array_equal(_u8(g), q), at
+
+
+def test_more_row_blocks_than_a_launch_has_threads_for():
+    """2^27 blocks of fp32 are 2^32 threads: a second slice of rows takes what the first cannot."""
+    rows, cols, lead = 1 << 27, 16, 1 << 20
+    say("quantize 1 x 128", rows, cols, "float32")
+    x = torch.empty((rows, cols), dtype=torch.float32, device="cuda")
+    head = torch.from_numpy(R.fill_normal((lead, cols), 9)).cuda()
+    x.view(rows // lead, lead, cols).copy_(head)                    # the same rows over and over
+    q, s = Q.quantize(x, torch.float8_e4m3fn, Q.QUANT_BLOCK_1x128)
+    del x
+    want_q, want_s = Q.quantize(head, torch.float8_e4m3fn, Q.QUANT_BLOCK_1x128)
+    assert torch.equal(s.view(rows // lead, lead, 1), want_s.expand(rows // lead, lead, 1))
+    assert torch.equal(q.view(torch.uint8).view(rows // lead, lead, cols), want_q.view(torch.uint8).expand(rows // lead, lead, cols))
+    del q, s
+    torch.cuda.empty_cache()
