@@ -1140,7 +1140,8 @@ double any_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N,
 // a wave's few blocks are rounded once more where the partial sums meet (relative error, tiles / few rows, int8 16 x 300 x 1031
 // 5.3e-8 / 6.4e-8, x 2051 6.8e-8 / 6.9e-8, but x 4001 8.4e-8 / 7.3e-8, fp8 x 7999 14.8e-8 / 8.3e-8; a 16-bit output hides it).
 double few_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N, size_t K) {
-    if (M > 128 || K >= ((size_t)1 << 30) || any_folded(in_dtype, out_dtype) || (block && out_dtype == QGEMM_DT_F32 && K < 3000)) return 1e30;
+    // (its 512 threads for 32 columns stay below the 2^32 of a launch; the tiles have 256 for 64 or 128)
+    if (M > 128 || (N + 31) / 32 >= ((size_t)1 << 23) || K >= ((size_t)1 << 30) || any_folded(in_dtype, out_dtype) || (block && out_dtype == QGEMM_DT_F32 && K < 3000)) return 1e30;
     struct FewModel {
         double fixed, round, alone, full;
         size_t per_cu;

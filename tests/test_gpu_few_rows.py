@@ -86,3 +86,21 @@ def test_special_values_stay_in_their_rows():
         got = c.cpu()
         assert torch.equal(got[keep_m][:, keep_n], want)
         assert torch.isnan(got[3]).all() and not torch.isfinite(got[0, 20])
+
+
+def test_more_columns_than_a_launch_has_threads_for():
+    """2^28 columns would be 2^32 threads of the kernel for few rows: the tiles take them."""
+    N, K, lead = 1 << 28, 129, 1 << 16
+    say("few rows", (1, N, K), "69 GB of B")
+    rng = np.random.default_rng(4)
+    a = rng.integers(-3, 4, size=(1, K)).astype(np.float32)
+    b = rng.integers(-3, 4, size=(lead, K)).astype(np.float32)
+    torch.cuda.empty_cache()
+    qb = torch.empty((N, K), dtype=torch.bfloat16, device="cuda")
+    qb.view(N // lead, lead, K).copy_(dev(b).bfloat16())             # the same rows over and over
+    c = torch.full((1, N), -7.0, dtype=torch.bfloat16, device="cuda")
+    Q.gemm(dev(a).bfloat16(), qb, c, "nk")
+    want = torch.from_numpy(R.gemm_f32acc(a, b)).bfloat16().cuda()
+    assert torch.equal(c.view(N // lead, lead), want.expand(N // lead, lead))
+    del qb, c
+    torch.cuda.empty_cache()
