@@ -112,11 +112,14 @@ __device__ inline v2i widen_fp8(uint32_t w) {
 }
 
 // A launch whose status is that of the launch itself.  The <<< >>> form passes the sizes through a stack of the runtime and leaves
-// the status to hipGetLastError: two calls and 0.1 - 0.3 us of host time more, of 3.3 a product.
+// the status to hipGetLastError: two calls and 0.1 - 0.3 us of host time more, of 3.3 a product.  A launch that fails leaves nothing in the
+// runtime's last error, where the next caller of hipGetLastError, here or in the program, would take it for its own.
 template <class... P>
 inline hipError_t launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, std::common_type_t<P>... args) {
     void *at[] = {(void *)&args...};
-    return hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, at, lds, stream);
+    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, at, lds, stream);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 // i / d and i % d with inv = inverse_of(d): the estimate is at most one too small.  Four scalar instructions where the values are
