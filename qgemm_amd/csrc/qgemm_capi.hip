@@ -1273,8 +1273,7 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
     pa.op[1].dst = bt;
     q.A = pack[0] ? at : a_src.p;
     q.B = pack[1] ? bt : b_src.p;
-    hipLaunchKernelGGL(eb == 2 ? pack_kernel<2> : pack_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, stream, pa);
-    if (hipGetLastError() != hipSuccess) return QGEMM_ERR_LAUNCH;
+    HIP_TRY(launch_kernel(eb == 2 ? pack_kernel<2> : pack_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, stream, pa));
     if (as_room) {
         st = scales_rows_contiguous(q, (char *)ws + split_room, stream);
         if (st != QGEMM_OK) return st;
@@ -1289,8 +1288,8 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
     const uint64_t elements = (uint64_t)a.a.rows * a.b.rows;
     if (a.a.end - a.a.p < 16 || a.b.end - a.b.p < 16 || (a.K < 16 && elements * a.K <= 1000000)) {
         if (elements >= (uint64_t)1 << 39) return QGEMM_ERR_TOO_LARGE;     // grid limit
-        hipLaunchKernelGGL((gemm_short_kernel<DT, BLOCK>), dim3((unsigned)((elements + 255) / 256)), dim3(256), 0, stream, a);
-        return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+        HIP_TRY(launch_kernel(gemm_short_kernel<DT, BLOCK>, dim3((unsigned)((elements + 255) / 256)), dim3(256), 0, stream, a));
+        return QGEMM_OK;
     }
     constexpr int W = BLOCK && DT == QGEMM_DT_I8 ? 64 : 128;
     const bool km = a.a.k_major || a.b.k_major;
@@ -1310,8 +1309,8 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
                           : (km ? gemm_any_kernel<DT, SUM, BLOCK ? 64 : W, true> : gemm_any_kernel<DT, SUM, W, false>);
     if constexpr (DT == QGEMM_DT_BF16 || DT == QGEMM_DT_F16)
         if (T == 64 && any_folded(DT, a.out_dtype)) kernel = km ? gemm_any_kernel<DT, ANY_FOLDED, 64, true> : gemm_any_kernel<DT, ANY_FOLDED, 64, false>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(256), 0, stream, a);
-    return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+    HIP_TRY(launch_kernel(kernel, dim3((unsigned)tiles), dim3(256), 0, stream, a));
+    return QGEMM_OK;
 }
 
 // The any-shape kernel on the operands as they stand (arguments as for launch_packed; M, N, K below 2^32)
@@ -1357,19 +1356,18 @@ int launch_transpose(int elem_bytes, const void *in, void *out, size_t M, size_t
         const bool aligned = M % 16 == 0 && N % 4 == 0 && (uintptr_t)in % 4 == 0 && (uintptr_t)out % 16 == 0;
         const dim3 g((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128));
         const auto kernel = aligned ? transpose_bytes_kernel<true> : transpose_bytes_kernel<false>;
-        hipLaunchKernelGGL(kernel, g, dim3(256), 0, stream, (const uint8_t *)in, (uint8_t *)out, (uint32_t)M, (uint32_t)N);
+        HIP_TRY(launch_kernel(kernel, g, dim3(256), 0, stream, (const uint8_t *)in, (uint8_t *)out, (uint32_t)M, (uint32_t)N));
     } else if (elem_bytes == 2) {
         const bool aligned = M % 8 == 0 && N % 8 == 0 && (uintptr_t)in % 16 == 0 && (uintptr_t)out % 16 == 0;
         const dim3 g((unsigned)((N + 255) / 256), (unsigned)((M + 63) / 64));
         const auto kernel = aligned ? transpose_u16_kernel<true> : transpose_u16_kernel<false>;
-        hipLaunchKernelGGL(kernel, g, dim3(256), 0, stream, (const uint16_t *)in, (uint16_t *)out, (uint32_t)M, (uint32_t)N);
+        HIP_TRY(launch_kernel(kernel, g, dim3(256), 0, stream, (const uint16_t *)in, (uint16_t *)out, (uint32_t)M, (uint32_t)N));
     } else if (elem_bytes == 4) {
-        hipLaunchKernelGGL(transpose_u32_kernel, grid, dim3(256), 0, stream, (const uint32_t *)in, (uint32_t *)out,
-                           (uint32_t)M, (uint32_t)N);
+        HIP_TRY(launch_kernel(transpose_u32_kernel, grid, dim3(256), 0, stream, (const uint32_t *)in, (uint32_t *)out, (uint32_t)M, (uint32_t)N));
     } else {
         return QGEMM_ERR_UNSUPPORTED;
     }
-    return hipGetLastError() == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+    return QGEMM_OK;
 }
 
 // Slices of rows of the 1 x 128 quantiser (QuantArgs::rows_per_slice; blockIdx.y) and workgroups of one slice.  A launch takes fewer
@@ -1859,8 +1857,7 @@ int scaled_gemm_entry(bool use_static, int in_dtype, int out_dtype, int scale_mo
             t.tiles0 = (uint32_t)(tk * t.tiles_n[0]);
             const size_t total = tk * ((size_t)t.tiles_n[0] + t.tiles_n[1]);
             if (total >= ((size_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
-            hipLaunchKernelGGL(transpose_bytes2_kernel, dim3((unsigned)total), dim3(256), 0, stream, t);
-            if (hipGetLastError() != hipSuccess) return QGEMM_ERR_LAUNCH;
+            HIP_TRY(launch_kernel(transpose_bytes2_kernel, dim3((unsigned)total), dim3(256), 0, stream, t));
         } else {
             st = launch_transpose(1, A, at, K, M, stream);
             if (st != QGEMM_OK) return st;
@@ -2005,9 +2002,8 @@ QGEMM_EXPORT int qgemm_selftest_layouts(char *buf, size_t buflen) {
         const uint32_t bases[3] = {0, 72 * 1024, 159 * 1024};
         const uint32_t soffs[3] = {0, 1024, 16};
         for (int t = 0; t < 3; ++t) {
-            hipLaunchKernelGGL(probe_lds_dma_kernel, dim3(1), dim3(64), 160 * 1024, 0, (const char *)dsrc,
-                               (const uint32_t *)doff, (uint32_t)nsrc, bases[t], soffs[t], (char *)dout);
-            HIP_TRY(hipGetLastError());
+            HIP_TRY(launch_kernel(probe_lds_dma_kernel, dim3(1), dim3(64), 160 * 1024, nullptr, (const char *)dsrc,
+                                  (const uint32_t *)doff, (uint32_t)nsrc, bases[t], soffs[t], (char *)dout));
             std::vector<uint8_t> hout(1024);
             HIP_TRY(hipMemcpy(hout.data(), dout, 1024, hipMemcpyDeviceToHost));
             int bad = 0, oob_zero = 0, oob_untouched = 0;
@@ -2045,9 +2041,8 @@ QGEMM_EXPORT int qgemm_selftest_layouts(char *buf, size_t buflen) {
         // four K blocks of a row per lane, whatever the number of K blocks in a row
         for (int l = 0; l < 64; ++l) hoff[l] = (uint32_t)(l < 56 ? 4 * (7 * l % 1000) : nsrc - 4 * (l - 55));
         HIP_TRY(hipMemcpy(doff, hoff.data(), 256, hipMemcpyHostToDevice));
-        hipLaunchKernelGGL(probe_lds_dma_kernel, dim3(1), dim3(64), 160 * 1024, 0, (const char *)dsrc, (const uint32_t *)doff,
-                           (uint32_t)nsrc, 0u, 0u, (char *)dout);
-        HIP_TRY(hipGetLastError());
+        HIP_TRY(launch_kernel(probe_lds_dma_kernel, dim3(1), dim3(64), 160 * 1024, nullptr, (const char *)dsrc, (const uint32_t *)doff,
+                              (uint32_t)nsrc, 0u, 0u, (char *)dout));
         std::vector<uint8_t> hout(1024);
         HIP_TRY(hipMemcpy(hout.data(), dout, 1024, hipMemcpyDeviceToHost));
         int bad = 0;
@@ -2074,8 +2069,7 @@ QGEMM_EXPORT int qgemm_selftest_layouts(char *buf, size_t buflen) {
         HIP_TRY(hipMalloc(&d, 64 * 4));
         HIP_TRY(hipMalloc(&o, 128 * 4));
         HIP_TRY(hipMemcpy(d, h.data(), 64 * 4, hipMemcpyHostToDevice));
-        hipLaunchKernelGGL(probe_b64_load_kernel, dim3(1), dim3(64), 0, 0, (const float *)d, (uint32_t)(n_in * 4), (int *)o);
-        HIP_TRY(hipGetLastError());
+        HIP_TRY(launch_kernel(probe_b64_load_kernel, dim3(1), dim3(64), 0, nullptr, (const float *)d, (uint32_t)(n_in * 4), (int *)o));
         std::vector<float> got(128);
         HIP_TRY(hipMemcpy(got.data(), o, 128 * 4, hipMemcpyDeviceToHost));
         int bad = 0;
@@ -2110,13 +2104,9 @@ QGEMM_EXPORT int qgemm_selftest_layouts(char *buf, size_t buflen) {
             }
             HIP_TRY(hipMemcpy(dx, hx.data(), 2048, hipMemcpyHostToDevice));
             HIP_TRY(hipMemcpy(dy, hy.data(), 2048, hipMemcpyHostToDevice));
-            switch (arith) {
-                case AR_I8: hipLaunchKernelGGL(probe_mfma_kernel<AR_I8>, dim3(1), dim3(64), 0, 0, (const char *)dx, (const char *)dy, (int *)dout); break;
-                case AR_F8: hipLaunchKernelGGL(probe_mfma_kernel<AR_F8>, dim3(1), dim3(64), 0, 0, (const char *)dx, (const char *)dy, (int *)dout); break;
-                case AR_BF16: hipLaunchKernelGGL(probe_mfma_kernel<AR_BF16>, dim3(1), dim3(64), 0, 0, (const char *)dx, (const char *)dy, (int *)dout); break;
-                default: hipLaunchKernelGGL(probe_mfma_kernel<AR_F16>, dim3(1), dim3(64), 0, 0, (const char *)dx, (const char *)dy, (int *)dout); break;
-            }
-            HIP_TRY(hipGetLastError());
+            auto probe = arith == AR_I8 ? probe_mfma_kernel<AR_I8> : arith == AR_F8 ? probe_mfma_kernel<AR_F8>
+                         : arith == AR_BF16 ? probe_mfma_kernel<AR_BF16> : probe_mfma_kernel<AR_F16>;
+            HIP_TRY(launch_kernel(probe, dim3(1), dim3(64), 0, nullptr, (const char *)dx, (const char *)dy, (int *)dout));
             std::vector<int> hout(256);
             HIP_TRY(hipMemcpy(hout.data(), dout, 1024, hipMemcpyDeviceToHost));
             // assumed: operand lane l = row (l & 15), K group (l >> 4); the same element position of
@@ -2153,8 +2143,7 @@ QGEMM_EXPORT int qgemm_selftest_layouts(char *buf, size_t buflen) {
         const int nwg = 64;
         void *dout = nullptr;
         HIP_TRY(hipMalloc(&dout, nwg * 8));
-        hipLaunchKernelGGL(probe_xcc_kernel, dim3(nwg), dim3(64), 0, 0, (uint32_t *)dout);
-        HIP_TRY(hipGetLastError());
+        HIP_TRY(launch_kernel(probe_xcc_kernel, dim3(nwg), dim3(64), 0, nullptr, (uint32_t *)dout));
         std::vector<uint32_t> h(nwg * 2);
         HIP_TRY(hipMemcpy(h.data(), dout, nwg * 8, hipMemcpyDeviceToHost));
         (void)hipFree(dout);
