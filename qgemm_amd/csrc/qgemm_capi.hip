@@ -549,21 +549,29 @@ uint32_t slices_for_few_tiles(size_t tiles, uint32_t ksteps, int cus) {
     return std::min<uint32_t>(want, ksteps / 4);
 }
 
-// us; 0: the estimate does not know the row
-double few_rows_estimate(const Variant &v, size_t M, size_t N, size_t ksteps, bool block, int cus, uint32_t nsplit) {
-    for (const FewRowsTile &t : kFewRows) {
-        if (t.bm != v.bm || t.bn != v.bn || t.kgroups != v.kgroups) continue;
-        const FewRowsModel &m = block ? t.block : t.plain;
-        const size_t steps = (ksteps + nsplit - 1) / nsplit, slices = (ksteps + steps - 1) / steps;
-        const size_t wgs = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * slices, slots = (size_t)cus * m.slots;
-        const double load = std::min(1.0, (double)wgs / slots), n = t.kgroups == 8 ? (steps + (steps + 7) / 8 * 8) * 0.5 : (double)steps;
-        const double rounds = (double)((wgs + slots - 1) / slots);
-        double us = std::max(m.fixed + rounds * (m.round + n * (m.alone + (m.full - m.alone) * load)),
-                             m.late + (double)N * ksteps * 128e-6 * m.stream);
-        if (slices > 1) us += 2.6 + (double)M * N * 4e-6 * (slices + 1) / 4.5;
-        return us;
+// K steps of a slice as a row counts them
+inline double few_rows_steps(int kgroups, uint32_t steps) { return kgroups == 8 ? (steps + (steps + 7) / 8 * 8) * 0.5 : (double)steps; }
+// us on `tiles` tiles
+double few_rows_estimate(const FewRowsTile &t, size_t M, size_t N, size_t tiles, uint32_t ksteps, bool block, int cus, uint32_t nsplit) {
+    const FewRowsModel &m = block ? t.block : t.plain;
+    uint32_t steps = ksteps, slices = 1;
+    if (nsplit > 1) {
+        steps = (ksteps + nsplit - 1) / nsplit;
+        slices = (ksteps + steps - 1) / steps;
     }
-    return 0;
+    const size_t wgs = tiles * slices, slots = (size_t)cus * m.slots;
+    double load = 1, rounds = 1;
+    if (wgs < slots) load = (double)wgs / slots;
+    else rounds = (double)((wgs + slots - 1) / slots);
+    double us = std::max(m.fixed + rounds * (m.round + few_rows_steps(t.kgroups, steps) * (m.alone + (m.full - m.alone) * load)),
+                         m.late + (double)N * ksteps * 128e-6 * m.stream);
+    if (slices > 1) us += 2.6 + (double)M * N * 4e-6 * (slices + 1) / 4.5;
+    return us;
+}
+// ... and what it cannot be below on any number of tiles, K in one slice
+inline double few_rows_least(const FewRowsTile &t, size_t N, uint32_t ksteps, bool block) {
+    const FewRowsModel &m = block ? t.block : t.plain;
+    return std::max(m.fixed + (m.round + few_rows_steps(t.kgroups, ksteps) * m.alone), m.late + (double)N * ksteps * 128e-6 * m.stream);
 }
 
 // How many partial sums an element of C is made of: K groups of the row times K slices.
@@ -596,38 +604,52 @@ int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t kst
                    bool may_split, bool whole, int out_dtype, uint32_t *nsplit_out) {
     const int vi = choose_by_rules(tab, count, M, N, ksteps, block, kmaj, cus, may_split, nsplit_out);
     if (vi < 0 || kmaj || !whole || M > 400 || tab[vi].arith == AR_F8W || !g_ctx.row_estimate || !g_ctx.small_tiles || !(ksteps < 32 || (block && M <= 128))) return vi;
+    // (tile sides are powers of two)
+    auto tiles_of = [&](int bm, int bn) { return ((M + bm - 1) >> __builtin_ctz(bm)) * ((N + bn - 1) >> __builtin_ctz(bn)); };
+    const uint32_t steps = (uint32_t)ksteps;
     uint32_t asked = std::max<uint32_t>(1, *nsplit_out);
-    if (*nsplit_out == 0 && may_split)
-        asked = std::max<uint32_t>(1, slices_for_few_tiles(((M + tab[vi].bm - 1) / tab[vi].bm) * ((N + tab[vi].bn - 1) / tab[vi].bn), (uint32_t)ksteps, cus));
-    const double t_rules = few_rows_estimate(tab[vi], M, N, ksteps, block, cus, asked);
-    if (t_rules == 0) return vi;
+    if (*nsplit_out == 0 && may_split) asked = std::max<uint32_t>(1, slices_for_few_tiles(tiles_of(tab[vi].bm, tab[vi].bn), steps, cus));
+    const FewRowsTile *rules = nullptr;
+    for (const FewRowsTile &t : kFewRows)
+        if (t.bm == tab[vi].bm && t.bn == tab[vi].bn && t.kgroups == tab[vi].kgroups) rules = &t;
+    if (!rules) return vi;
+    const size_t rules_tiles = tiles_of(rules->bm, rules->bn);
     // (with streamed weights tiles of a second round, rows without a K split inside the workgroup where they stand several on a CU, and
     // those rows behind long loops with block scales cost more than the estimate says, which is a mean of streamed and resident
     // weights: 32 x 14336 x 4096 with block scales 14.7 us on 224 tiles of 64 x 64, 16.2 on 448 of 32 x 32)
-    const bool one_round = ((M + tab[vi].bm - 1) / tab[vi].bm) * ((N + tab[vi].bn - 1) / tab[vi].bn) * asked <= (size_t)cus;
-    int best = vi;
+    const bool one_round = rules_tiles * asked <= (size_t)cus;
+    const FewRowsTile *best = nullptr;
     uint32_t best_ns = *nsplit_out;
-    double best_t = t_rules * (ksteps == 8 && !block ? 0.87 : ksteps >= 32 ? 0.93 : 0.97);
-    for (int i = 0; i < count; ++i) {
-        const Variant &v = tab[i];
-        if ((v.bm > 32 && (size_t)v.bm > 2 * M) || M > 12 * (size_t)v.bm) continue;
-        const size_t tiles = ((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn);
+    double best_t = few_rows_estimate(*rules, M, N, rules_tiles, steps, block, cus, asked) * (ksteps == 8 && !block ? 0.87 : ksteps >= 32 ? 0.93 : 0.97);
+    // (this is on the way of every eager call: rows that cannot win on any number of tiles are left out first, which in one slice is
+    // most of them, and only the winner is looked up in the table.  Host time of qgemm_plan, us, rules alone / every row of the table priced /
+    // so: fp8 1 x 2048 x 1024 0.13 / 0.30 / 0.17, bf16 64 x 4096 x 1024 0.14 / 0.46 / 0.24, block scales 100 x 4096 x 2992 0.39 / 0.69 / 0.42,
+    // 300 x 8192 x 3968 0.62 / 0.90 / 0.62)
+    for (const FewRowsTile &t : kFewRows) {
+        if ((t.bm > 32 && (size_t)t.bm > 2 * M) || M > 12 * (size_t)t.bm) continue;
+        if (asked == 1 && few_rows_least(t, N, steps, block) >= best_t) continue;
+        const size_t tiles = tiles_of(t.bm, t.bn);
         if (tiles > 1400) continue;
         for (uint32_t ns = 1; ns <= 8 && ns <= asked; ns *= 2) {
             if (ns > 1 && (ksteps / ns < 6 || tiles * ns > 300)) break;
-            if (!sums_as_exact(v.arith, block, out_dtype, {(uint32_t)tab[vi].kgroups, asked}, {(uint32_t)v.kgroups, ns})) continue;
-            double t = few_rows_estimate(v, M, N, ksteps, block, cus, ns);
-            if (tiles * ns > (size_t)cus && (one_round || v.kgroups == 1)) t *= 1.12;
-            if (ksteps >= 32 && v.kgroups != 8) t *= 1.15;
-            if (t > 0 && t < best_t) {
-                best = i;
+            if (!sums_as_exact(tab[vi].arith, block, out_dtype, {(uint32_t)rules->kgroups, asked}, {(uint32_t)t.kgroups, ns})) continue;
+            double us = few_rows_estimate(t, M, N, tiles, steps, block, cus, ns);
+            if (tiles * ns > (size_t)cus && (one_round || t.kgroups == 1)) us *= 1.12;
+            if (ksteps >= 32 && t.kgroups != 8) us *= 1.15;
+            if (us < best_t) {
+                best = &t;
                 best_ns = ns;
-                best_t = t;
+                best_t = us;
             }
         }
     }
-    *nsplit_out = best_ns;
-    return best;
+    if (!best) return vi;
+    for (int i = 0; i < count; ++i)
+        if (tab[i].bm == best->bm && tab[i].bn == best->bn && tab[i].kgroups == best->kgroups) {
+            *nsplit_out = best_ns;
+            return i;
+        }
+    return vi;
 }
 
 int choose_tile(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
