@@ -76,3 +76,13 @@ def test_fp32_sums_in_no_fewer_parts_than_by_the_rules(family):
         assert (ga, sa) == (gb, sb) or (family[1] == 0 and gb * sb > ga * sa), (family, shape, a, b)
         kept += b != f
     assert kept > 10 and fp32 != rules
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+def test_strips_of_64_columns_stay_where_the_rules_take_them(family):
+    """17 .. 64 rows against 8193 .. 16384 columns: a measured rule that the estimate, off by up to 30 % there, must not replace."""
+    es = 2 if family[0] in (Q.DT_BF16, Q.DT_F16) else 1
+    for M in (17, 24, 32, 36, 50, 64):
+        for N in (8208, 10512, 12336, 14336, 16288):
+            for K in (2048, 2512, 3296, 4096 - 16) + ((4752, 6064, 8048) if family[1] == Q.SCALE_BLOCK128 else ()):
+                assert Q.plan(*family, 0, M, N, K // es // 16 * 16) == "skinny_64x64_k8", (M, N, K)
