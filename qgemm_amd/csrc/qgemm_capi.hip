@@ -514,7 +514,7 @@ int choose_by_rules(const Variant *tab, int count, size_t M, size_t N, size_t ks
 // out of memory and weights resident.  The rules above were made on a few dozen shapes around 32 K steps, and with kernels that
 // started later; measured against the fastest row they are 15 % behind on average, at worst twice its time: 48 x 1200 x 1024 int8
 // 6.34 (two K slices) -> 4.05 us (16 x 16 tiles), 24 x 4432 x 1152 with block scales 7.52 -> 5.00, 110 x 1024 x 1280
-// 7.90 -> 3.97, 124 x 3072 x 1792 8.97 -> 5.87.  What the estimate takes is 2.5 % behind (on the third of the shapes that it was not fitted on 2.9).
+// 7.90 -> 3.97, 124 x 3072 x 1792 8.97 -> 5.87.  What the estimate takes (few_rows_doubtful left out) is 2.4 % behind.
 // A row costs `fixed`, and every round of `slots` workgroups per CU `round` plus its K steps at `alone` (few workgroups) .. `full`
 // (all CUs at work) us each, or, where that is longer, `late` and B at `stream` us/MB.  (The eight waves of the skinny-M kernel
 // take the steps in turn: halfway between the steps and the next multiple of eight.)
@@ -574,6 +574,37 @@ inline double few_rows_least(const FewRowsTile &t, size_t N, uint32_t ksteps, bo
     return std::max(m.fixed + (m.round + few_rows_steps(t.kgroups, ksteps) * m.alone), m.late + (double)N * ksteps * 128e-6 * m.stream);
 }
 
+// Changes of row that the estimate gets wrong, by the tile of the rules and the one it puts ahead: both timed on 5700 shapes (1 .. 400 rows
+// x 256 .. 100 000 columns x 512 .. 8192; fp8, int8, bf16 and the two with block scales), geometric mean of weights streamed and resident.
+// At each, the gain that the estimate promises and what was measured.  Of the other 5250 changes ten are more than 5 % behind
+// the rules, at worst 18 %; together they gain 26 %.
+bool few_rows_doubtful(const FewRowsTile &rules, size_t rules_tiles, const FewRowsTile &t, size_t tiles, size_t M, size_t N, uint32_t ksteps,
+                       bool block, int cus) {
+    const size_t round = (size_t)cus;
+    const bool two_rounds = N > 32 * round;                  // of strips of 32 columns
+    auto is = [](const FewRowsTile &x, int bm, int bn, int kgroups) { return x.bm == bm && x.bn == bn && x.kgroups == kgroups; };
+    // 1.33, 0.89: strips of 64 columns, up to 64 rows, where 32-column strips need a second round (64 x 128 tiles with block scales 0.78)
+    if (M <= 64 && is(rules, 64, 64, 8)) return true;
+    // 1.14, 0.77: 65 .. 128 rows x 11000 .. 16384 columns from 64 x 128 to one row of 128 x 128 tiles, two K groups each
+    if (is(t, 128, 128, 2)) return true;
+    // 1.18, 0.82: ... or to a second round of 64 x 64 tiles
+    if (!block && is(rules, 64, 128, 2) && is(t, 64, 64, 8) && tiles > round) return true;
+    // 1.15, 0.88: the same tile without its K groups; except strips of 16 x 32 in three rounds or more (1.24, 1.28), and in two up to 12 steps
+    // (1.24, 1.05; from 13 steps on 1.19, 0.92)
+    if (t.bm == rules.bm && t.bn == rules.bn && t.kgroups == 1)
+        return !(is(rules, 16, 32, 8) && (ksteps <= 12 || rules_tiles > 2 * round));
+    // 1.16, 0.81: strips of 16 x 32, many on a CU, to one row of the skinny-M kernel a CU, in a second round
+    if (is(rules, 16, 32, 1) && t.kgroups == 8 && two_rounds) return true;
+    // 1.11, 0.93: tiles of 64 rows on eight waves of which some have no step
+    if (t.kgroups == 8 && t.bm == 64 && ksteps < 8 && t.bn == (block ? 64 : 32)) return true;
+    // 1.06, 1.00, at worst 0.89: strips of 16 columns in a third round
+    if (!block && is(t, 16, 16, 8) && tiles > 2 * round) return true;
+    // 1.21, 0.89: block scales, strips of 64 x 32 to anything else in a second round; from 12 steps on, to 64 x 128 in a third round 1.44, 1.15
+    // and to the skinny-M kernel in a second 1.09, 1.05
+    return block && is(rules, 64, 32, 1) && two_rounds &&
+           !(ksteps >= 12 && (rules_tiles > 2 * round ? t.bm == 64 && t.bn == 128 : t.kgroups == 8));
+}
+
 // How many partial sums an element of C is made of: K groups of the row times K slices.
 struct PartialSums {
     uint32_t groups, slices;
@@ -612,14 +643,12 @@ int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t kst
     const FewRowsTile *rules = nullptr;
     for (const FewRowsTile &t : kFewRows)
         if (t.bm == tab[vi].bm && t.bn == tab[vi].bn && t.kgroups == tab[vi].kgroups) rules = &t;
-    // (up to 64 rows against columns whose 32-column strips need a second round of CUs the rules take 64-column strips, a measured rule:
-    // over 150 such shapes that the estimate would change it was 11 % slower on average, 64 x 128 tiles with block scales
-    // 29 %, and ahead of no shape by 5 %)
-    if (!rules || (M <= 64 && rules->bm == 64 && rules->bn == 64)) return vi;
+    if (!rules) return vi;
     const size_t rules_tiles = tiles_of(rules->bm, rules->bn);
-    // (with streamed weights tiles of a second round, rows without a K split inside the workgroup where they stand several on a CU, and
-    // those rows behind long loops with block scales cost more than the estimate says, which is a mean of streamed and resident
-    // weights: 32 x 14336 x 4096 with block scales 14.7 us on 224 tiles of 64 x 64, 16.2 on 448 of 32 x 32)
+    // Margins: with streamed weights tiles of a second round, rows without a K split inside the workgroup where they stand several on a CU,
+    // and those rows behind long loops with block scales cost more than the estimate says, which is a mean of streamed and
+    // resident weights.  What each keeps back, 110 shapes that it decides: 0.87 9.8 % of gain and one shape more than 5 % slower, 0.93 and 1.15
+    // together 7.4 % and seven, 1.12 9.5 % and eight.
     const bool one_round = rules_tiles * asked <= (size_t)cus;
     const FewRowsTile *best = nullptr;
     uint32_t best_ns = *nsplit_out;
@@ -632,7 +661,7 @@ int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t kst
         if ((t.bm > 32 && (size_t)t.bm > 2 * M) || M > 12 * (size_t)t.bm) continue;
         if (asked == 1 && few_rows_least(t, N, steps, block) >= best_t) continue;
         const size_t tiles = tiles_of(t.bm, t.bn);
-        if (tiles > 1400) continue;
+        if (tiles > 1400 || few_rows_doubtful(*rules, rules_tiles, t, tiles, M, N, steps, block, cus)) continue;
         for (uint32_t ns = 1; ns <= 8 && ns <= asked; ns *= 2) {
             if (ns > 1 && (ksteps / ns < 6 || tiles * ns > 300)) break;
             if (!sums_as_exact(tab[vi].arith, block, out_dtype, {(uint32_t)rules->kgroups, asked}, {(uint32_t)t.kgroups, ns})) continue;

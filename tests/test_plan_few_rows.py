@@ -86,3 +86,28 @@ def test_strips_of_64_columns_stay_where_the_rules_take_them(family):
         for N in (8208, 10512, 12336, 14336, 16288):
             for K in (2048, 2512, 3296, 4096 - 16) + ((4752, 6064, 8048) if family[1] == Q.SCALE_BLOCK128 else ()):
                 assert Q.plan(*family, 0, M, N, K // es // 16 * 16) == "skinny_64x64_k8", (M, N, K)
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+def test_one_row_of_128_x_128_tiles_does_not_replace_64_x_128(family):
+    """65 .. 128 rows against 11000 .. 16384 columns: the estimate likes the 128 x 128 row with two K groups, which is 15 - 30 % behind."""
+    es = 2 if family[0] in (Q.DT_BF16, Q.DT_F16) else 1
+    for M in (66, 76, 95, 109, 128):
+        for N in (11904, 13696, 14976, 16000):
+            for K in (1280, 2048, 2560, 3328, 3968):
+                shape = (M, N, K // es // 16 * 16)
+                rules, = _plans(family, [shape], row_estimate=0)
+                assert not Q.plan(*family, 0, *shape).startswith("128x128") or rules.startswith("128x128"), shape
+
+
+# shapes at which the estimate is ahead of the rules by itself and 7 - 37 % behind by the clock, one or two of each kind of change
+DOUBTFUL = [("bf16", 1, 10112, 1536), ("i8", 3, 10144, 3200), ("i8", 3, 10368, 2304), ("bf16", 9, 9616, 1088), ("i8b", 2, 23040, 640), ("f8", 3, 16256, 768),
+            ("i8b", 1, 22304, 688), ("i8b", 42, 13056, 896), ("i8b", 46, 76928, 512), ("f8b", 44, 15072, 976), ("f8b", 39, 61120, 752), ("f8b", 48, 32512, 992),
+            ("f8", 82, 15952, 2704), ("f8", 63, 7552, 3968), ("i8", 93, 15488, 3968), ("i8b", 73, 6784, 896), ("f8", 33, 7168, 640)]
+
+
+@pytest.mark.parametrize("kind,M,N,K", DOUBTFUL)
+def test_the_rules_stay_where_the_estimate_is_known_to_be_wrong(kind, M, N, K):
+    family = {"bf16": (Q.DT_BF16, 0), "f8": (Q.DT_F8E4M3, Q.SCALE_PER_MATRIX), "i8": (Q.DT_I8, Q.SCALE_PER_MATRIX),
+              "f8b": (Q.DT_F8E4M3, Q.SCALE_BLOCK128), "i8b": (Q.DT_I8, Q.SCALE_BLOCK128)}[kind]
+    assert _plans(family, [(M, N, K)]) == _plans(family, [(M, N, K)], row_estimate=0)
