@@ -184,7 +184,9 @@ int qgemm_quantize_grid(int in_dtype, size_t rows, size_t cols, uint32_t *rows_p
  *   empty last round of 256 x 256 tiles as a second launch where the estimate gains; 2 / 3: rows / columns wherever
  *   possible), "small_tiles" (0: 17 .. 256 rows against few columns keep a tall tile with a K split instead of several
  *   row tiles of the skinny-M kernel; row_estimate counts as 0 then), "row_estimate" (0: up to 400 rows follow the general
- *   rules instead of the estimate of every row that serves them below 32 K steps and, block scales, up to 128 rows), "c_plain" (0 / 1: non-temporal / ordinary stores for C; -1: the library's
+ *   rules instead of the estimate of every row that serves them below 32 K steps and, block scales, up to 128 rows), "few_rows"
+ *   (operands that option "any_shape" decides about, 1 .. 128 rows: 0 / 2: never / wherever it can the kernel for few rows
+ *   instead of the tiles of the any-shape kernel; 1: by an estimate), "c_plain" (0 / 1: non-temporal / ordinary stores for C; -1: the library's
  *   choice), "b_stream" (0 / 1: copies of B without / with the streaming hint; -1: the library's choice); "force_config" accepts only -1 (back to the heuristic).
  *   "k_rot": with at most 256 rows the workgroups of column tile i start their K loops 3 i steps in and wrap round
  *   (memory channels), so the order of an fp32 sum depends on the column tile: results are the same from run to
@@ -201,6 +203,9 @@ int qgemm_force_config(const char *name);
 int qgemm_variant_count(int in_dtype, int scale_mode, int k_major);
 int qgemm_variant_name(int in_dtype, int scale_mode, int k_major, int index, char *buf, size_t buflen);
 int qgemm_last_config(char *buf, size_t buflen);
+/* What the last product with qgemm_last_config "strided_any_shape" launched: "tiles_64x64" or "tiles_128x128" (the any-shape kernel),
+ * "few_rows_16x32" or "few_rows_32x32" (its form for 1 .. 128 rows), "short" (a few loads of single elements); "" before the first. */
+int qgemm_last_any_kernel(char *buf, size_t buflen);
 
 /* Which kernel configuration the library would run for a problem with dense, 16-byte aligned operands: the name
  * qgemm_last_config would report after the call ("256x256_w2x2_solo", "128x128_w2x2_dma_tn_splitk2", ...;

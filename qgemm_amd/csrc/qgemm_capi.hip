@@ -66,6 +66,7 @@ struct Context {
                                 // transposed copy of a_scale for the row with copying waves (see settle_scale_layout)
     long small_tiles = 1;       // 0: 17 .. 256 rows never go to several row tiles of the skinny-M kernel in place of a K split (and up to 400
                                 // rows follow the rules, as the estimate likes such tiles)
+    long few_rows = 1;          // ragged operands, up to 128 rows: 0: never gemm_few_kernel, 2: wherever it can, 1: by its estimate (few_estimate)
     long row_estimate = 1;      // 0: up to 400 rows follow the rules (choose_by_rules) instead of the estimate of every row (choose_variant)
     long k_rot = -1;            // -1: rotated K start for at most 256 rows (see plan_nt), 0: never, n: steps per column tile
     long stagger = -1;          // -1: staggered start where it pays (4-byte C, three or more rounds), else microseconds per group
@@ -80,6 +81,7 @@ struct Context {
     long kmajor = 1;            // 0: K-major operands (NN, reference fp8 layout) always go through the transposes; 2: never
                                 // where a K-major kernel fits the shape (for measurements and tests)
     std::string last_config;
+    const char *last_any_kernel = "";    // what launch_any_t launched last
 };
 
 Context g_ctx;
@@ -1196,6 +1198,7 @@ double any_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N,
 double few_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N, size_t K) {
     // (its 512 threads for 32 columns stay below the 2^32 of a launch; the tiles have 256 for 64 or 128)
     if (M > 128 || (N + 31) / 32 >= ((size_t)1 << 23) || K >= ((size_t)1 << 30) || any_folded(in_dtype, out_dtype) || (block && out_dtype == QGEMM_DT_F32 && K < 3000)) return 1e30;
+    if (g_ctx.few_rows != 1) return g_ctx.few_rows ? 0 : 1e30;
     struct FewModel {
         double fixed, round, alone, full;
         size_t per_cu;
@@ -1342,6 +1345,7 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
     const uint64_t elements = (uint64_t)a.a.rows * a.b.rows;
     if (a.a.end - a.a.p < 16 || a.b.end - a.b.p < 16 || (a.K < 16 && elements * a.K <= 1000000)) {
         if (elements >= (uint64_t)1 << 39) return QGEMM_ERR_TOO_LARGE;     // grid limit
+        g_ctx.last_any_kernel = "short";
         HIP_TRY(launch_kernel(gemm_short_kernel<DT, BLOCK>, dim3((unsigned)((elements + 255) / 256)), dim3(256), 0, stream, a));
         return QGEMM_OK;
     }
@@ -1350,6 +1354,7 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
     if (!km && few_estimate(DT, a.out_dtype, BLOCK, a.a.rows, a.b.rows, a.K) < any_estimate(DT, a.out_dtype, BLOCK, a.a.rows, a.b.rows, a.K)) {
         constexpr int ARITH = DT == QGEMM_DT_I8 ? AR_I8 : DT == QGEMM_DT_F8E4M3 ? AR_F8W : DT == QGEMM_DT_BF16 ? AR_BF16 : AR_F16;
         const bool one = a.a.rows <= 16;
+        g_ctx.last_any_kernel = one ? "few_rows_16x32" : "few_rows_32x32";
         const hipError_t e = launch_kernel(one ? gemm_few_kernel<ARITH, BLOCK, 1> : gemm_few_kernel<ARITH, BLOCK, 2>,
                                            dim3((a.b.rows + 31) / 32, one ? 1 : (a.a.rows + 31) / 32), dim3(512), 0, stream, a);
         return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
@@ -1358,6 +1363,7 @@ int launch_any_t(AnyArgs &a, hipStream_t stream) {
     const uint64_t tiles_m = ((uint64_t)a.a.rows + T - 1) / T, tiles_n = ((uint64_t)a.b.rows + T - 1) / T, tiles = tiles_m * tiles_n;
     if (tiles >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;    // grid limit
     a.map = make_tile_map((uint32_t)tiles_m, (uint32_t)tiles_n, 8);
+    g_ctx.last_any_kernel = T == 64 ? "tiles_64x64" : "tiles_128x128";
     constexpr int SUM = BLOCK ? ANY_SCALED : ANY_CHAIN;
     auto kernel = T == 64 ? (km ? gemm_any_kernel<DT, SUM, 64, true> : gemm_any_kernel<DT, SUM, 64, false>)
                           : (km ? gemm_any_kernel<DT, SUM, BLOCK ? 64 : W, true> : gemm_any_kernel<DT, SUM, W, false>);
@@ -1577,6 +1583,7 @@ QGEMM_EXPORT int qgemm_set_option(const char *key, long value) {
     else if (!std::strcmp(key, "k_rot")) g_ctx.k_rot = value;
     else if (!std::strcmp(key, "as_groups")) g_ctx.as_groups = value;
     else if (!std::strcmp(key, "small_tiles")) g_ctx.small_tiles = value;
+    else if (!std::strcmp(key, "few_rows")) g_ctx.few_rows = value;
     else if (!std::strcmp(key, "row_estimate")) g_ctx.row_estimate = value;
 #if QGEMM_DEBUG_BUILD
     else if (!std::strcmp(key, "dbg_ptr")) g_ctx.dbg_ptr = value;
@@ -1628,6 +1635,13 @@ QGEMM_EXPORT int qgemm_last_config(char *buf, size_t buflen) {
     if (!buf || buflen == 0) return QGEMM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lock(g_ctx.mu);
     std::snprintf(buf, buflen, "%s", g_ctx.last_config.c_str());
+    return QGEMM_OK;
+}
+
+QGEMM_EXPORT int qgemm_last_any_kernel(char *buf, size_t buflen) {
+    if (!buf || buflen == 0) return QGEMM_ERR_INVALID_ARG;
+    std::lock_guard<std::mutex> lock(g_ctx.mu);
+    std::snprintf(buf, buflen, "%s", g_ctx.last_any_kernel);
     return QGEMM_OK;
 }
 

@@ -52,6 +52,7 @@ SIGNATURES = {
     "qgemm_variant_count": (_i, [_i, _i, _i]),
     "qgemm_variant_name": (_i, [_i, _i, _i, _i, C.c_char_p, _sz]),
     "qgemm_last_config": (_i, [C.c_char_p, _sz]),
+    "qgemm_last_any_kernel": (_i, [C.c_char_p, _sz]),
     "qgemm_plan": (_i, [_i, _i, _i, _sz, _sz, _sz, C.c_char_p, _sz]),
     "qgemm_plan_out": (_i, [_i, _i, _i, _i, _sz, _sz, _sz, C.c_char_p, _sz]),
     "qgemm_selftest_layouts": (_i, [C.c_char_p, _sz]),

@@ -105,6 +105,13 @@ def last_config():
     return buf.value.decode()
 
 
+def last_any_kernel():
+    """Which kernel the last product with last_config() "strided_any_shape" ran."""
+    buf = C.create_string_buffer(64)
+    check(load_library().qgemm_last_any_kernel(buf, 64))
+    return buf.value.decode()
+
+
 def selftest_layouts():
     """-> (ok, report)"""
     buf = C.create_string_buffer(4096)

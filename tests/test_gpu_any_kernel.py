@@ -1,5 +1,6 @@
 """The any-shape kernel (option any_shape = 0) where its loads, tiles and steps end: K up to and around a 16-byte piece, a step
-and two steps, operands shorter than one piece, rows shorter than one, both tile sizes, rows of C with neighbours.  Small
+and two steps, operands shorter than one piece, rows shorter than one, both tile sizes, rows of C with neighbours; and the choice between
+the tiles and the kernel for few rows as it stands.  Small
 integers (and block scales that are powers of two) sum exactly, so the results equal the CPU oracle's."""
 import numpy as np
 import pytest
@@ -12,11 +13,13 @@ from tests.util import dev, say
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(autouse=True)
-def _any_shape_kernel():
+@pytest.fixture(autouse=True, params=[0, 1], ids=["tiles", "as_chosen"])
+def _any_shape_kernel(request):
     Q.set_option("any_shape", 0)
-    yield
+    Q.set_option("few_rows", request.param)
+    yield request.param
     Q.set_option("any_shape", 1)
+    Q.set_option("few_rows", 1)
 
 
 def _at_the_end(x, dtype):
@@ -39,22 +42,27 @@ SHAPES = [(1, 1, 1), (3, 5, 2), (2, 700, 7), (1, 15, 15), (40, 3, 16), (17, 9, 1
 @pytest.mark.parametrize("layout", ["nk", "kn"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.int8, torch.float8_e4m3fn])
 @pytest.mark.parametrize("shape", SHAPES)
-def test_products(shape, dtype, layout):
+def test_products(shape, dtype, layout, _any_shape_kernel):
     M, N, K = shape
+    if _any_shape_kernel and M > 128:
+        pytest.skip("tiles in either case")
     say("any-shape kernel", shape, dtype, layout)
     a, b = _operands(M, N, K)
     ref = torch.from_numpy(a.astype(np.float32)) @ torch.from_numpy(b.astype(np.float32)).t()
     c = torch.full((M, N + 3), 7.0, device="cuda")
     Q.gemm(_at_the_end(a, dtype), _at_the_end(b if layout == "nk" else np.ascontiguousarray(b.T), dtype), c[:, :N], layout)
     assert Q.last_config() == "strided_any_shape"
+    assert _any_shape_kernel or Q.last_any_kernel().startswith("tiles" if K >= 16 else ("tiles", "short"))
     assert torch.equal(c[:, :N].cpu(), ref)
     assert bool((c[:, N:] == 7).all())
 
 
 @pytest.mark.parametrize("dtype", [torch.int8, torch.float8_e4m3fn])
 @pytest.mark.parametrize("shape", [(1, 1, 3), (3, 300, 15), (70, 140, 63), (33, 257, 129), (65, 129, 193), (40, 70, 257), (2100, 2050, 191)])
-def test_block_scales(shape, dtype):
+def test_block_scales(shape, dtype, _any_shape_kernel):
     M, N, K = shape
+    if _any_shape_kernel and M > 128:
+        pytest.skip("tiles in either case")
     say("any-shape kernel, block scales", shape, dtype)
     a, b = _operands(M, N, K)
     KB, rng = (K + 127) // 128, np.random.default_rng(K)

@@ -16,8 +16,14 @@ TYPES = {"i8": torch.int8, "i8_block": torch.int8, "f8": torch.float8_e4m3fn, "f
 @pytest.fixture(autouse=True)
 def _reset_options():
     Q.set_option("any_shape", 0)
+    Q.set_option("few_rows", 2)
     yield
     Q.set_option("any_shape", 1)
+    Q.set_option("few_rows", 1)
+
+
+def _ran_for_few_rows(M):
+    return Q.last_config() == "strided_any_shape" and Q.last_any_kernel() == ("few_rows_16x32" if M <= 16 else "few_rows_32x32")
 
 
 def _operand(x, dt, shift):
@@ -56,10 +62,48 @@ def test_every_end_of_k(fam, M, N):
             one = dev(np.ones(1, np.float32))
             run = lambda: Q.scaled_gemm(qa, qb, one, one, c, M, N, K, Q.SCALE_PER_MATRIX)
         run()
-        assert Q.last_config() == "strided_any_shape", Q.last_config()
+        assert _ran_for_few_rows(M), (Q.last_config(), Q.last_any_kernel())
         want = torch.from_numpy(np.ascontiguousarray(ref, dtype=np.float32)).to(c.dtype if c.dtype != torch.int32 else torch.float32)
         got = c.cpu()
         assert torch.equal(got.to(want.dtype), want), (fam, M, N, K)
+
+
+@pytest.mark.parametrize("dt", [torch.int8, torch.float8_e4m3fn])
+@pytest.mark.parametrize("M,N,K", [(1, 33, 3000), (16, 100, 3001), (17, 200, 3199), (64, 31, 3333), (128, 140, 4097)])
+def test_block_scales_to_fp32(dt, M, N, K):
+    """From 3000 elements of K on (below, the tiles' sums are closer to 64 bits).  Products of small integers and powers of two within
+    2^24 units: every order of the sums gives the same fp32."""
+    say("few rows, block scales to fp32", dt, (M, N, K))
+    rng, kb = np.random.default_rng(K), (K + 127) // 128
+    a, b = rng.integers(-3, 4, size=(M, K)), rng.integers(-3, 4, size=(N, K))
+    as_, bs = ((2.0 ** rng.integers(-3, 4, size=(r, kb))).astype(np.float32) for r in (M, (N + 127) // 128))
+    c = torch.full((M, N), -7.0, device="cuda")
+    run = lambda: Q.scaled_gemm(_operand(a.astype(np.float32), dt, 3), _operand(b.astype(np.float32), dt, 1), dev(as_), dev(bs), c, M, N, K,  # noqa: E731
+                                Q.SCALE_BLOCK128)
+    run()
+    assert _ran_for_few_rows(M), Q.last_any_kernel()
+    scaled = lambda x, s: x * np.repeat(s.astype(np.float64), 128, 1)[:, :K]  # noqa: E731
+    want = torch.from_numpy((scaled(a, as_) @ scaled(b, np.repeat(bs, 128, 0)[:N]).T).astype(np.float32))
+    assert torch.equal(c.cpu(), want)
+    Q.set_option("few_rows", 0)
+    c.fill_(-7)
+    run()
+    assert Q.last_any_kernel().startswith("tiles") and torch.equal(c.cpu(), want)
+
+
+def test_where_it_does_not_run():
+    """Sums that the output would show to be less exact, more rows than 128, and B stored K x N, keep the tiles."""
+    def ran(M, N, K, dt, out, layout="nk"):
+        a, b = torch.ones(M, K, device="cuda").to(dt), torch.ones(*((N, K) if layout == "nk" else (K, N)), device="cuda").to(dt)
+        Q.gemm(a, b, torch.empty(M, N, dtype=out, device="cuda"), layout)
+        return Q.last_any_kernel()
+
+    bf16, fp32 = torch.bfloat16, torch.float32
+    assert ran(8, 40, 1001, bf16, bf16) == "few_rows_16x32" and ran(128, 40, 1001, bf16, bf16) == "few_rows_32x32"
+    assert ran(8, 40, 1001, bf16, fp32) == "tiles_64x64"
+    assert ran(129, 40, 1001, bf16, bf16) == "tiles_64x64"
+    assert ran(8, 41, 1001, bf16, bf16, "kn") == "tiles_64x64"
+    assert ran(8, 40, 7, bf16, bf16) == "short"
 
 
 def test_special_values_stay_in_their_rows():
@@ -74,6 +118,7 @@ def test_special_values_stay_in_their_rows():
     c = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
     g = torch.cuda.CUDAGraph()
     Q.gemm(qa, qb, c, "nk")
+    assert _ran_for_few_rows(M)
     torch.cuda.synchronize()
     with torch.cuda.graph(g):
         Q.gemm(qa, qb, c, "nk")
@@ -100,6 +145,7 @@ def test_more_columns_than_a_launch_has_threads_for():
     qb.view(N // lead, lead, K).copy_(dev(b).bfloat16())             # the same rows over and over
     c = torch.full((1, N), -7.0, dtype=torch.bfloat16, device="cuda")
     Q.gemm(dev(a).bfloat16(), qb, c, "nk")
+    assert Q.last_any_kernel() == "tiles_128x128"
     want = torch.from_numpy(R.gemm_f32acc(a, b)).bfloat16().cuda()
     assert torch.equal(c.view(N // lead, lead), want.expand(N // lead, lead))
     del qb, c
