@@ -261,8 +261,18 @@ gemm_skinny_kernel(QGEMM_HEAD, const GemmArgs p) {
     // A goes in front of B where the ring cannot take the round at once: the wait for it then does not include
     // the trip to HBM, and its slots turn over while B is still on its way.
     constexpr int SA = C::SA, SB = C::SB;
-    // (The scales of a round are requested behind its first copies, whose wait they share, and in front of the others.)
-    auto start_round = [&](int k, auto first_tag) {
+    // The scales of a round are requested behind its first copies, whose wait they share, and in front of the others; but EARLY, in
+    // front of all of them, on the tall 32-column tiles in every round but the first one of up to 36 K steps (which has
+    // to fetch arguments to locate them).  Their registers change hands at the end of the loop, where the compiler waits for as many
+    // copies as it can count behind them, and it cannot count B's, which stand behind branches: behind A0 that became a wait for
+    // B as well, and the rest of A was requested only then; in front of A0 it is the wait for A0 that comes next anyway.  64 x 32
+    // with block scales, time of this / of behind A0 in every round, 3700 shapes of 33 .. 64 rows x 4128 .. 8192 columns: 17 .. 22
+    // K steps 1.000, 23 .. 33 1.005, 34 .. 40 0.996, 41 .. 49 0.979, 50 .. 64 0.953 (42 x 6528 x 5936 17.9 -> 16.9 us); 128 x 32 0.95.
+    constexpr bool TALL = C::TM >= 4 && C::TN == 2;
+    typedef std::integral_constant<bool, true> yes;
+    typedef std::integral_constant<bool, false> no;
+    auto start_round = [&](int k, auto first_tag, auto early_tag) {
+        constexpr bool EARLY = decltype(early_tag)::value;
         auto scales = [&]() {
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (decltype(first_tag)::value) locate_scales();
@@ -281,14 +291,16 @@ gemm_skinny_kernel(QGEMM_HEAD, const GemmArgs p) {
             copy_a(k, 0, SA, 2 * SB);
             copy_a(k + C::NW, 0, SA, 2 * SB + SA);
         } else if constexpr (C::TM == 4) {
+            if constexpr (EARLY) scales();
             copy_a(k, 0, 8, 0);
-            scales();
+            if constexpr (!EARLY) scales();
             copy_b(k, 8);
             copy_b(k + C::NW, 12);
             copy_a(k + C::NW, 0, 4, 16);
         } else {
+            if constexpr (EARLY) scales();
             copy_a(k, 0, 12, 0);
-            scales();
+            if constexpr (!EARLY) scales();
             copy_b(k, 12);
             copy_b(k + C::NW, 16);
         }
@@ -356,11 +368,12 @@ gemm_skinny_kernel(QGEMM_HEAD, const GemmArgs p) {
             drain_a(1, 4, 4, 12);
         }
         drained();
-        if (next) start_round(k + 2 * C::NW, std::integral_constant<bool, false>{});
+        if (next) start_round(k + 2 * C::NW, no{}, std::integral_constant<bool, TALL>{});
         if (two) compute(1);
     };
     int k = wave;
-    start_round(k, std::integral_constant<bool, true>{});
+    if (C::BLOCK_SCALE && TALL && nk > 36) start_round(k, yes{}, std::integral_constant<bool, C::BLOCK_SCALE && TALL>{});
+    else start_round(k, yes{}, no{});
     QGEMM_STAMP(1);
     // (the scales of a matrix, fetched here: behind the barrier at the end they were a trip to memory of their own)
     float scale_a = 1.0f, scale_b = 1.0f;
