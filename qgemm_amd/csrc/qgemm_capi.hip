@@ -586,7 +586,11 @@ bool few_rows_doubtful(const FewRowsTile &rules, size_t rules_tiles, const FewRo
     const bool two_rounds = N > 32 * round;                  // of strips of 32 columns
     auto is = [](const FewRowsTile &x, int bm, int bn, int kgroups) { return x.bm == bm && x.bn == bn && x.kgroups == kgroups; };
     // 1.33, 0.89: strips of 64 columns, up to 64 rows, where 32-column strips need a second round (64 x 128 tiles with block scales 0.78)
-    if (M <= 64 && is(rules, 64, 64, 8)) return true;
+    // 1.11, 0.74: ... or with block scales 65 .. 128 rows from two such tiles of 64 rows to one of 128 x 32 (84 x 7632 x 6992 20.2 -> 30.7 us)
+    if (is(rules, 64, 64, 8) && (M <= 64 || is(t, 128, 32, 8))) return true;
+    // 1.10, 0.96: ... and 33 .. 64 rows from two K slices of 64 x 32 to two tiles of 32 rows over all of a K of 56 steps or more (39 x 4016 x
+    // 8112 13.2 -> 14.3 us; 48 .. 55 steps 1.08 ahead)
+    if (is(rules, 64, 32, 8) && is(t, 32, 32, 8) && rules_tiles < round && ksteps >= 56) return true;
     // 1.14, 0.77: 65 .. 128 rows x 11000 .. 16384 columns from 64 x 128 to one row of 128 x 128 tiles, two K groups each
     if (is(t, 128, 128, 2)) return true;
     // 1.18, 0.82: ... or to a second round of 64 x 64 tiles
