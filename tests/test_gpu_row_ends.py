@@ -17,7 +17,7 @@ def _reset_options():
     Q.set_option("any_shape", 1)
 
 
-@pytest.mark.parametrize("dt", [torch.int8, torch.bfloat16])
+@pytest.mark.parametrize("dt", [torch.int8, torch.bfloat16, torch.float32])
 def test_transpose_at_every_remainder(dt):
     rng = np.random.default_rng(3)
     for M in (1, 3, 8, 17, 130):
