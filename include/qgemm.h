@@ -124,7 +124,7 @@ int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int la
 
 /* Library workspace (no reference counterpart: the reference's entries take none).  Calls that split K, that
  * take operands or scales in an arrangement the kernels do not read directly, and the per-matrix quantiser (above
- * 256 KiB, where rows without gaps count as they are and others rounded up to 16 bytes each: 32768 x 1 with ld > 1 is 512 KiB) keep their intermediate data in one device block owned by the library and grown on demand.  A block that is
+ * 256 KiB, or, outside a capture and with gaps between the rows, which then count rounded up to 16 bytes each, above 128 KiB) keep their intermediate data in one device block owned by the library and grown on demand.  A block that is
  * outgrown is replaced but stays allocated until qgemm_shutdown, so launches already enqueued and graphs
  * already captured remain valid.  Calls on different streams share the block: each such call waits (on the
  * device, through an event) for the previous user on another stream.  While a stream is being captured into a

@@ -1466,8 +1466,12 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         }
         number((a.cols + P::VEC - 1) / P::VEC);
         const uint64_t pieces = (uint64_t)a.rows * a.per_row;
-        if (pieces * 16 <= kQuantSmallBytes) {
-            e = launch_kernel(a.rows == 1 ? quant_small_matrix_kernel<IN_DT, OUT_DT, true> : quant_small_matrix_kernel<IN_DT, OUT_DT, false>,
+        // (an empty matrix is for the forms that look whether a row has a piece: the others load without asking)
+        const bool row_ends = a.cols == 0 || a.cols % P::VEC != 0, one_row = a.rows == 1;
+        auto form = [&](auto one_ragged, auto one, auto rows_ragged, auto rows) { return one_row ? (row_ends ? one_ragged : one) : row_ends ? rows_ragged : rows; };
+        if (pieces * 16 <= kQuantSmallBytes && (one_row || pieces * 16 <= kQuantSmallRowsBytes || stream_is_capturing(stream))) {
+            e = launch_kernel(form(quant_small_matrix_kernel<IN_DT, OUT_DT, true, true>, quant_small_matrix_kernel<IN_DT, OUT_DT, true, false>,
+                                   quant_small_matrix_kernel<IN_DT, OUT_DT, false, true>, quant_small_matrix_kernel<IN_DT, OUT_DT, false, false>),
                               dim3((unsigned)std::max<uint64_t>(1, (pieces + 1023) / 1024)), dim3(1024), 0, stream, a);
             return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
         }
@@ -1480,10 +1484,12 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         int st = ensure_workspace_locked((size_t)a.npartial * sizeof(uint32_t), stream, &ws);
         if (st != QGEMM_OK) return st;
         a.partial = (uint32_t *)ws;
-        e = launch_kernel(a.rows == 1 ? quant_amax_kernel<IN_DT, true> : quant_amax_kernel<IN_DT, false>, dim3(nblk, slices), dim3(256), 0, stream, a);
+        e = launch_kernel(form(quant_amax_kernel<IN_DT, true, true>, quant_amax_kernel<IN_DT, true, false>,
+                               quant_amax_kernel<IN_DT, false, true>, quant_amax_kernel<IN_DT, false, false>), dim3(nblk, slices), dim3(256), 0, stream, a);
         if (e != hipSuccess) return QGEMM_ERR_LAUNCH;
         const uint32_t nq = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(2048, turns));
-        e = launch_kernel(a.rows == 1 ? quant_matrix_kernel<IN_DT, OUT_DT, true> : quant_matrix_kernel<IN_DT, OUT_DT, false>, dim3(nq, slices), dim3(256), 0, stream, a);
+        e = launch_kernel(form(quant_matrix_kernel<IN_DT, OUT_DT, true, true>, quant_matrix_kernel<IN_DT, OUT_DT, true, false>,
+                               quant_matrix_kernel<IN_DT, OUT_DT, false, true>, quant_matrix_kernel<IN_DT, OUT_DT, false, false>), dim3(nq, slices), dim3(256), 0, stream, a);
     } else if (mode == QGEMM_QUANT_BLOCK_1x128) {
         number((a.cols + 127) / 128);
         const RowBlockGrid g = row_block_grid(a.rows, a.per_row, 256 / P::LANES);

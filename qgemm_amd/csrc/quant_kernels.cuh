@@ -286,67 +286,93 @@ constexpr uint32_t kQuantNan = 0x80000000u;
 constexpr int kQuantTurn = 4;                    // pieces a lane has in flight (per-matrix passes)
 
 // ---- per matrix.  The host hands over a matrix without gaps as a single row (QuantArgs::per_row pieces), which saves the
-// divisions and all row ends but one.
+// divisions and all row ends but one.  RAGGED: rows may end inside a piece; where they do not, nothing has to be settled, and a single
+// row's maximum is that of its whole pieces and of its last one (start to now, us, graph replays: 500 x 7200 bf16 with gaps 7.6 -> 6.8,
+// 1435 x 3368 fp32 with gaps 11.7 -> 10.5, 64 x 2048 6.1 -> 4.9, 41 x 1001 5.1 -> 4.8).
 // Where piece i of `total` lies, loads and stores of it
-template <int IN_DT, bool ONE_ROW>
+template <int IN_DT, bool ONE_ROW, bool RAGGED>
 struct MatrixPieces {
     typedef Piece<IN_DT> P;
+    struct Place {
+        uint32_t r, c, valid;        // row, element of it, elements that the row has from there on (0: past the last piece)
+    };
     const QuantArgs &p;
     uint32_t row0, total;
     bool wide;
     __device__ MatrixPieces(const QuantArgs &a, uint32_t slice) : p(a) {
         row0 = slice * a.rows_per_slice;
         total = (a.rows - row0 < a.rows_per_slice ? a.rows - row0 : a.rows_per_slice) * a.per_row;
-        wide = a.cols >= (uint32_t)P::VEC;
+        wide = !RAGGED || a.cols >= (uint32_t)P::VEC;
     }
-    // element c of its row
-    __device__ void at(uint32_t i, size_t &r, uint32_t &c) const {
-        r = 0;
-        c = i;
-        if constexpr (!ONE_ROW) r = row0 + div_by_inv(i, p.per_row, p.inv, c);
-        c *= P::VEC;
+    // the whole pieces of a single row that ends inside one
+    __device__ explicit MatrixPieces(const MatrixPieces<IN_DT, ONE_ROW, true> &o) : p(o.p), row0(0), total(o.total - 1), wide(true) {}
+    __device__ Place place(uint32_t i) const {
+        const bool in = i < total;
+        Place o;
+        o.r = 0;
+        o.c = in ? i : 0;
+        if constexpr (!ONE_ROW) o.r = row0 + div_by_inv(o.c, p.per_row, p.inv, o.c);
+        o.c *= P::VEC;
+        o.valid = in ? p.cols - o.c : 0;
+        return o;
     }
-    // N pieces, `stride` apart: requested together, zeros past the end
-    template <int N>
-    __device__ void load(v4i (&v)[N], uint32_t first, uint32_t stride) const {
-        uint32_t valid[N];
-        size_t idx[N];
+    // as they come from memory, requested together; `settle` leaves zeros past the end  (WIDE: known to be `wide`)
+    template <int N, bool WIDE = false>
+    __device__ void request(v4i (&v)[N], const Place (&at)[N]) const {
+        auto idx = [&](int j) { return ONE_ROW ? (size_t)at[j].c : at[j].r * p.ld + at[j].c; };
+        if (WIDE || wide) {
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-            const uint32_t i = first + j * stride;
-            size_t r;
-            uint32_t c;
-            at(i < total ? i : 0, r, c);
-            idx[j] = ONE_ROW ? c : r * p.ld + c;
-            valid[j] = i < total ? p.cols - c : 0;
-        }
-        if (wide) {
-#pragma unroll
-            for (int j = 0; j < N; ++j) v[j] = P::load_whole(p.x, idx[j], valid[j]);
-#pragma unroll
-            for (int j = 0; j < N; ++j)
-                if (!valid[j]) v[j] = v4i{0, 0, 0, 0};
-#pragma unroll
-            for (int j = 0; j < N; ++j) P::settle(v[j], valid[j]);
+            for (int j = 0; j < N; ++j) v[j] = P::template load<RAGGED>(p.x, idx(j), at[j].valid, true);
         } else {
 #pragma unroll
-            for (int j = 0; j < N; ++j) v[j] = valid[j] ? P::load_elements(p.x, idx[j], valid[j]) : v4i{0, 0, 0, 0};
+            for (int j = 0; j < N; ++j) v[j] = at[j].valid ? P::load_elements(p.x, idx(j), at[j].valid) : v4i{0, 0, 0, 0};
         }
     }
-    __device__ void store(uint32_t i, v2i w) const {
-        if (i >= total) return;
-        size_t r;
-        uint32_t c;
-        at(i, r, c);
-        store_piece<IN_DT>(p.q, r * p.ldq + c, w, p.cols - c);
+    template <int N, bool WIDE = false>
+    __device__ void settle(v4i (&v)[N], const Place (&at)[N]) const {
+        if (!WIDE && !wide) return;
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (!at[j].valid) v[j] = v4i{0, 0, 0, 0};
+        if constexpr (RAGGED) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) P::settle(v[j], at[j].valid);
+        }
+    }
+    // both, for N pieces, `stride` apart
+    template <int N>
+    __device__ void load(v4i (&v)[N], Place (&at)[N], uint32_t first, uint32_t stride) const {
+#pragma unroll
+        for (int j = 0; j < N; ++j) at[j] = place(first + j * stride);
+        if (wide) {
+            request<N, true>(v, at);
+            settle<N, true>(v, at);
+        } else {
+            request<N>(v, at);
+        }
+    }
+    __device__ void store(const Place &at, v2i w) const {
+        if (at.valid) store_piece<IN_DT>(p.q, at.r * p.ldq + at.c, w, RAGGED ? at.valid : P::VEC);
     }
     // bits of the largest |x| that is a number, bit 31 set where there is something else, of N pieces, `stride` apart, from
-    // `first` on, N from first + `turn` on, ...
+    // `first` on, N from first + `turn` on, ...; a single row's last piece, if it is cut short, where `last` says so
     template <int N>
-    __device__ uint32_t maximum(uint32_t first, uint32_t stride, uint32_t turn) const {
+    __device__ uint32_t maximum(uint32_t first, uint32_t stride, uint32_t turn, bool last) const {
+        if constexpr (ONE_ROW && RAGGED) {
+            v4i end[1];
+            const Place at[1] = {place(last ? total - 1 : total)};
+            request<1>(end, at);
+            const uint32_t m = MatrixPieces<IN_DT, true, false>(*this).template maximum<N>(first, stride, turn, false);
+            settle<1>(end, at);
+            uint32_t b = P::max_bits(end[0]);
+            if (b > P::INF) b = P::max_bits_of_numbers(end[0]) | kQuantNan;
+            const uint32_t v = m & ~kQuantNan, w = b & ~kQuantNan;
+            return (v > w ? v : w) | ((m | b) & kQuantNan);
+        }
         v4i acc = v4i{0, 0, 0, 0}, v[N];
+        Place at[N];
         for (uint32_t i = first; i < total; i += turn) {
-            load<N>(v, i, stride);
+            load<N>(v, at, i, stride);
 #pragma unroll
             for (int j = 0; j < N; ++j) P::fold_max(acc, v[j]);
         }
@@ -356,7 +382,8 @@ struct MatrixPieces {
         for (uint32_t i = first; i < total; i += turn)
             for (int j = 0; j < N; ++j) {
                 v4i one[1];
-                load<1>(one, i + j * stride, 0);
+                Place there[1];
+                load<1>(one, there, i + j * stride, 0);
                 const uint32_t b = P::max_bits_of_numbers(one[0]);
                 m = b > m ? b : m;
             }
@@ -380,33 +407,39 @@ __device__ inline Divisor matrix_divisor(uint32_t m) {
 }
 
 // Small: one launch, no workspace.  Every workgroup takes the maximum of the whole matrix, then quantises its own 1024 pieces.
-// A workgroup reads some 100 GB/s, so this ends where that takes as long as a second launch: against the two passes below, us,
-// graph replays, bf16 16 x 2048 (64 KiB) 4.8 / 6.5, 64 x 2048 (256 KiB) 6.1 / 6.5, 64 x 3000 (375 KiB) 7.6 / 6.6.
-constexpr uint64_t kQuantSmallBytes = 256 << 10;
-template <int IN_DT, int OUT_DT, bool ONE_ROW>
+// A workgroup reads some 100 GB/s, so this ends where that takes as long as a second launch, or, with gaps between the rows and a
+// division for every piece, at half of that (kQuantSmallRowsBytes; a stream that is being captured, which has only the workspace that is
+// there, stays on one launch up to kQuantSmallBytes).  Against the two passes below, us, graph replays, bf16: 16 x 2048 (64 KiB) 3.6 / 4.7,
+// 48 x 2048 (192 KiB) 4.9 / 5.1, 64 x 2048 4.9 / 5.1; gaps: 64 x 512 (64 KiB) 4.3 / 4.8, 64 x 1024 4.4 / 5.2, 40 x 2176 (170 KiB) 7.6 / 5.2
+// (with the pieces of rows without ends as pieces of rows with them 7.6 / 6.3).
+constexpr uint64_t kQuantSmallBytes = 256 << 10, kQuantSmallRowsBytes = 128 << 10;
+template <int IN_DT, int OUT_DT, bool ONE_ROW, bool RAGGED>
 __global__ void __launch_bounds__(1024) quant_small_matrix_kernel(const QuantArgs p) {
-    const MatrixPieces<IN_DT, ONE_ROW> x(p, 0);
+    const MatrixPieces<IN_DT, ONE_ROW, RAGGED> x(p, 0);
     const uint32_t mine = blockIdx.x * 1024 + threadIdx.x;
     v4i own[1];
-    x.template load<1>(own, mine, 1);
-    const Divisor dv = matrix_divisor<IN_DT, OUT_DT>(workgroup_maximum<16>(x.template maximum<8>(threadIdx.x, 1024, 8 * 1024)));
+    typename MatrixPieces<IN_DT, ONE_ROW, RAGGED>::Place at[1] = {x.place(mine)};
+    x.template request<1>(own, at);                  // (settled behind the maximum: here it would wait for the piece in front of all others)
+    const Divisor dv = matrix_divisor<IN_DT, OUT_DT>(workgroup_maximum<16>(x.template maximum<8>(threadIdx.x, 1024, 8 * 1024, threadIdx.x == 0)));
+    x.template settle<1>(own, at);
     if (mine == 0) p.scales[0] = dv.s;
-    x.store(mine, quant_piece<IN_DT, OUT_DT>(own[0], dv));
+    x.store(at[0], quant_piece<IN_DT, OUT_DT>(own[0], dv));
 }
 
 // pass 1: one partial maximum per workgroup
-template <int IN_DT, bool ONE_ROW>
+template <int IN_DT, bool ONE_ROW, bool RAGGED>
 __global__ void __launch_bounds__(256) quant_amax_kernel(const QuantArgs p) {
-    const MatrixPieces<IN_DT, ONE_ROW> x(p, blockIdx.y);
-    const uint32_t m = workgroup_maximum<4>(x.template maximum<kQuantTurn>(blockIdx.x * 256 * kQuantTurn + threadIdx.x, 256, gridDim.x * 256 * kQuantTurn));
+    const MatrixPieces<IN_DT, ONE_ROW, RAGGED> x(p, blockIdx.y);
+    const uint32_t m = workgroup_maximum<4>(x.template maximum<kQuantTurn>(blockIdx.x * 256 * kQuantTurn + threadIdx.x, 256, gridDim.x * 256 * kQuantTurn,
+                                                                                 blockIdx.x == 0 && threadIdx.x == 0));
     if (threadIdx.x == 0) p.partial[blockIdx.y * gridDim.x + blockIdx.x] = m;
 }
 
 // pass 2: every workgroup reduces the partial maxima again (a few KB, L2 resident), then
 // quantises its share; workgroup 0 writes the scale
-template <int IN_DT, int OUT_DT, bool ONE_ROW>
+template <int IN_DT, int OUT_DT, bool ONE_ROW, bool RAGGED>
 __global__ void __launch_bounds__(256) quant_matrix_kernel(const QuantArgs p) {
-    const MatrixPieces<IN_DT, ONE_ROW> x(p, blockIdx.y);
+    const MatrixPieces<IN_DT, ONE_ROW, RAGGED> x(p, blockIdx.y);
     uint32_t m = 0, nan = 0;
     for (uint32_t i = threadIdx.x; i < p.npartial; i += 256) {
         const uint32_t b = p.partial[i];
@@ -417,9 +450,10 @@ __global__ void __launch_bounds__(256) quant_matrix_kernel(const QuantArgs p) {
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.scales[0] = dv.s;
     for (uint32_t first = blockIdx.x * 256 * kQuantTurn; first < x.total; first += gridDim.x * 256 * kQuantTurn) {
         v4i v[kQuantTurn];
-        x.template load<kQuantTurn>(v, first + threadIdx.x, 256);
+        typename MatrixPieces<IN_DT, ONE_ROW, RAGGED>::Place at[kQuantTurn];
+        x.template load<kQuantTurn>(v, at, first + threadIdx.x, 256);
 #pragma unroll
-        for (int j = 0; j < kQuantTurn; ++j) x.store(first + threadIdx.x + j * 256, quant_piece<IN_DT, OUT_DT>(v[j], dv));
+        for (int j = 0; j < kQuantTurn; ++j) x.store(at[j], quant_piece<IN_DT, OUT_DT>(v[j], dv));
     }
 }
 

@@ -38,9 +38,9 @@ def _strided(x, gap):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (3, 7), (129, 5), (2, 8), (16, 2045), (64, 2048), (64, 2049), (33, 1985), (260, 1027), (70, 4100), (16384, 1), (16385, 1)])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (3, 7), (129, 5), (2, 8), (16, 2045), (64, 2048), (64, 2049), (33, 1985), (260, 1027), (70, 4100), (16384, 1), (16385, 1), (8192, 8), (8193, 8), (8193, 9), (40, 2176)])
 def test_every_mode_at_row_ends_and_either_side_of_the_small_matrix(rows, cols, dt):
-    """64 x 2048 16-bit elements are the last small matrix, and 16384 rows of less than a piece where there is a gap between them; rows that end 1 .. 7 elements into a piece, shorter than one, with and
+    """64 x 2048 16-bit elements are the last small matrix, and 16384 rows of a piece or less in a capture (8192 outside one) where there is a gap between them; rows that end 1 .. 7 elements into a piece, shorter than one, with and
     without a gap between them; the largest element last."""
     say("quantize sizes", rows, cols, dt)
     x, xf = _input(rows, cols, dt, 33)
@@ -57,13 +57,34 @@ def test_every_mode_at_row_ends_and_either_side_of_the_small_matrix(rows, cols, 
                 assert np.array_equal(host(gs), s) and np.array_equal(_u8(g), q.view(np.uint8)), (rows, cols, qt, mode)
 
 
-@pytest.mark.parametrize("rows,cols", [(9, 517), (300, 1031)])
+def test_rows_with_gaps_in_a_capture():
+    """Between 128 and 256 KiB: two passes and the workspace outside a capture, one launch without it inside."""
+    x, xf = _input(10000, 8, torch.bfloat16, 37)
+    t = _strided(x, 3)
+    ref_q, ref_s = R.quantize_int8(xf)
+    for eager in (True, False):
+        say("quantize with gaps", "eager" if eager else "captured")
+        if eager:
+            g, gs = Q.quantize(t, torch.int8, Q.QUANT_PER_MATRIX)
+        else:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                g, gs = Q.quantize(t, torch.int8, Q.QUANT_PER_MATRIX)
+        for _ in range(1 if eager else 3):
+            if not eager:
+                g.zero_()
+                gs.zero_()
+                graph.replay()
+            assert host(gs)[0] == ref_s and np.array_equal(_u8(g), ref_q.view(np.uint8))
+
+
+@pytest.mark.parametrize("rows,cols", [(9, 517), (300, 1031), (3, 20), (40, 1024), (1, 5)])
 @pytest.mark.parametrize("special", [float("nan"), float("inf"), -float("inf")])
 def test_special_values_wherever_they_stand(rows, cols, special):
     """One NaN or infinity, in the last piece of a row and in the middle of one: the maximum is that of the numbers (infinity
     counts as one), every other element keeps its bytes, for the single launch as for the two passes."""
     x, _ = _input(rows, cols, torch.bfloat16, 35)
-    for at in ((rows - 1, cols - 1), (rows // 2, 128), (0, 3)):
+    for at in ((rows - 1, cols - 1), (rows // 2, min(128, cols - 1)), (0, 3)):
         say("quantize special", rows, cols, special, at)
         y = x.clone()
         y[at] = special
