@@ -1503,7 +1503,10 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
     } else {
         const uint64_t nblocks = (uint64_t)((a.rows + 127) / 128) * ((a.cols + 127) / 128);
         if (nblocks >= ((uint64_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
-        e = launch_kernel(ragged ? quant_square_block_kernel<IN_DT, OUT_DT, true> : quant_square_block_kernel<IN_DT, OUT_DT, false>, dim3((unsigned)nblocks), dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
+        if (a.rows <= kQuantFewRows)
+            e = launch_kernel(ragged ? quant_low_block_kernel<IN_DT, OUT_DT, true> : quant_low_block_kernel<IN_DT, OUT_DT, false>, dim3((unsigned)nblocks), dim3(256), 0, stream, a);
+        else
+            e = launch_kernel(ragged ? quant_square_block_kernel<IN_DT, OUT_DT, true> : quant_square_block_kernel<IN_DT, OUT_DT, false>, dim3((unsigned)nblocks), dim3(256), 0, stream, QGEMM_QUANT_HEAD_OF(a));
     }
     return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
 }

@@ -38,9 +38,9 @@ def _strided(x, gap):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (3, 7), (129, 5), (2, 8), (16, 2045), (64, 2048), (64, 2049), (33, 1985), (260, 1027), (70, 4100), (16384, 1), (16385, 1), (8192, 8), (8193, 8), (8193, 9), (40, 2176)])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (3, 7), (129, 5), (2, 8), (16, 2045), (64, 2048), (64, 2049), (33, 1985), (260, 1027), (70, 4100), (16384, 1), (16385, 1), (32, 300), (33, 300), (8192, 8), (8193, 8), (8193, 9), (40, 2176)])
 def test_every_mode_at_row_ends_and_either_side_of_the_small_matrix(rows, cols, dt):
-    """64 x 2048 16-bit elements are the last small matrix, and 16384 rows of a piece or less in a capture (8192 outside one) where there is a gap between them; rows that end 1 .. 7 elements into a piece, shorter than one, with and
+    """64 x 2048 16-bit elements are the last small matrix, and 16384 rows of a piece or less in a capture (8192 outside one) where there is a gap between them, 32 rows the last low block; rows that end 1 .. 7 elements into a piece, shorter than one, with and
     without a gap between them; the largest element last."""
     say("quantize sizes", rows, cols, dt)
     x, xf = _input(rows, cols, dt, 33)
