@@ -359,11 +359,11 @@ struct MatrixPieces {
     template <int N>
     __device__ uint32_t maximum(uint32_t first, uint32_t stride, uint32_t turn, bool last) const {
         if constexpr (ONE_ROW && RAGGED) {
-            v4i end[1];
-            const Place at[1] = {place(last ? total - 1 : total)};
-            request<1>(end, at);
+            v4i end[1] = {v4i{0, 0, 0, 0}};
+            const Place at[1] = {place(total - 1)};
+            if (last) request<1>(end, at);
             const uint32_t m = MatrixPieces<IN_DT, true, false>(*this).template maximum<N>(first, stride, turn, false);
-            settle<1>(end, at);
+            if (last) settle<1>(end, at);
             uint32_t b = P::max_bits(end[0]);
             if (b > P::INF) b = P::max_bits_of_numbers(end[0]) | kQuantNan;
             const uint32_t v = m & ~kQuantNan, w = b & ~kQuantNan;
@@ -448,12 +448,26 @@ __global__ void __launch_bounds__(256) quant_matrix_kernel(const QuantArgs p) {
     }
     const Divisor dv = matrix_divisor<IN_DT, OUT_DT>(workgroup_maximum<4>(m | nan));
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.scales[0] = dv.s;
-    for (uint32_t first = blockIdx.x * 256 * kQuantTurn; first < x.total; first += gridDim.x * 256 * kQuantTurn) {
-        v4i v[kQuantTurn];
-        typename MatrixPieces<IN_DT, ONE_ROW, RAGGED>::Place at[kQuantTurn];
-        x.template load<kQuantTurn>(v, at, first + threadIdx.x, 256);
+    auto quantise = [&](const auto &pieces) {
+        for (uint32_t first = blockIdx.x * 256 * kQuantTurn; first < pieces.total; first += gridDim.x * 256 * kQuantTurn) {
+            v4i v[kQuantTurn];
+            typename std::decay_t<decltype(pieces)>::Place at[kQuantTurn];
+            pieces.template load<kQuantTurn>(v, at, first + threadIdx.x, 256);
 #pragma unroll
-        for (int j = 0; j < kQuantTurn; ++j) x.store(at[j], quant_piece<IN_DT, OUT_DT>(v[j], dv));
+            for (int j = 0; j < kQuantTurn; ++j) pieces.store(at[j], quant_piece<IN_DT, OUT_DT>(v[j], dv));
+        }
+    };
+    if constexpr (ONE_ROW && RAGGED) {               // as in `maximum`
+        const bool last = blockIdx.x == 0 && threadIdx.x == 0;
+        v4i end[1];
+        const typename MatrixPieces<IN_DT, ONE_ROW, RAGGED>::Place at[1] = {x.place(x.total - 1)};
+        if (last) x.template request<1>(end, at);
+        quantise(MatrixPieces<IN_DT, true, false>(x));
+        if (!last) return;
+        x.template settle<1>(end, at);
+        x.store(at[0], quant_piece<IN_DT, OUT_DT>(end[0], dv));
+    } else {
+        quantise(x);
     }
 }
 
