@@ -577,7 +577,8 @@ inline double few_rows_least(const FewRowsTile &t, size_t N, uint32_t ksteps, bo
 }
 
 // Changes of row that the estimate gets wrong, by the tile of the rules and the one it puts ahead: both timed on 5700 shapes (1 .. 400 rows
-// x 256 .. 100 000 columns x 512 .. 8192; fp8, int8, bf16 and the two with block scales), geometric mean of weights streamed and resident.
+// x 256 .. 100 000 columns x 512 .. 8192; fp8, int8, bf16 and the two with block scales), geometric mean of weights streamed and resident,
+// and on 2500 of 17 .. 128 rows x 3000 .. 16384 x 4096 .. 8192 with block scales.
 // At each, the gain that the estimate promises and what was measured.  Of the other 5250 changes ten are more than 5 % behind
 // the rules, at worst 18 %; together they gain 26 %.
 bool few_rows_doubtful(const FewRowsTile &rules, size_t rules_tiles, const FewRowsTile &t, size_t tiles, size_t M, size_t N, uint32_t ksteps,

@@ -14,8 +14,8 @@
 //   * plain form (a finite maximum: no element is NaN or infinite, no quotient exceeds the type's largest value): the
 //     quotient of |x| without special cases, the sign moved over afterwards; anything else takes the careful form.
 // Before and now, us (to fp8 unless said): 1 x 128 6144 x 7168 bf16 45.7 -> 25.7 (5.1 TB/s, what a copy reaches), 500 x 7200
-// 7.3 -> 4.5; 128 x 128 7168 x 6144 fp32 43.4 -> 39.6 (5.6 TB/s); per matrix 1531 x 3004 bf16 to int8 4.9 + 8.5 -> 4.2 + 4.6
-// (a trace's times of the two passes).  A decoder's one row of 2048 1.98 -> 1.85: one trip to memory and back.
+// 7.3 -> 4.5; 128 x 128 7168 x 6144 fp32 43.4 -> 39.6 (5.6 TB/s); per matrix 1531 x 3004 bf16 to int8 4.9 + 8.5 -> 4.0 + 5.5
+// (a trace's times of the two passes; as a graph 11.3 -> 8.5).  A decoder's one row of 2048 1.98 -> 1.85: one trip to memory and back.
 #pragma once
 #include "common.h"
 
