@@ -124,15 +124,17 @@ int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int la
 
 /* Library workspace (no reference counterpart: the reference's entries take none).  Calls that split K, that
  * take operands or scales in an arrangement the kernels do not read directly, and the per-matrix quantiser (above
- * 256 KiB, or, outside a capture and with gaps between the rows, which then count rounded up to 16 bytes each, above 128 KiB) keep their intermediate data in one device block owned by the library and grown on demand.  A block that is
+ * 256 KiB, or, outside a capture and with gaps between the rows, which then count rounded up to 16 bytes each, above 128 KiB)
+ * keep their intermediate data in device blocks owned by the library and grown on demand.  A block that is
  * outgrown is replaced but stays allocated until qgemm_shutdown, so launches already enqueued and graphs
- * already captured remain valid.  Calls on different streams share the block: each such call waits (on the
- * device, through an event) for the previous user on another stream.  While a stream is being captured into a
- * graph the library neither allocates nor touches that event: a call that would have to grow the block returns
+ * already captured remain valid.  The first three streams that need one have a block each; calls on further streams share
+ * a fourth, and each such call waits (on the device, through an event) for the previous user on another stream.  While a
+ * stream is being captured into a graph the library neither allocates nor touches that event: such a call uses the largest
+ * block there is, one that would need more returns
  * QGEMM_ERR_ALLOC, and replays of graphs that use the workspace must not overlap other users of it.  (Products whose
  * operands would be packed into the block, see option "any_shape", do not use it while captured: they run the any-shape
  * kernel, whose fp32 sums have another order than those of an eager call.)
- * qgemm_reserve_workspace makes the block at least `bytes` large ahead of time (it allocates: call it before a
+ * qgemm_reserve_workspace makes the largest block at least `bytes` large ahead of time (it allocates: call it before a
  * capture begins, never during one; a block that has to grow at least doubles); qgemm_workspace_info reports
  * its address and size (NULL / 0 before first use). */
 int qgemm_reserve_workspace(size_t bytes);

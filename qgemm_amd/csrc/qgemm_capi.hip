@@ -37,23 +37,31 @@ struct WsBlock {
     void *p = nullptr;
     size_t bytes = 0;
 };
+constexpr int kOwnBlocks = 3;
 
 struct Context {
     std::mutex mu;
     bool ready = false;
     int device = -1;
     int num_cus = 256;
-    // Workspace (split-K partial planes, transposed operands and scales, quantiser partials): one block for
-    // the process.  A block that is outgrown is replaced and kept in `retired` until qgemm_shutdown: launches
-    // already enqueued and graphs already captured keep pointing at live memory.  Calls on different streams
-    // share the block and are ordered through ws_event: every call that used the workspace records it on its
-    // stream when it has enqueued its launches, and a call on another stream waits for it first.
-    WsBlock ws;
+    // Workspace (split-K partial planes, transposed and packed operands and scales, quantiser partials).  The first kOwnBlocks
+    // streams that use it have a block each, in which their calls follow one another as the stream has them; the streams beyond
+    // those (and hipStreamPerThread, one handle for many streams) share one more, ordered through ws_event: every call that
+    // used it records the event on its stream when it has enqueued its launches, and a call on another stream waits for it first.
+    // (Recording costs a call 4.3 - 5.4 us of host time, twice a launch, and the GPU a packet that the next launch waits for.  With
+    // one block for all streams every call that used the workspace paid that, eager calls, us: quantise 50 x 5296 fp16 to int8 per
+    // matrix 11.1 -> 8.0, quantise and multiply 1531 x 4100 x 3004 42.5 -> 36.2, forward and backward 505 x 531 x 1059 43.1 -> 37.0.)
+    // A block that is outgrown is replaced and kept in `retired` until qgemm_shutdown: launches
+    // already enqueued and graphs already captured keep pointing at live memory.
+    WsBlock ws[kOwnBlocks + 1];                // the last one is shared
+    hipStream_t ws_stream[kOwnBlocks] = {};    // whose the others are
+    int ws_owners = 0;
+    bool ws_all_share = false;                 // no memory for another block: every stream on the shared one from then on
     std::vector<void *> retired;
     hipEvent_t ws_event = nullptr;
     hipStream_t ws_last_stream = nullptr;
     bool ws_event_recorded = false;
-    bool ws_used_by_call = false;              // the running entry asked for the workspace
+    bool ws_shared_by_call = false;            // the running entry asked for the shared block
     bool static_call = false;                  // the running entry takes its workspace from the static scratch
     void *static_ptr[kMaxDevices] = {};        // device address of `scratch`, per device
     std::string force_config;   // name of a row of the variant tables, empty = heuristic (qgemm_force_config)
@@ -139,48 +147,88 @@ bool stream_is_capturing(hipStream_t stream) {
     return cap != hipStreamCaptureStatusNone;
 }
 
+// The largest block: what qgemm_reserve_workspace and qgemm_workspace_info speak of, and captured calls use
+WsBlock &largest_block() {
+    WsBlock *most = &g_ctx.ws[0];
+    for (WsBlock &b : g_ctx.ws)
+        if (b.bytes > most->bytes) most = &b;
+    return *most;
+}
+
+// Makes a block at least `bytes` large, twice its size if it has to grow; the old memory is retired (see Context).
+int grow_block(WsBlock &block, size_t bytes, size_t least) {
+    if (bytes <= block.bytes) return QGEMM_OK;
+    const size_t want = std::max({bytes, 2 * block.bytes, least});
+    // (another thread may be capturing a stream of its own: this allocation is none of its business)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    void *p = nullptr;
+    const hipError_t e = hipMalloc(&p, want);
+    if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return QGEMM_ERR_ALLOC;
+    }
+    if (block.p) g_ctx.retired.push_back(block.p);
+    block.p = p;
+    block.bytes = want;
+    return QGEMM_OK;
+}
+
+// Which block a stream uses: its own where it has one or there is one left, otherwise the shared one
+int block_of(hipStream_t stream) {
+    if (g_ctx.ws_all_share || stream == hipStreamPerThread) return kOwnBlocks;
+    for (int i = 0; i < g_ctx.ws_owners; ++i)
+        if (g_ctx.ws_stream[i] == stream) return i;
+    if (g_ctx.ws_owners == kOwnBlocks) return kOwnBlocks;
+    g_ctx.ws_stream[g_ctx.ws_owners] = stream;
+    return g_ctx.ws_owners++;
+}
+
 // Workspace of `bytes` for a call enqueued on `stream`.
 //   * qgemm_scaled_gemm_static: the static scratch; larger requests are an error, nothing is allocated.
-//   * otherwise the library's block, grown when too small.  Growing allocates a new block and retires the old
-//     one without freeing it (see Context).  While the stream is being captured into a graph nothing is
-//     allocated and no event is waited for or recorded: a call that would have to grow the block fails with
-//     QGEMM_ERR_ALLOC (the caller reserves the room before the capture, qgemm_reserve_workspace, or runs the
+//   * otherwise the stream's block (see Context), grown when too small.  While the stream is being captured into a graph nothing is
+//     allocated and no event is waited for or recorded: such a call takes the largest block there is, one that would need more
+//     fails with QGEMM_ERR_ALLOC (the caller reserves the room before the capture, qgemm_reserve_workspace, or runs the
 //     call once eagerly), and ordering replays against other users of the workspace is the caller's business.
 int ensure_workspace_locked(size_t bytes, hipStream_t stream, void **out) {
     if (g_ctx.static_call) {
         if (bytes > kStaticScratchBytes) return QGEMM_ERR_SCRATCH_TOO_SMALL;
         return static_scratch_locked(out);
     }
-    const bool capturing = stream_is_capturing(stream);
-    if (bytes > g_ctx.ws.bytes) {
-        if (capturing) return QGEMM_ERR_ALLOC;
-        const size_t want = std::max({bytes, 2 * g_ctx.ws.bytes, (size_t)64 << 20});
-        void *p = nullptr;
-        if (hipMalloc(&p, want) != hipSuccess) {
+    if (stream_is_capturing(stream)) {
+        *out = largest_block().p;
+        return bytes > largest_block().bytes ? QGEMM_ERR_ALLOC : QGEMM_OK;
+    }
+    WsBlock *block = &g_ctx.ws[block_of(stream)], &shared = g_ctx.ws[kOwnBlocks];
+    if (grow_block(*block, bytes, (size_t)64 << 20) != QGEMM_OK) {
+        // no memory, but a block of another stream would do: from here on all streams share that one, once it is idle
+        WsBlock &other = largest_block();
+        if (bytes > other.bytes || hipDeviceSynchronize() != hipSuccess) {
             (void)hipGetLastError();
             return QGEMM_ERR_ALLOC;
         }
-        if (g_ctx.ws.p) g_ctx.retired.push_back(g_ctx.ws.p);
-        g_ctx.ws.p = p;
-        g_ctx.ws.bytes = want;
+        std::swap(shared, other);
+        g_ctx.ws_all_share = true;
+        block = &shared;
     }
-    if (!capturing) {
-        if (g_ctx.ws_event_recorded && g_ctx.ws_last_stream != stream && !g_ctx.ws_used_by_call)
+    if (block == &shared && !g_ctx.ws_shared_by_call) {
+        if (g_ctx.ws_event_recorded && (g_ctx.ws_last_stream != stream || stream == hipStreamPerThread))
             HIP_TRY(hipStreamWaitEvent(stream, g_ctx.ws_event, 0));
-        g_ctx.ws_used_by_call = true;
+        g_ctx.ws_shared_by_call = true;
     }
-    *out = g_ctx.ws.p;
+    *out = block->p;
     return QGEMM_OK;
 }
 
-// Around the body of every entry that may use the workspace: when it did, the end of its launches is recorded
+// Around the body of every entry that may use the workspace: when it used the shared block, the end of its launches is recorded
 // on its stream for the next user on another stream to wait for.
 struct WorkspaceUse {
     hipStream_t stream;
-    explicit WorkspaceUse(hipStream_t s) : stream(s) { g_ctx.ws_used_by_call = false; }
+    explicit WorkspaceUse(hipStream_t s) : stream(s) { g_ctx.ws_shared_by_call = false; }
     ~WorkspaceUse() {
-        if (!g_ctx.ws_used_by_call) return;
-        g_ctx.ws_used_by_call = false;
+        if (!g_ctx.ws_shared_by_call) return;
+        g_ctx.ws_shared_by_call = false;
         if (!g_ctx.ws_event && hipEventCreateWithFlags(&g_ctx.ws_event, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
             g_ctx.ws_event = nullptr;
@@ -1530,13 +1578,16 @@ QGEMM_EXPORT int qgemm_init(void) {
 
 QGEMM_EXPORT int qgemm_shutdown(void) {
     std::lock_guard<std::mutex> lock(g_ctx.mu);
-    if (g_ctx.ws.p || !g_ctx.retired.empty()) {
+    if (largest_block().p || !g_ctx.retired.empty()) {
         (void)hipDeviceSynchronize();
-        if (g_ctx.ws.p) (void)hipFree(g_ctx.ws.p);
+        for (const WsBlock &b : g_ctx.ws)
+            if (b.p) (void)hipFree(b.p);
         for (void *p : g_ctx.retired) (void)hipFree(p);
     }
     if (g_ctx.ws_event) (void)hipEventDestroy(g_ctx.ws_event);
-    g_ctx.ws = WsBlock();
+    for (WsBlock &b : g_ctx.ws) b = WsBlock();
+    g_ctx.ws_owners = 0;
+    g_ctx.ws_all_share = false;
     g_ctx.retired.clear();
     g_ctx.ws_event = nullptr;
     g_ctx.ws_event_recorded = false;
@@ -1982,27 +2033,15 @@ QGEMM_EXPORT int qgemm_reserve_workspace(size_t bytes) {
     std::lock_guard<std::mutex> lock(g_ctx.mu);
     int st = ensure_init_locked();
     if (st != QGEMM_OK) return st;
-    if (bytes <= g_ctx.ws.bytes) return QGEMM_OK;
     // (takes no stream, so it cannot tell whether one is being captured: the caller reserves before a capture)
-    // grow geometrically, as ensure_workspace_locked does: a caller that reserves step by step then retires
-    // O(log n) blocks, not one per call
-    const size_t want = std::max(bytes, 2 * g_ctx.ws.bytes);
-    void *p = nullptr;
-    if (hipMalloc(&p, want) != hipSuccess) {
-        (void)hipGetLastError();
-        return QGEMM_ERR_ALLOC;
-    }
-    if (g_ctx.ws.p) g_ctx.retired.push_back(g_ctx.ws.p);
-    g_ctx.ws.p = p;
-    g_ctx.ws.bytes = want;
-    return QGEMM_OK;
+    return grow_block(largest_block(), bytes, 0);
 }
 
 QGEMM_EXPORT int qgemm_workspace_info(void **base, size_t *bytes) {
     if (!base || !bytes) return QGEMM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lock(g_ctx.mu);
-    *base = g_ctx.ws.p;
-    *bytes = g_ctx.ws.bytes;
+    *base = largest_block().p;
+    *bytes = largest_block().bytes;
     return QGEMM_OK;
 }
 

@@ -154,3 +154,26 @@ def test_packed_operands_on_two_streams():
     for _, _, ref, _, c in jobs:
         for r in range(rounds):
             assert np.array_equal(host(c[r]), ref), r
+
+
+@pytest.mark.parametrize("streams", [2, 6])
+def test_streams_with_blocks_of_their_own_and_beyond(streams):
+    """Split-K products of different operands on several streams at once, more than there are blocks to own: whoever shares
+    a block is ordered, whoever has one needs no order, and every result is the oracle's."""
+    say("workspace blocks", streams)
+    M, N, K, rounds = 96, 256, 2048, 10
+    jobs = []
+    for i in range(streams):
+        qa, sa, qb, sb = int8_inputs(M, N, K, seed=130 + i)
+        jobs.append((dev(qa), dev(qb), scalar(sa), scalar(sb), R.gemm_i8_i32(qa, qb), torch.cuda.Stream(),
+                     [torch.zeros((M, N), dtype=torch.int32, device="cuda") for _ in range(rounds)]))
+    torch.cuda.synchronize()
+    for r in range(rounds):
+        for a, b, sa, sb, _, stream, c in jobs:
+            with torch.cuda.stream(stream):
+                Q.int8_mm(a, b, sa, sb, c[r], split_k=8)
+            assert "splitk" in Q.last_config()
+    torch.cuda.synchronize()
+    for i, job in enumerate(jobs):
+        for r in range(rounds):
+            assert np.array_equal(host(job[6][r]), job[4]), (i, r)
