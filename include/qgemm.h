@@ -123,10 +123,10 @@ int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int la
                              size_t K, int split_k, void *stream);
 
 /* Library workspace (no reference counterpart: the reference's entries take none).  Calls that split K, that
- * take operands or scales in an arrangement the kernels do not read directly, and the per-matrix quantiser (above
- * 256 KiB, or, outside a capture and with gaps between the rows, which then count rounded up to 16 bytes each, above 128 KiB)
- * keep their intermediate data in device blocks owned by the library and grown on demand.  A block that is
- * outgrown is replaced but stays allocated until qgemm_shutdown, so launches already enqueued and graphs
+ * take operands or scales in an arrangement the kernels do not read directly, and the per-matrix quantiser where it makes two passes
+ * (above 256 KiB while captured; otherwise above 128 KiB with gaps between the rows, which then count rounded up to 16 bytes each, or at
+ * addresses that are no multiple of 4, and above 32 MiB) keep their intermediate data in device blocks owned by the library
+ * and grown on demand.  A block that is outgrown is replaced but stays allocated until qgemm_shutdown, so launches already enqueued and graphs
  * already captured remain valid.  The first three streams that need one have a block each; calls on further streams share
  * a fourth, and each such call waits (on the device, through an event) for the previous user on another stream.  While a
  * stream is being captured into a graph the library neither allocates nor touches that event: such a call uses the largest
@@ -185,7 +185,8 @@ int qgemm_quantize_grid(int in_dtype, size_t rows, size_t cols, uint32_t *rows_p
  *   "stagger_groups", "as_groups", "row_split" (0: one launch always; 1: the rows "a+b" or columns "a|b" of a partly
  *   empty last round of 256 x 256 tiles as a second launch where the estimate gains; 2 / 3: rows / columns wherever
  *   possible), "small_tiles" (0: 17 .. 256 rows against few columns keep a tall tile with a K split instead of several
- *   row tiles of the skinny-M kernel; row_estimate counts as 0 then), "row_estimate" (0: up to 400 rows follow the general
+ *   row tiles of the skinny-M kernel; row_estimate counts as 0 then), "quant_wait" (microseconds for which the workgroups of a per-matrix
+ *   quantisation in one launch wait for one another before each reads the whole matrix, 2000; -1: two passes instead), "row_estimate" (0: up to 400 rows follow the general
  *   rules instead of the estimate of every row that serves them below 32 K steps and, block scales, up to 128 rows), "few_rows"
  *   (operands that option "any_shape" decides about, 1 .. 128 rows: 0 / 2: never / wherever it can the kernel for few rows
  *   instead of the tiles of the any-shape kernel; 1: by an estimate), "c_plain" (0 / 1: non-temporal / ordinary stores for C; -1: the library's

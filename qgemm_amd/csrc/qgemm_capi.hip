@@ -62,6 +62,8 @@ struct Context {
     hipStream_t ws_last_stream = nullptr;
     bool ws_event_recorded = false;
     bool ws_shared_by_call = false;            // the running entry asked for the shared block
+    uint32_t quant_launches = 0;               // of quant_whole_matrix_kernel, which number them
+    long quant_wait = 2000;     // microseconds its workgroups wait for one another; -1: per-matrix scales in two passes
     bool static_call = false;                  // the running entry takes its workspace from the static scratch
     void *static_ptr[kMaxDevices] = {};        // device address of `scratch`, per device
     std::string force_config;   // name of a row of the variant tables, empty = heuristic (qgemm_force_config)
@@ -1518,10 +1520,25 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         // (an empty matrix is for the forms that look whether a row has a piece: the others load without asking)
         const bool row_ends = a.cols == 0 || a.cols % P::VEC != 0, one_row = a.rows == 1;
         auto form = [&](auto one_ragged, auto one, auto rows_ragged, auto rows) { return one_row ? (row_ends ? one_ragged : one) : row_ends ? rows_ragged : rows; };
-        if (pieces * 16 <= kQuantSmallBytes && (one_row || pieces * 16 <= kQuantSmallRowsBytes || stream_is_capturing(stream))) {
+        const bool capturing = pieces * 16 > kQuantSmallBytes && stream_is_capturing(stream);
+        if (pieces * 16 <= kQuantSmallBytes || (capturing && pieces * 16 <= kQuantSmallCapturedBytes)) {
             e = launch_kernel(form(quant_small_matrix_kernel<IN_DT, OUT_DT, true, true>, quant_small_matrix_kernel<IN_DT, OUT_DT, true, false>,
                                    quant_small_matrix_kernel<IN_DT, OUT_DT, false, true>, quant_small_matrix_kernel<IN_DT, OUT_DT, false, false>),
                               dim3((unsigned)std::max<uint64_t>(1, (pieces + 1023) / 1024)), dim3(1024), 0, stream, a);
+            return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
+        }
+        const uint64_t most = (uint64_t)std::min(g_ctx.num_cus, kQuantGroups) * 1024;        // lanes of a launch that fits the chip
+        if (g_ctx.quant_wait >= 0 && one_row && pieces <= most * kQuantMostPieces && (uintptr_t)a.x % 4 == 0 && !capturing) {
+            const uint32_t whole = a.cols / P::VEC, each = (uint32_t)((whole + most - 1) / most);
+            const uint32_t groups = std::max<uint32_t>(1, std::min<uint32_t>((uint32_t)(most / 1024), (whole + 1023) / 1024));
+            a.share = (whole + groups - 1) / groups;
+            if (++g_ctx.quant_launches == 0) g_ctx.quant_launches = 1;
+            a.tag = g_ctx.quant_launches;
+            a.set = a.tag % kQuantSets;
+            a.wait = (uint32_t)g_ctx.quant_wait * 100;
+            e = launch_kernel(each <= 1 ? quant_whole_matrix_kernel<IN_DT, OUT_DT, 1> : each <= 2 ? quant_whole_matrix_kernel<IN_DT, OUT_DT, 2> :
+                              each <= 4 ? quant_whole_matrix_kernel<IN_DT, OUT_DT, 4> : quant_whole_matrix_kernel<IN_DT, OUT_DT, kQuantMostPieces>,
+                              dim3(groups), dim3(1024), 0, stream, a);
             return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
         }
         // two passes: partial maxima (one per workgroup) into the workspace, then scale and cast
@@ -1649,6 +1666,7 @@ QGEMM_EXPORT int qgemm_set_option(const char *key, long value) {
     else if (!std::strcmp(key, "as_groups")) g_ctx.as_groups = value;
     else if (!std::strcmp(key, "small_tiles")) g_ctx.small_tiles = value;
     else if (!std::strcmp(key, "few_rows")) g_ctx.few_rows = value;
+    else if (!std::strcmp(key, "quant_wait")) g_ctx.quant_wait = std::max(-1L, std::min(value, 1000000L));
     else if (!std::strcmp(key, "row_estimate")) g_ctx.row_estimate = value;
 #if QGEMM_DEBUG_BUILD
     else if (!std::strcmp(key, "dbg_ptr")) g_ctx.dbg_ptr = value;

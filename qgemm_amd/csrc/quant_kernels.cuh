@@ -31,6 +31,8 @@ struct QuantArgs {
     // Work is numbered along rows in units of a piece (per matrix) or of a 1 x 128 block: `per_row` of them in a row,
     // inv = inverse_of(per_row).  blockIdx.y counts slices of rows_per_slice rows, so that a number fits 32 bits.
     uint32_t per_row, inv, rows_per_slice;
+    uint32_t share, set, tag, wait; // quant_whole_matrix_kernel: whole pieces of a workgroup; where, under which number and for how long
+                                    // (ticks of the 100 MHz clock) maxima meet
 };
 
 // What the kernels start with, in front of QuantArgs: arguments of their own arrive in scalar registers with the wave (kernarg
@@ -407,12 +409,11 @@ __device__ inline Divisor matrix_divisor(uint32_t m) {
 }
 
 // Small: one launch, no workspace.  Every workgroup takes the maximum of the whole matrix, then quantises its own 1024 pieces.
-// A workgroup reads some 100 GB/s, so this ends where that takes as long as a second launch, or, with gaps between the rows and a
-// division for every piece, at half of that (kQuantSmallRowsBytes; a stream that is being captured, which has only the workspace that is
-// there, stays on one launch up to kQuantSmallBytes).  Against the two passes below, us, graph replays, bf16: 16 x 2048 (64 KiB) 3.6 / 4.7,
-// 48 x 2048 (192 KiB) 4.9 / 5.1, 64 x 2048 4.9 / 5.1; gaps: 64 x 512 (64 KiB) 4.3 / 4.8, 64 x 1024 4.4 / 5.2, 40 x 2176 (170 KiB) 7.6 / 5.2
-// (with the pieces of rows without ends as pieces of rows with them 7.6 / 6.3).
-constexpr uint64_t kQuantSmallBytes = 256 << 10, kQuantSmallRowsBytes = 128 << 10;
+// A workgroup reads some 100 GB/s, so this ends where that takes as long as the exchange of quant_whole_matrix_kernel (bf16, us, this /
+// exchange: 16 x 2048 (64 KiB) 6.2 / 6.2, 48 x 2048 (192 KiB) 7.2 / 6.5, 64 x 2048 7.2 / 6.5) or, with gaps between the rows and a division for
+// every piece, as a second launch (graph replays, us, this / two passes: 64 x 512 (64 KiB) 4.3 / 4.8, 64 x 1024 4.4 / 5.2, 40 x 2176 (170 KiB) 7.6 /
+// 5.2).  A stream that is being captured, which has neither the exchange nor more workspace than is there, stays on this to kQuantSmallCapturedBytes.
+constexpr uint64_t kQuantSmallBytes = 128 << 10, kQuantSmallCapturedBytes = 256 << 10;
 template <int IN_DT, int OUT_DT, bool ONE_ROW, bool RAGGED>
 __global__ void __launch_bounds__(1024) quant_small_matrix_kernel(const QuantArgs p) {
     const MatrixPieces<IN_DT, ONE_ROW, RAGGED> x(p, 0);
@@ -424,6 +425,85 @@ __global__ void __launch_bounds__(1024) quant_small_matrix_kernel(const QuantArg
     x.template settle<1>(own, at);
     if (mine == 0) p.scales[0] = dv.s;
     x.store(at[0], quant_piece<IN_DT, OUT_DT>(own[0], dv));
+}
+
+// One launch for a matrix without gaps that the chip can hold: every lane keeps its pieces in registers, the workgroups exchange their
+// maxima through memory and each quantises what it holds.  The matrix is read once and a launch saved, for an exchange of some 2 us.
+// Eager calls one after another, bf16 to int8, us, two passes / so: 50 x 5296 7.9 / 5.3, 378 x 4632 9.2 / 6.6, 1531 x 3004 7.7 / 7.1, 1000 x
+// 7168 8.6 / 7.9, 4096 x 4096 14.1 / 12.9; fp32 50 x 5296 7.9 / 5.1, 500 x 4096 7.4 / 6.1, 2048 x 4096 11.0 / 9.9.  Bound by the exchange up to
+// some 10 MiB, by memory above.
+// A workgroup writes its maximum and the launch's number as one 64-bit word, with the device's scope, and reads everybody's words
+// until they carry that number: nothing has to be reset, ordered or fenced (a fence of that scope writes back the L2: 27 us), and a
+// word is either this launch's or it is not.  kQuantSets launches have words of their own; should two that far apart run at the same time,
+// or should workgroups not all find room beside another stream's kernel, the wait ends after QuantArgs::wait and the workgroup takes the
+// maximum of the whole matrix itself: slow, and the same result.  A replayed graph would bring the same number again: captured calls take the two passes below.
+constexpr int kQuantSets = 64, kQuantGroups = 256, kQuantMostPieces = 8;
+static __device__ uint64_t quant_words[kQuantSets][kQuantGroups];
+// maximum of all workgroups' m (as workgroup_maximum gives it), false where some of them did not come in time
+__device__ inline bool launch_maximum(uint32_t &m, uint32_t set, uint32_t tag, uint32_t wait) {
+    uint64_t *const words = quant_words[set];
+    const uint32_t t = threadIdx.x;
+    if (t == 0) __hip_atomic_store(words + blockIdx.x, (uint64_t)tag << 32 | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint64_t w = 0;
+    bool late = false;
+    if (t < gridDim.x) {
+        const uint64_t start = __builtin_amdgcn_s_memrealtime();
+        while (w = __hip_atomic_load(words + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), (uint32_t)(w >> 32) != tag) {
+            late = __builtin_amdgcn_s_memrealtime() - start > wait;
+            if (late) break;
+        }
+    } else if (blockIdx.x == 0 && t < (uint32_t)kQuantGroups) {          // (numbers come round: no old word stays for longer than kQuantSets launches)
+        __hip_atomic_store(words + t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    late = __syncthreads_or(late);
+    m = workgroup_maximum<16>((uint32_t)w);
+    return !late;
+}
+template <int IN_DT, int OUT_DT, int N>
+__global__ void __launch_bounds__(1024, 8) quant_whole_matrix_kernel(const QuantArgs p) {
+    typedef Piece<IN_DT> P;
+    const MatrixPieces<IN_DT, true, true> x(p, 0);
+    const uint32_t whole = p.cols / P::VEC, first = blockIdx.x * p.share;
+    const uint32_t mine = first < whole ? (whole - first < p.share ? whole - first : p.share) : 0;
+    // (lanes past the workgroup's share are out of the buffer's range and get zeros: no branch between the loads)
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>((const char *)p.x + (size_t)first * 16), 0, mine * 16, 0x00020000);
+    v4i v[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, threadIdx.x * 16, j * 1024 * 16, 0));
+    // the last piece of a matrix that ends inside one is one lane's
+    const bool last = whole < x.total && blockIdx.x == 0 && threadIdx.x == 0;
+    v4i end[1] = {v4i{0, 0, 0, 0}};
+    const typename MatrixPieces<IN_DT, true, true>::Place at[1] = {x.place(x.total - 1)};
+    if (last) x.template request<1>(end, at);
+    v4i acc = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < N; ++j) P::fold_max(acc, v[j]);
+    if (last) {
+        x.template settle<1>(end, at);
+        P::fold_max(acc, end[0]);
+    }
+    uint32_t m = P::max_bits(acc);
+    if (m > P::INF) {
+        m = P::max_bits_of_numbers(end[0]);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const uint32_t b = P::max_bits_of_numbers(v[j]);
+            m = b > m ? b : m;
+        }
+        m |= kQuantNan;
+    }
+    m = workgroup_maximum<16>(m);
+    if (!launch_maximum(m, p.set, p.tag, p.wait)) {
+        __syncthreads();
+        m = workgroup_maximum<16>(x.template maximum<1>(threadIdx.x, 1024, 1024, threadIdx.x == 0));
+    }
+    const Divisor dv = matrix_divisor<IN_DT, OUT_DT>(m);
+    if (blockIdx.x == 0 && threadIdx.x == 0) p.scales[0] = dv.s;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        if (j * 1024 + threadIdx.x < mine)
+            store_piece<IN_DT>(p.q, (size_t)(first + j * 1024 + threadIdx.x) * P::VEC, quant_piece<IN_DT, OUT_DT>(v[j], dv), P::VEC);
+    if (last) x.store(at[0], quant_piece<IN_DT, OUT_DT>(end[0], dv));
 }
 
 // pass 1: one partial maximum per workgroup
