@@ -114,7 +114,7 @@ int qgemm_scaled_gemm(int in_dtype, int out_dtype, int scale_mode, int layout, c
  * more returns QGEMM_ERR_SCRATCH_TOO_SMALL and launches nothing.  All calls on one GPU share the array: two
  * calls whose kernels overlap in time on one GPU (different streams, or threads) race.
  * Operands that qgemm_scaled_gemm packs into the workspace first (K not a multiple of 16, unaligned pointers: option
- * "any_shape") are not packed here: the any-shape kernel reads them as they stand, and such calls take nothing from
+ * "any_shape") are not packed here: the kernels read them as they stand, and such calls take nothing from
  * the array.  int8 operands with one scale give the same bits either way; block-scaled ones are the same products and
  * the same folds, summed in another order. */
 #define QGEMM_STATIC_SCRATCH_BYTES ((size_t)32 << 20)
@@ -132,8 +132,8 @@ int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int la
  * stream is being captured into a graph the library neither allocates nor touches that event: such a call uses the largest
  * block there is, one that would need more returns
  * QGEMM_ERR_ALLOC, and replays of graphs that use the workspace must not overlap other users of it.  (Products whose
- * operands would be packed into the block, see option "any_shape", do not use it while captured: they run the any-shape
- * kernel, whose fp32 sums have another order than those of an eager call.)
+ * operands would be packed into the block, see option "any_shape", do not use it while captured: their operands are read as
+ * they stand, and fp32 sums have another order than those of an eager call.)
  * qgemm_reserve_workspace makes the largest block at least `bytes` large ahead of time (it allocates: call it before a
  * capture begins, never during one; a block that has to grow at least doubles); qgemm_workspace_info reports
  * its address and size (NULL / 0 before first use). */
@@ -180,8 +180,8 @@ int qgemm_quantize_grid(int in_dtype, size_t rows, size_t cols, uint32_t *rows_p
  * src/include/gemm_config.h:30-36).
  * qgemm_set_option(key, value): "force_split" (K slices, 0 = heuristic), "group_m", "kmajor", "any_shape" (operands whose K
  *   bytes are no multiple of 16, or whose rows or pointers are unaligned: 0 the any-shape kernel, which reads them as they
- *   stand, 1 packed into the workspace for the other kernels where that is faster, 2 packed wherever possible; captured
- *   calls and qgemm_scaled_gemm_static always run the any-shape kernel), "stagger", "k_rot",
+ *   stand, 2 packed into the workspace for the other kernels wherever possible, 3 read by the other kernels as they stand wherever
+ *   possible, 1 what is estimated fastest; captured calls and qgemm_scaled_gemm_static never pack), "stagger", "k_rot",
  *   "stagger_groups", "as_groups", "row_split" (0: one launch always; 1: the rows "a+b" or columns "a|b" of a partly
  *   empty last round of 256 x 256 tiles as a second launch where the estimate gains; 2 / 3: rows / columns wherever
  *   possible), "small_tiles" (0: 17 .. 256 rows against few columns keep a tall tile with a K split instead of several

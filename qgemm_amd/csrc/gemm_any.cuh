@@ -1,7 +1,7 @@
 // The any-shape GEMM: operands at any address, with any distance between rows and any number of elements in them, read where
 // they stand.  It asks for no memory but its operands: captured calls and calls on the static scratch, whose kernels may
-// overlap with other users of the workspace, run it, as do products too small to be worth packing, and
-// whatever exceeds what the other kernels index.  int32 sums for int8, fp32 otherwise; block scales are folded in once per
+// overlap with other users of the workspace, run it where the MFMA rows do not read their operands as they stand, as do small
+// products, and whatever exceeds what the other kernels index.  int32 sums for int8, fp32 otherwise; block scales are folded in once per
 // 128 elements of K as (P * as) * bs (hip_mix_gemm_kernel.cpp:231-244), in the form for few rows (gemm_few_kernel, at the end) as
 // P * (as * bs), like the kernels for whole rows: two roundings either way.
 //

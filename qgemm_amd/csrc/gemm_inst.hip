@@ -31,20 +31,20 @@ static hipError_t allow_lds(K kernel, int bytes) {
     return e;
 }
 
-template <class C>
+template <class C, bool REST = false>
 static hipError_t launch_variant(const GemmArgs &a, uint32_t grid, hipStream_t s) {
-    hipError_t e = allow_lds(gemm_nt_kernel<C>, C::LDS_BYTES);
+    hipError_t e = allow_lds(gemm_nt_kernel<C, REST>, C::LDS_BYTES);
     if (e != hipSuccess) return e;
     const LaunchHead h(a, a.map.inv_group, a.map.inv_gm, a.map.inv_last, a.inv_nk);
-    return launch_kernel(gemm_nt_kernel<C>, dim3(grid), dim3(C::THREADS), C::LDS_BYTES, s, QGEMM_HEAD_OF(h), a);
+    return launch_kernel(gemm_nt_kernel<C, REST>, dim3(grid), dim3(C::THREADS), C::LDS_BYTES, s, QGEMM_HEAD_OF(h), a);
 }
 
-template <class C>
+template <class C, bool REST = false>
 static hipError_t launch_skinny(const GemmArgs &a, uint32_t grid, hipStream_t s) {
-    hipError_t e = allow_lds(gemm_skinny_kernel<C>, C::LDS_BYTES);
+    hipError_t e = allow_lds(gemm_skinny_kernel<C, REST>, C::LDS_BYTES);
     if (e != hipSuccess) return e;
     const LaunchHead h(a, C::TN == 4 ? a.map.inv_group : a.inv_tiles_m, a.map.inv_gm, a.map.inv_last, a.inv_nk);
-    return launch_kernel(gemm_skinny_kernel<C>, dim3(grid), dim3(C::THREADS), C::LDS_BYTES, s, QGEMM_HEAD_OF(h), a);
+    return launch_kernel(gemm_skinny_kernel<C, REST>, dim3(grid), dim3(C::THREADS), C::LDS_BYTES, s, QGEMM_HEAD_OF(h), a);
 }
 
 constexpr int kElemBytes = (INST_ARITH == AR_BF16 || INST_ARITH == AR_F16) ? 2 : 1;
@@ -53,6 +53,7 @@ constexpr bool kBlock = (bool)INST_BLOCK;
 // (128 x 128 with two K groups: 164 bytes of scratch a lane, 308 with block scales; 256 x 256 on eight waves 272 and 676;
 // 256 x 128 with copying waves 148 and 1756; 128 rows of the skinny-M kernel 148 with block scales).
 constexpr bool kWide = INST_ARITH == AR_F8W;
+constexpr bool kRest = INST_ARITH != AR_F8;         // (fp8 rows that end inside a chunk run widened)
 // A K-major operand needs whole 128-byte panels of its tile side and a multiple of four waves (GemmCfg's
 // static_asserts); tiles that cannot have that are left out of a K-major family.
 constexpr bool kmajor_can(int bm, int bn, int nw) {
@@ -63,7 +64,7 @@ constexpr bool kmajor_can(int bm, int bn, int nw) {
 template <class C>
 static Variant gemm_row(const char *name, bool auto_ok) {
     return Variant{name, C::ARITH, C::BLOCK_SCALE, C::BM, C::BN, C::THREADS, C::LDS_BYTES, auto_ok, C::COPYW, C::KG, C::ASK,
-                   C::AS_ANY_STRIDE, -1, 0, &launch_variant<C>};
+                   C::AS_ANY_STRIDE, -1, 0, &launch_variant<C>, kRest ? &launch_variant<C, kRest> : nullptr};
 }
 // row of the skinny-M kernel (gemm_skinny.cuh): 16 * TM rows x 16 * TN columns, eight waves splitting K between them.
 // Picked by choose_variant in place of the narrow simple-pipeline tiles, never by the table scan (auto_ok = false).
@@ -71,7 +72,7 @@ template <int TM, int TN = 2>
 static Variant skinny_row(const char *name) {
     using C = SkinnyCfg<INST_ARITH, TM, kBlock, TN>;
     return Variant{name, C::ARITH, C::BLOCK_SCALE, C::BM, C::BN, C::THREADS, C::LDS_BYTES, false, false, 8, false, C::BLOCK_SCALE,
-                   -1, 0, &launch_skinny<C>};
+                   -1, 0, &launch_skinny<C>, kRest ? &launch_skinny<C, kRest> : nullptr};
 }
 
 // simple pipeline

@@ -57,6 +57,7 @@ struct GemmArgs {
     uint32_t M, N;
     uint32_t ksteps;      // K steps of 128 bytes in total, the last one possibly partial
     uint32_t k_tail;      // bytes of K in the last step when it is partial (a multiple of 16), 0 when it is whole
+    uint32_t k_rest;      // bytes of K behind those steps (1 .. 15: rows that do not end with a chunk of 16 bytes, see gemm_rest), 0 mostly
     uint32_t lda, ldb;    // bytes
     uint32_t ldc;         // elements
     TileMap map;          // tiles of the launch
@@ -295,6 +296,97 @@ __device__ inline void mma128_inplace(v4i x0, v4i x1, v4i y0, v4i y1, typename A
     }
 }
 
+// ---- Rows at any address, of any length.  The copies fetch 16 bytes a lane from whatever address a row has, but only chunks that lie
+// wholly inside a row; what K has left behind the last of them, `rest` bytes (1 .. 15), is one MFMA more per tile at the end of the
+// loop, whose fragments come from memory straight into registers: the last 16 bytes of the row, moved down, zeros above, in the lanes of K
+// group 0.  So that the trip to memory is short the K loop has just fetched the same lines.
+// (Packing such operands into aligned rows first is a launch that reads and writes both of them: 7.6 us in front of a product of 23.7, int8
+// 1531 x 4100 x 3004.)
+// 16 bytes that start at k_end - 16 of a row, as the fragment of K group 0
+__device__ __forceinline__ v4i rest_fragment(const char *row_end, uint32_t rest, bool group0) {
+    const v4i v = *(const v4i_any *)(row_end - 16);
+    uint32_t w[4] = {(uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]};
+    move_down<4>(w, group0 ? 16 - rest : 16);
+    return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+}
+// the same out of an operand stored K x N (16-bit elements): up to seven rows of k, column `at` of them
+__device__ __forceinline__ v4i rest_column(const char *at, uint32_t ld, uint32_t rest, bool group0) {
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (uint32_t i = 0; i < 7; ++i) {
+        const uint32_t in = 2 * i < rest;
+        const uint32_t e = *(const uint16_t *)(at + (in ? i * (size_t)ld : 0));
+        w[i / 2] |= (in && group0 ? e : 0u) << (16 * (i & 1));
+    }
+    return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+}
+template <int ARITH>
+__device__ __forceinline__ typename AccT<ARITH>::type mma_rest(v4i x, v4i y, typename AccT<ARITH>::type c) {
+    if constexpr (ARITH == AR_F8W) {
+        auto wide = [](int lo, int hi) {
+            const v2i a = widen_fp8((uint32_t)lo), b = widen_fp8((uint32_t)hi);
+            return __builtin_bit_cast(v8bf, v4i{a[0], a[1], b[0], b[1]});
+        };
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wide(x[0], x[1]), wide(y[0], y[1]), c, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(wide(x[2], x[3]), wide(y[2], y[3]), c, 0, 0, 0);
+    } else if constexpr (ARITH == AR_I8) {
+        return __builtin_amdgcn_mfma_i32_16x16x64_i8(x, y, c, 0, 0, 0);
+    } else if constexpr (ARITH == AR_BF16) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, x), __builtin_bit_cast(v8bf, y), c, 0, 0, 0);
+    } else {
+        static_assert(ARITH == AR_F16, "");
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, x), __builtin_bit_cast(v8h, y), c, 0, 0, 0);
+    }
+}
+// Adds the rest of K to a wave's TM x TN tiles, which start at row m0 of A and n0 of B (rows past M and N repeat the last one and are
+// not stored).  k_bytes: the K that the loop has done.
+template <class C, bool KMB, bool PINNED, int TM, int TN, class Acc>
+__device__ __forceinline__ void gemm_rest(Acc (&acc)[TM][TN], const GemmArgs &p, const char *A, const char *B, uint32_t lda, uint32_t ldb, uint32_t M,
+                                          uint32_t N, uint32_t k_bytes, uint32_t m0, uint32_t n0, int lane) {
+    typedef typename AccT<C::ARITH>::type part_t;
+    const uint32_t rest = p.k_rest, r = lane & 15;
+    const bool group0 = lane < 16;
+    v4i x[TN], y[TM];
+#pragma unroll
+    for (int a = 0; a < TM; ++a) {
+        const uint32_t m = m0 + a * 16 + r;
+        y[a] = rest_fragment(A + (size_t)(m < M ? m : M - 1) * lda + k_bytes + rest, rest, group0);
+    }
+#pragma unroll
+    for (int b = 0; b < TN; ++b) {
+        const uint32_t n = n0 + b * 16 + r, nn = n < N ? n : N - 1;
+        if constexpr (KMB) x[b] = rest_column(B + (size_t)(k_bytes / 2) * ldb + (size_t)nn * 2, ldb, rest, group0);
+        else x[b] = rest_fragment(B + (size_t)nn * ldb + k_bytes + rest, rest, group0);
+    }
+    if constexpr (C::BLOCK_SCALE) {
+        const uint32_t kb = (k_bytes + rest - 1) / 128;
+#pragma unroll
+        for (int a = 0; a < TM; ++a) {
+            const uint32_t m = m0 + a * 16 + r;
+            const float as = p.as[(size_t)(m < M ? m : M - 1) * p.as_ms + (size_t)kb * p.as_ks];
+#pragma unroll
+            for (int b = 0; b < TN; ++b) {
+                const uint32_t nb = (n0 + b * 16) / 128;
+                const float f = as * p.bs[(size_t)(nb < p.nb_max ? nb : p.nb_max) * p.bs_ns + (size_t)kb * p.bs_ks];
+                const part_t part = mma_rest<C::ARITH>(x[b], y[a], part_t{0, 0, 0, 0});
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[a][b][e] += (float)part[e] * f;
+            }
+        }
+    } else {
+        // (the compiler does not see what the pinned MFMAs need between a vector instruction and themselves)
+        if constexpr (PINNED) asm volatile("s_nop 15" ::: "memory");
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+            for (int b = 0; b < TN; ++b) {
+                if constexpr (PINNED) mma128_inplace<C::ARITH>(x[b], x[b], y[a], y[a], acc[a][b], 0);
+                else acc[a][b] = mma_rest<C::ARITH>(x[b], y[a], acc[a][b]);
+            }
+        if constexpr (PINNED) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    }
+}
+
 // What a wave needs for its first copies travels in front of GemmArgs as arguments of its own: such arguments arrive in scalar
 // registers with the wave (kernarg preloading, at most 14 dwords: -amdgpu-kernarg-preload-count in the Makefile), while a field
 // of a struct is a scalar load, a trip to memory that every launch starts with.  The divisions are multiplications with inverses
@@ -325,7 +417,9 @@ struct LaunchHead {
                    k_bytes = (uint32_t)kf_, flags = (uint32_t)(kf_ >> 32), inv0 = (uint32_t)inv01_, inv1 = (uint32_t)(inv01_ >> 32), \
                    inv2 = (uint32_t)inv23_
 
-template <class C>
+// REST: K ends in GemmArgs::k_rest bytes behind the last whole chunk (an instantiation of its own: in the others the code behind the loop
+// cost the narrow tiles twice their accumulation registers)
+template <class C, bool REST = false>
 __global__ void __launch_bounds__(C::THREADS)
 gemm_nt_kernel(QGEMM_HEAD, const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the launch stub
@@ -1092,7 +1186,8 @@ gemm_nt_kernel(QGEMM_HEAD, const GemmArgs p) {
             const uint32_t line_a = (uint32_t)((uintptr_t)A >> 4) + (lane >> 3) * (lda >> 4);    // for row & 7 == lane >> 3
             const uint32_t line_b = (uint32_t)((uintptr_t)B >> 4) + (lane >> 3) * (ldb >> 4);
             constexpr bool LATE_FORM = C::KMAJ == 0 && (!C::BLOCK_SCALE || C::BM >= 128);
-            const bool late = LATE_FORM && nk >= (C::BLOCK_SCALE ? 32 : 1) && (((uint32_t)(uintptr_t)A | (uint32_t)(uintptr_t)B | lda | ldb) & 127u) != 0;
+            const uint32_t addresses = (uint32_t)(uintptr_t)A | (uint32_t)(uintptr_t)B | lda | ldb;
+            const bool late = LATE_FORM && nk >= (C::BLOCK_SCALE ? 32 : 1) && (addresses & 127u) != 0 && (addresses & 15u) == 0;
             constexpr int NPC = C::NLOAD / C::NPROD;                        // operand copies per stage and copying wave
             constexpr int CPS = NPC + (C::BLOCK_SCALE ? 1 : 0);
             static_assert(C::NPROD == 4 && C::NLOAD % 4 == 0 && C::RBA % 2 == 0 && (NS - 2) * CPS <= 63,
@@ -1403,6 +1498,12 @@ gemm_nt_kernel(QGEMM_HEAD, const GemmArgs p) {
         }
     }
 
+    if constexpr (REST) {
+        static_assert(C::ARITH != AR_F8 && !C::KMA, "fp8 rows of any length run on the family that widens them");
+        if (kend == ksteps && kg == 0)
+            gemm_rest<C, C::KMB, C::PIPE == PIPE_SOLO && C::NW == 4 && !C::COPYW>(acc, p, A, B, lda, ldb, M, N, k_bytes, row0 + wm * C::WM,
+                                                                                    col0 + wn * C::WN, lane);
+    }
     QGEMM_STAMP(2);
     // ---- epilogue: lane holds C[m][n0 .. n0+3] of every 16x16 tile
     float scale = 1.0f;

@@ -62,7 +62,8 @@ __device__ inline void wait_landed() {
 }
 
 // (arguments in front of `p`: see LaunchHead; inverses of the row tiles, or, 64 x 64 form, the three of TileMap, then of the K steps)
-template <class C>
+// REST: as for gemm_nt_kernel
+template <class C, bool REST = false>
 __global__ void __launch_bounds__(C::THREADS)
 gemm_skinny_kernel(QGEMM_HEAD, const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -385,6 +386,10 @@ gemm_skinny_kernel(QGEMM_HEAD, const GemmArgs p) {
     // (a wave without a step has copies of zeros on their way into its ring, which now takes the partial sums)
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0) & 0xF0FF);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (REST) {
+        if (kend == ksteps && wave == C::NW - 1)
+            gemm_rest<C, false, false>(acc, p, A, B, lda, ldb, M, N, k_bytes, row0, col0, lane);
+    }
     QGEMM_STAMP(3);
 
     // ---- the eight partial sums meet in LDS: partial of wave w, tile t at smem + w * RING_BYTES + t * 1 KiB, lane-linear

@@ -285,6 +285,11 @@ bool out_dtype_ok(int in_dtype, int out_dtype) {
     return out_dtype == QGEMM_DT_I32 && in_dtype == QGEMM_DT_I8;
 }
 
+// What copying 128 bytes of a row of A or B into LDS takes a CU, us, where it is known to bound a step: rows that do not start on 16 bytes
+// (0: the planner's times per step have it).
+struct RowCopies {
+    double a = 0, b = 0;
+};
 struct NtProblem {
     int arith;
     bool block;
@@ -293,21 +298,23 @@ struct NtProblem {
     size_t lda_bytes, ldb_bytes, ldc;   // ldc in elements; lda / ldb: stride between rows of m / n, or, for a
                                         // K-major operand (kmaj), between rows of k
     size_t M, N, Kbytes;
+    size_t k_rest;                      // bytes of K behind Kbytes, which then ends with the last whole 16-byte chunk (GemmArgs::k_rest)
     int kmaj;                           // bit 0: A is stored K x M, bit 1: B is stored K x N
     const float *as, *bs;
     uint32_t as_ms, as_ks, bs_ns, bs_ks;
     int out_dtype, per_matrix, split_k;
+    RowCopies copies;
 };
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 size_t ksteps_of(const NtProblem &q) { return (q.Kbytes + 127) / 128; }      // the last one may be partial
 
-// Shapes the MFMA kernel takes (pointer alignment is checked separately); everything else goes to the any-shape
-// kernel.  K is a whole number of 16-byte chunks (the unit of a copy); a last K step of fewer than 128 bytes is
+// Shapes the MFMA kernel takes (mfma_shape_ok: with whole rows, pointer alignment checked separately; everything else: launch_unaligned,
+// launch_packed, launch_any).  K is a whole number of 16-byte chunks (the unit of a copy); a last K step of fewer than 128 bytes is
 // filled up with zeros on the way into LDS (GemmArgs::k_tail), which the reference's dispatch covers with its
 // 64- and 32-wide K tiles (hip_mix_gemm_kernel.cpp:442-463).
-bool mfma_shape_ok(const NtProblem &q) {
+bool mfma_sizes_ok(const NtProblem &q) {
     const size_t es = (q.arith == AR_BF16 || q.arith == AR_F16) ? 2 : 1, krows = q.Kbytes / es;
     // 32-bit buffer offsets: 256 tile rows of a K-contiguous operand (plus the 3072 bytes by which the solo kernels
     // shift their descriptors), every k row of a K-major one.  With a partial last K step the lanes past the end of
@@ -319,9 +326,9 @@ bool mfma_shape_ok(const NtProblem &q) {
                                    : q.ldb_bytes * 256 + 4096 < lim;
     // block scales: the kernel addresses a_scale with 32-bit byte offsets ((kb * as_ks + m) * 4)
     const bool s_ok = !q.block || ((q.Kbytes + 127) / 128) * std::max<size_t>(q.M, q.as_ks) * 4 < ((size_t)1 << 32);
-    return q.Kbytes % 16 == 0 && q.Kbytes > 0 && q.lda_bytes % 16 == 0 && q.ldb_bytes % 16 == 0 && a_ok && b_ok && s_ok &&
-           q.M < ((size_t)1 << 31) && q.N < ((size_t)1 << 31) && q.ldc < ((size_t)1 << 32);
+    return q.Kbytes % 16 == 0 && q.Kbytes > 0 && a_ok && b_ok && s_ok && q.M < ((size_t)1 << 31) && q.N < ((size_t)1 << 31) && q.ldc < ((size_t)1 << 32);
 }
+bool mfma_shape_ok(const NtProblem &q) { return q.lda_bytes % 16 == 0 && q.ldb_bytes % 16 == 0 && mfma_sizes_ok(q); }
 
 // Which tile, and how many K slices.
 //
@@ -389,7 +396,7 @@ double rounds_cost(size_t wgs, size_t slots, size_t cus, size_t steps, double sh
 bool is_kgroup_row(const Variant &v) { return v.kgroups == 2; }
 
 int choose_by_cost(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int cus, bool may_split,
-                   uint32_t *nsplit_out, double *cost_out = nullptr) {
+                   uint32_t *nsplit_out, double *cost_out = nullptr, RowCopies copies = {}) {
     int best = -1;
     double best_t = 0;
     const bool wide = tab[0].arith == AR_F8W;
@@ -404,7 +411,9 @@ int choose_by_cost(const Variant *tab, int count, size_t M, size_t N, size_t kst
         for (uint32_t ns = 1; ns <= 8; ns *= 2) {
             if (ns > 1 && (!may_split || ksteps / ns < 4)) break;
             const size_t wgs = tiles * ns, slots = (size_t)cus * (block ? tm.blk_per_cu : tm.per_cu), steps = (ksteps + ns - 1) / ns;
-            double t = rounds_cost(wgs, slots, cus, steps, block ? tm.blk_shared : tm.step_shared, block ? tm.blk_alone : tm.step_alone, tm.fixed);
+            const double copy = tm.bm * copies.a + tm.bn * copies.b;
+            double t = rounds_cost(wgs, slots, cus, steps, std::max(block ? tm.blk_shared : tm.step_shared, copy * (block ? tm.blk_per_cu : tm.per_cu)),
+                                   std::max(block ? tm.blk_alone : tm.step_alone, copy), tm.fixed);
             if (ns > 1) t += 4.0 + (double)M * N * 4.0 * (ns + 1) / 3.0e6;
             if (best < 0 || t < best_t) {
                 best = vi;
@@ -418,11 +427,11 @@ int choose_by_cost(const Variant *tab, int count, size_t M, size_t N, size_t kst
 }
 
 int choose_tile(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
-                bool may_split, uint32_t *nsplit_out);
+                bool may_split, uint32_t *nsplit_out, RowCopies copies);
 size_t rows_for_full_rounds(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int cus,
-                            double t_single, double *t_split = nullptr, size_t *padding = nullptr);
+                            double t_single, double *t_split = nullptr, size_t *padding = nullptr, RowCopies copies = {});
 size_t cols_for_full_rounds(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int cus,
-                            double t_single, double *t_split = nullptr, size_t *padding = nullptr, bool whatever_the_estimate = false);
+                            double t_single, double *t_split = nullptr, size_t *padding = nullptr, bool whatever_the_estimate = false, RowCopies copies = {});
 
 // The skinny-M kernel (gemm_skinny.cuh: the K split inside the workgroup, eight waves each on every eighth K step)
 // takes over from the narrow simple-pipeline tiles where it is faster: one row tile (M <= 128), a strip of 32
@@ -441,8 +450,8 @@ size_t cols_for_full_rounds(const Variant *tab, int count, size_t M, size_t N, s
 // against 9.5 with two slices) and none where the strips fill the CUs (16 x 8192 x 8192 15.2 against 18.8).
 // kmaj: the table is a K-major family, which has no narrow tiles: the estimate then serves every M
 int choose_by_rules(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
-                   bool may_split, uint32_t *nsplit_out) {
-    const int vi = choose_tile(tab, count, M, N, ksteps, block, kmaj, cus, may_split, nsplit_out);
+                   bool may_split, uint32_t *nsplit_out, RowCopies copies) {
+    const int vi = choose_tile(tab, count, M, N, ksteps, block, kmaj, cus, may_split, nsplit_out, copies);
     // The same kernel on 64 x 64 tiles: shapes with several row tiles whose 64 x 64 tiles fit one
     // round of CUs and give most of them work, 16 K steps or more.  Against whatever the estimate picks (narrow
     // tiles, K-group tiles with a K split) it is 13 - 33 % faster over 512 .. 2048 rows x 256 .. 3000 columns x 2 .. 8 KiB
@@ -689,8 +698,8 @@ bool sums_as_exact(int arith, bool block, int out_dtype, PartialSums a, PartialS
 // Where an fp32 output would show it, only rows whose sums are as exact as those of the rules' row (sums_as_exact): bf16 8 x 8788 x 544
 // is 7.4e-8 of the result off on eight groups, which the rules ask for, 13.0e-8 in the one chain that the estimate likes.
 int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
-                   bool may_split, bool whole, int out_dtype, uint32_t *nsplit_out) {
-    const int vi = choose_by_rules(tab, count, M, N, ksteps, block, kmaj, cus, may_split, nsplit_out);
+                   bool may_split, bool whole, int out_dtype, uint32_t *nsplit_out, RowCopies copies) {
+    const int vi = choose_by_rules(tab, count, M, N, ksteps, block, kmaj, cus, may_split, nsplit_out, copies);
     if (vi < 0 || kmaj || !whole || M > 400 || tab[vi].arith == AR_F8W || !g_ctx.row_estimate || !g_ctx.small_tiles || !(ksteps < 32 || (block && M <= 128))) return vi;
     // (tile sides are powers of two)
     auto tiles_of = [&](int bm, int bn) { return ((M + bm - 1) >> __builtin_ctz(bm)) * ((N + bn - 1) >> __builtin_ctz(bn)); };
@@ -742,10 +751,10 @@ int choose_variant(const Variant *tab, int count, size_t M, size_t N, size_t kst
 }
 
 int choose_tile(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int kmaj, int cus,
-                bool may_split, uint32_t *nsplit_out) {
+                bool may_split, uint32_t *nsplit_out, RowCopies copies) {
     *nsplit_out = 0;                                       // 0: no opinion, plan_nt decides
     if (M > 64 || kmaj) {
-        int vi = choose_by_cost(tab, count, M, N, ksteps, block, cus, may_split, nsplit_out);
+        int vi = choose_by_cost(tab, count, M, N, ksteps, block, cus, may_split, nsplit_out, nullptr, copies);
         if (vi >= 0) {
             // 256 x 256, int8 and 16-bit types: the 8-wave form needs fewer cycles per tile, the 4-wave form a third
             // fewer LDS reads.  With at least one full round of CUs the part runs at its power limit and the 4-wave
@@ -866,7 +875,7 @@ size_t padded_area(size_t bm, size_t bn, size_t M, size_t N) {
 // second) is not at least 2.5 % below the estimate t_single of the one (config 4 with block scales: estimate
 // 160.5 against 164.8 us, 2.6 %; measured 170.9 - 172.5 against 175.1 - 176.9 us in three interleaved runs).
 size_t rows_for_full_rounds(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int cus,
-                            double t_single, double *t_split, size_t *padding) {
+                            double t_single, double *t_split, size_t *padding, RowCopies copies) {
     if (!g_ctx.row_split) return 0;
     const size_t tn = (N + 255) / 256, tiles = ((M + 255) / 256) * tn, full = tiles / cus;
     if (full == 0 || tiles % cus == 0) return 0;
@@ -874,11 +883,11 @@ size_t rows_for_full_rounds(const Variant *tab, int count, size_t M, size_t N, s
     if (m_main == 0 || m_main >= M) return 0;
     uint32_t ns = 0;
     double t_main = 0, t_rest = 0;
-    const int vm = choose_by_cost(tab, count, m_main, N, ksteps, block, cus, false, &ns, &t_main);
+    const int vm = choose_by_cost(tab, count, m_main, N, ksteps, block, cus, false, &ns, &t_main, copies);
     if (vm < 0 || tab[vm].bm != 256 || tab[vm].bn != 256) return 0;
     size_t pad = padded_area(256, 256, m_main, N);
     if (M - m_main > 128) {
-        const int vr = choose_by_cost(tab, count, M - m_main, N, ksteps, block, cus, false, &ns, &t_rest);
+        const int vr = choose_by_cost(tab, count, M - m_main, N, ksteps, block, cus, false, &ns, &t_rest, copies);
         if (vr < 0) return 0;
         pad += padded_area(tab[vr].bm, tab[vr].bn, M - m_main, N);
     } else {
@@ -895,7 +904,7 @@ size_t rows_for_full_rounds(const Variant *tab, int count, size_t M, size_t N, s
 // 48 of its 56 column tiles are exactly three, and the 4096 x 2048 to their right fill a round of smaller tiles.
 // Returns the columns of the first launch (a multiple of 256, so the right part starts on a 128-block of b_scale).
 size_t cols_for_full_rounds(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int cus,
-                            double t_single, double *t_split, size_t *padding, bool whatever_the_estimate) {
+                            double t_single, double *t_split, size_t *padding, bool whatever_the_estimate, RowCopies copies) {
     if (!g_ctx.row_split) return 0;
     const size_t tm = (M + 255) / 256, tiles = tm * ((N + 255) / 256), full = tiles / cus;
     if (full == 0 || tiles % cus == 0) return 0;
@@ -903,9 +912,9 @@ size_t cols_for_full_rounds(const Variant *tab, int count, size_t M, size_t N, s
     if (n_main == 0 || n_main >= N) return 0;
     uint32_t ns = 0;
     double t_main = 0, t_rest = 0;
-    const int vm = choose_by_cost(tab, count, M, n_main, ksteps, block, cus, false, &ns, &t_main);
+    const int vm = choose_by_cost(tab, count, M, n_main, ksteps, block, cus, false, &ns, &t_main, copies);
     if (vm < 0 || tab[vm].bm != 256 || tab[vm].bn != 256) return 0;
-    const int vr = choose_by_cost(tab, count, M, N - n_main, ksteps, block, cus, false, &ns, &t_rest);
+    const int vr = choose_by_cost(tab, count, M, N - n_main, ksteps, block, cus, false, &ns, &t_rest, copies);
     if (vr < 0) return 0;
     if (t_split) *t_split = t_main + t_rest + 6.0;
     if (padding) *padding = padded_area(256, 256, M, n_main) + padded_area(tab[vr].bm, tab[vr].bn, M, N - n_main);
@@ -919,18 +928,18 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     if (!tab) return QGEMM_ERR_UNSUPPORTED;
     uint32_t model_split = 0;
     int vi = choose_variant(tab, count, q.M, q.N, ksteps_of(q), q.block, q.kmaj, g_ctx.num_cus, q.split_k == 0, may_split_rows, q.out_dtype,
-                            &model_split);
+                            &model_split, q.copies);
     if (may_split_rows && vi >= 0 && !forced() && g_ctx.force_split <= 0 && q.split_k == 0 && model_split <= 1 &&
         q.M > 128 && q.kmaj == 0) {
         uint32_t ns = 0;
         double t_single = 0;
-        const int ci = choose_by_cost(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, false, &ns, &t_single);
+        const int ci = choose_by_cost(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, false, &ns, &t_single, q.copies);
         if (ci >= 0 && tab[ci].bm == tab[vi].bm && tab[ci].bn == tab[vi].bn && tab[ci].kgroups == tab[vi].kgroups) {
             double t_rows = 0, t_cols = 0;
             size_t pad_rows = 0, pad_cols = 0;
-            size_t m_main = rows_for_full_rounds(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, t_single, &t_rows, &pad_rows);
+            size_t m_main = rows_for_full_rounds(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, t_single, &t_rows, &pad_rows, q.copies);
             size_t n_main = g_ctx.row_split == 2 ? 0
-                                : cols_for_full_rounds(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, t_single, &t_cols, &pad_cols, m_main != 0);
+                                : cols_for_full_rounds(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, t_single, &t_cols, &pad_cols, m_main != 0, q.copies);
             // The columns by themselves where they are estimated at least 2.5 % ahead of the single launch, as the rows are.
             // Where the rows pass that test, the columns take their place if they are estimated 5 % faster, or no more
             // than 5 % slower with tiles that compute less beyond the matrix: the estimate prices tiles, not the rows in
@@ -979,6 +988,8 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     a.N = (uint32_t)q.N;
     a.ksteps = (uint32_t)ksteps_of(q);
     a.k_tail = (uint32_t)(q.Kbytes % 128);
+    a.k_rest = (uint32_t)q.k_rest;
+    if (q.k_rest && !v.launch_rest) return QGEMM_ERR_UNSUPPORTED;
     a.lda = (uint32_t)q.lda_bytes;
     a.ldb = (uint32_t)q.ldb_bytes;
     const uint32_t tiles_m = (uint32_t)((q.M + v.bm - 1) / v.bm), tiles_n = (uint32_t)((q.N + v.bn - 1) / v.bn);
@@ -1107,7 +1118,7 @@ int run_nt(const NtProblem &q, Plan &pl, void *split_ws, hipStream_t stream) {
                                        : (v.bm == 256 && v.bn == 256 && ob == 4 && pl.tiles < 3 * (size_t)g_ctx.num_cus);
         a.stagger_wgs = (uint32_t)g_ctx.num_cus;
         a.stagger_groups = (uint32_t)std::max<long>(1, std::min<long>(32, g_ctx.stagger_groups));
-        hipError_t e = v.launch(a, (uint32_t)pl.tiles, stream);
+        hipError_t e = (a.k_rest ? v.launch_rest : v.launch)(a, (uint32_t)pl.tiles, stream);
         g_ctx.last_config = std::string(v.name) + kmaj_suffix(q.kmaj);
         return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
     }
@@ -1119,7 +1130,7 @@ int run_nt(const NtProblem &q, Plan &pl, void *split_ws, hipStream_t stream) {
     a.split_stride = plane;
     a.out_dtype = i32_acc ? QGEMM_DT_I32 : QGEMM_DT_F32;
     a.per_matrix_scale = 0;
-    hipError_t e = v.launch(a, (uint32_t)(pl.tiles * a.nsplit), stream);
+    hipError_t e = (a.k_rest ? v.launch_rest : v.launch)(a, (uint32_t)(pl.tiles * a.nsplit), stream);
     if (e != hipSuccess) return QGEMM_ERR_LAUNCH;
 
     const uint32_t per_row = (uint32_t)((q.N + 3) / 4);
@@ -1267,32 +1278,60 @@ double few_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N,
     return m.fixed + (double)((wgs + slots - 1) / slots) * (m.round + n * (m.alone + (m.full - m.alone) * load));
 }
 
-// Is a product on the any-shape path faster packed?  Estimates of both, in microseconds, fitted on 240 ragged shapes (1 .. 4096
-// rows x 1024 .. 7168 columns x K = 777 .. 7161; fp8 and int8 with one scale and with block scales, bf16), eager calls, before
-// gemm_few_kernel and faster row ends in pack_kernel; on 150 other shapes with both the way chosen is 1.1 % behind the faster one
-// on average, 59 % at worst (bf16 657 x 4159 x 4585 79.2 / 49.7), and a smaller constant part (7 .. 10.5 for 12) is level with it
-// (0.9 - 1.3 %).  Two thresholds on the sizes, K and M N, were 21 % behind on average.  Unpacked / packed: int8 1 x 2048 x 1032
-// 7.9 / 11.5, 512 x 3000 x 1500 11.3 / 18.5, 1024 x 4096 x 2001 26.5 / 23.7, 4096 x 4096 x 2001 74.9 / 42.0, fp8 64 x 7168 x 2056
-// 10.3 / 19.1, 512 x 2048 x 1032 11.2 / 14.7, 4096 x 4608 x 7161 357 / 229, bf16 512 x 2048 x 1036 11.5 / 15.8, 2048 x 3000 x 1500
-// 39.7 / 31.6.
+// Is a product on the any-shape path faster packed?  Estimates of both, in microseconds, fitted on ragged shapes (1 .. 4096
+// rows x 1024 .. 7168 columns x K = 777 .. 7161; fp8 and int8 with one scale and with block scales, bf16), eager calls; two thresholds on
+// the sizes, K and M N, were 21 % behind on average.  (The constant part of packing was 12 as long as every call that used the workspace
+// recorded an event.  Unpacked / packed: int8 1002 x 2558 x 2881 with block scales 39.5 / 26.0, 353 x 11549 x 2008 30.5 / 26.1, bf16 485 x
+// 1024 x 2075 18.6 / 16.0, 344 x 1664 x 515 8.0 / 9.5, fp8 501 x 2190 x 1638 18.6 / 16.1.)
 // Operands that are transposed on the way (km) make the any-shape kernel twice as slow: thresholds do there (bf16 with B stored
 // K x N 1024 x 2049 x 261 15.5 / 15.7, x 401 18.4 / 16.7).
+// Rows at any address.  Share of them that start at no multiple of four (any distance between them), and RowCopies of such an operand: the
+// copies of one CU, out of the L2 and with nothing else to do, reach 110 GB/s on whole lines, 75 off them and 36 where addresses are no
+// multiple of four; fitted on products, 60 and 30.
+double odd_rows(const void *p, size_t ld) {
+    int odd = 0;
+    for (size_t r = 0; r < 4; ++r) odd += ((uintptr_t)p + r * ld) % 4 != 0;
+    return odd / 4.0;
+}
+double row_copy(const void *p, size_t ld) {
+    if (((uintptr_t)p | ld) % 16 == 0) return 0;
+    const double odd = odd_rows(p, ld);
+    return 128.0 * ((1 - odd) / 60.0e3 + odd / 30.0e3);
+}
+// Time of a product on the MFMA rows, us: the tiles' estimate or, up to `few` rows, the skinny-M kernel's (see choose_variant), < 0 for none
+double rows_estimate(const NtProblem &q, size_t few) {
+    int count = 0;
+    const Variant *tab = table_for(q.arith, q.block, q.kmaj, &count);
+    uint32_t nsplit = 0;
+    double t = 0;
+    const size_t steps = ksteps_of(q), cus = g_ctx.num_cus;
+    if (!tab) return -1;
+    const int vi = choose_by_cost(tab, count, q.M, q.N, steps, q.block, (int)cus, q.split_k == 0, &nsplit, &t, q.copies);
+    if (vi < 0) return -1;
+    if (q.kmaj) return tab[vi].copy_waves ? t : 1.15 * t;
+    if (q.M <= few) {
+        const size_t bm = q.M <= 16 ? 16 : (q.M <= 32 ? 32 : 64), strips = ((q.M + 63) / 64) * ((q.N + 31) / 32);
+        const double piece = 128.0 / 50.0e3;
+        t = std::min(t, std::max(4.0, (bm * std::max(piece, q.copies.a) + 32 * std::max(piece, q.copies.b)) * steps) * std::max(1.0, (double)strips / cus));
+    }
+    return t;
+}
+// Packed: another launch that reads and writes both operands, then rows of whole K steps (q: the product; kbytes: its K).  Where an fp32
+// output shows how sums are made, packed rows sum less exactly than the any-shape kernel (bf16 1445 x 640 x 1095 8.5e-8 / 7.8e-8 of the
+// result) and keep the 12 us that a call with workspace once had as its constant part, so that no product comes to them for being faster now.
+double packed_estimate(NtProblem q, size_t kbytes) {
+    q.Kbytes = kbytes;
+    q.kmaj = 0;
+    q.copies = {};
+    const bool shows = output_shows_sums(q.arith, q.block, q.out_dtype);
+    const double t = rows_estimate(q, shows || q.arith != AR_F8W ? 256 : 64);
+    return t < 0 ? 1e30 : (shows ? 12.0 : 6.3) + 0.2e-6 * (double)(q.M + q.N) * kbytes + (shows ? 1.0 : 1.05) * t;
+}
 enum class Packing { NO, YES, UNLESS_FEW_ROWS };        // UNLESS_FEW_ROWS: gemm_few_kernel is faster still
 Packing pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
-    const size_t kbytes = K * dtype_bytes(in_dtype), cus = g_ctx.num_cus;
+    const size_t kbytes = K * dtype_bytes(in_dtype);
     if (km) return kbytes > 512 || (double)q.M * q.N >= 4e6 ? Packing::YES : Packing::NO;
-    // packed: two launches and the packing, then the tiles' estimate or the skinny-M kernel's (see choose_variant)
-    int count = 0;
-    const Variant *tab = table_for(q.arith, q.block, 0, &count);
-    uint32_t nsplit = 0;
-    double t_rows = 0;
-    const size_t steps = (kbytes + 127) / 128;
-    if (!tab || choose_by_cost(tab, count, q.M, q.N, steps, q.block, (int)cus, true, &nsplit, &t_rows) < 0) return Packing::NO;
-    if (q.M <= 256) {
-        const size_t bm = q.M <= 16 ? 16 : (q.M <= 32 ? 32 : 64), strips = ((q.M + 63) / 64) * ((q.N + 31) / 32);
-        t_rows = std::min(t_rows, std::max(4.0, (bm + 32) * steps * 128.0 / 50.0e3) * std::max(1.0, (double)strips / cus));
-    }
-    const double t_packed = 12.0 + 0.2e-6 * (double)(q.M + q.N) * kbytes + t_rows;
+    const double t_packed = packed_estimate(q, kbytes);
     if (t_packed >= any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K)) return Packing::NO;
     return t_packed >= few_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K) ? Packing::UNLESS_FEW_ROWS : Packing::YES;
 }
@@ -1302,7 +1341,7 @@ Packing pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
 // the operands as the caller has them, ld in bytes between rows, or, k_major, between rows of k.  q: everything else, with
 // the caller's K.  *taken = false, and nothing launched, where the any-shape kernel is the one to run (launch_any), which
 // needs no memory but the operands:
-//   * calls that are captured and calls on the static scratch: replays of a captured graph, and the calls of several threads
+//   * calls that are captured and calls on the static scratch (which launch_unaligned may take first): replays of a captured graph, and the calls of several threads
 //     on the scratch, are ordered by nobody, and packed operands in a block that they share would overwrite each other.
 //     (The choice does not depend on how much room there happens to be: a call captured twice gives the same bits.)
 //   * the device has no memory left for the workspace, or the shape exceeds what the MFMA kernels index;
@@ -1392,6 +1431,74 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
     }
     st = run_nt(q, pl, ws, stream);
     g_ctx.last_config = "pack+" + g_ctx.last_config;
+    return st;
+}
+
+// Operands whose rows start or end anywhere, on the MFMA kernels as they stand: A, and B where it is N x K, may have any address, row
+// distance and K of 16 bytes or more (see gemm_rest); B stored K x N only lets K end inside a chunk.  Which of the three ways a product
+// goes is a matter of estimates, fitted on drawn ragged products: the tiles' own estimate runs low here, the copies being bound by a rate
+// that LDS reads share, more so off multiples of four; on 70 programs that quantise and multiply, multiply or train a layer, operands changing
+// from pass to pass, the way chosen is 2.3 % behind the fastest of the three.  Whole programs, us, as they stand / packed / any-shape kernel:
+// fp16 510 x 3024 x 3026 with B stored K x N 23.5 / 29.4 / 41.0, 203 x 4320 x 1381 14.2 / 20.4 / 22.3, int8 7523 x 1024 x 1548 21.0 / 25.8 /
+// 27.8, fp8 with block scales 164 x 1152 x 2407 15.2 / 17.4 / 25.4, training 2759 x 768 x 2304 55.7 / 59.1 / 76.3; but fp16 779 x 3968 x 3615 59.0 /
+// 39.0 / 80.6, int8 1531 x 4100 x 3004 38.7 / 36.9 / 52.4, fp8 block 3942 x 4992 x 2901 135 / 122 / 187.
+bool unaligned_pays(NtProblem &q, int in_dtype, size_t K, bool may_pack) {
+    const double few = q.kmaj ? 1e30 : few_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K);
+    if (few < 1e30) q.split_k = 1;               // (that kernel needs no second launch)
+    double t = rows_estimate(q, q.arith == AR_F8W ? 64 : 256);
+    if (t < 0) return false;
+    t *= 1.25 + (q.arith == AR_F8W ? 0 : 0.2) * (odd_rows(q.A, q.lda_bytes) + (q.kmaj ? 0 : odd_rows(q.B, q.ldb_bytes))) / 2;
+    if (!q.kmaj) {
+        if (few < 1e30) t *= 1.35;
+        constexpr double least = 4.3;            // (what a call takes the host)
+        if (std::max(least, t) >= std::max(least, std::min(few, any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K)))) return false;
+    }
+    return !may_pack || t < packed_estimate(q, K * dtype_bytes(in_dtype));
+}
+// *taken as for launch_packed.
+//   * Captured calls and calls on the static scratch run without a K split, and so without workspace.
+//   * fp32 output that shows how sums are made (output_shows_sums): 16-bit operands, where the packed rows would run, in as many parts; not
+//     with block scales, whose last block is folded in two parts here.
+int launch_unaligned(NtProblem q, int in_dtype, const SourceOperand &a_src, const SourceOperand &b_src, size_t K, hipStream_t stream,
+                     bool *taken) {
+    *taken = false;
+    const size_t eb = dtype_bytes(in_dtype);
+    if (g_ctx.any_shape != 1 && g_ctx.any_shape != 3) return QGEMM_OK;
+    if (q.arith == AR_F8) q.arith = AR_F8W;
+    if (a_src.k_major || (b_src.k_major && (eb != 2 || b_src.ld % 16 != 0 || !aligned16(b_src.p)))) return QGEMM_OK;
+    if (q.M >= ((size_t)1 << 31) || q.N >= ((size_t)1 << 31) || K >= ((size_t)1 << 30) || K * eb < 16) return QGEMM_OK;
+    const bool may_pack = !g_ctx.static_call && !stream_is_capturing(stream), choose = g_ctx.any_shape == 1;
+    const NtProblem whole = q;
+    q.k_rest = K * eb % 16;
+    q.Kbytes = K * eb - q.k_rest;
+    q.A = a_src.p;
+    q.B = b_src.p;
+    q.lda_bytes = a_src.ld;
+    q.ldb_bytes = b_src.ld;
+    q.kmaj = b_src.k_major ? 2 : 0;
+    q.copies = {row_copy(q.A, q.lda_bytes), q.kmaj ? 0 : row_copy(q.B, q.ldb_bytes)};
+    if (!may_pack) q.split_k = 1;
+    if (!mfma_sizes_ok(q) || (choose && !unaligned_pays(q, in_dtype, K, may_pack))) return QGEMM_OK;
+    Plan pl;
+    if (plan_nt(q, pl) != QGEMM_OK || !settle_scale_layout(q, pl)) return QGEMM_OK;
+    if (choose && output_shows_sums(q.arith, q.block, q.out_dtype)) {
+        NtProblem packed = whole;
+        packed.arith = q.arith;
+        packed.Kbytes = packed.lda_bytes = packed.ldb_bytes = (K * eb + 127) / 128 * 128;
+        Plan other;
+        if (!may_pack || q.block || q.arith == AR_F8W || pl.rest || pack_pays(packed, in_dtype, K, b_src.k_major) != Packing::YES || plan_nt(packed, other) != QGEMM_OK || other.rest ||
+            !sums_as_exact(q.arith, q.block, q.out_dtype, {(uint32_t)other.v->kgroups, other.a.nsplit}, {(uint32_t)pl.v->kgroups, pl.a.nsplit}))
+            return QGEMM_OK;
+    }
+    void *ws = nullptr;
+    if (pl.split_bytes) {
+        const int st = ensure_workspace_locked(pl.split_bytes, stream, &ws);
+        if (st == QGEMM_ERR_ALLOC) return QGEMM_OK;
+        if (st != QGEMM_OK) return st;
+    }
+    *taken = true;
+    const int st = run_nt(q, pl, ws, stream);
+    g_ctx.last_config = "unaligned+" + g_ctx.last_config;
     return st;
 }
 
@@ -1744,8 +1851,7 @@ QGEMM_EXPORT int qgemm_plan_out(int in_dtype, int out_dtype, int scale_mode, int
     if (!out_dtype_ok(in_dtype, out_dtype) || (scale_mode == QGEMM_SCALE_BLOCK128 && out_dtype == QGEMM_DT_I32)) return QGEMM_ERR_UNSUPPORTED;
     std::lock_guard<std::mutex> lock(g_ctx.mu);          // no device call below: 256 CUs are assumed before qgemm_init
     const size_t eb = (arith == AR_BF16 || arith == AR_F16) ? 2 : 1;
-    NtProblem q;
-    std::memset(&q, 0, sizeof(q));
+    NtProblem q = NtProblem();
     q.arith = arith;
     q.block = scale_mode == QGEMM_SCALE_BLOCK128;
     q.M = M;
@@ -1860,8 +1966,7 @@ QGEMM_EXPORT int qgemm_gemm(int in_dtype, int out_dtype, int layout_b, const voi
     WorkspaceUse ws_use(stream);
 
     const size_t eb = dtype_bytes(in_dtype);
-    NtProblem q;
-    std::memset(&q, 0, sizeof(q));
+    NtProblem q = NtProblem();
     q.arith = arith;
     q.block = false;
     q.A = A;
@@ -1908,6 +2013,8 @@ QGEMM_EXPORT int qgemm_gemm(int in_dtype, int out_dtype, int layout_b, const voi
     if (M >= ((size_t)1 << 32) || N >= ((size_t)1 << 32) || K >= ((size_t)1 << 32)) return QGEMM_ERR_TOO_LARGE;
     const SourceOperand a_src{A, ldA * eb, false}, b_src{B, ldB * eb, layout_b == QGEMM_B_KN};
     bool taken = false;
+    st = launch_unaligned(q, in_dtype, a_src, b_src, K, stream, &taken);
+    if (taken || st != QGEMM_OK) return st;
     st = launch_packed(q, in_dtype, a_src, b_src, K, stream, &taken);
     return taken ? st : launch_any(q, in_dtype, a_src, b_src, K, stream);
 }
@@ -1949,8 +2056,7 @@ int scaled_gemm_entry(bool use_static, int in_dtype, int out_dtype, int scale_mo
 
     const bool block = scale_mode == QGEMM_SCALE_BLOCK128;
     const uint32_t KB = (uint32_t)((K + 127) / 128), NBLK = (uint32_t)((N + 127) / 128);
-    NtProblem q;
-    std::memset(&q, 0, sizeof(q));
+    NtProblem q = NtProblem();
     q.arith = arith_of(in_dtype);
     q.block = block;
     q.C = C;
@@ -2025,6 +2131,8 @@ int scaled_gemm_entry(bool use_static, int in_dtype, int out_dtype, int scale_mo
     const bool km = layout == QGEMM_LAYOUT_REFERENCE;
     const SourceOperand a_src{A, km ? M : K, km}, b_src{B, km ? N : K, km};
     bool taken = false;
+    st = launch_unaligned(q, in_dtype, a_src, b_src, K, stream, &taken);
+    if (taken || st != QGEMM_OK) return st;
     st = launch_packed(q, in_dtype, a_src, b_src, K, stream, &taken);
     return taken ? st : launch_any(q, in_dtype, a_src, b_src, K, stream);
 }
@@ -2303,3 +2411,4 @@ QGEMM_EXPORT int qgemm_selftest_layouts(char *buf, size_t buflen) {
 }
 
 }  // extern "C"
+

@@ -25,6 +25,7 @@ struct Variant {
     int twin;
     int ks_blocks;
     hipError_t (*launch)(const GemmArgs &, uint32_t grid, hipStream_t);
+    hipError_t (*launch_rest)(const GemmArgs &, uint32_t grid, hipStream_t);      // where K ends inside a chunk (GemmArgs::k_rest); null: never
 };
 
 // one translation unit per arithmetic family defines one of these
