@@ -124,8 +124,8 @@ int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int la
 
 /* Library workspace (no reference counterpart: the reference's entries take none).  Calls that split K, that
  * take operands or scales in an arrangement the kernels do not read directly, and the per-matrix quantiser where it makes two passes
- * (above 256 KiB while captured; otherwise above 128 KiB with gaps between the rows, which then count rounded up to 16 bytes each, or at
- * addresses that are no multiple of 4, and above 32 MiB) keep their intermediate data in device blocks owned by the library
+ * (above 256 KiB: while captured, at addresses that are no multiple of 4, and above 32 MiB; outside a capture above 128 KiB with gaps
+ * between the rows, which count rounded up to 16 bytes each) keep their intermediate data in device blocks owned by the library
  * and grown on demand.  A block that is outgrown is replaced but stays allocated until qgemm_shutdown, so launches already enqueued and graphs
  * already captured remain valid.  The first three streams that need one have a block each; calls on further streams share
  * a fourth, and each such call waits (on the device, through an event) for the previous user on another stream.  While a

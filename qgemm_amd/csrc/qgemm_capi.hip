@@ -1627,8 +1627,8 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         // (an empty matrix is for the forms that look whether a row has a piece: the others load without asking)
         const bool row_ends = a.cols == 0 || a.cols % P::VEC != 0, one_row = a.rows == 1;
         auto form = [&](auto one_ragged, auto one, auto rows_ragged, auto rows) { return one_row ? (row_ends ? one_ragged : one) : row_ends ? rows_ragged : rows; };
-        const bool capturing = pieces * 16 > kQuantSmallBytes && stream_is_capturing(stream);
-        if (pieces * 16 <= kQuantSmallBytes || (capturing && pieces * 16 <= kQuantSmallCapturedBytes)) {
+        const bool small = pieces * 16 <= (one_row ? kQuantSmallBytes : kQuantSmallRowsBytes), capturing = !small && stream_is_capturing(stream);
+        if (small || (capturing && pieces * 16 <= kQuantSmallBytes)) {
             e = launch_kernel(form(quant_small_matrix_kernel<IN_DT, OUT_DT, true, true>, quant_small_matrix_kernel<IN_DT, OUT_DT, true, false>,
                                    quant_small_matrix_kernel<IN_DT, OUT_DT, false, true>, quant_small_matrix_kernel<IN_DT, OUT_DT, false, false>),
                               dim3((unsigned)std::max<uint64_t>(1, (pieces + 1023) / 1024)), dim3(1024), 0, stream, a);

@@ -409,11 +409,12 @@ __device__ inline Divisor matrix_divisor(uint32_t m) {
 }
 
 // Small: one launch, no workspace.  Every workgroup takes the maximum of the whole matrix, then quantises its own 1024 pieces.
-// A workgroup reads some 100 GB/s, so this ends where that takes as long as the exchange of quant_whole_matrix_kernel (bf16, us, this /
-// exchange: 16 x 2048 (64 KiB) 6.2 / 6.2, 48 x 2048 (192 KiB) 7.2 / 6.5, 64 x 2048 7.2 / 6.5) or, with gaps between the rows and a division for
-// every piece, as a second launch (graph replays, us, this / two passes: 64 x 512 (64 KiB) 4.3 / 4.8, 64 x 1024 4.4 / 5.2, 40 x 2176 (170 KiB) 7.6 /
-// 5.2).  A stream that is being captured, which has neither the exchange nor more workspace than is there, stays on this to kQuantSmallCapturedBytes.
-constexpr uint64_t kQuantSmallBytes = 128 << 10, kQuantSmallCapturedBytes = 256 << 10;
+// A workgroup reads some 100 GB/s, so this ends where the exchange of quant_whole_matrix_kernel, which a call has to look for a capture for (0.25 us
+// of host time, and calls of this size are bound by that), is ahead of it by as much: bf16, us a call among others / on the GPU alone, this: 48 x 2048
+// (192 KiB) 5.0 / 7.2, exchange 5.1 / 6.5; 128 x 2048 (512 KiB) 7.1 / 9.4 and 6.7 / 7.2.  With gaps between the rows and a division for every piece it
+// ends where two passes are ahead (kQuantSmallRowsBytes; graph replays, us, this / two passes: 64 x 512 (64 KiB) 4.3 / 4.8, 64 x 1024 4.4 / 5.2,
+// 40 x 2176 (170 KiB) 7.6 / 5.2), but for a stream that is being captured, which has no more workspace than is there.
+constexpr uint64_t kQuantSmallBytes = 256 << 10, kQuantSmallRowsBytes = 128 << 10;
 template <int IN_DT, int OUT_DT, bool ONE_ROW, bool RAGGED>
 __global__ void __launch_bounds__(1024) quant_small_matrix_kernel(const QuantArgs p) {
     const MatrixPieces<IN_DT, ONE_ROW, RAGGED> x(p, 0);

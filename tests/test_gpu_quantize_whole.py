@@ -35,7 +35,7 @@ def _check(x, xf):
 def test_either_side_of_every_form(dt, vec, elements):
     """`small`: the last matrix whose maximum every workgroup takes by itself; `groups`: the first that needs all workgroups; n: the
     last of n pieces a lane."""
-    at = {"small": 8192 * vec, "first": 9 * 1024 * vec, "groups": (LANES - 1024) * vec}.get(elements) or elements * LANES * vec
+    at = {"small": 16384 * vec, "first": 17 * 1024 * vec, "groups": (LANES - 1024) * vec}.get(elements) or elements * LANES * vec
     for n in (at - 1, at, at + 1, at + vec):
         say("quantize whole", dt, n)
         x = torch.from_numpy(R.fill_normal((1, n), 71)).to(dt).cuda()
