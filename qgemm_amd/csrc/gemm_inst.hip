@@ -108,8 +108,8 @@ static std::vector<Variant> build_table() {
     // no more tiles than CUs, where the two-stage row above would sit alone on its CU
     // (K-major families too: the waves that read the tile with the transposing LDS reads have no copies in flight)
     if constexpr (kmajor_can(128, 128, 4) && !kWide) add(gemm_row<Simple<128, 128, 2, 2, kBlock ? 4 : 5, 2>>("128x128_w2x2_k2", true));
-    // the same for the 64 x 128 tile, with six stages
-    if constexpr (kmajor_can(64, 128, 4)) add(gemm_row<Simple<64, 128, 1, 4, 6, 2>>("64x128_w1x4_k2", true));
+    // the same for the 64 x 128 tile, with six stages (K-major bytes: see GemmCfg::KMA64)
+    if constexpr (kmajor_can(64, 128, 4) || (INST_KMAJ == 3 && kElemBytes == 1)) add(gemm_row<Simple<64, 128, 1, 4, 6, 2>>("64x128_w1x4_k2", true));
     if constexpr (INST_KMAJ == 0) {
         // The 256 x 256 tile: fp8 per-matrix runs fastest on the 4-wave solo schedule (a third fewer LDS reads: 3 % in
         // interleaved runs); for int8 and the 16-bit types the table marks the 8-wave one and choose_variant swaps in

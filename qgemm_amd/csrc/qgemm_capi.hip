@@ -355,6 +355,8 @@ bool mfma_shape_ok(const NtProblem &q) { return q.lda_bytes % 16 == 0 && q.ldb_b
 // rounds; fp8 165.9 -> 163.7 us, block scales 206.9 -> 198.1, bf16 327.4 -> 318.5; over the 71 of 1440 grid shapes
 // whose plan changed the new plan is 3.0 % faster on average, at worst 1.6 % slower).
 // A K split adds 4 us and the partial planes at 3 TB/s.
+// The reference's storage has 64 x 128 with two K groups as well: few rows left most of a 128-row tile empty and most CUs idle (fp8_mm, us,
+// 128 x 128 / so: 32 x 1280 x 832 7.4 / 6.3, 96 x 1536 x 3328 11.3 / 10.0, 288 x 4736 x 3840 18.0 / 15.8, 544 x 1792 x 3072 15.8 / 13.2).
 //
 // M <= 64 (bandwidth-bound, B is streamed once): the largest tile that still gives three quarters of the CUs a
 // workgroup, else the shortest tile that covers the rows; narrow tiles instead of a K split.  (65 .. 128 rows go
