@@ -110,6 +110,10 @@ static std::vector<Variant> build_table() {
     if constexpr (kmajor_can(128, 128, 4) && !kWide) add(gemm_row<Simple<128, 128, 2, 2, kBlock ? 4 : 5, 2>>("128x128_w2x2_k2", true));
     // the same for the 64 x 128 tile, with six stages (K-major bytes: see GemmCfg::KMA64)
     if constexpr (kmajor_can(64, 128, 4) || (INST_KMAJ == 3 && kElemBytes == 1)) add(gemm_row<Simple<64, 128, 1, 4, 6, 2>>("64x128_w1x4_k2", true));
+    // 64 x 64 with as many stages as let two workgroups share a CU, for mid-sized products of few tiles (eight stages, one workgroup per CU,
+    // are level or slower); K-contiguous families take it by a rule of choose_by_rules only
+    if constexpr ((kmajor_can(64, 64, 4) || (INST_KMAJ == 3 && kElemBytes == 1)) && !kWide)
+        add(gemm_row<Simple<64, 64, 2, 2, kBlock ? 4 : 5, 2>>("64x64_w2x2_k2", INST_KMAJ != 0));
     if constexpr (INST_KMAJ == 0) {
         // The 256 x 256 tile: fp8 per-matrix runs fastest on the 4-wave solo schedule (a third fewer LDS reads: 3 % in
         // interleaved runs); for int8 and the 16-bit types the table marks the 8-wave one and choose_variant swaps in

@@ -178,9 +178,9 @@ struct GemmCfg {
                   "solo with block scales: the accumulators have to live in the 256 vector registers of a wave");
     static_assert(PIPE == PIPE_SIMPLE || (RBA * 2) % NW == 0, "A loads must divide evenly over the waves");
     static_assert(KMAJ == 0 || NW % 4 == 0, "K-major tiles: the swizzle of a copy must not depend on the instruction");
-    // KMA64: the K-major A side is half a panel (see kmajor_swz64); the rows with two K groups, whose copying waves know it
-    static constexpr bool KMA64 = KMA && BM * ES == 64 && ES == 1 && KGROUPS_ == 2;
-    static_assert((!KMA || KMA64 || (BM * ES) % 128 == 0) && (!KMB || (BN * ES) % 128 == 0),
+    // KMA64, KMB64: a K-major side is half a panel (see kmajor_swz64); the rows with two K groups, whose copying waves know it
+    static constexpr bool KMA64 = KMA && BM * ES == 64 && ES == 1 && KGROUPS_ == 2, KMB64 = KMB && BN * ES == 64 && ES == 1 && KGROUPS_ == 2;
+    static_assert((!KMA || KMA64 || (BM * ES) % 128 == 0) && (!KMB || KMB64 || (BN * ES) % 128 == 0),
                   "K-major tiles are made of whole 128-byte panels");
     // The compiler makes every transposing LDS read wait for all global->LDS copies in flight (vmcnt(0)): it cannot
     // tell that they target another buffer.  The simple pipeline issues the next stage's copies behind the reads
@@ -517,8 +517,9 @@ gemm_nt_kernel(QGEMM_HEAD, const GemmArgs p) {
     const int ld_chunk_km = (lane & 7) ^ kmajor_swz<C::ES>(ld_r + 16 * ((lw >> 1) & 1));
     // (KMA64: an instruction brings 16 k rows)
     const int ld_chunk_64 = (lane & 7) ^ (((lane >> 4) & 1) | ((lw & 1) << 1));
-    const uint32_t voff_a = C::KMA64 ? (2 * (lane >> 3) + (ld_chunk_64 >> 2)) * lda + (ld_chunk_64 & 3) * 16 : ld_r * lda + (C::KMA ? ld_chunk_km : ld_chunk) * 16;
-    const uint32_t voff_b = ld_r * ldb + (C::KMB ? ld_chunk_km : ld_chunk) * 16;
+    const int ld_r_64 = 2 * (lane >> 3) + (ld_chunk_64 >> 2);
+    const uint32_t voff_a = C::KMA64 ? ld_r_64 * lda + (ld_chunk_64 & 3) * 16 : ld_r * lda + (C::KMA ? ld_chunk_km : ld_chunk) * 16;
+    const uint32_t voff_b = C::KMB64 ? ld_r_64 * ldb + (ld_chunk_64 & 3) * 16 : ld_r * ldb + (C::KMB ? ld_chunk_km : ld_chunk) * 16;
     // (the chunk of a lane is the same in every copy instruction of every pipeline: (lane & 7) - (lane >> 3) mod 8)
     const uint32_t tail_or = (has_tail && (uint32_t)ld_chunk * 16 >= k_tail) ? 0x80000000u : 0u;
     const uint32_t voff_a_t = C::KMA ? voff_a : (voff_a | tail_or), voff_b_t = C::KMB ? voff_b : (voff_b | tail_or);
@@ -656,17 +657,20 @@ gemm_nt_kernel(QGEMM_HEAD, const GemmArgs p) {
     // the lane's part of a fragment address in a tile of 64-byte k rows: k = 16 fg + (fr >> 1), LDS row k >> 1
     const int km64_row = 8 * fg + (fr >> 2);
     const int km64_lane = km64_row * 128 + 16 * ((((fr >> 1) & 1) << 2) ^ kmajor_swz64(km64_row)) + 8 * (fr & 1);
+    auto frag_km64 = [&](const char *tile, int x16, int half) {
+        const char *q = tile + half * (C::KE / 4) * 128 + (km64_lane ^ (16 * x16));
+        const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)q);
+        const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(q + 4 * 128));      // (eight k rows on)
+        return v4i{lo[0], lo[1], hi[0], hi[1]};
+    };
     auto frag_a = [&](const char *stage, int a, int half) {
-        if constexpr (C::KMA64) {
-            const char *q = stage + half * (C::KE / 4) * 128 + (km64_lane ^ (16 * (wm * C::TM + a)));
-            const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)q);
-            const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(q + 4 * 128));      // (eight k rows on)
-            return v4i{lo[0], lo[1], hi[0], hi[1]};
-        } else if constexpr (C::KMA) return frag_km(stage, wm * C::TM + a, half);
+        if constexpr (C::KMA64) return frag_km64(stage, wm * C::TM + a, half);
+        else if constexpr (C::KMA) return frag_km(stage, wm * C::TM + a, half);
         else return *(const v4i *)(stage + a_blk0 + a * 2048 + (half ? off1 : off0));
     };
     auto frag_b = [&](const char *stage, int b, int half) {
-        if constexpr (C::KMB) return frag_km(stage + C::RBA * 2048, wn * C::TN + b, half);
+        if constexpr (C::KMB64) return frag_km64(stage + C::RBA * 2048, wn * C::TN + b, half);
+        else if constexpr (C::KMB) return frag_km(stage + C::RBA * 2048, wn * C::TN + b, half);
         else return *(const v4i *)(stage + b_blk0 + b * 2048 + (half ? off1 : off0));
     };
 
@@ -1251,6 +1255,8 @@ gemm_nt_kernel(QGEMM_HEAD, const GemmArgs p) {
                             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, va, ((uint32_t)k * C::KE + (pw + 4 * j) * 16) * lda, 0, 0);
                         else if (2 * j < C::RBA)
                             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, va, soff_k2(C::KMA, blk, lda, kt) - back, 0, 0);
+                        else if (C::KMB64)
+                            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst, 16, vb, ((uint32_t)k * C::KE + (pw + 4 * j - 2 * C::RBA) * 16) * ldb, 0, B_NT ? 2 : 0);
                         else
                             __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst, 16, vb, soff_k2(C::KMB, blk - C::RBA, ldb, kt) - back, 0, B_NT ? 2 : 0);
                     }

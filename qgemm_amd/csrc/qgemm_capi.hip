@@ -289,6 +289,7 @@ bool out_dtype_ok(int in_dtype, int out_dtype) {
 // (0: the planner's times per step have it).
 struct RowCopies {
     double a = 0, b = 0;
+    bool tile64 = true;          // 64 x 64 with two K groups may be chosen (see copies_of)
 };
 struct NtProblem {
     int arith;
@@ -357,6 +358,13 @@ bool mfma_shape_ok(const NtProblem &q) { return q.lda_bytes % 16 == 0 && q.ldb_b
 // A K split adds 4 us and the partial planes at 3 TB/s.
 // The reference's storage has 64 x 128 with two K groups as well: few rows left most of a 128-row tile empty and most CUs idle (fp8_mm, us,
 // 128 x 128 / so: 32 x 1280 x 832 7.4 / 6.3, 96 x 1536 x 3328 11.3 / 10.0, 288 x 4736 x 3840 18.0 / 15.8, 544 x 1792 x 3072 15.8 / 13.2).
+// The K-major families have 64 x 64 with two K groups too, two workgroups a CU: mid-sized products make few tiles, and a CU's work on one is
+// latency (start, first copies, a step of 0.18 us, the way out).  Graph replays, us, the best other row / so: B stored K x N bf16 505 x 1056 x
+// 531 8.7 / 6.6, 512 x 512 x 2048 11.7 / 9.2, 384 x 1280 x 1184 8.2 / 7.0, 64 x 2816 x 560 6.1 / 5.1; fp8_mm 160 x 3168 x 448 5.7 / 4.6, 1024 x
+// 544 x 2080 9.7 / 7.7, 512 x 1984 x 1792 9.0 / 7.4.  136 shapes of 32 .. 1280 rows: 7 - 24 % ahead wherever there are no more tiles than
+// CUs; with more, two share a CU and most shapes are behind (fp8_mm 640 x 2432 x 3136, 380 tiles, 13.6 / 18.3).  In the K-contiguous
+// families, whose other rows need no transposing reads, it is level or behind, but for what choose_by_rules gives it.  From 1024 x 1024 on it is left out: more tiles than CUs,
+// but for that square itself, whose plan is pinned by name (x 1024 bf16 7.8 / 6.9).
 //
 // M <= 64 (bandwidth-bound, B is streamed once): the largest tile that still gives three quarters of the CUs a
 // workgroup, else the shortest tile that covers the rows; narrow tiles instead of a K split.  (65 .. 128 rows go
@@ -378,7 +386,8 @@ struct TileModel {
 const TileModel kTileModels[] = {{256, 256, 1, 1.25, 1.25, 4.0, false, 1, 1.40, 1.40}, {128, 128, 2, 0.85, 0.66, 2.0, false, 2, 1.32, 1.04},
                                  {128, 128, 1, 0.43, 0.43, 4.5, true, 1, 0.50, 0.50},  {64, 128, 1, 0.52, 0.52, 1.5, false, 3, 1.21, 0.83},
                                  {64, 128, 1, 0.27, 0.27, 4.5, true, 1, 0.34, 0.34},   {128, 32, 1, 0.39, 0.39, 1.0, false, 2, 0.74, 0.60},
-                                 {256, 128, 1, 0.71, 0.58, 6.0, false, 1, 0.93, 0.76}, {192, 256, 1, 1.03, 0.97, 6.0, false, 1, 1.27, 1.18}};
+                                 {256, 128, 1, 0.71, 0.58, 6.0, false, 1, 0.93, 0.76}, {192, 256, 1, 1.03, 0.97, 6.0, false, 1, 1.27, 1.18},
+                                 {64, 64, 2, 0.47, 0.23, 2.9, true, 2, 0.56, 0.24}};
 // Widened fp8 (AR_F8W: packed operands): twice the matrix instructions of a 16-bit step and the conversions in front of them, on
 // the rows that family has.  Fitted on 56 ragged shapes of 1 .. 4096 rows x 1024 .. 7168 columns x 777 .. 7161, every row forced
 // (within 5 % of the measured time on average).  Priced as fp8 before, us in a kernel trace: 512 x 4608 x 7161 58.5 (128 x 128) ->
@@ -397,6 +406,14 @@ double rounds_cost(size_t wgs, size_t slots, size_t cus, size_t steps, double sh
 // rows with two K groups: two sets of computing waves on a tile that otherwise has one (one workgroup per CU)
 bool is_kgroup_row(const Variant &v) { return v.kgroups == 2; }
 
+// An fp32 output that shows how its sums are made keeps the rows, and with them the parts of a sum, that it had before the 64 x 64 tile.
+bool output_shows_sums(int arith, bool block, int out_dtype);
+RowCopies copies_of(const NtProblem &q) {
+    RowCopies c = q.copies;
+    c.tile64 = !output_shows_sums(q.arith, q.block, q.out_dtype);
+    return c;
+}
+
 int choose_by_cost(const Variant *tab, int count, size_t M, size_t N, size_t ksteps, bool block, int cus, bool may_split,
                    uint32_t *nsplit_out, double *cost_out = nullptr, RowCopies copies = {}) {
     int best = -1;
@@ -408,7 +425,7 @@ int choose_by_cost(const Variant *tab, int count, size_t M, size_t N, size_t kst
         int vi = -1;
         for (int i = 0; i < count; ++i)
             if (tab[i].auto_ok && tab[i].bm == tm.bm && tab[i].bn == tm.bn && is_kgroup_row(tab[i]) == tm.kgroups) vi = i;
-        if (vi < 0) continue;
+        if (vi < 0 || (tm.bm == 64 && tm.bn == 64 && (!copies.tile64 || (M >= 1024 && N >= 1024)))) continue;
         const size_t tiles = ((M + tm.bm - 1) / tm.bm) * ((N + tm.bn - 1) / tm.bn);
         for (uint32_t ns = 1; ns <= 8; ns *= 2) {
             if (ns > 1 && (!may_split || ksteps / ns < 4)) break;
@@ -513,6 +530,18 @@ int choose_by_rules(const Variant *tab, int count, size_t M, size_t N, size_t ks
                     return i;
                 }
     }
+    // 64 x 64 with two K groups where such tiles fit a round and 9 .. 15 K steps (block scales: 8 .. 15) are too few for the eight waves above;
+    // fewer do not pay for its start.  More than 400 rows (below, the estimate of choose_variant decides) that start on whole chunks.  Graph
+    // replays, us, the rows of the estimate (128 x 32, 64 x 128 with K groups) / so: int8 600 x 512 x 1152 5.6 / 5.3, fp8 600 x 1536 x 1792 7.3 /
+    // 6.4, bf16 896 x 688 x 768 7.1 / 6.4, block scales fp8 416 x 1728 x 1792 8.7 / 7.0, int8 1200 x 832 x 1152 7.4 / 6.0; 4 steps 4.1 / 4.5,
+    // 6 steps 4.7 / 4.8; 24 steps against the eight waves 8.3 / 8.5, 32 steps 8.6 / 10.3.
+    if (vi >= 0 && !kmaj && M > 400 && ksteps >= (block ? 8 : 9) && ksteps <= 15 && copies.tile64 && copies.a == 0 && copies.b == 0 &&
+        ((M + 63) / 64) * ((N + 63) / 64) <= (size_t)cus)
+        for (int i = 0; i < count; ++i)
+            if (tab[i].kgroups == 2 && tab[i].bm == 64 && tab[i].bn == 64) {
+                *nsplit_out = 1;
+                return i;
+            }
     if (vi < 0 || kmaj || M > 128) return vi;
     const size_t strips = (N + 31) / 32;
     // Up to 32 rows against so few columns that 32-column strips leave half of the CUs idle, 32 .. 112 K steps: strips of
@@ -828,7 +857,7 @@ bool kmajor_problem_ok(NtProblem q, int kmaj, size_t lda_bytes, size_t ldb_bytes
     const bool may_split = q.split_k == 0;
     uint32_t ns = 0;
     double t_km = 0, t_nt = 8.0;                    // a skinny K-contiguous launch: about 8 us
-    const int vk = choose_by_cost(tab_km, count_km, q.M, q.N, ksteps, q.block, g_ctx.num_cus, may_split, &ns, &t_km);
+    const int vk = choose_by_cost(tab_km, count_km, q.M, q.N, ksteps, q.block, g_ctx.num_cus, may_split, &ns, &t_km, copies_of(q));
     if (vk < 0) return false;
     if (q.M > 128 && choose_by_cost(tab, count, q.M, q.N, ksteps, q.block, g_ctx.num_cus, may_split, &ns, &t_nt) < 0)
         return false;
@@ -930,18 +959,18 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     if (!tab) return QGEMM_ERR_UNSUPPORTED;
     uint32_t model_split = 0;
     int vi = choose_variant(tab, count, q.M, q.N, ksteps_of(q), q.block, q.kmaj, g_ctx.num_cus, q.split_k == 0, may_split_rows, q.out_dtype,
-                            &model_split, q.copies);
+                            &model_split, copies_of(q));
     if (may_split_rows && vi >= 0 && !forced() && g_ctx.force_split <= 0 && q.split_k == 0 && model_split <= 1 &&
         q.M > 128 && q.kmaj == 0) {
         uint32_t ns = 0;
         double t_single = 0;
-        const int ci = choose_by_cost(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, false, &ns, &t_single, q.copies);
+        const int ci = choose_by_cost(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, false, &ns, &t_single, copies_of(q));
         if (ci >= 0 && tab[ci].bm == tab[vi].bm && tab[ci].bn == tab[vi].bn && tab[ci].kgroups == tab[vi].kgroups) {
             double t_rows = 0, t_cols = 0;
             size_t pad_rows = 0, pad_cols = 0;
-            size_t m_main = rows_for_full_rounds(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, t_single, &t_rows, &pad_rows, q.copies);
+            size_t m_main = rows_for_full_rounds(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, t_single, &t_rows, &pad_rows, copies_of(q));
             size_t n_main = g_ctx.row_split == 2 ? 0
-                                : cols_for_full_rounds(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, t_single, &t_cols, &pad_cols, m_main != 0, q.copies);
+                                : cols_for_full_rounds(tab, count, q.M, q.N, ksteps_of(q), q.block, g_ctx.num_cus, t_single, &t_cols, &pad_cols, m_main != 0, copies_of(q));
             // The columns by themselves where they are estimated at least 2.5 % ahead of the single launch, as the rows are.
             // Where the rows pass that test, the columns take their place if they are estimated 5 % faster, or no more
             // than 5 % slower with tiles that compute less beyond the matrix: the estimate prices tiles, not the rows in
@@ -1308,7 +1337,7 @@ double rows_estimate(const NtProblem &q, size_t few) {
     double t = 0;
     const size_t steps = ksteps_of(q), cus = g_ctx.num_cus;
     if (!tab) return -1;
-    const int vi = choose_by_cost(tab, count, q.M, q.N, steps, q.block, (int)cus, q.split_k == 0, &nsplit, &t, q.copies);
+    const int vi = choose_by_cost(tab, count, q.M, q.N, steps, q.block, (int)cus, q.split_k == 0, &nsplit, &t, copies_of(q));
     if (vi < 0) return -1;
     if (q.kmaj) return tab[vi].copy_waves ? t : 1.15 * t;
     if (q.M <= few) {
