@@ -1270,13 +1270,14 @@ int any_tile(int in_dtype, int out_dtype, bool block, bool km, size_t M, size_t 
 }
 
 // Time of the any-shape kernel on operands that are not transposed on the way, us: 64 x 64 tiles, three on a CU, and 128 x 128, two
-// on a CU.  (fitted as pack_pays says)
+// on a CU.  (fitted as pack_pays says; fp8 on several 64 x 64 tiles a CU had been 15 % low in whole programs: block scales 1206 x 2045 x 2481 ran
+// 43.9 us there, 37.0 packed)
 double any_estimate(int in_dtype, int out_dtype, bool block, size_t M, size_t N, size_t K) {
     struct AnyModel {
         double shared64, alone64, fixed64, shared128, alone128, fixed128;
     };
-    static const AnyModel kAny16{0.68, 0.45, 3.6, 1.29, 0.90, 10.4}, kAnyF8{0.63, 0.43, 3.2, 1.11, 0.72, 8.6},
-        kAnyF8Block{0.72, 0.48, 2.7, 1.37, 0.99, 6.6}, kAnyI8{0.81, 0.47, 3.4, 1.37, 0.94, 8.9}, kAnyI8Block{1.18, 0.67, 1.6, 0, 0, 0};
+    static const AnyModel kAny16{0.68, 0.45, 3.6, 1.29, 0.90, 10.4}, kAnyF8{0.72, 0.43, 3.2, 1.11, 0.72, 8.6},
+        kAnyF8Block{0.82, 0.48, 2.7, 1.37, 0.99, 6.6}, kAnyI8{0.81, 0.47, 3.4, 1.37, 0.94, 8.9}, kAnyI8Block{1.18, 0.67, 1.6, 0, 0, 0};
     const AnyModel &m = in_dtype == QGEMM_DT_F8E4M3 ? (block ? kAnyF8Block : kAnyF8) : (in_dtype == QGEMM_DT_I8 ? (block ? kAnyI8Block : kAnyI8) : kAny16);
     const size_t cus = g_ctx.num_cus, tile = any_tile(in_dtype, out_dtype, block, false, M, N), steps = (K - 1) / (in_dtype == QGEMM_DT_I8 ? 128 : 64) + 1;
     const size_t tiles = ((M + tile - 1) / tile) * ((N + tile - 1) / tile);
@@ -1344,6 +1345,12 @@ double rows_estimate(const NtProblem &q, size_t few) {
         const size_t bm = q.M <= 16 ? 16 : (q.M <= 32 ? 32 : 64), strips = ((q.M + 63) / 64) * ((q.N + 31) / 32);
         const double piece = 128.0 / 50.0e3;
         t = std::min(t, std::max(4.0, (bm * std::max(piece, q.copies.a) + 32 * std::max(piece, q.copies.b)) * steps) * std::max(1.0, (double)strips / cus));
+    }
+    // (widening rows of 65 rows and more: the 64 x 64 form of the skinny-M kernel, as choose_by_rules takes it; without it fp8 with block
+    // scales 184 x 4800 x 2037 ran on the any-shape kernel, 25.4 against 15.4 us)
+    if (q.arith == AR_F8W && q.M > 64 && steps >= 16 && steps <= 48) {
+        const size_t t64 = ((q.M + 63) / 64) * ((q.N + 63) / 64);
+        if (t64 >= 128 && t64 <= cus) t = std::min(t, 0.52 * steps);
     }
     return t;
 }
@@ -1476,14 +1483,17 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
 bool unaligned_pays(NtProblem &q, int in_dtype, size_t K, bool may_pack) {
     const double few = q.kmaj ? 1e30 : few_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K);
     if (few < 1e30) q.split_k = 1;               // (that kernel needs no second launch)
+    constexpr double least = 4.3;                // (what a call takes the host)
+    const double as_any = q.kmaj ? 1e30 : std::min(few, any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K));
+    if (as_any <= least) return false;
     double t = rows_estimate(q, q.arith == AR_F8W ? 64 : 256);
     if (t < 0) return false;
     t *= 1.25 + (q.arith == AR_F8W ? 0 : 0.2) * (odd_rows(q.A, q.lda_bytes) + (q.kmaj ? 0 : odd_rows(q.B, q.ldb_bytes))) / 2;
-    if (!q.kmaj) {
-        if (few < 1e30) t *= 1.35;
-        constexpr double least = 4.3;            // (what a call takes the host)
-        if (std::max(least, t) >= std::max(least, std::min(few, any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K)))) return false;
-    }
+    if (few < 1e30) t *= 1.35;
+    if (std::max(least, t) >= as_any) return false;
+    // (against packing the estimate of the widening rows runs low by 1.4, not 1.25: fp8 with block scales 2287 x 6912 x 859 as they stand /
+    // packed 52.9 / 45.1 us, 2727 x 3136 x 2283 58.5 / 54.7, one scale 3384 x 6208 x 691 54.2 / 49.0)
+    if (q.arith == AR_F8W) t *= 1.12;
     return !may_pack || t < packed_estimate(q, K * dtype_bytes(in_dtype));
 }
 // *taken as for launch_packed.
