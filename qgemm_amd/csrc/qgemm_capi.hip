@@ -38,6 +38,7 @@ struct WsBlock {
     size_t bytes = 0;
 };
 constexpr int kOwnBlocks = 3;
+constexpr size_t kLeastBlock = (size_t)64 << 20;        // what a first call allocates
 
 struct Context {
     std::mutex mu;
@@ -203,7 +204,7 @@ int ensure_workspace_locked(size_t bytes, hipStream_t stream, void **out) {
         return bytes > largest_block().bytes ? QGEMM_ERR_ALLOC : QGEMM_OK;
     }
     WsBlock *block = &g_ctx.ws[block_of(stream)], &shared = g_ctx.ws[kOwnBlocks];
-    if (grow_block(*block, bytes, (size_t)64 << 20) != QGEMM_OK) {
+    if (grow_block(*block, bytes, kLeastBlock) != QGEMM_OK) {
         // no memory, but a block of another stream would do: from here on all streams share that one, once it is idle
         WsBlock &other = largest_block();
         if (bytes > other.bytes || hipDeviceSynchronize() != hipSuccess) {
@@ -1675,11 +1676,18 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
                               dim3((unsigned)std::max<uint64_t>(1, (pieces + 1023) / 1024)), dim3(1024), 0, stream, a);
             return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
         }
+        // two passes: partial maxima, one per workgroup, in the workspace
+        const uint32_t slices = std::max<uint32_t>(1, (a.rows + a.rows_per_slice - 1) / a.rows_per_slice);
+        const uint64_t turns = ((uint64_t)a.rows_per_slice * a.per_row + 256 * kQuantTurn - 1) / (256 * kQuantTurn);
+        const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(1024, turns));
+        const size_t room = (size_t)nblk * slices * sizeof(uint32_t);
         const uint64_t most = (uint64_t)std::min(g_ctx.num_cus, kQuantGroups) * 1024;        // lanes of a launch that fits the chip
         if (g_ctx.quant_wait >= 0 && one_row && pieces <= most * kQuantMostPieces && (uintptr_t)a.x % 4 == 0 && !capturing) {
             const uint32_t whole = a.cols / P::VEC, each = (uint32_t)((whole + most - 1) / most);
             const uint32_t groups = std::max<uint32_t>(1, std::min<uint32_t>((uint32_t)(most / 1024), (whole + 1023) / 1024));
             a.share = (whole + groups - 1) / groups;
+            // (captured, the same call makes two passes in the room that an eager one has left: one that needs none itself leaves it too)
+            (void)grow_block(largest_block(), room, kLeastBlock);
             if (++g_ctx.quant_launches == 0) g_ctx.quant_launches = 1;
             a.tag = g_ctx.quant_launches;
             a.set = a.tag % kQuantSets;
@@ -1689,13 +1697,9 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
                               dim3(groups), dim3(1024), 0, stream, a);
             return e == hipSuccess ? QGEMM_OK : QGEMM_ERR_LAUNCH;
         }
-        // two passes: partial maxima (one per workgroup) into the workspace, then scale and cast
-        const uint32_t slices = std::max<uint32_t>(1, (a.rows + a.rows_per_slice - 1) / a.rows_per_slice);
-        const uint64_t turns = ((uint64_t)a.rows_per_slice * a.per_row + 256 * kQuantTurn - 1) / (256 * kQuantTurn);
-        const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(1024, turns));
         a.npartial = nblk * slices;
         void *ws = nullptr;
-        int st = ensure_workspace_locked((size_t)a.npartial * sizeof(uint32_t), stream, &ws);
+        int st = ensure_workspace_locked(room, stream, &ws);
         if (st != QGEMM_OK) return st;
         a.partial = (uint32_t *)ws;
         e = launch_kernel(form(quant_amax_kernel<IN_DT, true, true>, quant_amax_kernel<IN_DT, true, false>,

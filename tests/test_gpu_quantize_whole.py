@@ -7,6 +7,7 @@ import torch
 
 import qgemm_amd as Q
 from oracle import cpu_ref as R
+from qgemm_amd import lib as L
 from tests.util import host, say
 
 pytestmark = pytest.mark.gpu
@@ -77,6 +78,25 @@ def test_in_a_capture():
     Q.set_option("quant_wait", -1)
     Q.quantize(x, torch.int8, Q.QUANT_PER_MATRIX)            # (the workspace, outside the capture)
     Q.set_option("quant_wait", 2000)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        g, gs = Q.quantize(x, torch.int8, Q.QUANT_PER_MATRIX)
+    for i in range(4):
+        x.mul_(1.5 if i % 2 else 0.25)
+        graph.replay()
+        torch.cuda.synchronize()
+        e, es = Q.quantize(x, torch.int8, Q.QUANT_PER_MATRIX)
+        assert torch.equal(g, e) and torch.equal(gs, es), i
+
+
+def test_in_a_capture_after_one_eager_call():
+    """An eager call with the options as they are is all that a capture needs, also where nothing has used the workspace."""
+    say("quantize whole, eager, captured, replayed")
+    x = torch.from_numpy(R.fill_normal((500, 1000), 78)).bfloat16().cuda()
+    torch.cuda.synchronize()
+    L.check(L.load_library().qgemm_shutdown())
+    Q.quantize(x, torch.int8, Q.QUANT_PER_MATRIX)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
