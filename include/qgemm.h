@@ -125,18 +125,22 @@ int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int la
 /* Library workspace (no reference counterpart: the reference's entries take none).  Calls that split K, that
  * take operands or scales in an arrangement the kernels do not read directly, and the per-matrix quantiser where it makes two passes
  * (above 256 KiB: while captured, at addresses that are no multiple of 4, and above 32 MiB; outside a capture above 128 KiB with gaps
- * between the rows, which count rounded up to 16 bytes each) keep their intermediate data in device blocks owned by the library
- * and grown on demand.  A block that is outgrown is replaced but stays allocated until qgemm_shutdown, so launches already enqueued and graphs
- * already captured remain valid.  The first three streams that need one have a block each; calls on further streams share
- * a fourth, and each such call waits (on the device, through an event) for the previous user on another stream.  While a
- * stream is being captured into a graph the library neither allocates nor touches that event: such a call uses the largest
- * block there is, one that would need more returns
+ * between the rows, which count rounded up to 16 bytes each) keep their intermediate data in device blocks owned by the library:
+ * a shared one, which every call outside a capture makes as large as it needs (it at least doubles, and has 64 MiB or more), and
+ * 128 MiB each for the first three streams that ask.  A shared block that is outgrown is replaced but stays allocated until qgemm_shutdown, so
+ * launches already enqueued and graphs already captured remain valid.  Calls that need more than 128 MiB, calls on further streams, and
+ * calls for whose stream there is no memory left use the shared block, and each such call waits (on the device, through an event) for the
+ * previous user on another stream.  The first three streams keep their blocks until qgemm_shutdown, also when they are destroyed:
+ * programs should make their streams once.  While a
+ * stream is being captured into a graph the library neither allocates nor touches that event: such a call uses the shared
+ * block, one that would need more returns
  * QGEMM_ERR_ALLOC, and replays of graphs that use the workspace must not overlap other users of it.  (Products whose
  * operands would be packed into the block, see option "any_shape", do not use it while captured: their operands are read as
  * they stand, and fp32 sums have another order than those of an eager call.)
- * qgemm_reserve_workspace makes the largest block at least `bytes` large ahead of time (it allocates: call it before a
- * capture begins, never during one; a block that has to grow at least doubles); qgemm_workspace_info reports
- * its address and size (NULL / 0 before first use). */
+ * qgemm_reserve_workspace makes the shared block at least `bytes` large and the three others ahead of time, as far as there is memory for
+ * those: calls that need no more than `bytes` then allocate nothing, on any stream (it allocates: call it before a
+ * capture begins, never during one); qgemm_workspace_info reports the shared block's
+ * address and size (NULL / 0 before first use). */
 int qgemm_reserve_workspace(size_t bytes);
 int qgemm_workspace_info(void **base, size_t *bytes);
 

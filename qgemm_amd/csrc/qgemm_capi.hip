@@ -38,26 +38,30 @@ struct WsBlock {
     size_t bytes = 0;
 };
 constexpr int kOwnBlocks = 3;
-constexpr size_t kLeastBlock = (size_t)64 << 20;        // what a first call allocates
+constexpr size_t kOwnBytes = (size_t)128 << 20;         // fits all but the largest calls, whose time hides an event
+constexpr size_t kLeastBlock = (size_t)64 << 20;        // of the shared block, what a first call allocates
 
 struct Context {
     std::mutex mu;
     bool ready = false;
     int device = -1;
     int num_cus = 256;
-    // Workspace (split-K partial planes, transposed and packed operands and scales, quantiser partials).  The first kOwnBlocks
-    // streams that use it have a block each, in which their calls follow one another as the stream has them; the streams beyond
-    // those (and hipStreamPerThread, one handle for many streams) share one more, ordered through ws_event: every call that
+    // Workspace (split-K partial planes, transposed and packed operands and scales, quantiser partials): one shared block, which every
+    // eager call makes as large as it needs, and kOwnBlocks blocks of kOwnBytes, one each for the first streams that ask.  In its own
+    // block a stream's calls follow one another as the stream has them.  The shared block is for calls that need more, for the streams beyond
+    // those (and hipStreamPerThread, one handle for many streams), where there is no memory for another block, and for captured
+    // calls; its eager users are ordered through ws_event: every call that
     // used it records the event on its stream when it has enqueued its launches, and a call on another stream waits for it first.
     // (Recording costs a call 4.3 - 5.4 us of host time, twice a launch, and the GPU a packet that the next launch waits for.  With
     // one block for all streams every call that used the workspace paid that, eager calls, us: quantise 50 x 5296 fp16 to int8 per
-    // matrix 11.1 -> 8.0, quantise and multiply 1531 x 4100 x 3004 42.5 -> 36.2, forward and backward 505 x 531 x 1059 43.1 -> 37.0.)
-    // A block that is outgrown is replaced and kept in `retired` until qgemm_shutdown: launches
+    // matrix 11.1 -> 8.0, forward and backward 505 x 531 x 1059 43.1 -> 37.0, fp8_mm 2080 x 4096 x 4096 50.6 -> 47.5.)
+    // A shared block that is outgrown is replaced and kept in `retired` until qgemm_shutdown: launches
     // already enqueued and graphs already captured keep pointing at live memory.
-    WsBlock ws[kOwnBlocks + 1];                // the last one is shared
-    hipStream_t ws_stream[kOwnBlocks] = {};    // whose the others are
+    WsBlock ws;
+    WsBlock ws_own[kOwnBlocks];
+    hipStream_t ws_stream[kOwnBlocks] = {};    // whose they are
     int ws_owners = 0;
-    bool ws_all_share = false;                 // no memory for another block: every stream on the shared one from then on
+    bool ws_own_failed = false;                // there was no memory for one of them: no more are tried
     std::vector<void *> retired;
     hipEvent_t ws_event = nullptr;
     hipStream_t ws_last_stream = nullptr;
@@ -150,14 +154,6 @@ bool stream_is_capturing(hipStream_t stream) {
     return cap != hipStreamCaptureStatusNone;
 }
 
-// The largest block: what qgemm_reserve_workspace and qgemm_workspace_info speak of, and captured calls use
-WsBlock &largest_block() {
-    WsBlock *most = &g_ctx.ws[0];
-    for (WsBlock &b : g_ctx.ws)
-        if (b.bytes > most->bytes) most = &b;
-    return *most;
-}
-
 // Makes a block at least `bytes` large, twice its size if it has to grow; the old memory is retired (see Context).
 int grow_block(WsBlock &block, size_t bytes, size_t least) {
     if (bytes <= block.bytes) return QGEMM_OK;
@@ -178,21 +174,26 @@ int grow_block(WsBlock &block, size_t bytes, size_t least) {
     return QGEMM_OK;
 }
 
-// Which block a stream uses: its own where it has one or there is one left, otherwise the shared one
-int block_of(hipStream_t stream) {
-    if (g_ctx.ws_all_share || stream == hipStreamPerThread) return kOwnBlocks;
-    for (int i = 0; i < g_ctx.ws_owners; ++i)
-        if (g_ctx.ws_stream[i] == stream) return i;
-    if (g_ctx.ws_owners == kOwnBlocks) return kOwnBlocks;
-    g_ctx.ws_stream[g_ctx.ws_owners] = stream;
-    return g_ctx.ws_owners++;
+// The stream's own block, null where it has none
+void *own_block(hipStream_t stream) {
+    if (stream == hipStreamPerThread) return nullptr;
+    int i = 0;
+    while (i < g_ctx.ws_owners && g_ctx.ws_stream[i] != stream) ++i;
+    if (i == kOwnBlocks) return nullptr;
+    if (!g_ctx.ws_own[i].p) {
+        if (g_ctx.ws_own_failed) return nullptr;
+        g_ctx.ws_own_failed = grow_block(g_ctx.ws_own[i], kOwnBytes, 0) != QGEMM_OK;
+        if (g_ctx.ws_own_failed) return nullptr;
+    }
+    if (i == g_ctx.ws_owners) g_ctx.ws_stream[g_ctx.ws_owners++] = stream;
+    return g_ctx.ws_own[i].p;
 }
 
 // Workspace of `bytes` for a call enqueued on `stream`.
 //   * qgemm_scaled_gemm_static: the static scratch; larger requests are an error, nothing is allocated.
-//   * otherwise the stream's block (see Context), grown when too small.  While the stream is being captured into a graph nothing is
-//     allocated and no event is waited for or recorded: such a call takes the largest block there is, one that would need more
-//     fails with QGEMM_ERR_ALLOC (the caller reserves the room before the capture, qgemm_reserve_workspace, or runs the
+//   * otherwise the stream's own block or the shared one (see Context), which grows when too small.  While the stream is being captured into
+//     a graph nothing is allocated and no event is waited for or recorded: such a call takes the shared block, and one that would need
+//     more fails with QGEMM_ERR_ALLOC (the caller reserves the room before the capture, qgemm_reserve_workspace, or runs the
 //     call once eagerly), and ordering replays against other users of the workspace is the caller's business.
 int ensure_workspace_locked(size_t bytes, hipStream_t stream, void **out) {
     if (g_ctx.static_call) {
@@ -200,27 +201,19 @@ int ensure_workspace_locked(size_t bytes, hipStream_t stream, void **out) {
         return static_scratch_locked(out);
     }
     if (stream_is_capturing(stream)) {
-        *out = largest_block().p;
-        return bytes > largest_block().bytes ? QGEMM_ERR_ALLOC : QGEMM_OK;
+        *out = g_ctx.ws.p;
+        return bytes > g_ctx.ws.bytes ? QGEMM_ERR_ALLOC : QGEMM_OK;
     }
-    WsBlock *block = &g_ctx.ws[block_of(stream)], &shared = g_ctx.ws[kOwnBlocks];
-    if (grow_block(*block, bytes, kLeastBlock) != QGEMM_OK) {
-        // no memory, but a block of another stream would do: from here on all streams share that one, once it is idle
-        WsBlock &other = largest_block();
-        if (bytes > other.bytes || hipDeviceSynchronize() != hipSuccess) {
-            (void)hipGetLastError();
-            return QGEMM_ERR_ALLOC;
-        }
-        std::swap(shared, other);
-        g_ctx.ws_all_share = true;
-        block = &shared;
-    }
-    if (block == &shared && !g_ctx.ws_shared_by_call) {
+    const int st = grow_block(g_ctx.ws, bytes, kLeastBlock);
+    *out = bytes <= kOwnBytes ? own_block(stream) : nullptr;
+    if (*out) return QGEMM_OK;
+    if (st != QGEMM_OK) return st;
+    if (!g_ctx.ws_shared_by_call) {
         if (g_ctx.ws_event_recorded && (g_ctx.ws_last_stream != stream || stream == hipStreamPerThread))
             HIP_TRY(hipStreamWaitEvent(stream, g_ctx.ws_event, 0));
         g_ctx.ws_shared_by_call = true;
     }
-    *out = block->p;
+    *out = g_ctx.ws.p;
     return QGEMM_OK;
 }
 
@@ -1687,7 +1680,7 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
             const uint32_t groups = std::max<uint32_t>(1, std::min<uint32_t>((uint32_t)(most / 1024), (whole + 1023) / 1024));
             a.share = (whole + groups - 1) / groups;
             // (captured, the same call makes two passes in the room that an eager one has left: one that needs none itself leaves it too)
-            (void)grow_block(largest_block(), room, kLeastBlock);
+            (void)grow_block(g_ctx.ws, room, kLeastBlock);
             if (++g_ctx.quant_launches == 0) g_ctx.quant_launches = 1;
             a.tag = g_ctx.quant_launches;
             a.set = a.tag % kQuantSets;
@@ -1747,16 +1740,16 @@ QGEMM_EXPORT int qgemm_init(void) {
 
 QGEMM_EXPORT int qgemm_shutdown(void) {
     std::lock_guard<std::mutex> lock(g_ctx.mu);
-    if (largest_block().p || !g_ctx.retired.empty()) {
-        (void)hipDeviceSynchronize();
-        for (const WsBlock &b : g_ctx.ws)
-            if (b.p) (void)hipFree(b.p);
-        for (void *p : g_ctx.retired) (void)hipFree(p);
-    }
+    for (const WsBlock &b : g_ctx.ws_own)
+        if (b.p) g_ctx.retired.push_back(b.p);
+    if (g_ctx.ws.p) g_ctx.retired.push_back(g_ctx.ws.p);
+    if (!g_ctx.retired.empty()) (void)hipDeviceSynchronize();
+    for (void *p : g_ctx.retired) (void)hipFree(p);
     if (g_ctx.ws_event) (void)hipEventDestroy(g_ctx.ws_event);
-    for (WsBlock &b : g_ctx.ws) b = WsBlock();
+    g_ctx.ws = WsBlock();
+    for (WsBlock &b : g_ctx.ws_own) b = WsBlock();
     g_ctx.ws_owners = 0;
-    g_ctx.ws_all_share = false;
+    g_ctx.ws_own_failed = false;
     g_ctx.retired.clear();
     g_ctx.ws_event = nullptr;
     g_ctx.ws_event_recorded = false;
@@ -2205,14 +2198,18 @@ QGEMM_EXPORT int qgemm_reserve_workspace(size_t bytes) {
     int st = ensure_init_locked();
     if (st != QGEMM_OK) return st;
     // (takes no stream, so it cannot tell whether one is being captured: the caller reserves before a capture)
-    return grow_block(largest_block(), bytes, 0);
+    if (grow_block(g_ctx.ws, bytes, 0) != QGEMM_OK) return QGEMM_ERR_ALLOC;
+    // calls that need no more than this allocate nothing from here on, on any stream
+    for (WsBlock &b : g_ctx.ws_own)
+        if (!b.p && !g_ctx.ws_own_failed) g_ctx.ws_own_failed = grow_block(b, kOwnBytes, 0) != QGEMM_OK;
+    return QGEMM_OK;
 }
 
 QGEMM_EXPORT int qgemm_workspace_info(void **base, size_t *bytes) {
     if (!base || !bytes) return QGEMM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lock(g_ctx.mu);
-    *base = largest_block().p;
-    *bytes = largest_block().bytes;
+    *base = g_ctx.ws.p;
+    *bytes = g_ctx.ws.bytes;
     return QGEMM_OK;
 }
 

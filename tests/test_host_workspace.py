@@ -26,3 +26,65 @@ runtime.host_budget(0)                                          # without memory
 lib.qgemm_shutdown()
 assert quantize(500, 1000) == 0 and quantize(500, 1000, stream=64) == 5
 """)
+
+
+def test_a_reservation_serves_every_stream(host):
+    """No call that needs no more than was reserved allocates, on whichever stream, also above what a stream has for itself."""
+    host("""
+need = 4 * 4096 * 4096 * 4                                      # planes of four K slices: 256 MiB
+assert lib.qgemm_reserve_workspace(need) == 0
+events()
+for stream in (0, 64, 128, 192, 256, 2):                        # (2: hipStreamPerThread)
+    for M, split in ((4096, 4), (192, 4), (4096, 2)):
+        assert product(M, 4096, 2048, stream=stream, split=split) == 0 and "splitk%d" % split in config()
+assert not any(e.startswith(("malloc", "synchronize")) for e in events())
+lib.qgemm_shutdown()
+runtime.host_budget(need)                                       # room for the reservation and nothing else
+assert lib.qgemm_reserve_workspace(need) == 0
+events()
+for stream in (0, 64, 128, 192, 256, 2):
+    assert product(4096, 4096, 2048, stream=stream, split=4) == 0 and product(192, 4096, 2048, stream=stream, split=4) == 0
+assert not any(e.startswith(("malloc", "synchronize")) for e in events())
+""")
+
+
+def test_whose_block(host):
+    """Three streams have a block each and no events; further streams, hipStreamPerThread and calls beyond 128 MiB share one and wait for
+    one another; captured calls touch no event."""
+    host("""
+def block(stream, M=192, split=4):
+    assert product(M, 4096, 2048, stream=stream, split=split) == 0
+    log = events()
+    return [re.search("first (0x[0-9a-f]+)", e).group(1) for e in log if "splitk_reduce" in e][0], [e.split()[0] for e in log if e[:4] in ("wait", "reco")]
+own = [block(s) for s in (0, 64, 128)]
+shared = block(192)
+assert len({b for b, _ in own} | {shared[0]}) == 4 and all(not e for _, e in own) and shared[1] == ["record"]
+assert block(192) == (shared[0], ["record"]) and block(256) == (shared[0], ["wait", "record"])
+assert block(2) == block(2) == (shared[0], ["wait", "record"])
+assert [block(s) for s in (0, 64, 128)] == own
+large = block(64, 4096)                                         # (the shared block grows)
+assert large[1] == ["wait", "record"] and large[0] not in {b for b, _ in own} | {shared[0]}
+assert block(192) == (large[0], ["wait", "record"])
+runtime.host_capture(64, 1)
+assert block(64) == (large[0], []) and block(64, 4096) == (large[0], [])
+runtime.host_capture(64, 0)
+assert block(64) == own[1]
+""")
+
+
+def test_without_memory_for_another_block(host):
+    """A stream for which there is no block left uses the shared one, which is as large as any call has needed: nothing is waited for on
+    the host, and no other stream's block is touched."""
+    host("""
+runtime.host_budget((64 + 128) << 20)
+def call(stream, M=192):
+    return product(M, 4096, 2048, stream=stream, split=4), [e.split()[0] for e in events() if not e.startswith("launch")]
+assert call(0) == (0, ["malloc", "malloc"])
+assert call(64) == (0, ["malloc", "record"])
+assert call(64) == (0, ["record"]) and call(128) == (0, ["wait", "record"]) and call(0) == (0, [])
+assert call(64, 4096) == (5, ["malloc"]) and call(0, 4096) == (5, ["malloc"])       # (more than the shared block, and none to be had)
+assert call(64) == (0, ["wait", "record"])
+lib.qgemm_shutdown()
+runtime.host_budget(1 << 40)
+assert call(64) == (0, ["synchronize", "malloc", "malloc"]) and call(64) == (0, [])
+""")
