@@ -190,7 +190,7 @@ int qgemm_quantize_grid(int in_dtype, size_t rows, size_t cols, uint32_t *rows_p
  *   empty last round of 256 x 256 tiles as a second launch where the estimate gains; 2 / 3: rows / columns wherever
  *   possible), "small_tiles" (0: 17 .. 256 rows against few columns keep a tall tile with a K split instead of several
  *   row tiles of the skinny-M kernel; row_estimate counts as 0 then), "quant_wait" (microseconds for which the workgroups of a per-matrix
- *   quantisation in one launch wait for one another before each reads the whole matrix, 2000; -1: two passes instead), "row_estimate" (0: up to 400 rows follow the general
+ *   quantisation in one launch wait for one another before each reads the whole matrix; -2: 20 and 1 for each 100 KB; -1: two passes instead), "row_estimate" (0: up to 400 rows follow the general
  *   rules instead of the estimate of every row that serves them below 32 K steps and, block scales, up to 128 rows), "few_rows"
  *   (operands that option "any_shape" decides about, 1 .. 128 rows: 0 / 2: never / wherever it can the kernel for few rows
  *   instead of the tiles of the any-shape kernel; 1: by an estimate), "c_plain" (0 / 1: non-temporal / ordinary stores for C; -1: the library's

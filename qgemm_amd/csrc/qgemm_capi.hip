@@ -68,7 +68,13 @@ struct Context {
     bool ws_event_recorded = false;
     bool ws_shared_by_call = false;            // the running entry asked for the shared block
     uint32_t quant_launches = 0;               // of quant_whole_matrix_kernel, which number them
-    long quant_wait = 2000;     // microseconds its workgroups wait for one another; -1: per-matrix scales in two passes
+    long quant_wait = -2;       // microseconds its workgroups wait for one another; -1: per-matrix scales in two passes; -2: quant_wait_of
+    struct QuantStream {
+        hipStream_t stream;
+        uint64_t last;                         // number of its last call
+        bool whole_chip;                       // its kernels may run on every CU
+    } quant_streams[2] = {};                   // see may_exchange_maxima
+    uint64_t quant_calls = 0;
     bool static_call = false;                  // the running entry takes its workspace from the static scratch
     void *static_ptr[kMaxDevices] = {};        // device address of `scratch`, per device
     std::string force_config;   // name of a row of the variant tables, empty = heuristic (qgemm_force_config)
@@ -1642,6 +1648,35 @@ RowBlockGrid row_block_grid(uint32_t rows, uint32_t per_row, uint32_t per_group)
     return g;
 }
 
+// May a per-matrix quantisation on this stream be one launch whose workgroups wait for one another (quant_whole_matrix_kernel)?  Two such
+// launches have room on the chip side by side (two workgroups of 1024 threads and at most 64 registers a CU): kernels that wait for nobody
+// then only delay them.  Three could each hold a part of it and wait for the rest until the wait ends.  So two streams may, those whose last
+// such call lies fewer than 64 back; calls on others, on hipStreamPerThread and on streams that are kept to some of the CUs make two passes.
+bool may_exchange_maxima(hipStream_t stream) {
+    if (stream == hipStreamPerThread) return false;
+    const uint64_t now = ++g_ctx.quant_calls;
+    Context::QuantStream *oldest = &g_ctx.quant_streams[0];
+    for (Context::QuantStream &q : g_ctx.quant_streams) {
+        if (q.last && q.stream == stream) {
+            q.last = now;
+            return q.whole_chip;
+        }
+        if (q.last < oldest->last) oldest = &q;
+    }
+    if (oldest->last && now - oldest->last < 64) return false;
+    uint32_t mask[64] = {}, bits = 0;
+    const bool known = hipExtStreamGetCUMask(stream, 64, mask) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    for (uint32_t w : mask) bits += __builtin_popcount(w);
+    *oldest = {stream, now, !known || bits >= (uint32_t)g_ctx.num_cus};
+    return oldest->whole_chip;
+}
+// How long its workgroups wait, us: what the exchange may take beside other work, and as long as reading `bytes` again takes a workgroup
+// (some 100 GB/s), so that a wait in vain costs about twice what not waiting would have
+uint32_t quant_wait_of(uint64_t bytes) {
+    return g_ctx.quant_wait >= 0 ? (uint32_t)g_ctx.quant_wait : 20 + (uint32_t)(bytes / 100000);
+}
+
 template <int IN_DT, int OUT_DT>
 int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
     typedef Piece<IN_DT> P;
@@ -1675,7 +1710,7 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(1024, turns));
         const size_t room = (size_t)nblk * slices * sizeof(uint32_t);
         const uint64_t most = (uint64_t)std::min(g_ctx.num_cus, kQuantGroups) * 1024;        // lanes of a launch that fits the chip
-        if (g_ctx.quant_wait >= 0 && one_row && pieces <= most * kQuantMostPieces && (uintptr_t)a.x % 4 == 0 && !capturing) {
+        if (g_ctx.quant_wait != -1 && one_row && pieces <= most * kQuantMostPieces && (uintptr_t)a.x % 4 == 0 && !capturing && may_exchange_maxima(stream)) {
             const uint32_t whole = a.cols / P::VEC, each = (uint32_t)((whole + most - 1) / most);
             const uint32_t groups = std::max<uint32_t>(1, std::min<uint32_t>((uint32_t)(most / 1024), (whole + 1023) / 1024));
             a.share = (whole + groups - 1) / groups;
@@ -1684,7 +1719,7 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
             if (++g_ctx.quant_launches == 0) g_ctx.quant_launches = 1;
             a.tag = g_ctx.quant_launches;
             a.set = a.tag % kQuantSets;
-            a.wait = (uint32_t)g_ctx.quant_wait * 100;
+            a.wait = quant_wait_of(pieces * 16) * 100;
             e = launch_kernel(each <= 1 ? quant_whole_matrix_kernel<IN_DT, OUT_DT, 1> : each <= 2 ? quant_whole_matrix_kernel<IN_DT, OUT_DT, 2> :
                               each <= 4 ? quant_whole_matrix_kernel<IN_DT, OUT_DT, 4> : quant_whole_matrix_kernel<IN_DT, OUT_DT, kQuantMostPieces>,
                               dim3(groups), dim3(1024), 0, stream, a);
@@ -1811,7 +1846,7 @@ QGEMM_EXPORT int qgemm_set_option(const char *key, long value) {
     else if (!std::strcmp(key, "as_groups")) g_ctx.as_groups = value;
     else if (!std::strcmp(key, "small_tiles")) g_ctx.small_tiles = value;
     else if (!std::strcmp(key, "few_rows")) g_ctx.few_rows = value;
-    else if (!std::strcmp(key, "quant_wait")) g_ctx.quant_wait = std::max(-1L, std::min(value, 1000000L));
+    else if (!std::strcmp(key, "quant_wait")) g_ctx.quant_wait = std::max(-2L, std::min(value, 1000000L));
     else if (!std::strcmp(key, "row_estimate")) g_ctx.row_estimate = value;
 #if QGEMM_DEBUG_BUILD
     else if (!std::strcmp(key, "dbg_ptr")) g_ctx.dbg_ptr = value;

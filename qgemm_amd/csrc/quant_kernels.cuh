@@ -436,7 +436,8 @@ __global__ void __launch_bounds__(1024) quant_small_matrix_kernel(const QuantArg
 // A workgroup writes its maximum and the launch's number as one 64-bit word, with the device's scope, and reads everybody's words
 // until they carry that number: nothing has to be reset, ordered or fenced (a fence of that scope writes back the L2: 27 us), and a
 // word is either this launch's or it is not.  kQuantSets launches have words of their own; should two that far apart run at the same time,
-// or should workgroups not all find room beside another stream's kernel, the wait ends after QuantArgs::wait and the workgroup takes the
+// or should workgroups not all find room beside another program's kernels (beside this library's they do: may_exchange_maxima), the wait ends
+// after QuantArgs::wait and the workgroup takes the
 // maximum of the whole matrix itself: slow, and the same result.  A replayed graph would bring the same number again: captured calls take the two passes below.
 constexpr int kQuantSets = 64, kQuantGroups = 256, kQuantMostPieces = 8;
 static __device__ uint64_t quant_words[kQuantSets][kQuantGroups];

@@ -1,6 +1,8 @@
 """Per-matrix quantisation in one launch, whose workgroups exchange their maxima: at the sizes where a lane holds one piece more
 and where the launch gives way to others, against the CPU oracle bit for bit; also where the workgroups do not wait for one
 another (each then takes the maximum of the whole matrix), and on several streams at once."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -18,7 +20,7 @@ LANES = 256 * 1024
 @pytest.fixture(autouse=True)
 def _reset_options():
     yield
-    Q.set_option("quant_wait", 2000)
+    Q.set_option("quant_wait", -2)
 
 
 def _check(x, xf):
@@ -125,4 +127,35 @@ def test_several_streams():
     torch.cuda.synchronize()
     for x, q, s, _, got in jobs:
         for g, gs in got:
+            assert gs.cpu().numpy()[0] == s and np.array_equal(g.cpu().numpy(), q)
+
+
+def test_launches_do_not_crowd_one_another_out():
+    """Quantisations that take the whole chip each, on four streams, beside products on a fifth: with a wait of a quarter of a second
+    a single launch that waited in vain would take longer than all of them together."""
+    say("quantize whole, four streams, whole chip")
+    n, rounds = 2048, 40
+    xs = [torch.from_numpy(R.fill_normal((n, 4096), 90 + i)).bfloat16().cuda() for i in range(4)]
+    want = [R.quantize_int8(x.float().cpu().numpy()) for x in xs]
+    w = torch.zeros(4096, 4096, dtype=torch.int8, device="cuda")
+    c, one = torch.empty(4096, 4096, dtype=torch.int32, device="cuda"), torch.ones(1, device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(5)]
+    Q.set_option("quant_wait", 250000)
+    for x, stream in zip(xs, streams):                      # (first launches of every kernel, and the workspace)
+        with torch.cuda.stream(stream):
+            Q.quantize(x, torch.int8, Q.QUANT_PER_MATRIX)
+    Q.int8_mm(w, w, one, one, c)
+    torch.cuda.synchronize()
+    start = time.perf_counter()
+    got = [[] for _ in xs]
+    for _ in range(rounds):
+        with torch.cuda.stream(streams[4]):
+            Q.int8_mm(w, w, one, one, c)
+        for i, x in enumerate(xs):
+            with torch.cuda.stream(streams[i]):
+                got[i].append(Q.quantize(x, torch.int8, Q.QUANT_PER_MATRIX))
+    torch.cuda.synchronize()
+    assert time.perf_counter() - start < 0.25
+    for (q, s), results in zip(want, got):
+        for g, gs in results:
             assert gs.cpu().numpy()[0] == s and np.array_equal(g.cpu().numpy(), q)

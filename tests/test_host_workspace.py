@@ -88,3 +88,28 @@ lib.qgemm_shutdown()
 runtime.host_budget(1 << 40)
 assert call(64) == (0, ["synchronize", "malloc", "malloc"]) and call(64) == (0, [])
 """)
+
+
+def test_two_streams_exchange_maxima_at_a_time(host):
+    """Quantisations whose workgroups wait for one another need room for all of them: two streams launch such kernels, others make two
+    passes, until one of the two has not been seen for a while."""
+    host("""
+WHOLE, PASSES = ["quant_whole_matrix_kernel"], ["quant_amax_kernel", "quant_matrix_kernel"]
+def way(stream, rows=2048):
+    assert quantize(rows, 4096, stream=stream) == 0
+    return kernels()
+for _ in range(100):
+    assert way(0) == way(64) == WHOLE and way(128) == way(192) == way(2) == PASSES
+for _ in range(59):
+    assert way(64) == WHOLE
+assert way(128) == PASSES                                       # the 63rd call since stream 0's
+assert way(128) == WHOLE and way(0) == PASSES and way(64) == WHOLE
+assert way(0, 16) == way(128, 16) == ["quant_small_matrix_kernel"]
+""")
+    host("""
+runtime.host_masked_cus(255)
+assert quantize(2048, 4096) == 0 and kernels() == ["quant_amax_kernel", "quant_matrix_kernel"]
+assert quantize(2048, 4096) == 0 and kernels() == ["quant_amax_kernel", "quant_matrix_kernel"]
+runtime.host_masked_cus(0)
+assert quantize(2048, 4096, stream=64) == 0 and kernels() == ["quant_whole_matrix_kernel"]
+""")
