@@ -98,7 +98,8 @@ int qgemm_gemm(int in_dtype, int out_dtype, int layout_b, const void *A, size_t 
  *                          reference only has for fp8)
  *   layout     see qgemm_layout_t;  C is row-major with leading dimension ldC
  *   split_k    0 = choose, 1 = never split, n > 1 = split K into n slices (deterministic
- *              two-pass reduction through the library workspace)
+ *              two-pass reduction through the library workspace; the any-shape kernel does not split, nor do captured calls and
+ *              qgemm_scaled_gemm_static on operands that option "any_shape" is about)
  * QGEMM_LAYOUT_REFERENCE enforces the reference's dispatch contract and
  * returns QGEMM_ERR_NOT_DIVISIBLE_{M,N,K} where the reference throws. */
 int qgemm_scaled_gemm(int in_dtype, int out_dtype, int scale_mode, int layout, const void *A, const void *B,

@@ -304,6 +304,7 @@ struct NtProblem {
     const float *as, *bs;
     uint32_t as_ms, as_ks, bs_ns, bs_ks;
     int out_dtype, per_matrix, split_k;
+    bool no_planes;                     // never a K split (a second launch for rows or columns all the same)
     RowCopies copies;
 };
 
@@ -958,9 +959,9 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     const Variant *tab = table_for(q.arith, q.block, q.kmaj, &count);
     if (!tab) return QGEMM_ERR_UNSUPPORTED;
     uint32_t model_split = 0;
-    int vi = choose_variant(tab, count, q.M, q.N, ksteps_of(q), q.block, q.kmaj, g_ctx.num_cus, q.split_k == 0, may_split_rows, q.out_dtype,
+    int vi = choose_variant(tab, count, q.M, q.N, ksteps_of(q), q.block, q.kmaj, g_ctx.num_cus, q.split_k == 0 && !q.no_planes, may_split_rows, q.out_dtype,
                             &model_split, copies_of(q));
-    if (may_split_rows && vi >= 0 && !forced() && g_ctx.force_split <= 0 && q.split_k == 0 && model_split <= 1 &&
+    if (may_split_rows && vi >= 0 && !forced() && (g_ctx.force_split <= 0 || q.no_planes) && q.split_k == 0 && model_split <= 1 &&
         q.M > 128 && q.kmaj == 0) {
         uint32_t ns = 0;
         double t_single = 0;
@@ -1051,7 +1052,8 @@ int plan_nt(const NtProblem &q, Plan &pl, bool may_split_rows = true) {
     if (pl.tiles * 64 >= ((size_t)1 << 31)) return QGEMM_ERR_TOO_LARGE;
 
     uint32_t nsplit = 1;
-    if (q.split_k > 1) nsplit = (uint32_t)q.split_k;
+    if (q.no_planes) nsplit = 1;
+    else if (q.split_k > 1) nsplit = (uint32_t)q.split_k;
     else if (q.split_k == 0) {
         if (g_ctx.force_split > 0) nsplit = (uint32_t)g_ctx.force_split;
         else if (model_split > 0) nsplit = model_split;
@@ -1338,7 +1340,8 @@ double rows_estimate(const NtProblem &q, size_t few) {
     double t = 0;
     const size_t steps = ksteps_of(q), cus = g_ctx.num_cus;
     if (!tab) return -1;
-    const int vi = choose_by_cost(tab, count, q.M, q.N, steps, q.block, (int)cus, q.split_k == 0, &nsplit, &t, copies_of(q));
+    // (slices that the caller asks for are priced as those that the estimate would take)
+    const int vi = choose_by_cost(tab, count, q.M, q.N, steps, q.block, (int)cus, q.split_k != 1 && !q.no_planes, &nsplit, &t, copies_of(q));
     if (vi < 0) return -1;
     if (q.kmaj) return tab[vi].copy_waves ? t : 1.15 * t;
     if (q.M <= few) {
@@ -1361,6 +1364,7 @@ double packed_estimate(NtProblem q, size_t kbytes) {
     q.Kbytes = kbytes;
     q.kmaj = 0;
     q.copies = {};
+    q.no_planes = false;
     const bool shows = output_shows_sums(q.arith, q.block, q.out_dtype);
     const double t = rows_estimate(q, shows || q.arith != AR_F8W ? 256 : 64);
     return t < 0 ? 1e30 : (shows ? 12.0 : 6.3) + 0.2e-6 * (double)(q.M + q.N) * kbytes + (shows ? 1.0 : 1.05) * t;
@@ -1482,7 +1486,7 @@ int launch_packed(NtProblem q, int in_dtype, const SourceOperand &a_src, const S
 // 39.0 / 80.6, int8 1531 x 4100 x 3004 38.7 / 36.9 / 52.4, fp8 block 3942 x 4992 x 2901 135 / 122 / 187.
 bool unaligned_pays(NtProblem &q, int in_dtype, size_t K, bool may_pack) {
     const double few = q.kmaj ? 1e30 : few_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K);
-    if (few < 1e30) q.split_k = 1;               // (that kernel needs no second launch)
+    if (few < 1e30 && q.split_k == 0 && g_ctx.force_split <= 0) q.no_planes = true;       // (that kernel needs no second launch)
     constexpr double least = 4.3;                // (what a call takes the host)
     const double as_any = q.kmaj ? 1e30 : std::min(few, any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K));
     if (as_any <= least) return false;
@@ -1497,7 +1501,7 @@ bool unaligned_pays(NtProblem &q, int in_dtype, size_t K, bool may_pack) {
     return !may_pack || t < packed_estimate(q, K * dtype_bytes(in_dtype));
 }
 // *taken as for launch_packed.
-//   * Captured calls and calls on the static scratch run without a K split, and so without workspace.
+//   * Captured calls and calls on the static scratch run without a K split, also where the caller asks for one, and so without workspace.
 //   * fp32 output that shows how sums are made (output_shows_sums): 16-bit operands, where the packed rows would run, in as many parts; not
 //     with block scales, whose last block is folded in two parts here.
 int launch_unaligned(NtProblem q, int in_dtype, const SourceOperand &a_src, const SourceOperand &b_src, size_t K, hipStream_t stream,
@@ -1518,7 +1522,12 @@ int launch_unaligned(NtProblem q, int in_dtype, const SourceOperand &a_src, cons
     q.ldb_bytes = b_src.ld;
     q.kmaj = b_src.k_major ? 2 : 0;
     q.copies = {row_copy(q.A, q.lda_bytes), q.kmaj ? 0 : row_copy(q.B, q.ldb_bytes)};
-    if (!may_pack) q.split_k = 1;
+    if (!may_pack) {
+        q.no_planes = true;
+        q.split_k = std::min(q.split_k, 1);         // (1: nor a second launch)
+    }
+    // (K one element or more past whole steps, and as many slices asked for as there are steps with that one: packed rows have it)
+    if (choose && q.split_k > 1 && ksteps_of(q) < std::min<size_t>(q.split_k, (K * eb + 127) / 128)) return QGEMM_OK;
     if (!mfma_sizes_ok(q) || (choose && !unaligned_pays(q, in_dtype, K, may_pack))) return QGEMM_OK;
     Plan pl;
     if (plan_nt(q, pl) != QGEMM_OK || !settle_scale_layout(q, pl)) return QGEMM_OK;

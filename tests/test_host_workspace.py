@@ -113,3 +113,42 @@ assert quantize(2048, 4096) == 0 and kernels() == ["quant_amax_kernel", "quant_m
 runtime.host_masked_cus(0)
 assert quantize(2048, 4096, stream=64) == 0 and kernels() == ["quant_whole_matrix_kernel"]
 """)
+
+
+def test_slices_that_the_caller_asks_for(host):
+    """Rows that start or end anywhere, split_k = n: n slices wherever another kernel than the any-shape one runs, none while captured or
+    on the static scratch, which launch nothing but the product."""
+    host("""
+import random
+rng = random.Random(3)
+ran = {"unaligned": 0, "pack": 0}
+for i in range(1500):
+    dt, mode, slices = rng.choice([I8, F8]), rng.choice([1, 2]), rng.choice([2, 3, 4])
+    shape = [int(2 ** rng.uniform(0, 12)), int(2 ** rng.uniform(6, 13)), int(2 ** rng.uniform(7.1, 13))]
+    a, b = (1 << 32) + rng.choice([0, 1, 4, 8]), (1 << 33) + rng.choice([0, 2, 16])
+    call = dict(dt=dt, mode=mode, out=rng.choice([F32, BF16]), split=slices, a=a, b=b)
+    assert product(*shape, **call) == 0
+    way = config()
+    if not way.startswith(("unaligned+", "pack+")):
+        continue
+    ran[way.split("+")[0]] += 1
+    steps = (shape[2] + 127) // 128
+    each = -(-steps // min(slices, steps))
+    got = int(way.split("_splitk")[1]) if "_splitk" in way else 1
+    assert got in (-(-steps // each), -(-(steps - 1) // -(-(steps - 1) // min(slices, steps - 1 or 1)))), (shape, call, way)
+    events()
+    runtime.host_capture(0, 1)
+    assert product(*shape, **call) == 0 and "_splitk" not in config() and not config().startswith("pack+"), config()
+    runtime.host_capture(0, 0)
+    assert all(e.startswith("launch") for e in events())
+    assert product(*shape, static=True, **call) == 0 and "_splitk" not in config() and not config().startswith("pack+"), config()
+assert min(ran.values()) > 30, ran
+option("force_split", 3)
+found = 0
+for i in range(300):
+    assert product(rng.randrange(17, 129), rng.randrange(512, 8192), rng.randrange(1000, 8000), dt=I8, out=BF16) == 0
+    if config().startswith("unaligned+"):
+        found += 1
+        assert config().endswith("_splitk3"), config()
+assert found > 10
+""")
