@@ -362,10 +362,11 @@ bool mfma_shape_ok(const NtProblem &q) { return q.lda_bytes % 16 == 0 && q.ldb_b
 // The K-major families have 64 x 64 with two K groups too, two workgroups a CU: mid-sized products make few tiles, and a CU's work on one is
 // latency (start, first copies, a step of 0.18 us, the way out).  Graph replays, us, the best other row / so: B stored K x N bf16 505 x 1056 x
 // 531 8.7 / 6.6, 512 x 512 x 2048 11.7 / 9.2, 384 x 1280 x 1184 8.2 / 7.0, 64 x 2816 x 560 6.1 / 5.1; fp8_mm 160 x 3168 x 448 5.7 / 4.6, 1024 x
-// 544 x 2080 9.7 / 7.7, 512 x 1984 x 1792 9.0 / 7.4.  136 shapes of 32 .. 1280 rows: 7 - 24 % ahead wherever there are no more tiles than
-// CUs; with more, two share a CU and most shapes are behind (fp8_mm 640 x 2432 x 3136, 380 tiles, 13.6 / 18.3).  In the K-contiguous
-// families, whose other rows need no transposing reads, it is level or behind, but for what choose_by_rules gives it.  From 1024 x 1024 on it is left out: more tiles than CUs,
-// but for that square itself, whose plan is pinned by name (x 1024 bf16 7.8 / 6.9).
+// 544 x 2080 9.7 / 7.7, 512 x 1984 x 1792 9.0 / 7.4, 1024 x 1024 x 1024 6.8 / 5.5, bf16 7.7 / 6.6.  136 shapes of 32 .. 1280 rows: 7 - 24 % ahead
+// wherever there are no more tiles than CUs.  With more, two share a CU: up to five K steps level with the best other row and ahead of
+// what the estimates would take instead (fp8_mm 352 x 2848 x 352 5.8 / 5.0); beyond, with block scales, level to 60 % behind (224 shapes; 1280 x 1280 x
+// 1024 7.2 / 8.1, 608 x 3232 x 3008 16.8 / 21.0), where the estimate is up to 29 % low; 16-bit types are behind by as much, and the estimate knows it.
+// In the K-contiguous families, whose other rows need no transposing reads, it is level or behind, but for what choose_by_rules gives it.
 //
 // M <= 64 (bandwidth-bound, B is streamed once): the largest tile that still gives three quarters of the CUs a
 // workgroup, else the shortest tile that covers the rows; narrow tiles instead of a K split.  (65 .. 128 rows go
@@ -426,8 +427,8 @@ int choose_by_cost(const Variant *tab, int count, size_t M, size_t N, size_t kst
         int vi = -1;
         for (int i = 0; i < count; ++i)
             if (tab[i].auto_ok && tab[i].bm == tm.bm && tab[i].bn == tm.bn && is_kgroup_row(tab[i]) == tm.kgroups) vi = i;
-        if (vi < 0 || (tm.bm == 64 && tm.bn == 64 && (!copies.tile64 || (M >= 1024 && N >= 1024)))) continue;
         const size_t tiles = ((M + tm.bm - 1) / tm.bm) * ((N + tm.bn - 1) / tm.bn);
+        if (vi < 0 || (tm.bm == 64 && tm.bn == 64 && (!copies.tile64 || (block && tiles > (size_t)cus && ksteps > 5)))) continue;
         for (uint32_t ns = 1; ns <= 8; ns *= 2) {
             if (ns > 1 && (!may_split || ksteps / ns < 4)) break;
             const size_t wgs = tiles * ns, slots = (size_t)cus * (block ? tm.blk_per_cu : tm.per_cu), steps = (ksteps + ns - 1) / ns;

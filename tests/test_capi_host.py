@@ -201,7 +201,10 @@ def test_plan_names_the_kernel_without_a_device():
     assert plan(Q.DT_F8E4M3, Q.SCALE_BLOCK128, 3, 2048, 2048, 2048) == "128x128_w2x2_k2_tn"
     assert plan(Q.DT_F8E4M3, Q.SCALE_BLOCK128, 3, 4096, 2048, 2048) == "256x128_w2x2_cw_tn"
     assert plan(Q.DT_F8E4M3, Q.SCALE_BLOCK128, 3, 6144, 4608, 7168) == "transpose+256x256_w2x4_solo8|192x256_w2x4_solo8"
-    assert plan(Q.DT_BF16, 0, 2, 1024, 1024, 1024) == "64x128_w1x4_k2_nn"
+    assert plan(Q.DT_BF16, 0, 2, 1024, 1024, 1024) == "64x64_w2x2_k2_nn"                    # (64 x 128: 7.7 us against 6.6)
+    assert plan(Q.DT_BF16, 0, 2, 1024, 1088, 1024) == "64x128_w1x4_k2_nn"                   # more tiles of 64 x 64 than CUs
+    assert plan(Q.DT_F8E4M3, Q.SCALE_BLOCK128, 3, 1024, 1024, 1024) == "64x64_w2x2_k2_tn"
+    assert plan(Q.DT_F8E4M3, Q.SCALE_BLOCK128, 3, 608, 3232, 3008) == "128x128_w2x2_k2_tn"
     assert plan(Q.DT_BF16, 0, 2, 8192, 8192, 8192) == "transpose+256x256_w2x2_solo"
     # large shapes whose transposes are a sizeable part: as stored, on the K-major 256 x 128 row with copying waves
     assert plan(Q.DT_F8E4M3, Q.SCALE_BLOCK128, 3, 4096, 4096, 4096) == "256x128_w2x2_cw_tn"
