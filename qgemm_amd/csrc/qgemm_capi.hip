@@ -427,8 +427,9 @@ int choose_by_cost(const Variant *tab, int count, size_t M, size_t N, size_t kst
         int vi = -1;
         for (int i = 0; i < count; ++i)
             if (tab[i].auto_ok && tab[i].bm == tm.bm && tab[i].bn == tm.bn && is_kgroup_row(tab[i]) == tm.kgroups) vi = i;
+        if (vi < 0) continue;
         const size_t tiles = ((M + tm.bm - 1) / tm.bm) * ((N + tm.bn - 1) / tm.bn);
-        if (vi < 0 || (tm.bm == 64 && tm.bn == 64 && (!copies.tile64 || (block && tiles > (size_t)cus && ksteps > 5)))) continue;
+        if (tm.bm == 64 && tm.bn == 64 && (!copies.tile64 || (block && tiles > (size_t)cus && ksteps > 5))) continue;
         for (uint32_t ns = 1; ns <= 8; ns *= 2) {
             if (ns > 1 && (!may_split || ksteps / ns < 4)) break;
             const size_t wgs = tiles * ns, slots = (size_t)cus * (block ? tm.blk_per_cu : tm.per_cu), steps = (ksteps + ns - 1) / ns;
@@ -1358,24 +1359,43 @@ double rows_estimate(const NtProblem &q, size_t few) {
     }
     return t;
 }
+// What rows_estimate is never below: the start and the steps of the row that is fastest by itself, in eight slices where that is allowed.
+// It spares products of few rows, whose calls the host bounds, two or three estimates of all rows (int8 block scales 5 x 1024 x 1213, one
+// scale 1 x 2048 x 1037: 2.9 and 2.8 -> 2.2 us of host time a call).
+double least_rows_estimate(const NtProblem &q) {
+    const size_t steps = ksteps_of(q), eighth = (steps + 7) / 8;
+    const bool wide = q.arith == AR_F8W, split = q.split_k != 1 && !q.no_planes;
+    const TileModel *models = wide ? kWideTileModels : kTileModels;
+    double t = wide || q.M <= 256 ? std::max(4.0, 0.12 * steps) : 1e30;             // (the skinny-M kernel)
+    for (size_t i = 0; i < (wide ? std::size(kWideTileModels) : std::size(kTileModels)); ++i) {
+        const TileModel &m = models[i];
+        const double step = q.block ? std::min(m.blk_shared, m.blk_alone) : std::min(m.step_shared, m.step_alone);
+        t = std::min(t, m.fixed + steps * step);
+        if (split) t = std::min(t, m.fixed + eighth * step + 4.0);
+    }
+    return t;
+}
 // Packed: another launch that reads and writes both operands, then rows of whole K steps (q: the product; kbytes: its K).  Where an fp32
 // output shows how sums are made, packed rows sum less exactly than the any-shape kernel (bf16 1445 x 640 x 1095 8.5e-8 / 7.8e-8 of the
 // result) and keep the 12 us that a call with workspace once had as its constant part, so that no product comes to them for being faster now.
-double packed_estimate(NtProblem q, size_t kbytes) {
+// (enough: an estimate that is known not to be below this is as good as none)
+double packed_estimate(NtProblem q, size_t kbytes, double enough) {
     q.Kbytes = kbytes;
     q.kmaj = 0;
     q.copies = {};
     q.no_planes = false;
     const bool shows = output_shows_sums(q.arith, q.block, q.out_dtype);
+    const double packing = (shows ? 12.0 : 6.3) + 0.2e-6 * (double)(q.M + q.N) * kbytes, rate = shows ? 1.0 : 1.05;
+    if (packing + rate * least_rows_estimate(q) >= enough) return 1e30;
     const double t = rows_estimate(q, shows || q.arith != AR_F8W ? 256 : 64);
-    return t < 0 ? 1e30 : (shows ? 12.0 : 6.3) + 0.2e-6 * (double)(q.M + q.N) * kbytes + (shows ? 1.0 : 1.05) * t;
+    return t < 0 ? 1e30 : packing + rate * t;
 }
 enum class Packing { NO, YES, UNLESS_FEW_ROWS };        // UNLESS_FEW_ROWS: gemm_few_kernel is faster still
 Packing pack_pays(const NtProblem &q, int in_dtype, size_t K, bool km) {
     const size_t kbytes = K * dtype_bytes(in_dtype);
     if (km) return kbytes > 512 || (double)q.M * q.N >= 4e6 ? Packing::YES : Packing::NO;
-    const double t_packed = packed_estimate(q, kbytes);
-    if (t_packed >= any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K)) return Packing::NO;
+    const double as_any = any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K), t_packed = packed_estimate(q, kbytes, as_any);
+    if (t_packed >= as_any) return Packing::NO;
     return t_packed >= few_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K) ? Packing::UNLESS_FEW_ROWS : Packing::YES;
 }
 
@@ -1491,6 +1511,7 @@ bool unaligned_pays(NtProblem &q, int in_dtype, size_t K, bool may_pack) {
     constexpr double least = 4.3;                // (what a call takes the host)
     const double as_any = q.kmaj ? 1e30 : std::min(few, any_estimate(in_dtype, q.out_dtype, q.block, q.M, q.N, K));
     if (as_any <= least) return false;
+    if (!q.kmaj && least_rows_estimate(q) * 1.25 * (few < 1e30 ? 1.35 : 1.0) >= as_any) return false;
     double t = rows_estimate(q, q.arith == AR_F8W ? 64 : 256);
     if (t < 0) return false;
     t *= 1.25 + (q.arith == AR_F8W ? 0 : 0.2) * (odd_rows(q.A, q.lda_bytes) + (q.kmaj ? 0 : odd_rows(q.B, q.ldb_bytes))) / 2;
@@ -1499,7 +1520,7 @@ bool unaligned_pays(NtProblem &q, int in_dtype, size_t K, bool may_pack) {
     // (against packing the estimate of the widening rows runs low by 1.4, not 1.25: fp8 with block scales 2287 x 6912 x 859 as they stand /
     // packed 52.9 / 45.1 us, 2727 x 3136 x 2283 58.5 / 54.7, one scale 3384 x 6208 x 691 54.2 / 49.0)
     if (q.arith == AR_F8W) t *= 1.12;
-    return !may_pack || t < packed_estimate(q, K * dtype_bytes(in_dtype));
+    return !may_pack || t < packed_estimate(q, K * dtype_bytes(in_dtype), t * (1 + 1e-9));
 }
 // *taken as for launch_packed.
 //   * Captured calls and calls on the static scratch run without a K split, also where the caller asks for one, and so without workspace.
