@@ -67,12 +67,12 @@ struct Context {
     hipStream_t ws_last_stream = nullptr;
     bool ws_event_recorded = false;
     bool ws_shared_by_call = false;            // the running entry asked for the shared block
-    uint32_t quant_launches = 0;               // of quant_whole_matrix_kernel, which number them
     long quant_wait = -2;       // microseconds its workgroups wait for one another; -1: per-matrix scales in two passes; -2: quant_wait_of
     struct QuantStream {
         hipStream_t stream;
         uint64_t last;                         // number of its last call
         bool whole_chip;                       // its kernels may run on every CU
+        uint32_t launches;                     // of quant_whole_matrix_kernel from this place, which number them
     } quant_streams[2] = {};                   // see may_exchange_maxima
     uint64_t quant_calls = 0;
     bool static_call = false;                  // the running entry takes its workspace from the static scratch
@@ -1679,28 +1679,29 @@ RowBlockGrid row_block_grid(uint32_t rows, uint32_t per_row, uint32_t per_group)
     return g;
 }
 
-// May a per-matrix quantisation on this stream be one launch whose workgroups wait for one another (quant_whole_matrix_kernel)?  Two such
+// May a per-matrix quantisation on this stream be one launch whose workgroups wait for one another (quant_whole_matrix_kernel), and which
+// of the places for such streams is its?  Two such
 // launches have room on the chip side by side (two workgroups of 1024 threads and at most 64 registers a CU): kernels that wait for nobody
 // then only delay them.  Three could each hold a part of it and wait for the rest until the wait ends.  So two streams may, those whose last
 // such call lies fewer than 64 back; calls on others, on hipStreamPerThread and on streams that are kept to some of the CUs make two passes.
-bool may_exchange_maxima(hipStream_t stream) {
-    if (stream == hipStreamPerThread) return false;
+Context::QuantStream *may_exchange_maxima(hipStream_t stream) {
+    if (stream == hipStreamPerThread) return nullptr;
     const uint64_t now = ++g_ctx.quant_calls;
     Context::QuantStream *oldest = &g_ctx.quant_streams[0];
     for (Context::QuantStream &q : g_ctx.quant_streams) {
         if (q.last && q.stream == stream) {
             q.last = now;
-            return q.whole_chip;
+            return q.whole_chip ? &q : nullptr;
         }
         if (q.last < oldest->last) oldest = &q;
     }
-    if (oldest->last && now - oldest->last < 64) return false;
+    if (oldest->last && now - oldest->last < 64) return nullptr;
     uint32_t mask[64] = {}, bits = 0;
     const bool known = hipExtStreamGetCUMask(stream, 64, mask) == hipSuccess;
     if (!known) (void)hipGetLastError();
     for (uint32_t w : mask) bits += __builtin_popcount(w);
-    *oldest = {stream, now, !known || bits >= (uint32_t)g_ctx.num_cus};
-    return oldest->whole_chip;
+    *oldest = {stream, now, !known || bits >= (uint32_t)g_ctx.num_cus, oldest->launches};
+    return oldest->whole_chip ? oldest : nullptr;
 }
 // How long its workgroups wait, us: what the exchange may take beside other work, and as long as reading `bytes` again takes a workgroup
 // (some 100 GB/s), so that a wait in vain costs about twice what not waiting would have
@@ -1741,15 +1742,17 @@ int quantize_t(int mode, QuantArgs &a, hipStream_t stream) {
         const uint32_t nblk = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(1024, turns));
         const size_t room = (size_t)nblk * slices * sizeof(uint32_t);
         const uint64_t most = (uint64_t)std::min(g_ctx.num_cus, kQuantGroups) * 1024;        // lanes of a launch that fits the chip
-        if (g_ctx.quant_wait != -1 && one_row && pieces <= most * kQuantMostPieces && (uintptr_t)a.x % 4 == 0 && !capturing && may_exchange_maxima(stream)) {
+        const bool whole_fits = one_row && pieces <= most * kQuantMostPieces && (uintptr_t)a.x % 4 == 0;
+        Context::QuantStream *const place = g_ctx.quant_wait != -1 && whole_fits && !capturing ? may_exchange_maxima(stream) : nullptr;
+        if (place) {
             const uint32_t whole = a.cols / P::VEC, each = (uint32_t)((whole + most - 1) / most);
             const uint32_t groups = std::max<uint32_t>(1, std::min<uint32_t>((uint32_t)(most / 1024), (whole + 1023) / 1024));
             a.share = (whole + groups - 1) / groups;
             // (captured, the same call makes two passes in the room that an eager one has left: one that needs none itself leaves it too)
             (void)grow_block(g_ctx.ws, room, kLeastBlock);
-            if (++g_ctx.quant_launches == 0) g_ctx.quant_launches = 1;
-            a.tag = g_ctx.quant_launches;
-            a.set = a.tag % kQuantSets;
+            if (++place->launches == 0) place->launches = 1;
+            a.tag = place->launches;
+            a.set = (uint32_t)(place - g_ctx.quant_streams) * (kQuantSets / 2) + a.tag % (kQuantSets / 2);
             a.wait = quant_wait_of(pieces * 16) * 100;
             e = launch_kernel(each <= 1 ? quant_whole_matrix_kernel<IN_DT, OUT_DT, 1> : each <= 2 ? quant_whole_matrix_kernel<IN_DT, OUT_DT, 2> :
                               each <= 4 ? quant_whole_matrix_kernel<IN_DT, OUT_DT, 4> : quant_whole_matrix_kernel<IN_DT, OUT_DT, kQuantMostPieces>,

@@ -435,9 +435,9 @@ __global__ void __launch_bounds__(1024) quant_small_matrix_kernel(const QuantArg
 // some 10 MiB, by memory above.
 // A workgroup writes its maximum and the launch's number as one 64-bit word, with the device's scope, and reads everybody's words
 // until they carry that number: nothing has to be reset, ordered or fenced (a fence of that scope writes back the L2: 27 us), and a
-// word is either this launch's or it is not.  kQuantSets launches have words of their own; should two that far apart run at the same time,
-// or should workgroups not all find room beside another program's kernels (beside this library's they do: may_exchange_maxima), the wait ends
-// after QuantArgs::wait and the workgroup takes the
+// word is either this launch's or it is not.  The two streams that launch it at a time (may_exchange_maxima) have half of the sets each, which
+// their launches take in turn; should another stream take a place over before the last one's launches are done, should workgroups not all
+// find room beside another program's kernels, the wait ends after QuantArgs::wait and the workgroup takes the
 // maximum of the whole matrix itself: slow, and the same result.  A replayed graph would bring the same number again: captured calls take the two passes below.
 constexpr int kQuantSets = 64, kQuantGroups = 256, kQuantMostPieces = 8;
 static __device__ uint64_t quant_words[kQuantSets][kQuantGroups];
@@ -454,7 +454,7 @@ __device__ inline bool launch_maximum(uint32_t &m, uint32_t set, uint32_t tag, u
             late = __builtin_amdgcn_s_memrealtime() - start > wait;
             if (late) break;
         }
-    } else if (blockIdx.x == 0 && t < (uint32_t)kQuantGroups) {          // (numbers come round: no old word stays for longer than kQuantSets launches)
+    } else if (blockIdx.x == 0 && t < (uint32_t)kQuantGroups) {          // (numbers come round: no old word stays for longer than a place's sets)
         __hip_atomic_store(words + t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     late = __syncthreads_or(late);
