@@ -488,16 +488,16 @@ gemm_nt_kernel(QGEMM_HEAD, const GemmArgs p) {
     const bool has_tail = k_tail != 0 && kend == ksteps && nk > 0;
     const uint32_t kbytes = has_tail ? (uint32_t)(nk - 1) * C::BKB + k_tail : (uint32_t)nk * C::BKB;
     // K-major operand: rows are k (stride lda / ldb bytes), the tile starts at column row0 / col0; the range ends
-    // with the last column of the last k row of this K slice.  Columns past M / N inside an earlier row read
+    // with the last column of the last k row of this K slice, and as the range check is one of whole dwords, with the dword
+    // that column is in (rows start on 16 bytes).  Columns past M / N inside an earlier row read
     // the neighbouring row instead (valid memory) and, as above, only feed outputs that are not stored.
     const uint32_t krows = nk > 0 ? kbytes / C::ES : 1;
+    auto kmajor_bytes = [&](uint32_t ld, uint32_t columns) { return (krows - 1) * ld + ((columns * C::ES + 3) & ~3u); };
     const __amdgpu_buffer_rsrc_t ra =
-        C::KMA ? make_rsrc(A + (size_t)kbeg * C::KE * lda + (size_t)row0 * C::ES,
-                           (krows - 1) * lda + (M - row0) * C::ES)
+        C::KMA ? make_rsrc(A + (size_t)kbeg * C::KE * lda + (size_t)row0 * C::ES, kmajor_bytes(lda, M - row0))
                : make_rsrc(A + (size_t)row0 * lda + (size_t)kbeg * C::BKB, (a_rows - 1) * lda + kbytes);
     const __amdgpu_buffer_rsrc_t rb =
-        C::KMB ? make_rsrc(B + (size_t)kbeg * C::KE * ldb + (size_t)col0 * C::ES,
-                           (krows - 1) * ldb + (N - col0) * C::ES)
+        C::KMB ? make_rsrc(B + (size_t)kbeg * C::KE * ldb + (size_t)col0 * C::ES, kmajor_bytes(ldb, N - col0))
                : make_rsrc(B + (size_t)col0 * ldb + (size_t)kbeg * C::BKB, (b_rows - 1) * ldb + kbytes);
 
     // ---- the LPT load instructions of this wave.  Instruction q = wave + i*NW (0 .. NLOAD-1) covers

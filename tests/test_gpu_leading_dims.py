@@ -115,3 +115,33 @@ def test_bf16_padded_lda_ldb_ldc(variant, pads):
     assert "strided" not in Q.last_config(), Q.last_config()
     assert np.array_equal(host(c), ref), Q.last_config()
     assert _poison_intact(whole, M, N, -77.0), Q.last_config()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(130, 1001, 256), (300, 513, 200), (64, 2815, 560), (33, 7, 136), (257, 999, 1003)])
+def test_b_stored_k_by_n_with_an_odd_number_of_columns(dtype, M, N, K):
+    """Rows of B on 16 bytes, an odd number of columns in them: the last column of the last k row (of every K slice) shares its dword with
+    what lies behind the operand.  Small integers, exact; NaNs around the operand."""
+    rng = np.random.default_rng(N)
+    a, b = rng.integers(-4, 5, (M, K)).astype(np.float32), rng.integers(1, 5, (K, N)).astype(np.float32)
+    ref = torch.from_numpy(a @ b)
+    flat = torch.full((K * ((N + 8) // 8 * 8) + 8,), float("nan"), dtype=dtype, device="cuda")
+    bt = flat[:-8].view(K, -1)[:, :N]
+    bt.copy_(torch.from_numpy(b))
+    at = torch.from_numpy(a).to(dtype).cuda()
+    Q.set_option("any_shape", 3)
+    try:
+        for row in [None] + Q.variant_names(Q.DT_BF16, 0, 2):
+            for split in (0, 1, 3):
+                say("odd columns", dtype, M, N, K, row, split)
+                Q.set_option("kmajor", 1 if row is None else 2)
+                Q.force_config(row)
+                Q.set_option("force_split", split)
+                c = torch.full((M, N), 7.0, dtype=torch.float32, device="cuda")
+                Q.gemm(at, bt, c, "kn")
+                assert row is None or row + "_nn" in Q.last_config(), Q.last_config()
+                assert torch.equal(c.cpu(), ref), (row, split, Q.last_config())
+    finally:
+        Q.set_option("any_shape", 1)
+        Q.set_option("kmajor", 1)
+        Q.force_config(None)
