@@ -51,7 +51,9 @@ constexpr int kElemBytes = (INST_ARITH == AR_BF16 || INST_ARITH == AR_F16) ? 2 :
 constexpr bool kBlock = (bool)INST_BLOCK;
 // Widened fp8 keeps the rows whose fragments, twice their size once widened, leave the registers of a wave without spills
 // (128 x 128 with two K groups: 164 bytes of scratch a lane, 308 with block scales; 256 x 256 on eight waves 272 and 676;
-// 256 x 128 with copying waves 148 and 1756; 128 rows of the skinny-M kernel 148 with block scales).
+// 256 x 128 with copying waves 148 and 1756; 128 rows of the skinny-M kernel 148 with block scales).  Rows that spill all the
+// same: 64 x 128 with two K groups and block scales 32 bytes, and int8 block scales on 256 x 256 and 256 x 128 116 - 132, 184 where rows end
+// inside a chunk.
 constexpr bool kWide = INST_ARITH == AR_F8W;
 constexpr bool kRest = INST_ARITH != AR_F8;         // (fp8 rows that end inside a chunk run widened)
 // A K-major operand needs whole 128-byte panels of its tile side and a multiple of four waves (GemmCfg's
