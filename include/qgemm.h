@@ -138,8 +138,8 @@ int qgemm_scaled_gemm_static(int in_dtype, int out_dtype, int scale_mode, int la
  * QGEMM_ERR_ALLOC, and replays of graphs that use the workspace must not overlap other users of it.  (Products whose
  * operands would be packed into the block, see option "any_shape", do not use it while captured: their operands are read as
  * they stand, and fp32 sums have another order than those of an eager call.)
- * qgemm_reserve_workspace makes the shared block at least `bytes` large and the three others ahead of time, as far as there is memory for
- * those: calls that need no more than `bytes` then allocate nothing, on any stream (it allocates: call it before a
+ * qgemm_reserve_workspace makes the shared block at least `bytes` large and the three others that large or 128 MiB ahead of time, as far as
+ * there is memory for those: calls that need no more than `bytes` then allocate nothing, on any stream (it allocates: call it before a
  * capture begins, never during one); qgemm_workspace_info reports the shared block's
  * address and size (NULL / 0 before first use). */
 int qgemm_reserve_workspace(size_t bytes);

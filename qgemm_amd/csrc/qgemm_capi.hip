@@ -47,7 +47,7 @@ struct Context {
     int device = -1;
     int num_cus = 256;
     // Workspace (split-K partial planes, transposed and packed operands and scales, quantiser partials): one shared block, which every
-    // eager call makes as large as it needs, and kOwnBlocks blocks of kOwnBytes, one each for the first streams that ask.  In its own
+    // eager call makes as large as it needs, and kOwnBlocks blocks of kOwnBytes (or what was reserved), one each for the first streams that ask.  In its own
     // block a stream's calls follow one another as the stream has them.  The shared block is for calls that need more, for the streams beyond
     // those (and hipStreamPerThread, one handle for many streams), where there is no memory for another block, and for captured
     // calls; its eager users are ordered through ws_event: every call that
@@ -181,17 +181,22 @@ int grow_block(WsBlock &block, size_t bytes, size_t least) {
     return QGEMM_OK;
 }
 
-// The stream's own block, null where it has none
-void *own_block(hipStream_t stream) {
+// An own block of `bytes`, unless it is as large already; false where there is no memory for it
+bool make_own_block(WsBlock &block, size_t bytes) {
+    if (bytes <= block.bytes) return true;
+    WsBlock larger;
+    if (!g_ctx.ws_own_failed) g_ctx.ws_own_failed = grow_block(larger, bytes, 0) != QGEMM_OK;
+    if (g_ctx.ws_own_failed) return false;
+    if (block.p) g_ctx.retired.push_back(block.p);
+    block = larger;
+    return true;
+}
+// The stream's own block for a call that needs `bytes` (kOwnBytes at most), null where it has none
+void *own_block(hipStream_t stream, size_t bytes) {
     if (stream == hipStreamPerThread) return nullptr;
     int i = 0;
     while (i < g_ctx.ws_owners && g_ctx.ws_stream[i] != stream) ++i;
-    if (i == kOwnBlocks) return nullptr;
-    if (!g_ctx.ws_own[i].p) {
-        if (g_ctx.ws_own_failed) return nullptr;
-        g_ctx.ws_own_failed = grow_block(g_ctx.ws_own[i], kOwnBytes, 0) != QGEMM_OK;
-        if (g_ctx.ws_own_failed) return nullptr;
-    }
+    if (i == kOwnBlocks || (bytes > g_ctx.ws_own[i].bytes && !make_own_block(g_ctx.ws_own[i], kOwnBytes))) return nullptr;
     if (i == g_ctx.ws_owners) g_ctx.ws_stream[g_ctx.ws_owners++] = stream;
     return g_ctx.ws_own[i].p;
 }
@@ -212,7 +217,7 @@ int ensure_workspace_locked(size_t bytes, hipStream_t stream, void **out) {
         return bytes > g_ctx.ws.bytes ? QGEMM_ERR_ALLOC : QGEMM_OK;
     }
     const int st = grow_block(g_ctx.ws, bytes, kLeastBlock);
-    *out = bytes <= kOwnBytes ? own_block(stream) : nullptr;
+    *out = bytes <= kOwnBytes ? own_block(stream, bytes) : nullptr;
     if (*out) return QGEMM_OK;
     if (st != QGEMM_OK) return st;
     if (!g_ctx.ws_shared_by_call) {
@@ -2272,8 +2277,7 @@ QGEMM_EXPORT int qgemm_reserve_workspace(size_t bytes) {
     // (takes no stream, so it cannot tell whether one is being captured: the caller reserves before a capture)
     if (grow_block(g_ctx.ws, bytes, 0) != QGEMM_OK) return QGEMM_ERR_ALLOC;
     // calls that need no more than this allocate nothing from here on, on any stream
-    for (WsBlock &b : g_ctx.ws_own)
-        if (!b.p && !g_ctx.ws_own_failed) g_ctx.ws_own_failed = grow_block(b, kOwnBytes, 0) != QGEMM_OK;
+    for (WsBlock &b : g_ctx.ws_own) (void)make_own_block(b, std::min(bytes, kOwnBytes));
     return QGEMM_OK;
 }
 

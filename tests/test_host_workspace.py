@@ -48,6 +48,19 @@ assert not any(e.startswith(("malloc", "synchronize")) for e in events())
 """)
 
 
+def test_a_small_reservation(host):
+    """It takes no more memory than it says, four times; a call that needs more allocates as if nothing had been reserved."""
+    host("""
+assert lib.qgemm_reserve_workspace(0) == 0 and events() == []
+assert lib.qgemm_reserve_workspace(1 << 20) == 0 and events() == ["malloc 1048576"] * 4
+assert product(32, 512, 2048, split=4) == 0 and "splitk4" in config() and all(e.startswith("launch") for e in events())
+assert product(192, 4096, 2048, split=4) == 0
+assert [e for e in events() if not e.startswith("launch")] == ["malloc %d" % (64 << 20), "malloc %d" % (128 << 20)]
+assert lib.qgemm_reserve_workspace(1 << 20) == 0 and events() == []
+assert product(192, 4096, 2048, split=4) == 0 and all(e.startswith("launch") for e in events())
+""")
+
+
 def test_whose_block(host):
     """Three streams have a block each and no events; further streams, hipStreamPerThread and calls beyond 128 MiB share one and wait for
     one another; captured calls touch no event."""
